@@ -29,6 +29,14 @@ struct hg_graph {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   void *tables = nullptr;  // grouped: the views and block tables the launches read
+  // grouped: what its launches were captured with, for capturing them again
+  // when a context's metric no longer has the zeros they leave out
+  std::vector<hg_ctx *> ctxs;
+  std::vector<unsigned> total;
+  const hg_mlp *mlp = nullptr;
+  size_t vpad = 0;
+  int nsteps = 0, ns = 0, mode = 0;
+  bool ucum = false, ks = false;
 };
 
 #define HIPTRY(call)                                                               \
@@ -247,6 +255,67 @@ const char *grouped_unsupported(const hg_ctx *c, const hg_ctx *c0) {
   return nullptr;
 }
 
+bool all_ks(const hg_graph *g) {
+  for (const hg_ctx *c : g->ctxs)
+    if (!c->d.ks) return false;
+  return true;
+}
+
+// the grouped launches of g's steps into a new executable graph
+int capture_grouped(hg_graph *g) {
+  int rc = 0;
+  const int n = (int)g->ctxs.size();
+  const GridView *dv = (const GridView *)g->tables;
+  const unsigned *dfirst = (const unsigned *)((char *)g->tables + g->vpad);
+  const bool ks = all_ks(g);
+  hipStream_t cap = nullptr;
+  HIPTRY(hipStreamCreateWithFlags(&cap, hipStreamNonBlocking));
+  if (!rc) HIPTRY(hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal));
+  if (!rc) {
+    auto L = [&](int k, int sub) {
+      const GridView *vs = dv + (size_t)sub * n;
+      const unsigned *fs = dfirst + (size_t)k * (n + 1);
+      if (k == GK_MLP) launch_group_mlp(g->mlp, vs, fs, n, g->total[k], cap);
+      else launch_group(k, vs, fs, n, g->total[k], g->mode, ks, cap);
+    };
+    // one substep of step_ch.c:94-166 on every grid: fluxcalc (directions in
+    // turn, every direction's dP/P indicator in one launch), update, the
+    // learned start's features and network, inversion, dt on the final
+    // substep, bound_prim, post_fixup, bound_prim
+    const int order[] = {GK_PREP, GK_DPI, GK_WENO1, GK_FLUX1, GK_WENO2, GK_FLUX2, GK_WENO3, GK_FLUX3,
+                         GK_EMF, g->ucum ? GK_UPDATEU : GK_UPDATE, GK_FEATURES, GK_MLP, GK_INVERT, GK_DT, GK_BOUND1,
+                         GK_BOUND2, GK_BOUND3, GK_FXCHECK, GK_FXRESOLVE, GK_FXAVG, GK_FXAPPLY, GK_BOUND1,
+                         GK_BOUND2, GK_BOUND3};
+    for (int step = 0; step < g->nsteps; step++)
+      for (int sub = 0; sub < g->ns; sub++)
+        for (int k : order) {
+          if (k == GK_DT && sub != g->ns - 1) continue;
+          if ((k == GK_FEATURES || k == GK_MLP) && g->mode != 2) continue;
+          L(k, sub);
+        }
+    HIPTRY(hipGetLastError());
+    hipGraph_t graph = nullptr;
+    hipError_t e = hipStreamEndCapture(cap, &graph);
+    if (e != hipSuccess && !rc) {
+      set_error("hg_graph_create_grouped: capture failed: %s", hipGetErrorString(e));
+      rc = 1;
+    }
+    hipGraphExec_t exec = nullptr;
+    if (!rc) HIPTRY(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
+    if (!rc) {
+      if (g->exec) (void)hipGraphExecDestroy(g->exec);
+      if (g->graph) (void)hipGraphDestroy(g->graph);
+      g->graph = graph;
+      g->exec = exec;
+      g->ks = ks;
+    } else if (graph) {
+      (void)hipGraphDestroy(graph);
+    }
+  }
+  if (cap) (void)hipStreamDestroy(cap);
+  return rc;
+}
+
 }  // namespace
 
 extern "C" int hg_graph_create_grouped(hg_ctx *const *ctxs, int n, int nsteps, hg_graph **out) {
@@ -314,46 +383,16 @@ extern "C" int hg_graph_create_grouped(hg_ctx *const *ctxs, int n, int nsteps, h
   if (!rc) HIPTRY(hipMemcpy(g->tables, views.data(), vbytes, hipMemcpyHostToDevice));
   if (!rc) HIPTRY(hipMemcpy((char *)g->tables + vpad, first.data(), first.size() * sizeof(unsigned),
                             hipMemcpyHostToDevice));
-  const GridView *dv = (const GridView *)g->tables;
-  const unsigned *dfirst = (const unsigned *)((char *)g->tables + vpad);
+  g->ctxs.assign(ctxs, ctxs + n);
+  g->total.assign(total, total + GK_NCLASS);
+  g->mlp = ctxs[0]->mlp;
+  g->vpad = vpad;
+  g->nsteps = nsteps;
+  g->ns = ns;
   const int cm = ctxs[0]->c2p_mode;
-  const int mode = cm == HG_C2P_MIXED ? 1 : cm == HG_C2P_LEARNED ? 2 : 0;
-  hipStream_t cap = nullptr;
-  if (!rc) HIPTRY(hipStreamCreateWithFlags(&cap, hipStreamNonBlocking));
-  if (!rc) HIPTRY(hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal));
-  if (!rc) {
-    auto L = [&](int k, int sub) {
-      const GridView *vs = dv + (size_t)sub * n;
-      const unsigned *fs = dfirst + (size_t)k * (n + 1);
-      if (k == GK_MLP) launch_group_mlp(ctxs[0]->mlp, vs, fs, n, total[k], cap);
-      else launch_group(k, vs, fs, n, total[k], mode, cap);
-    };
-    // one substep of step_ch.c:94-166 on every grid: fluxcalc (directions in
-    // turn, every direction's dP/P indicator in one launch), update, the
-    // learned start's features and network, inversion, dt on the final
-    // substep, bound_prim, post_fixup, bound_prim
-    const int order[] = {GK_PREP, GK_DPI, GK_WENO1, GK_FLUX1, GK_WENO2, GK_FLUX2, GK_WENO3, GK_FLUX3,
-                         GK_EMF, ucum ? GK_UPDATEU : GK_UPDATE, GK_FEATURES, GK_MLP, GK_INVERT, GK_DT, GK_BOUND1,
-                         GK_BOUND2, GK_BOUND3, GK_FXCHECK, GK_FXRESOLVE, GK_FXAVG, GK_FXAPPLY, GK_BOUND1,
-                         GK_BOUND2, GK_BOUND3};
-    for (int step = 0; step < nsteps; step++)
-      for (int sub = 0; sub < ns; sub++)
-        for (int k : order) {
-          if (k == GK_DT && sub != ns - 1) continue;
-          if ((k == GK_FEATURES || k == GK_MLP) && mode != 2) continue;
-          L(k, sub);
-        }
-    HIPTRY(hipGetLastError());
-    hipGraph_t graph = nullptr;
-    hipError_t e = hipStreamEndCapture(cap, &graph);
-    if (e != hipSuccess && !rc) {
-      set_error("hg_graph_create_grouped: capture failed: %s", hipGetErrorString(e));
-      rc = 1;
-    }
-    g->graph = graph;
-    if (!rc) HIPTRY(hipGraphInstantiate(&g->exec, g->graph, nullptr, nullptr, 0));
-  }
-  if (cap) (void)hipStreamDestroy(cap);
+  g->mode = cm == HG_C2P_MIXED ? 1 : cm == HG_C2P_LEARNED ? 2 : 0;
+  g->ucum = ucum;
+  if (!rc) rc = capture_grouped(g);
   if (rc) {
     (void)hg_graph_destroy(g);
     return 1;
@@ -373,6 +412,10 @@ extern "C" int hg_graph_launch(hg_graph *g, void *stream) {
   if (!g || !g->exec) {
     set_error("hg_graph_launch: no graph");
     return 1;
+  }
+  if (g->ks && !all_ks(g)) {
+    // earlier launches still read the executable graph that is replaced
+    if (hipDeviceSynchronize() != hipSuccess || capture_grouped(g)) return 1;
   }
   hipError_t e = hipGraphLaunch(g->exec, (hipStream_t)stream);
   if (e != hipSuccess) {

@@ -72,18 +72,20 @@ __device__ __forceinline__ void newton_dx(const C2PInv &c, double igr, double W,
 // Setup of Utoprim_new_body up to the Newton guess (utoprim_2d_final.c:152-300).
 // U is alpha * U_geomfree; prim holds the guess.  Returns a failure code (4)
 // when the guess is unusable, else 0, and sets W_last and the invariants.
-__device__ __forceinline__ int c2p_setup(const double *U, const Geom &G, const double *prim,
+template <class GT>
+__device__ __forceinline__ int c2p_setup(const double *U, const GT &G, const double *prim,
                                          double gam, C2PInv &c, double &W_last) {
-  double Bcov[4], Qcov[4], ncov[4];
+  double Bcov[4], Qcov[4];
   c.Bcon[0] = 0.;
   c.Bcon[1] = U[B1];
   c.Bcon[2] = U[B2];
   c.Bcon[3] = U[B3];
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
+  for (int i = 1; i < 4; i++) {
     Bcov[i] = 0.;
 #pragma unroll
-    for (int j = 0; j < 4; j++) Bcov[i] += G.gcov[i][j] * c.Bcon[j];
+    for (int j = 1; j < 4; j++)
+      if (!GT::cov0(i, j)) Bcov[i] += G.gcov[i][j] * c.Bcon[j];
   }
 #pragma unroll
   for (int i = 0; i < 4; i++) Qcov[i] = U[UU + i];
@@ -91,27 +93,20 @@ __device__ __forceinline__ int c2p_setup(const double *U, const Geom &G, const d
   for (int i = 0; i < 4; i++) {
     c.Qcon[i] = 0.;
 #pragma unroll
-    for (int j = 0; j < 4; j++) c.Qcon[i] += G.gcon[i][j] * Qcov[j];
+    for (int j = 0; j < 4; j++)
+      if (!GT::con0(i, j)) c.Qcon[i] += G.gcon[i][j] * Qcov[j];
   }
   c.Bsq = 0.;
 #pragma unroll
   for (int i = 1; i < 4; i++) c.Bsq += c.Bcon[i] * Bcov[i];
   c.QdotB = 0.;
 #pragma unroll
-  for (int i = 0; i < 4; i++) c.QdotB += Qcov[i] * c.Bcon[i];
+  for (int i = 1; i < 4; i++) c.QdotB += Qcov[i] * c.Bcon[i];  // B^t = 0
   c.QdotBsq = c.QdotB * c.QdotB;
-  double lapse = sqrt(-1. / G.gcon[0][0]);
-  ncov[0] = -lapse;
-  ncov[1] = 0.;
-  ncov[2] = 0.;
-  ncov[3] = 0.;
+  const double ncov0 = -sqrt(-1. / G.gcon[0][0]);  // the only nonzero n_mu
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    c.ncon[i] = 0.;
-#pragma unroll
-    for (int j = 0; j < 4; j++) c.ncon[i] += G.gcon[i][j] * ncov[j];
-  }
-  c.Qdotn = c.Qcon[0] * ncov[0];
+  for (int i = 0; i < 4; i++) c.ncon[i] = GT::con0(i, 0) ? 0. : 0. + G.gcon[i][0] * ncov0;
+  c.Qdotn = c.Qcon[0] * ncov0;
   double Qsq = 0.;
 #pragma unroll
   for (int i = 0; i < 4; i++) Qsq += Qcov[i] * c.Qcon[i];
@@ -122,7 +117,8 @@ __device__ __forceinline__ int c2p_setup(const double *U, const Geom &G, const d
 #pragma unroll
   for (int i = 1; i < 4; i++)
 #pragma unroll
-    for (int j = 1; j < 4; j++) utsq += G.gcov[i][j] * prim[U1 + i - 1] * prim[U1 + j - 1];
+    for (int j = 1; j < 4; j++)
+      if (!GT::cov0(i, j)) utsq += G.gcov[i][j] * prim[U1 + i - 1] * prim[U1 + j - 1];
   if ((utsq < 0.) && (fabs(utsq) < MAXNEGUTSQ)) utsq = 0.0;
   const double utsq_too_big = (GAMMAFAIL - 1.0) * (GAMMAFAIL - 1.0);
   if (utsq < 0. || utsq > utsq_too_big) return FAIL_CONVGUESSUTSQ;
@@ -185,7 +181,8 @@ __device__ __forceinline__ int c2p_finish(const C2PInv &c, double W, int retval,
 // U: evolved conserved variables (with gdet); pr: guess in, solution out.
 // The core also returns the invariants and the final Newton iterate (x0 = W,
 // x1 = vsq); newton is false when the set-up failed before the iteration.
-__device__ __forceinline__ int utoprimgen_fp64_core(const double *U, const Geom &G, double gam, double *pr,
+template <class GT>
+__device__ __forceinline__ int utoprimgen_fp64_core(const double *U, const GT &G, double gam, double *pr,
                                                     int &iters, C2PInv &c, double &x0, double &x1,
                                                     bool &newton) {
   double Ug[NPR], Ut[NPR];
@@ -240,7 +237,8 @@ __device__ __forceinline__ int utoprimgen_fp64_core(const double *U, const Geom 
   return code;
 }
 
-__device__ __forceinline__ int utoprimgen_fp64(const double *U, const Geom &G, double gam, double *pr,
+template <class GT>
+__device__ __forceinline__ int utoprimgen_fp64(const double *U, const GT &G, double gam, double *pr,
                                                int &iters) {
   C2PInv c;
   double x0 = 0., x1 = 0.;
@@ -487,7 +485,8 @@ __device__ __forceinline__ int c2p_finish_dd(const C2PInv &c, double W, double i
 // values), then, for a zone it solves, the polish from its final iterate and
 // the primitives in double-double; these replace the reference's values
 // when the polish converges.  *polished tells whether they did.
-__device__ __forceinline__ int utoprimgen_refined(const double *U, const Geom &G, double gam, double *pr,
+template <class GT>
+__device__ __forceinline__ int utoprimgen_refined(const double *U, const GT &G, double gam, double *pr,
                                                   int &iters, bool &polished) {
   C2PInv c;
   double x0 = 0., x1 = 0.;

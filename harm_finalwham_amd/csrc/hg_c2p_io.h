@@ -102,7 +102,8 @@ __device__ __forceinline__ void c2p_features(const C2PInv &c, double W_last, dou
 }
 
 // the FP64 set-up shared by features and the learned inversion
-__device__ __forceinline__ int c2p_setup_zone(const double *U, const Geom &G, double gam, const double *guess,
+template <class GT>
+__device__ __forceinline__ int c2p_setup_zone(const double *U, const GT &G, double gam, const double *guess,
                                           C2PInv &c, double &W_last, double &alpha, double *Ug) {
   double Ut[NPR];
 #pragma unroll

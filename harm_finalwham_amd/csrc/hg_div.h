@@ -35,6 +35,29 @@ __device__ __forceinline__ bool div_num_ok(double x) {
 
 __device__ __forceinline__ bool div_den_ok(double d) { return d >= 0x1p-300 && d <= 0x1p300; }
 
+// x[k] / d for K numerators of one divisor of either sign, whose reciprocal
+// y = rcp_refined(d) the caller formed.  The residual is taken as d q - x:
+// where it is zero its negative is -0, which leaves a zero quotient's sign
+// alone, so unlike div_core this keeps x / d for x = -0 too.
+template <int K>
+__device__ __forceinline__ void div_group(double *x, double d, double y) {
+  double q[K];
+  bool ok = div_den_ok(fabs(d));
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    const double q0 = x[k] * y;
+    q[k] = fma(-fma(d, q0, -x[k]), y, q0);
+    ok = ok && div_num_ok(x[k]);
+  }
+  if (ok) {
+#pragma unroll
+    for (int k = 0; k < K; k++) x[k] = q[k];
+  } else {
+#pragma unroll
+    for (int k = 0; k < K; k++) x[k] /= d;
+  }
+}
+
 // x[k] / d for K numerators of one positive divisor, none of them -0.  SD
 // false: K full divisions.  The shuffle kernel along i runs faster with the
 // shared reciprocal, the marching kernels (whose loop the range checks and

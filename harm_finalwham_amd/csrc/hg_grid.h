@@ -30,6 +30,7 @@ struct Dims {
   int n1, n2, n3;
   int nb1, nb2, nb3;
   int m1, m2, m3;
+  int ks;                // the metric tables hold the Kerr-Schild zeros (GeomT, hg_phys.h)
   int g1, g2;            // geometry table extents (m1+1, m2+1)
   int64_t sj, sk, spl;   // strides of j, k, pl in a[pl][k][j][i]
   int64_t gplane;        // g1*g2
@@ -43,6 +44,7 @@ struct Dims {
 
 inline Dims make_dims(int n1, int n2, int n3, int nb) {
   Dims d;
+  d.ks = 0;
   d.n1 = n1; d.n2 = n2; d.n3 = n3;
   d.nb1 = (n1 > 1) ? nb : 0;
   d.nb2 = (n2 > 1) ? nb : 0;

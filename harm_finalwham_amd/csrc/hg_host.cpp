@@ -12,6 +12,7 @@
 #include "hg_grid.h"
 #include "hg_host.h"
 #include "hg_kernels.h"
+#include "hg_phys.h"
 
 using namespace hg;
 
@@ -182,6 +183,16 @@ int hg::upload_geometry_tables(hg_ctx *c, const double *gcov, const double *gcon
       fl[g] = c->cfg.rhomin * pow(r, -1.5);
       fl[d.cplane + g] = c->cfg.uumin * pow(r, -2.5);
     }
+  // whether the metric has the zeros GeomT<true> leaves out, each +0
+  bool ks = true;
+  for (int l = 0; l < 4; l++)
+    for (int a = 0; a < 16; a++)
+      for (int part = 0; part < 2; part++) {
+        if (!(part ? GeomT<true>::con0(a / 4, a % 4) : GeomT<true>::cov0(a / 4, a % 4))) continue;
+        const double *b = &geo[((size_t)l * GCOMP + 16 * part + a) * d.gplane];
+        for (int64_t z = 0; z < d.gplane && ks; z++) ks = b[z] == 0. && !std::signbit(b[z]);
+      }
+  c->d.ks = ks ? 1 : 0;
   HIPCHECK(hipMemcpy(c->geo, geo.data(), geo.size() * sizeof(double), hipMemcpyHostToDevice));
   HIPCHECK(hipMemcpy(c->corn, corn.data(), corn.size() * sizeof(double), hipMemcpyHostToDevice));
   HIPCHECK(hipMemcpy(c->conn, cn.data(), cn.size() * sizeof(double), hipMemcpyHostToDevice));
@@ -415,10 +426,20 @@ extern "C" const char *hg_profile_class_name(int k) {
   return (k >= 0 && k < HG_PROF_NCLASS) ? names[k] : "";
 }
 
+// The grid as the next launches on s see it.  A captured launch may be
+// replayed after the caller has uploaded another geometry, so what a capture
+// records reads the whole metric (Dims::ks 0).
+static Dims launch_dims(const hg_ctx *c, hipStream_t s, bool &captured) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  captured = c->capturing || hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
+  Dims d = c->d;
+  if (captured) d.ks = 0;
+  return d;
+}
+
 // fluxcalc (flux.c:7) on primitives pb: per-direction fluxes and ndt bits,
 // then the flux-CT EMFs (fluxct.c:10)
-static void enqueue_fluxcalc(hg_ctx *c, const double *pb, hipStream_t s) {
-  const Dims &d = c->d;
+static void enqueue_fluxcalc(hg_ctx *c, const double *pb, const Dims &d, bool captured, hipStream_t s) {
   const hg_config &f = c->cfg;
   c->flux_state = pb;
   c->dg_faces_valid = false;
@@ -430,11 +451,7 @@ static void enqueue_fluxcalc(hg_ctx *c, const double *pb, hipStream_t s) {
   // caller's: the fork records the context's own events onto its own side
   // streams, which a capture would pull into the graph, and that path is
   // kept out of captures (a graph runs its grids side by side instead).
-  bool conc = c->tune.concurrent && !c->prof_on && !c->capturing;
-  if (conc) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) conc = false;
-  }
+  const bool conc = c->tune.concurrent && !c->prof_on && !captured;
   // Run one after another, the three directions' dP/P indicators take one
   // launch with the shared inputs' (fewer launches for the small grids of a
   // graph); a profile keeps them with their directions, as the concurrent
@@ -493,7 +510,9 @@ static void enqueue_fluxcalc(hg_ctx *c, const double *pb, hipStream_t s) {
 extern "C" int hg_fluxcalc(hg_ctx *c, double *F1, double *F2, double *F3, double ndt[3], void *stream) {
   if (need_geometry(c, "hg_fluxcalc")) return 1;
   hipStream_t s = (hipStream_t)stream;
-  enqueue_fluxcalc(c, c->p, s);
+  bool captured;
+  const Dims ld = launch_dims(c, s, captured);
+  enqueue_fluxcalc(c, c->p, ld, captured, s);
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipStreamSynchronize(s));
   if (check_err(c)) return 1;
@@ -531,7 +550,9 @@ extern "C" int hg_fluxcalc(hg_ctx *c, double *F1, double *F2, double *F3, double
 static void enqueue_substep(hg_ctx *c, double *pi, double *pb, double *pf, const RkStage &rk, int stage,
                             int finalstep, hipStream_t s) {
   const hg_config &f = c->cfg;
-  enqueue_fluxcalc(c, pb, s);
+  bool captured;
+  const Dims d = launch_dims(c, s, captured);
+  enqueue_fluxcalc(c, pb, d, captured, s);
   const bool rk4 = f.timeorder == 4;
   if (c->dg_record && (finalstep || rk4)) {
     // diag_flux of advance.c:130, where the reference's p is still pi; the
@@ -542,13 +563,13 @@ static void enqueue_substep(hg_ctx *c, double *pi, double *pb, double *pf, const
   }
   prof_mark(c, HG_PROF_UPDATE, s);
   launch_update(pi, pb, c->uf, c->F[0], c->F[1], c->F[2], c->emf[0], c->emf[1], c->emf[2], c->geo, c->conn, c->dt,
-                rk, c->d, f.gam, f.dx, c->err, c->tune, s);
+                rk, d, f.gam, f.dx, c->err, c->tune, s);
   if (c->c2p_mode == HG_C2P_LEARNED) {
     // the network's start for every inversion of this substep
     launch_step_features(c->uf, pb, c->geo, c->d, f.gam, c->lx, s);
     launch_mlp_forward(c->mlp, (int64_t)c->d.n1 * c->d.n2 * c->d.n3, c->lx, c->ly, s);
   }
-  launch_invert(c->uf, pb, pf, c->geo, c->floors, rk, finalstep, c->d, f.gam, f.gammamax, c->counters, c->pflag,
+  launch_invert(c->uf, pb, pf, c->geo, c->floors, rk, finalstep, d, f.gam, f.gammamax, c->counters, c->pflag,
                 c->c2p_mode == HG_C2P_MIXED ? 1 : c->c2p_mode == HG_C2P_LEARNED ? 2 : 0, c->ly, c->fx_count,
                 c->err, c->tune, s);
   if (finalstep) launch_dt(c->ndt_bits, c->dt, f.defcon, f.safe, s);

@@ -149,11 +149,12 @@ enum GroupClass {
 // FP64, 1 mixed, 2 mixed from the learned start; GK_MLP goes through
 // launch_group_mlp, which needs the network)
 unsigned group_blocks(int k, const GridView &v);
-void launch_group(int k, const GridView *views, const unsigned *first, int n, unsigned total, int mode,
+void launch_group(int k, const GridView *views, const unsigned *first, int n, unsigned total, int mode, bool ks,
                   hipStream_t s);
 // the per-TU parts of the two above
 unsigned group_blocks_weno(int k, const GridView &v);
-void launch_group_weno(int k, const GridView *views, const unsigned *first, int n, unsigned total, hipStream_t s);
+void launch_group_weno(int k, const GridView *views, const unsigned *first, int n, unsigned total, bool ks,
+                       hipStream_t s);
 unsigned group_blocks_fixup(int k, const GridView &v);
 void launch_group_fixup(int k, const GridView *views, const unsigned *first, int n, unsigned total, hipStream_t s);
 // the reconstruction's line segments of a view (v.d set), as launch_weno

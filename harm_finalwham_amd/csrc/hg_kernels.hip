@@ -18,15 +18,16 @@
 
 namespace hg {
 
+template <class GT>
 __device__ __forceinline__ void load_geom(const double *__restrict__ full, int loc, int64_t gplane, int64_t gi,
-                                          Geom &G) {
+                                          GT &G) {
   const double *b = full + (int64_t)loc * GCOMP * gplane + gi;
 #pragma unroll
   for (int a = 0; a < 4; a++)
 #pragma unroll
     for (int c = 0; c < 4; c++) {
-      G.gcov[a][c] = b[(a * 4 + c) * gplane];
-      G.gcon[a][c] = b[(16 + a * 4 + c) * gplane];
+      if (!GT::cov0(a, c)) G.gcov[a][c] = b[(a * 4 + c) * gplane];
+      if (!GT::con0(a, c)) G.gcon[a][c] = b[(16 + a * 4 + c) * gplane];
     }
   G.gpert0 = b[32 * gplane];
   G.g = b[33 * gplane];
@@ -36,13 +37,14 @@ __device__ __forceinline__ void load_geom(const double *__restrict__ full, int l
 // maxwell() forms depend on the geometry alone; without this barrier the
 // compiler keeps the products of one state alive for the next state that
 // uses the same geometry, which costs more registers than recomputing them.
-__device__ __forceinline__ void geom_barrier(Geom &G) {
+template <class GT>
+__device__ __forceinline__ void geom_barrier(GT &G) {
 #pragma unroll
   for (int a = 0; a < 4; a++)
 #pragma unroll
     for (int c = 0; c < 4; c++) {
-      asm volatile("" : "+v"(G.gcov[a][c]));
-      asm volatile("" : "+v"(G.gcon[a][c]));
+      if (!GT::cov0(a, c)) asm volatile("" : "+v"(G.gcov[a][c]));
+      if (!GT::con0(a, c)) asm volatile("" : "+v"(G.gcon[a][c]));
     }
   asm volatile("" : "+v"(G.gpert0));
   asm volatile("" : "+v"(G.g));
@@ -189,7 +191,8 @@ __global__ void k_bound_x3(double *__restrict__ p, Dims d) { bound_x3_body(p, d,
 // ---------------------------------------------------------------------------
 // Riemann flux at one face from left/right states, fluxcompute.c:12
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ bool face_flux(int dir, Geom &G, double *p_l, double *p_r, double gam,
+template <class GT>
+__device__ __forceinline__ bool face_flux(int dir, GT &G, double *p_l, double *p_r, double gam,
                                           int fluxmethod, double *F, double &ctop) {
   // flux.c:629 BDIRCONT
   double bav = 0.5 * (p_l[B1 + dir - 1] + p_r[B1 + dir - 1]);
@@ -199,9 +202,10 @@ __device__ __forceinline__ bool face_flux(int dir, Geom &G, double *p_l, double 
   // starts, so only its results stay live
   double F_l[NPR], F_r[NPR], U_l[NPR], U_r[NPR];
   double cmax_l, cmin_l, cmax_r, cmin_r;
+  const double alpha = lapse_of(G);
   {
     State ql;
-    if (get_state(p_l, G, ql)) return true;
+    if (get_state(p_l, G, alpha, ql)) return true;
     Maxwell M;
     maxwell(p_l, ql, G, M);
     double p1 = one_plus_ud0(ql, G);
@@ -212,7 +216,7 @@ __device__ __forceinline__ bool face_flux(int dir, Geom &G, double *p_l, double 
   geom_barrier(G);
   {
     State qr;
-    if (get_state(p_r, G, qr)) return true;
+    if (get_state(p_r, G, alpha, qr)) return true;
     Maxwell M;
     maxwell(p_r, qr, G, M);
     double p1 = one_plus_ud0(qr, G);
@@ -229,7 +233,9 @@ __device__ __forceinline__ bool face_flux(int dir, Geom &G, double *p_l, double 
   if (fluxmethod == 1 && (lmax + lmin != 0.0)) {
 #pragma unroll
     for (int pl = 0; pl < NPR; pl++)
-      F[pl] = ((lmax * F_l[pl] + lmin * F_r[pl]) - (lmax * lmin) * (U_r[pl] - U_l[pl])) / (lmax + lmin);
+      F[pl] = (lmax * F_l[pl] + lmin * F_r[pl]) - (lmax * lmin) * (U_r[pl] - U_l[pl]);
+    const double ls = lmax + lmin;
+    div_by<NPR>(F, ls, div_rcp(ls));
   } else {
 #pragma unroll
     for (int pl = 0; pl < NPR; pl++) F[pl] = 0.5 * ((F_l[pl] + F_r[pl]) - ctop * (U_r[pl] - U_l[pl]));
@@ -469,7 +475,7 @@ __device__ __forceinline__ void para4(const double y[5], double &lout, double &r
 // point-type reconstruction fused with the Riemann flux (flux.c:469
 // fluxcalc_standard): MC slopes (interppoint.c:387) or PARA interface values
 // (interppoint.c:289), turned into the face states by flux.c:753 getp2interplr
-template <int DIR, bool PARA, bool EXT = false>
+template <int DIR, bool PARA, bool EXT = false, bool KS = false>
 __device__ __forceinline__ void flux_point_body(const double *__restrict__ p, const double *__restrict__ geo,
                                                 double *__restrict__ F, const Dims &d, const FaceRange &fr,
                                                 double gam, double cour, double dxdir, int fluxmethod, int slim,
@@ -510,11 +516,13 @@ __device__ __forceinline__ void flux_point_body(const double *__restrict__ p, co
         }
       }
     }
-    Geom G;
+    GeomT<KS> G;
     load_geom(geo, DIR, d.gplane, d.gidx(i, j), G);
     double Fz[NPR], ctop;
-    if (EXT ? face_flux_ext(DIR, G, p_l, p_r, gam, fluxmethod, Fz, ctop)
-            : face_flux(DIR, G, p_l, p_r, gam, fluxmethod, Fz, ctop)) {
+    bool bad;
+    if constexpr (EXT) bad = face_flux_ext(DIR, G, p_l, p_r, gam, fluxmethod, Fz, ctop);
+    else bad = face_flux(DIR, G, p_l, p_r, gam, fluxmethod, Fz, ctop);
+    if (bad) {
       atomicOr(err, 2);
     } else {
 #pragma unroll
@@ -525,34 +533,34 @@ __device__ __forceinline__ void flux_point_body(const double *__restrict__ p, co
   block_min_to(dtij, ndt_bits);
 }
 
-template <int DIR>
+template <int DIR, bool KS>
 __global__ void __launch_bounds__(256) k_flux_mc(const double *__restrict__ p, const double *__restrict__ geo,
                                                  double *__restrict__ F, Dims d, double gam, double cour,
                                                  double dxdir, int fluxmethod, int slim,
                                                  unsigned long long *__restrict__ ndt_bits, int *__restrict__ err) {
   FaceRange fr = face_range(d, DIR);
-  flux_point_body<DIR, false>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err);
+  flux_point_body<DIR, false, false, KS>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err);
 }
 
-template <int DIR>
+template <int DIR, bool KS>
 __global__ void __launch_bounds__(256) k_flux_para(const double *__restrict__ p, const double *__restrict__ geo,
                                                    double *__restrict__ F, Dims d, double gam, double cour,
                                                    double dxdir, int fluxmethod, int slim,
                                                    unsigned long long *__restrict__ ndt_bits,
                                                    int *__restrict__ err) {
   FaceRange fr = face_range(d, DIR);
-  flux_point_body<DIR, true>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err);
+  flux_point_body<DIR, true, false, KS>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err);
 }
 
 // the finite-volume flux loops (every transverse ghost row)
-template <int DIR, bool PARA>
+template <int DIR, bool PARA, bool KS>
 __global__ void __launch_bounds__(256) k_flux_pt_fv(const double *__restrict__ p, const double *__restrict__ geo,
                                                     double *__restrict__ F, Dims d, double gam, double cour,
                                                     double dxdir, int fluxmethod, int slim,
                                                     unsigned long long *__restrict__ ndt_bits,
                                                     int *__restrict__ err) {
   FaceRange fr = face_range_fv(d, DIR);
-  flux_point_body<DIR, PARA>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err);
+  flux_point_body<DIR, PARA, false, KS>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err);
 }
 
 // MC or PARA with the FORCE / MUSTA / HLLLAXF1 fluxes
@@ -566,7 +574,7 @@ __global__ void __launch_bounds__(256) k_flux_pt_ext(const double *__restrict__ 
   flux_point_body<DIR, PARA, true>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err);
 }
 
-template <int DIR, bool EXT>
+template <int DIR, bool EXT, bool KS = false>
 __device__ __forceinline__ void flux_lr_body(const double *__restrict__ pleft,
                                                  const double *__restrict__ pright,
                                                  const double *__restrict__ geo, double *__restrict__ F, Dims d,
@@ -591,11 +599,13 @@ __device__ __forceinline__ void flux_lr_body(const double *__restrict__ pleft,
       p_l[pl] = pright[z - s + pl * d.spl];
       p_r[pl] = pleft[z + pl * d.spl];
     }
-    Geom G;
+    GeomT<KS> G;
     load_geom(geo, DIR, d.gplane, d.gidx(i, j), G);
     double Fz[NPR], ctop;
-    if (EXT ? face_flux_ext(DIR, G, p_l, p_r, gam, fluxmethod, Fz, ctop)
-            : face_flux(DIR, G, p_l, p_r, gam, fluxmethod, Fz, ctop)) {
+    bool bad;
+    if constexpr (EXT) bad = face_flux_ext(DIR, G, p_l, p_r, gam, fluxmethod, Fz, ctop);
+    else bad = face_flux(DIR, G, p_l, p_r, gam, fluxmethod, Fz, ctop);
+    if (bad) {
       atomicOr(err, 2);
     } else {
 #pragma unroll
@@ -606,18 +616,18 @@ __device__ __forceinline__ void flux_lr_body(const double *__restrict__ pleft,
   block_min_to(dtij, ndt_bits);
 }
 
-template <int DIR>
+template <int DIR, bool KS>
 __global__ void __launch_bounds__(256) k_flux_lr(const double *__restrict__ pleft,
                                                  const double *__restrict__ pright,
                                                  const double *__restrict__ geo, double *__restrict__ F, Dims d,
                                                  double gam, double cour, double dxdir, int fluxmethod,
                                                  unsigned long long *__restrict__ ndt_bits, int *__restrict__ err) {
   FaceRange fr = face_range(d, DIR);
-  flux_lr_body<DIR, false>(pleft, pright, geo, F, d, fr, gam, cour, dxdir, fluxmethod, ndt_bits, err, blockIdx.x);
+  flux_lr_body<DIR, false, KS>(pleft, pright, geo, F, d, fr, gam, cour, dxdir, fluxmethod, ndt_bits, err, blockIdx.x);
 }
 
 // the finite-volume flux loops (every transverse ghost row)
-template <int DIR>
+template <int DIR, bool KS>
 __global__ void __launch_bounds__(256) k_flux_lr_fv(const double *__restrict__ pleft,
                                                     const double *__restrict__ pright,
                                                     const double *__restrict__ geo, double *__restrict__ F, Dims d,
@@ -625,7 +635,7 @@ __global__ void __launch_bounds__(256) k_flux_lr_fv(const double *__restrict__ p
                                                     unsigned long long *__restrict__ ndt_bits,
                                                     int *__restrict__ err) {
   FaceRange fr = face_range_fv(d, DIR);
-  flux_lr_body<DIR, false>(pleft, pright, geo, F, d, fr, gam, cour, dxdir, fluxmethod, ndt_bits, err, blockIdx.x);
+  flux_lr_body<DIR, false, KS>(pleft, pright, geo, F, d, fr, gam, cour, dxdir, fluxmethod, ndt_bits, err, blockIdx.x);
 }
 
 // WENO5BND states with the FORCE / MUSTA / HLLLAXF1 fluxes
@@ -709,7 +719,7 @@ __global__ void k_emf(const double *__restrict__ F1, const double *__restrict__ 
 // (one kernel holding both needs more registers than either, and the Uf
 // round trip through HBM costs less than the occupancy it loses)
 // ---------------------------------------------------------------------------
-template <bool UCUM, bool FV>
+template <bool UCUM, bool FV, bool KS>
 __device__ __forceinline__ void update_body(const double *__restrict__ pi, const double *__restrict__ pb,
                                             double *__restrict__ ubuf, const double *__restrict__ F1,
                                             const double *__restrict__ F2, const double *__restrict__ F3,
@@ -729,7 +739,7 @@ __device__ __forceinline__ void update_body(const double *__restrict__ pi, const
     int s1 = d.n1 > 1, s2 = d.n2 > 1, s3 = d.n3 > 1;
     int64_t z = d.idx(i, j, k);
     const int64_t P = d.spl;
-    Geom G;
+    GeomT<KS> G;
     load_geom(geo, GL_CENT, d.gplane, d.gidx(i, j), G);
     double Ui[NPR], dUg[NPR], prb[NPR];
     bool bad = false;
@@ -745,9 +755,12 @@ __device__ __forceinline__ void update_body(const double *__restrict__ pi, const
       bad = primtoU(pri, G, gam, Ui);
     }
     // the three phases (U of p_i, source of p_b, flux divergence) are kept
-    // apart: interleaved, their live values exceed the register file
+    // apart: interleaved, their live values take 256 VGPRs (0.50 against 0.31
+    // ms at 256x128x64).  The full metric is held back from one phase to the
+    // next as well; the 18 numbers of the Kerr-Schild one need not be (112
+    // VGPRs and 0.31 ms without, 154 and 0.38 ms with)
     value_barrier(Ui, NPR);
-    geom_barrier(G);
+    if (!KS) geom_barrier(G);
     asm volatile("" ::: "memory");
 #pragma unroll
     for (int pl = 0; pl < NPR; pl++) prb[pl] = pb[z + pl * P];
@@ -783,7 +796,7 @@ __device__ __forceinline__ void update_body(const double *__restrict__ pi, const
       dUg[B3] = 0.0 + G.g * 0;
     }
     value_barrier(dUg, NPR);
-    geom_barrier(G);
+    if (!KS) geom_barrier(G);
     asm volatile("" ::: "memory");
     // advance.c:741 flux2dUavg, field components from the flux-CT EMFs (fluxct.c:720-781)
     double Uf[NPR];
@@ -852,7 +865,7 @@ __device__ __forceinline__ void update_body(const double *__restrict__ pi, const
   }
 }
 
-template <bool UCUM, bool FV>
+template <bool UCUM, bool FV, bool KS>
 __global__ void __launch_bounds__(256) k_update(const double *__restrict__ pi, const double *__restrict__ pb,
                                                 double *__restrict__ ubuf, const double *__restrict__ F1,
                                                 const double *__restrict__ F2, const double *__restrict__ F3,
@@ -861,7 +874,7 @@ __global__ void __launch_bounds__(256) k_update(const double *__restrict__ pi, c
                                                 const double *__restrict__ conn, const double *__restrict__ dtp,
                                                 RkStage rk, Dims d, double gam, double idx1, double idx2,
                                                 double idx3, int *__restrict__ err) {
-  update_body<UCUM, FV>(pi, pb, ubuf, F1, F2, F3, emf1, emf2, emf3, geo, conn, dtp, rk, d, gam, idx1, idx2, idx3, err,
+  update_body<UCUM, FV, KS>(pi, pb, ubuf, F1, F2, F3, emf1, emf2, emf3, geo, conn, dtp, rk, d, gam, idx1, idx2, idx3, err,
                         blockIdx.x);
 }
 
@@ -872,8 +885,8 @@ __global__ void __launch_bounds__(256) k_update(const double *__restrict__ pi, c
 // primitives) with the converged-root reference inversion (HG_C2P_REFINED)
 // from the plain guess for any zone that path does not settle
 constexpr int INV_FP64 = 0, INV_MIXED = 1, INV_LEARNED = 2;
-template <int MODE>
-__device__ __forceinline__ int invert_zone(const double *Uf, const Geom &G, double gam, double *pr, float ylearn,
+template <int MODE, class GT>
+__device__ __forceinline__ int invert_zone(const double *Uf, const GT &G, double gam, double *pr, float ylearn,
                                            int &iters) {
   if (MODE == INV_FP64) return utoprimgen_fp64(Uf, G, gam, pr, iters);
   {
@@ -904,7 +917,7 @@ __device__ __forceinline__ int invert_zone(const double *Uf, const Geom &G, doub
   return utoprimgen_refined(Uf, G, gam, pr, iters, pol);
 }
 
-template <bool FV, int MODE>
+template <bool FV, int MODE, bool KS>
 __device__ __forceinline__ void invert_body(const double *__restrict__ ubuf, const double *__restrict__ pb,
                                             double *__restrict__ pf, const double *__restrict__ geo,
                                             const double *__restrict__ floors, int finalstep, const Dims &d,
@@ -925,7 +938,7 @@ __device__ __forceinline__ void invert_body(const double *__restrict__ ubuf, con
     int j = (int)(r / d.n3);
     int64_t z = d.idx(i, j, k);
     const int64_t P = d.spl;
-    Geom G;
+    GeomT<KS> G;
     load_geom(geo, GL_CENT, d.gplane, d.gidx(i, j), G);
     double Uf[NPR], pr[NPR];
 #pragma unroll
@@ -978,7 +991,7 @@ __device__ __forceinline__ void invert_body(const double *__restrict__ ubuf, con
   block_sum_to(nfail, nit, &counters[0], &counters[1]);
 }
 
-template <bool FV, int MODE>
+template <bool FV, int MODE, bool KS>
 __global__ void __launch_bounds__(256) k_invert(const double *__restrict__ ubuf, const double *__restrict__ pb,
                                                 double *__restrict__ pf, const double *__restrict__ geo,
                                                 const double *__restrict__ floors, int finalstep, Dims d,
@@ -987,7 +1000,7 @@ __global__ void __launch_bounds__(256) k_invert(const double *__restrict__ ubuf,
                                                 int8_t *__restrict__ pflag, double *__restrict__ ucons,
                                                 const float *__restrict__ ylearn, unsigned *__restrict__ fx_reset,
                                                 int *__restrict__ err) {
-  invert_body<FV, MODE>(ubuf, pb, pf, geo, floors, finalstep, d, gam, gammamax, counters, pflag, ucons, ylearn,
+  invert_body<FV, MODE, KS>(ubuf, pb, pf, geo, floors, finalstep, d, gam, gammamax, counters, pflag, ucons, ylearn,
                         fx_reset, err, blockIdx.x);
 }
 
@@ -1033,11 +1046,11 @@ __global__ void __launch_bounds__(256) kg_bound_x3(const GridView *__restrict__ 
   bound_x3_body(v.pf, v.d, bid);
 }
 
-template <int DIR>
+template <int DIR, bool KS>
 __global__ void __launch_bounds__(256) kg_flux_lr(const GridView *__restrict__ views,
                                                   const unsigned *__restrict__ first, int n) {
   HG_GROUP_PRELUDE
-  flux_lr_body<DIR, false>(v.pl[DIR - 1], v.pr[DIR - 1], v.geo, v.F[DIR - 1], v.d, face_range(v.d, DIR), v.gam,
+  flux_lr_body<DIR, false, KS>(v.pl[DIR - 1], v.pr[DIR - 1], v.geo, v.F[DIR - 1], v.d, face_range(v.d, DIR), v.gam,
                            v.cour, v.dx[DIR], v.fluxmethod, v.ndt_bits + DIR - 1, v.err, bid);
 }
 
@@ -1047,19 +1060,19 @@ __global__ void __launch_bounds__(256) kg_emf(const GridView *__restrict__ views
   emf_body(v.F[0], v.F[1], v.F[2], v.geo, v.corn, v.emf[0], v.emf[1], v.emf[2], v.d, bid);
 }
 
-template <bool UCUM>
+template <bool UCUM, bool KS>
 __global__ void __launch_bounds__(256) kg_update(const GridView *__restrict__ views,
                                                  const unsigned *__restrict__ first, int n) {
   HG_GROUP_PRELUDE
-  update_body<UCUM, false>(v.pi, v.pb, v.uf, v.F[0], v.F[1], v.F[2], v.emf[0], v.emf[1], v.emf[2], v.geo, v.conn,
+  update_body<UCUM, false, KS>(v.pi, v.pb, v.uf, v.F[0], v.F[1], v.F[2], v.emf[0], v.emf[1], v.emf[2], v.geo, v.conn,
                             v.dt, v.rk, v.d, v.gam, v.idx[1], v.idx[2], v.idx[3], v.err, bid);
 }
 
-template <int MODE>
+template <int MODE, bool KS>
 __global__ void __launch_bounds__(256) kg_invert(const GridView *__restrict__ views,
                                                  const unsigned *__restrict__ first, int n) {
   HG_GROUP_PRELUDE
-  invert_body<false, MODE>(v.uf, v.pb, v.pf, v.geo, v.floors, v.finalstep, v.d, v.gam, v.gammamax, v.counters,
+  invert_body<false, MODE, KS>(v.uf, v.pb, v.pf, v.geo, v.floors, v.finalstep, v.d, v.gam, v.gammamax, v.counters,
                            v.pflag, nullptr, MODE == INV_LEARNED ? v.ly : nullptr, v.fx.count, v.err, bid);
 }
 
@@ -1122,6 +1135,19 @@ void launch_gather_inversions(const double *ubuf, const double *pb, const double
 // ---------------------------------------------------------------------------
 static inline unsigned nblocks(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
+// the instance of a kernel template for the grid's metric (Dims::ks, GeomT):
+// its last template argument
+#define HG_LAUNCH_KS(ks, K, A, g, b, ...)                                            \
+  do {                                                                               \
+    if (ks) hipLaunchKernelGGL((K<A, true>), g, b, 0, s, __VA_ARGS__);               \
+    else hipLaunchKernelGGL((K<A, false>), g, b, 0, s, __VA_ARGS__);                 \
+  } while (0)
+#define HG_LAUNCH_KS2(ks, K, A, B, g, b, ...)                                        \
+  do {                                                                               \
+    if (ks) hipLaunchKernelGGL((K<A, B, true>), g, b, 0, s, __VA_ARGS__);            \
+    else hipLaunchKernelGGL((K<A, B, false>), g, b, 0, s, __VA_ARGS__);              \
+  } while (0)
+
 void launch_bound(double *p, const double *geo, const Dims &d, double gammamax, int *err, hipStream_t s) {
   if (d.n1 > 1) {
     int64_t n = 2LL * d.nb1 * d.n2 * d.n3;
@@ -1158,25 +1184,25 @@ void launch_flux_point(int dir, int lim, bool fv, const double *p, const double 
   }
   if (fv) {
     if (para) {
-      if (dir == 1) hipLaunchKernelGGL((k_flux_pt_fv<1, true>), g, b, 0, s, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
-      if (dir == 2) hipLaunchKernelGGL((k_flux_pt_fv<2, true>), g, b, 0, s, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
-      if (dir == 3) hipLaunchKernelGGL((k_flux_pt_fv<3, true>), g, b, 0, s, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+      if (dir == 1) HG_LAUNCH_KS2(d.ks, k_flux_pt_fv, 1, true, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+      if (dir == 2) HG_LAUNCH_KS2(d.ks, k_flux_pt_fv, 2, true, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+      if (dir == 3) HG_LAUNCH_KS2(d.ks, k_flux_pt_fv, 3, true, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
     } else {
-      if (dir == 1) hipLaunchKernelGGL((k_flux_pt_fv<1, false>), g, b, 0, s, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
-      if (dir == 2) hipLaunchKernelGGL((k_flux_pt_fv<2, false>), g, b, 0, s, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
-      if (dir == 3) hipLaunchKernelGGL((k_flux_pt_fv<3, false>), g, b, 0, s, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+      if (dir == 1) HG_LAUNCH_KS2(d.ks, k_flux_pt_fv, 1, false, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+      if (dir == 2) HG_LAUNCH_KS2(d.ks, k_flux_pt_fv, 2, false, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+      if (dir == 3) HG_LAUNCH_KS2(d.ks, k_flux_pt_fv, 3, false, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
     }
     return;
   }
   if (para) {
-    if (dir == 1) hipLaunchKernelGGL(k_flux_para<1>, g, b, 0, s, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
-    if (dir == 2) hipLaunchKernelGGL(k_flux_para<2>, g, b, 0, s, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
-    if (dir == 3) hipLaunchKernelGGL(k_flux_para<3>, g, b, 0, s, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+    if (dir == 1) HG_LAUNCH_KS(d.ks, k_flux_para, 1, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+    if (dir == 2) HG_LAUNCH_KS(d.ks, k_flux_para, 2, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+    if (dir == 3) HG_LAUNCH_KS(d.ks, k_flux_para, 3, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
     return;
   }
-  if (dir == 1) hipLaunchKernelGGL(k_flux_mc<1>, g, b, 0, s, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
-  if (dir == 2) hipLaunchKernelGGL(k_flux_mc<2>, g, b, 0, s, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
-  if (dir == 3) hipLaunchKernelGGL(k_flux_mc<3>, g, b, 0, s, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+  if (dir == 1) HG_LAUNCH_KS(d.ks, k_flux_mc, 1, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+  if (dir == 2) HG_LAUNCH_KS(d.ks, k_flux_mc, 2, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+  if (dir == 3) HG_LAUNCH_KS(d.ks, k_flux_mc, 3, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
 }
 
 // initbase.c:18 init_conservatives (primtoU of every active zone) into the
@@ -1221,14 +1247,14 @@ void launch_flux_lr(int dir, const double *pleft, const double *pright, const do
     return;
   }
   if (fv) {
-    if (dir == 1) hipLaunchKernelGGL(k_flux_lr_fv<1>, g, b, 0, s, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
-    if (dir == 2) hipLaunchKernelGGL(k_flux_lr_fv<2>, g, b, 0, s, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
-    if (dir == 3) hipLaunchKernelGGL(k_flux_lr_fv<3>, g, b, 0, s, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
+    if (dir == 1) HG_LAUNCH_KS(d.ks, k_flux_lr_fv, 1, g, b, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
+    if (dir == 2) HG_LAUNCH_KS(d.ks, k_flux_lr_fv, 2, g, b, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
+    if (dir == 3) HG_LAUNCH_KS(d.ks, k_flux_lr_fv, 3, g, b, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
     return;
   }
-  if (dir == 1) hipLaunchKernelGGL(k_flux_lr<1>, g, b, 0, s, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
-  if (dir == 2) hipLaunchKernelGGL(k_flux_lr<2>, g, b, 0, s, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
-  if (dir == 3) hipLaunchKernelGGL(k_flux_lr<3>, g, b, 0, s, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
+  if (dir == 1) HG_LAUNCH_KS(d.ks, k_flux_lr, 1, g, b, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
+  if (dir == 2) HG_LAUNCH_KS(d.ks, k_flux_lr, 2, g, b, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
+  if (dir == 3) HG_LAUNCH_KS(d.ks, k_flux_lr, 3, g, b, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
 }
 
 void launch_emf(const double *F1, const double *F2, const double *F3, const double *geo, const double *corn,
@@ -1285,13 +1311,13 @@ void launch_update(const double *pi, const double *pb, double *ubuf, const doubl
   dim3 g(nblocks(n, tu.bs_update)), b(tu.bs_update);
   const double i1 = 1.0 / dx[1], i2 = 1.0 / dx[2], i3 = 1.0 / dx[3];
   if (rk.ucons)
-    hipLaunchKernelGGL((k_update<true, true>), g, b, 0, s, pi, pb, ubuf, F1, F2, F3, e1, e2, e3, geo, conn, dtp, rk, d,
+    HG_LAUNCH_KS2(d.ks, k_update, true, true, g, b, pi, pb, ubuf, F1, F2, F3, e1, e2, e3, geo, conn, dtp, rk, d,
                        gam, i1, i2, i3, err);
   else if (rk.ucum)
-    hipLaunchKernelGGL((k_update<true, false>), g, b, 0, s, pi, pb, ubuf, F1, F2, F3, e1, e2, e3, geo, conn, dtp, rk,
+    HG_LAUNCH_KS2(d.ks, k_update, true, false, g, b, pi, pb, ubuf, F1, F2, F3, e1, e2, e3, geo, conn, dtp, rk,
                        d, gam, i1, i2, i3, err);
   else
-    hipLaunchKernelGGL((k_update<false, false>), g, b, 0, s, pi, pb, ubuf, F1, F2, F3, e1, e2, e3, geo, conn, dtp, rk,
+    HG_LAUNCH_KS2(d.ks, k_update, false, false, g, b, pi, pb, ubuf, F1, F2, F3, e1, e2, e3, geo, conn, dtp, rk,
                        d, gam, i1, i2, i3, err);
 }
 
@@ -1303,10 +1329,10 @@ static void launch_invert_mode(const double *ubuf, const double *pb, double *pf,
   int64_t n = (int64_t)d.n1 * d.n2 * d.n3;
   dim3 gi(nblocks(n, tu.bs_invert)), bi(tu.bs_invert);
   if (rk.ucons && finalstep)
-    hipLaunchKernelGGL((k_invert<true, MODE>), gi, bi, 0, s, ubuf, pb, pf, geo, floors, finalstep, d, gam, gammamax,
+    HG_LAUNCH_KS2(d.ks, k_invert, true, MODE, gi, bi, ubuf, pb, pf, geo, floors, finalstep, d, gam, gammamax,
                        counters, pflag, rk.ucons, ylearn, fx_reset, err);
   else
-    hipLaunchKernelGGL((k_invert<false, MODE>), gi, bi, 0, s, ubuf, pb, pf, geo, floors, finalstep, d, gam, gammamax,
+    HG_LAUNCH_KS2(d.ks, k_invert, false, MODE, gi, bi, ubuf, pb, pf, geo, floors, finalstep, d, gam, gammamax,
                        counters, pflag, nullptr, ylearn, fx_reset, err);
 }
 
@@ -1411,7 +1437,7 @@ unsigned group_blocks(int k, const GridView &v) {
   }
 }
 
-void launch_group(int k, const GridView *views, const unsigned *first, int n, unsigned total, int mode,
+void launch_group(int k, const GridView *views, const unsigned *first, int n, unsigned total, int mode, bool ks,
                   hipStream_t s) {
   if (total == 0) return;
   const dim3 g(total);
@@ -1419,23 +1445,23 @@ void launch_group(int k, const GridView *views, const unsigned *first, int n, un
     case GK_BOUND1: hipLaunchKernelGGL(kg_bound_x1, g, dim3(128), 0, s, views, first, n); return;
     case GK_BOUND2: hipLaunchKernelGGL(kg_bound_x2, g, dim3(256), 0, s, views, first, n); return;
     case GK_BOUND3: hipLaunchKernelGGL(kg_bound_x3, g, dim3(256), 0, s, views, first, n); return;
-    case GK_FLUX1: hipLaunchKernelGGL(kg_flux_lr<1>, g, dim3(256), 0, s, views, first, n); return;
-    case GK_FLUX2: hipLaunchKernelGGL(kg_flux_lr<2>, g, dim3(256), 0, s, views, first, n); return;
-    case GK_FLUX3: hipLaunchKernelGGL(kg_flux_lr<3>, g, dim3(256), 0, s, views, first, n); return;
+    case GK_FLUX1: HG_LAUNCH_KS(ks, kg_flux_lr, 1, g, dim3(256), views, first, n); return;
+    case GK_FLUX2: HG_LAUNCH_KS(ks, kg_flux_lr, 2, g, dim3(256), views, first, n); return;
+    case GK_FLUX3: HG_LAUNCH_KS(ks, kg_flux_lr, 3, g, dim3(256), views, first, n); return;
     case GK_EMF: hipLaunchKernelGGL(kg_emf, g, dim3(256), 0, s, views, first, n); return;
-    case GK_UPDATE: hipLaunchKernelGGL(kg_update<false>, g, dim3(256), 0, s, views, first, n); return;
-    case GK_UPDATEU: hipLaunchKernelGGL(kg_update<true>, g, dim3(256), 0, s, views, first, n); return;
+    case GK_UPDATE: HG_LAUNCH_KS(ks, kg_update, false, g, dim3(256), views, first, n); return;
+    case GK_UPDATEU: HG_LAUNCH_KS(ks, kg_update, true, g, dim3(256), views, first, n); return;
     case GK_INVERT:
-      if (mode == INV_MIXED) hipLaunchKernelGGL(kg_invert<INV_MIXED>, g, dim3(256), 0, s, views, first, n);
-      else if (mode == INV_LEARNED) hipLaunchKernelGGL(kg_invert<INV_LEARNED>, g, dim3(256), 0, s, views, first, n);
-      else hipLaunchKernelGGL(kg_invert<INV_FP64>, g, dim3(256), 0, s, views, first, n);
+      if (mode == INV_MIXED) HG_LAUNCH_KS(ks, kg_invert, INV_MIXED, g, dim3(256), views, first, n);
+      else if (mode == INV_LEARNED) HG_LAUNCH_KS(ks, kg_invert, INV_LEARNED, g, dim3(256), views, first, n);
+      else HG_LAUNCH_KS(ks, kg_invert, INV_FP64, g, dim3(256), views, first, n);
       return;
     case GK_FEATURES: hipLaunchKernelGGL(kg_step_features, g, dim3(256), 0, s, views, first, n); return;
     case GK_DT: hipLaunchKernelGGL(kg_dt, g, dim3(64), 0, s, views, first, n); return;
     case GK_FXCHECK: case GK_FXRESOLVE: case GK_FXAVG: case GK_FXAPPLY:
       launch_group_fixup(k, views, first, n, total, s);
       return;
-    default: launch_group_weno(k, views, first, n, total, s);
+    default: launch_group_weno(k, views, first, n, total, ks, s);
   }
 }
 

@@ -315,7 +315,7 @@ void ucon2pr_rel4(const double ucon[4], const Geom &G, double *pr) {
 // relative 4-velocity goes through u^mu and back
 bool rel4_round_trip(double *pr, const Geom &G) {
   double ucon[4];
-  if (ucon_calc(pr, G, ucon)) return true;
+  if (ucon_calc(pr, G, lapse_of(G), ucon)) return true;
   ucon2pr_rel4(ucon, G, pr);
   return false;
 }

@@ -327,6 +327,7 @@ __device__ __forceinline__ void stage_e(const double *y, double m0, double w0, d
 // stage A inputs per zone: par = (1 + u_t) u^t, upar = gam u u^t u_t + (gam-1) u
 // over the box [-2, n+1] of every direction with more than one zone
 // ---------------------------------------------------------------------------
+template <bool KS>
 __device__ __forceinline__ void weno_prep_body(const double *__restrict__ p, const double *__restrict__ geo,
                                                double *__restrict__ aux, const Dims &d, double gam, int wide,
                                                unsigned long long *__restrict__ ndt_reset, unsigned bid) {
@@ -346,15 +347,15 @@ __device__ __forceinline__ void weno_prep_body(const double *__restrict__ p, con
   double pr[NPR];
 #pragma unroll
   for (int pl = 0; pl < NPR; pl++) pr[pl] = p[z + pl * d.spl];
-  Geom G;
+  GeomT<KS> G;
   {
     const double *b = geo + (int64_t)GL_CENT * GCOMP * d.gplane + d.gidx(i, j);
 #pragma unroll
     for (int a = 0; a < 4; a++)
 #pragma unroll
       for (int c = 0; c < 4; c++) {
-        G.gcov[a][c] = b[(a * 4 + c) * d.gplane];
-        G.gcon[a][c] = b[(16 + a * 4 + c) * d.gplane];
+        if (!G.cov0(a, c)) G.gcov[a][c] = b[(a * 4 + c) * d.gplane];
+        if (!G.con0(a, c)) G.gcon[a][c] = b[(16 + a * 4 + c) * d.gplane];
       }
     G.gpert0 = b[32 * d.gplane];
     G.g = b[33 * d.gplane];
@@ -366,10 +367,11 @@ __device__ __forceinline__ void weno_prep_body(const double *__restrict__ p, con
   aux[z + d.spl] = gam * pr[UU] * (q.ucon[0] * q.ucov[0]) + (gam - 1.0) * pr[UU];
 }
 
+template <bool KS>
 __global__ void __launch_bounds__(256) k_weno_prep(const double *__restrict__ p, const double *__restrict__ geo,
                                                    double *__restrict__ aux, Dims d, double gam, int wide,
                                                    unsigned long long *__restrict__ ndt_reset) {
-  weno_prep_body(p, geo, aux, d, gam, wide, ndt_reset, blockIdx.x);
+  weno_prep_body<KS>(p, geo, aux, d, gam, wide, ndt_reset, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -645,10 +647,11 @@ __global__ void __launch_bounds__(256) k_weno_m(const double *__restrict__ p, co
   const unsigned bid = blockIdx.x - first[g_], nblk = first[g_ + 1] - first[g_]; \
   (void)nblk;
 
+template <bool KS>
 __global__ void __launch_bounds__(256) kg_weno_prep(const GridView *__restrict__ views,
                                                     const unsigned *__restrict__ first, int n) {
   WG_PRELUDE
-  weno_prep_body(v.pb, v.geo, v.aux, v.d, v.gam, 0, v.ndt_bits, bid);
+  weno_prep_body<KS>(v.pb, v.geo, v.aux, v.d, v.gam, 0, v.ndt_bits, bid);
 }
 
 __global__ void __launch_bounds__(256) kg_weno_dpi(const GridView *__restrict__ views,
@@ -677,9 +680,10 @@ void launch_weno_prep(const double *p, const double *geo, double *aux, const Dim
   const int e1 = d.n1 > 1 ? (wide ? d.nb1 : 2) : 0, e2 = d.n2 > 1 ? (wide ? d.nb2 : 2) : 0;
   const int e3 = d.n3 > 1 ? (wide ? d.nb3 : 2) : 0;
   int64_t n = (int64_t)(d.n1 + 2 * e1) * (d.n2 + 2 * e2) * (d.n3 + 2 * e3);
-  hipLaunchKernelGGL(k_weno_prep, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p, geo, aux, d, gam, wide,
-                     ndt_reset);
-  if (all_dpi) hipLaunchKernelGGL(k_weno_dpi<0>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p, aux, d, wide);
+  const dim3 gb((unsigned)((n + 255) / 256));
+  if (d.ks) hipLaunchKernelGGL(k_weno_prep<true>, gb, dim3(256), 0, s, p, geo, aux, d, gam, wide, ndt_reset);
+  else hipLaunchKernelGGL(k_weno_prep<false>, gb, dim3(256), 0, s, p, geo, aux, d, gam, wide, ndt_reset);
+  if (all_dpi) hipLaunchKernelGGL(k_weno_dpi<0>, gb, dim3(256), 0, s, p, aux, d, wide);
 }
 
 static void weno_march_shape(int dir, const Dims &d, const Tune &tu, int wide, int &nseg, int &seglen, int &nlb) {
@@ -771,9 +775,13 @@ unsigned group_blocks_weno(int k, const GridView &v) {
   }
 }
 
-void launch_group_weno(int k, const GridView *views, const unsigned *first, int n, unsigned total, hipStream_t s) {
+void launch_group_weno(int k, const GridView *views, const unsigned *first, int n, unsigned total, bool ks,
+                       hipStream_t s) {
   const dim3 g(total), b(256);
-  if (k == GK_PREP) hipLaunchKernelGGL(kg_weno_prep, g, b, 0, s, views, first, n);
+  if (k == GK_PREP) {
+    if (ks) hipLaunchKernelGGL(kg_weno_prep<true>, g, b, 0, s, views, first, n);
+    else hipLaunchKernelGGL(kg_weno_prep<false>, g, b, 0, s, views, first, n);
+  }
   if (k == GK_DPI) hipLaunchKernelGGL(kg_weno_dpi, g, b, 0, s, views, first, n);
   if (k == GK_WENO1) hipLaunchKernelGGL(kg_weno_x, g, b, 0, s, views, first, n);
   if (k == GK_WENO2) hipLaunchKernelGGL(kg_weno_m<2>, g, b, 0, s, views, first, n);
