@@ -35,14 +35,15 @@ __device__ __forceinline__ bool div_num_ok(double x) {
 
 __device__ __forceinline__ bool div_den_ok(double d) { return d >= 0x1p-300 && d <= 0x1p300; }
 
-// x[k] / d for K numerators of one divisor of either sign, whose reciprocal
-// y = rcp_refined(d) the caller formed.  The residual is taken as d q - x:
-// where it is zero its negative is -0, which leaves a zero quotient's sign
-// alone, so unlike div_core this keeps x / d for x = -0 too.
+// x[k] / d for K numerators of one divisor, whose reciprocal y = rcp_refined(d)
+// the caller formed; a divisor that is not positive takes full divisions.  The
+// residual is taken as d q - x: where it is zero its negative is -0, which
+// leaves a zero quotient's sign alone, so unlike div_core this keeps x / d for
+// x = -0 too.
 template <int K>
 __device__ __forceinline__ void div_group(double *x, double d, double y) {
   double q[K];
-  bool ok = div_den_ok(fabs(d));
+  bool ok = div_den_ok(d);
 #pragma unroll
   for (int k = 0; k < K; k++) {
     const double q0 = x[k] * y;
@@ -55,50 +56,6 @@ __device__ __forceinline__ void div_group(double *x, double d, double y) {
   } else {
 #pragma unroll
     for (int k = 0; k < K; k++) x[k] /= d;
-  }
-}
-
-// x[k] / d for K numerators of one positive divisor, none of them -0.  SD
-// false: K full divisions.  The shuffle kernel along i runs faster with the
-// shared reciprocal, the marching kernels (whose loop the range checks and
-// their branches lengthen) without.
-template <int K, bool SD>
-__device__ __forceinline__ void div_shared(double *x, double d) {
-  if (!SD) {
-#pragma unroll
-    for (int k = 0; k < K; k++) x[k] /= d;
-    return;
-  }
-  const double y = rcp_refined(d);
-  double q[K];
-  bool ok = div_den_ok(d);
-#pragma unroll
-  for (int k = 0; k < K; k++) {
-    q[k] = div_core(x[k], d, y);
-    ok = ok && div_num_ok(x[k]);
-  }
-  if (ok) {
-#pragma unroll
-    for (int k = 0; k < K; k++) x[k] = q[k];
-  } else {
-#pragma unroll
-    for (int k = 0; k < K; k++) x[k] /= d;
-  }
-}
-
-// the mixed-sign numerators n[0..3] of one constant divisor d, whose
-// reciprocal yd = rcp_refined(d) the caller forms once: q[k] = n[k] / d
-// bit for bit, except that a zero quotient is +0 for both signs of n[k]
-__device__ __forceinline__ void div_const4(const double *n, double d, double yd, double *q) {
-  bool ok = true;
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    q[k] = div_core(n[k], d, yd);
-    ok = ok && div_num_ok(n[k]);
-  }
-  if (!ok) {
-#pragma unroll
-    for (int k = 0; k < 4; k++) q[k] = n[k] / d;
   }
 }
 

@@ -22,7 +22,7 @@ __device__ __forceinline__ uint64_t mixh(uint64_t z) {
 // an operand from hash h: the biased exponent anywhere, inside the divisor's
 // range, around the numerator's range or at the edges of both; a random
 // mantissa, one just below or just above a power of two, or a pattern
-__device__ __forceinline__ double operand(uint64_t h, bool positive) {
+__device__ __forceinline__ double operand(uint64_t h) {
   const uint64_t h2 = mixh(h);
   int e;
   switch ((h >> 60) & 3) {
@@ -43,8 +43,8 @@ __device__ __forceinline__ double operand(uint64_t h, bool positive) {
     default: m = h2 & 0x5555555555555ull; break;
   }
   uint64_t bits = ((uint64_t)e << 52) | m;
-  if ((h & 0x3FF) == 7) bits = 0;
-  if (!positive && ((h >> 12) & 1)) bits |= 0x8000000000000000ull;
+  if ((h & 0x3FF) == 7) bits = 0;  // zeros of either sign
+  if ((h >> 12) & 1) bits |= 0x8000000000000000ull;
   return __longlong_as_double((long long)bits);
 }
 
@@ -52,36 +52,33 @@ __device__ __forceinline__ bool same(double a, double b) {
   return __double_as_longlong(a) == __double_as_longlong(b) || (a != a && b != b);
 }
 
-// out: [0] mismatches of div_shared<3, true> (non-negative numerators, one
-// positive divisor), [1] of 1 / d through div_shared<1, true>, [2] of
-// div_const4 by 12 (mixed signs; a zero quotient may differ in sign only),
-// [3] operand sets div_shared took its shortcut for
+// out: [0] mismatches of div_group<3> (one divisor, either sign;
+// a negative one takes full divisions), [1] of 1 / d
+// through div_group<1>, [2] of div_group<4> by 12, [3] operand sets the first
+// took its shortcut for
 __global__ void k_check_div(int64_t n, uint64_t seed, unsigned long long *out) {
   const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   unsigned long long bad = 0, badr = 0, badc = 0, fast = 0;
   if (t < n) {
     const uint64_t h = mixh(seed ^ mixh((uint64_t)t));
-    const double d = fabs(operand(h, true));
+    const double d = (h & 0xC00) ? fabs(operand(h)) : operand(h);
     double x[3], ref[3];
     bool ok = div_den_ok(d);
     for (int k = 0; k < 3; k++) {
-      x[k] = fabs(operand(mixh(h + 1 + k), true));
+      x[k] = operand(mixh(h + 1 + k));
       ref[k] = x[k] / d;
       ok = ok && div_num_ok(x[k]);
     }
     fast = ok ? 1ull : 0ull;
-    div_shared<3, true>(x, d);
+    div_group<3>(x, d, rcp_refined(d));
     for (int k = 0; k < 3; k++) bad += !same(x[k], ref[k]);
     double r[1] = {1.0};
-    div_shared<1, true>(r, d);
+    div_group<1>(r, d, rcp_refined(d));
     badr += !same(r[0], 1.0 / d);
     double nn[4], q[4];
-    for (int k = 0; k < 4; k++) nn[k] = operand(mixh(h + 11 + k), false);
-    div_const4(nn, 12., rcp_refined(12.), q);
-    for (int k = 0; k < 4; k++) {
-      const double rq = nn[k] / 12.;
-      badc += !(same(q[k], rq) || (q[k] == 0.0 && rq == 0.0));
-    }
+    for (int k = 0; k < 4; k++) nn[k] = q[k] = operand(mixh(h + 11 + k));
+    div_group<4>(q, 12., rcp_refined(12.));
+    for (int k = 0; k < 4; k++) badc += !same(q[k], nn[k] / 12.);
   }
   if (bad) atomicAdd(&out[0], bad);
   if (badr) atomicAdd(&out[1], badr);

@@ -50,40 +50,70 @@ __device__ __forceinline__ double wmin(double a, double b) { return ((a) < (b)) 
 __device__ __forceinline__ double wminmod(double a, double b) {
   return ((a) * (b) <= 0) ? 0.0 : ((fabs(a) < fabs(b)) ? (a) : (b));
 }
-__device__ __forceinline__ double wsign(double a) { return (a > 0.0) ? 1.0 : ((a < 0.0) ? -1.0 : 0.0); }
 
-// reconstructeno.c:1920 get_sum_of_elements, symmetric pairing
-__device__ __forceinline__ double sum3(double a0, double a1, double a2) {
-  double s = 0.0;
-  s += a0 + a2;
-  s += a1 * 1;
-  return s;
+// reconstructeno.c:1920 get_sum_of_elements, symmetric pairing.  The reference
+// adds to 0. first; that and a last term a[1] * 0 change a value only where it
+// is a zero of the other sign, so they are left out where the terms are
+// squares or weights (never -0) and where the caller adds the sum to 0.
+__device__ __forceinline__ double sum3(double a0, double a1, double a2) { return (a0 + a2) + a1; }
+__device__ __forceinline__ double sum5(const double *a) { return ((a[0] + a[4]) + (a[1] + a[3])) + a[2]; }
+
+// The quotients of the weights.  Every numerator and divisor of these
+// functions but the smoothness indicators' is bounded by the step that formed
+// it, so the hardware division's scaling and fix-up steps have nothing to do
+// and are left out (div_core, hg_div.h):
+//   indicators over their sum   si in [0, ss]; div_weights looks at the range
+//   1 / t^2, t = si + 1e-26     si is such a quotient, in [0, 1]
+//   w / sum of w                w = 1 / t^2 in [0.99, 1e52]
+//   stage D, stage E, order 2   weights in [1e-70, 1] and 1e-26 more, or sums
+//                               of weights that add up to 1
+// A NaN stays one on either way.  With the two readings off before a division
+// (cusp, mono_eno5) the reconstruction at 256x128x64 went from 0.428 / 0.514 /
+// 0.538 to 0.310 / 0.355 / 0.355 ms along i / j / k: FP64 issue bounds it, and
+// about 33 full divisions a point were half of that.
+template <int K>
+__device__ __forceinline__ void div_bounded(double *x, double d) {
+  const double y = rcp_refined(d);
+#pragma unroll
+  for (int k = 0; k < K; k++) x[k] = div_core(x[k], d, y);
 }
-__device__ __forceinline__ double sum2(double a0, double a1) {
-  double s = 0.0;
-  s += a0 + a1;
-  s += a1 * 0;
-  return s;
+__device__ __forceinline__ double rcp_bounded(double d) {
+  const double y = rcp_refined(d);
+  return fma(fma(-d, y, 1.0), y, y);
 }
-__device__ __forceinline__ double sum5(const double *a) {
-  double s = 0.0;
-  s += a[0] + a[4];
-  s += a[1] + a[3];
-  s += a[2] * 1;
-  return s;
+// indicators si >= e >= 0 over d = their sum ss + DBL_MIN: in the steps' range
+// when e >= 2^-600 and d <= 2^600, or when ss = 0 (a line of zeros: every
+// quotient is +0); full divisions otherwise
+template <int K>
+__device__ __forceinline__ void div_weights(double *si, double ss, double e) {
+  const double d = ss + DBL_MIN;
+  double q[K];
+#pragma unroll
+  for (int k = 0; k < K; k++) q[k] = si[k];
+  div_bounded<K>(q, d);
+  if (__builtin_expect((e >= 0x1p-600 && d <= 0x1p600) || ss == 0.0, 1)) {
+#pragma unroll
+    for (int k = 0; k < K; k++) si[k] = q[k];
+  } else {
+#pragma unroll
+    for (int k = 0; k < K; k++) si[k] /= d;
+  }
+}
+// indicators normalised by their sum -> weights normalised by theirs
+template <int K>
+__device__ __forceinline__ void norm_weights(const double *si, double *w) {
+#pragma unroll
+  for (int s = 0; s < K; s++) {
+    double t = si[s] + WENO_EPS / 1.;
+    t *= t;
+    w[s] = rcp_bounded(t);
+  }
+  div_bounded<K>(w, K == 3 ? sum3(w[0], w[1], w[K - 1]) : w[0] + w[1]);
 }
 
 // order-3 unoptimised weights (reconstructeno.c:1406) for a point far from
-// the line ends; u points at the cell.  Returns the cusp-driven lower-order
-// fraction (1 for a cusp, else 0).
-template <bool SD>
-__device__ __forceinline__ double weights3(double mono0, double mono1, const double *u, double *w) {
-  if (mono0 == 1) {
-    double sw = 1.0 / 3;
-    w[0] = sw; w[1] = sw; w[2] = sw;
-    return 0.;
-  }
-  double lof = (mono0 == 0 && mono1 != 0) ? 1.0 : 0.;
+// the line ends; u points at the cell
+__device__ __forceinline__ void weights3(const double *u, double *w) {
   double fd0 = -(3 * u[0] + u[2]) + 4 * u[1];
   double fd1 = u[1] - u[-1];
   double fd2 = (3 * u[0] + u[-2]) - 4 * u[-1];
@@ -97,65 +127,35 @@ __device__ __forceinline__ double weights3(double mono0, double mono1, const dou
   double u2[5];
 #pragma unroll
   for (int i = -2; i < 3; i++) u2[i + 2] = u[i] * u[i];
-  double e = sum5(u2) * WENO_EPS;
+  const double e = sum5(u2) * WENO_EPS;
 #pragma unroll
   for (int s = 0; s < 3; s++) si[s] += e;
-  double ss = sum3(si[0], si[1], si[2]);
-  // sums of squares and positive terms: no numerator is -0
-  div_shared<3, SD>(si, ss + DBL_MIN);
-#pragma unroll
-  for (int s = 0; s < 3; s++) {
-    double t = si[s] + WENO_EPS / 1.;
-    t *= t;
-    w[s] = 1.;
-    div_shared<1, SD>(&w[s], t);
-  }
-  double sw = sum3(w[0], w[1], w[2]);
-  div_shared<3, SD>(w, sw + 0);
-  return lof;
+  div_weights<3>(si, sum3(si[0], si[1], si[2]), e);
+  norm_weights<3>(si, w);
 }
 
 // order-2 unoptimised + optimised weights (reconstructeno.c:1406 and :1617 with order 2)
-template <bool SD>
-__device__ __forceinline__ void weights2(double mono0, const double *u, double *wl, double *wr) {
+__device__ __forceinline__ void weights2(const double *u, double *wl, double *wr) {
   double w[2];
-  if (mono0 == 1) {
-    // equal weights; compute_optimized_cf_stencil_weights returns without
-    // setting the optimised ones, which are then never read (mono0 == 1)
-    wl[0] = wl[1] = wr[0] = wr[1] = 0.0;
-    return;
-  }
   double fd0 = u[1] - u[0];
   double fd1 = u[0] - u[-1];
   double si[2] = {fd0 * fd0, fd1 * fd1};
-  double u2[3] = {u[-1] * u[-1], u[0] * u[0], u[1] * u[1]};
-  double e = sum3(u2[0], u2[1], u2[2]) * WENO_EPS;
+  const double e = sum3(u[-1] * u[-1], u[0] * u[0], u[1] * u[1]) * WENO_EPS;
   si[0] += e;
   si[1] += e;
-  double ss = sum2(si[0], si[1]);
-  // squares, positive sums and their products with positive constants: no
-  // numerator is -0
-  div_shared<2, SD>(si, ss + DBL_MIN);
-#pragma unroll
-  for (int s = 0; s < 2; s++) {
-    double t = si[s] + WENO_EPS / 1.;
-    t *= t;
-    w[s] = 1.;
-    div_shared<1, SD>(&w[s], t);
-  }
-  double sw = sum2(w[0], w[1]);
-  div_shared<2, SD>(w, sw + 0);
+  div_weights<2>(si, si[0] + si[1], e);
+  norm_weights<2>(si, w);
   wl[0] = w[0] * (1. / 4.);
   wl[1] = w[1] * (3. / 4);
   wr[0] = w[0] * (3. / 4.);
   wr[1] = w[1] * (1. / 4.);
-  double sl = sum2(wl[0], wl[1]);
-  div_shared<2, SD>(wl, sl + DBL_MIN);
-  double sr = sum2(wr[0], wr[1]);
-  div_shared<2, SD>(wr, sr + DBL_MIN);
+  div_bounded<2>(wl, wl[0] + wl[1] + DBL_MIN);
+  div_bounded<2>(wr, wr[0] + wr[1] + DBL_MIN);
 }
 
-// reconstructeno.c:730 eno_cvt for order 3, left (C2L) or right (C2R) face
+// reconstructeno.c:730 eno_cvt for order 3, left (C2L) or right (C2R) face.
+// The reference skips a stencil of weight 0; its term is then a zero here too
+// (a stencil that is not finite makes its weights NaN, not 0).
 __device__ __forceinline__ double cvt3(bool right, const double *sw, const double *u) {
   double su[3];
   // rows of the center-to-face matrices (Lagrange interpolation on 3 points)
@@ -166,8 +166,7 @@ __device__ __forceinline__ double cvt3(bool right, const double *sw, const doubl
     double pu0 = (right ? R[s][0] : L[s][0]) * u[0 - s];
     double pu1 = (right ? R[s][1] : L[s][1]) * u[1 - s];
     double pu2 = (right ? R[s][2] : L[s][2]) * u[2 - s];
-    su[s] = 0.0;
-    if (sw[s] != 0.0) su[s] = sw[s] * sum3(pu0, pu1, pu2);
+    su[s] = sw[s] * sum3(pu0, pu1, pu2);
   }
   return sum3(su[0], su[1], su[2]);
 }
@@ -180,64 +179,71 @@ __device__ __forceinline__ double cvt2(bool right, const double *sw, const doubl
   for (int s = 0; s < 2; s++) {
     double pu0 = (right ? R[s][0] : L[s][0]) * u[0 - s];
     double pu1 = (right ? R[s][1] : L[s][1]) * u[1 - s];
-    su[s] = 0.0;
-    if (sw[s] != 0.0) su[s] = sw[s] * sum2(pu0, pu1);
+    su[s] = sw[s] * (pu0 + pu1);
   }
-  return sum2(su[0], su[1]);
+  return su[0] + su[1];
 }
 
-// smonointerp.c:439 check_for_cusp_new; y points at the cell
-__device__ __forceinline__ bool cusp(const double *y) {
-  double df[4], ddf[3];  // df[-1..2] -> df[0..3], ddf[-1..1] -> ddf[0..2]
-#pragma unroll
-  for (int a = -1; a <= 2; a++) df[a + 1] = y[a] - y[a - 1];
-#pragma unroll
-  for (int a = -1; a <= 1; a++) ddf[a + 1] = df[a + 2] - df[a + 1];
-  double norm = (fabs(y[-2]) + fabs(y[-1]) + fabs(y[0]) + fabs(y[1]) + fabs(y[2]) + W_SMALL);
-  norm = norm * SQRT_WENO_EPS;
-  double d_1 = df[0], d0 = df[1], d1 = df[2], d2 = df[3];
-  double f1a = fabs(d0) - norm;
-  double f1 = ddf[0] * wsign(d0) - norm;
-  double f2 = -ddf[1] * wsign(d0) - norm;
-  double f3 = -d2 * wsign(d0) - norm;
-  double f3a = fabs(-d2 - d0) - 0.25 * (fabs(d2) + fabs(d0));
-  double f4 = -d1 * wsign(d0) - norm;
-  double f4a = fabs(-d1 - d0) - 0.25 * (fabs(d1) + fabs(d0));
-  if (f1a > 0 && f1 > 0 && f2 > 0 && ((f3 > 0 && f3a > 0) || (f4 > 0 && f4a > 0))) return true;
-  double f5a = fabs(d1) - norm;
-  double f5 = -ddf[2] * wsign(d1) - norm;
-  double f6 = ddf[1] * wsign(d1) - norm;
-  double f7 = -d_1 * wsign(d1) - norm;
-  double f7a = fabs(-d_1 - d1) - 0.25 * (fabs(d_1) + fabs(d1));
-  double f8 = -d0 * wsign(d1) - norm;
-  double f8a = fabs(-d0 - d1) - 0.25 * (fabs(d0) + fabs(d1));
-  if (f5a > 0 && f5 > 0 && f6 > 0 && ((f7 > 0 && f7a > 0) || (f8 > 0 && f8a > 0))) return true;
-  return false;
+// x with its sign flipped where s is negative
+__device__ __forceinline__ double flip(double x, double s) {
+  return __hiloint2double(__double2hiint(x) ^ (__double2hiint(s) & (int)0x80000000), __double2loint(x));
 }
 
-// smonointerp.c:296 compute_mono_indicator_point_eno5
-__device__ __forceinline__ double mono_eno5(const double *yin) {
-  // the four divisions by 12 (their zero quotients' signs cannot reach the
-  // result: the minmods below return a literal 0 for a zero argument)
-  const double n[4] = {(((-3 * yin[-2] + yin[2]) + (-10 * yin[-1] - 6 * yin[1])) + 18 * yin[0]),
-                        (((11 * yin[-2] - yin[2]) + (-20 * yin[-1] + 4 * yin[1])) + 6 * yin[0]),
-                        (((-yin[-2] + 3 * yin[2]) + (6 * yin[-1] + 10 * yin[1])) - 18 * yin[0]),
-                        (((-yin[-2] + 11 * yin[2]) + (4 * yin[-1] - 20 * yin[1])) + 6 * yin[0])};
-  double q[4];
-  div_const4(n, 12., rcp_refined(12.), q);
-  double ld1 = q[0], ld2 = q[1], rd1 = q[2], rd2 = q[3];
-  double ld3 = (((-3 * yin[-2] - yin[2]) + (10 * yin[-1] + 6 * yin[1])) - 12 * yin[0]) / 2.;
-  double rd3 = (((yin[-2] + 3 * yin[2]) - (6 * yin[-1] + 10 * yin[1])) + 12 * yin[0]) / 2.;
+// smonointerp.c:439 check_for_cusp_new; d_1..d2 the differences y[a] - y[a-1]
+// for a = -1..2, norm the reference's.  Its tests f = x - norm > 0 are x > norm.
+__device__ __forceinline__ bool cusp(double d_1, double d0, double d1, double d2, double norm) {
+  const double dd0 = d0 - d_1, dd1 = d1 - d0, dd2 = d2 - d1;
+  const bool c1 = fabs(d0) > norm && flip(dd0, d0) > norm && -flip(dd1, d0) > norm;
+  const bool c2 = fabs(d1) > norm && -flip(dd2, d1) > norm && flip(dd1, d1) > norm;
+  bool r = false;
+  if (c1)
+    r = (-flip(d2, d0) > norm && fabs(d2 + d0) > 0.25 * (fabs(d2) + fabs(d0))) ||
+        (-flip(d1, d0) > norm && fabs(d1 + d0) > 0.25 * (fabs(d1) + fabs(d0)));
+  if (c2 && !r)
+    r = (-flip(d_1, d1) > norm && fabs(d_1 + d1) > 0.25 * (fabs(d_1) + fabs(d1))) ||
+        (-flip(d0, d1) > norm && fabs(d0 + d1) > 0.25 * (fabs(d0) + fabs(d1)));
+  return r;
+}
+
+// smonointerp.c:296 compute_mono_indicator_point_eno5: the smallest of three
+// minmods over a cutoff, held to [0, 1]
+__device__ __forceinline__ double mono_quotient(const double *yin, const double *n, double l3, double r3) {
+  double ld1 = n[0] / 12., ld2 = n[1] / 12., rd1 = n[2] / 12., rd2 = n[3] / 12.;
   ld1 = wminmod(ld1, yin[-1] - yin[-2]);
   rd1 = wminmod(rd1, yin[2] - yin[1]);
   double minabs = W_BIG;
   minabs = wmin(minabs, fabs(wminmod(ld1, rd1)));
   minabs = wmin(minabs, fabs(wminmod(ld2, rd2)));
-  minabs = wmin(minabs, fabs(wminmod(ld3, rd3)));
+  minabs = wmin(minabs, fabs(wminmod(l3 / 2., r3 / 2.)));
   double norm = fabs(yin[0]) + ((fabs(yin[-1]) + fabs(yin[1])) + (fabs(yin[-2]) + fabs(yin[2])));
   double cutoff = norm * SQRT_WENO_EPS + DBL_MIN;
   double x = (minabs - 0.0) / (cutoff - 0.0);
   return wmax(0., wmin(1., x));
+}
+// It is 0 where two values of a minmod differ in sign or one is zero, and 1
+// where every value reaches the cutoff; those two are read off the values
+// before their divisions (norm is cusp's, which is the cutoff but for its
+// order of summing, so that 1.00001 norm is above the cutoff; at least 1e-63,
+// so that no product of the minmods underflows).  Only a point between, or one
+// that is not finite, takes the quotient.
+__device__ __forceinline__ double mono_eno5(const double *yin, double d_1, double d2, double norm) {
+  const double n[4] = {(((-3 * yin[-2] + yin[2]) + (-10 * yin[-1] - 6 * yin[1])) + 18 * yin[0]),
+                        (((11 * yin[-2] - yin[2]) + (-20 * yin[-1] + 4 * yin[1])) + 6 * yin[0]),
+                        (((-yin[-2] + 3 * yin[2]) + (6 * yin[-1] + 10 * yin[1])) - 18 * yin[0]),
+                        (((-yin[-2] + 11 * yin[2]) + (4 * yin[-1] - 20 * yin[1])) + 6 * yin[0])};
+  const double l3 = (((-3 * yin[-2] - yin[2]) + (10 * yin[-1] + 6 * yin[1])) - 12 * yin[0]);
+  const double r3 = (((yin[-2] + 3 * yin[2]) - (6 * yin[-1] + 10 * yin[1])) + 12 * yin[0]);
+  const int h0 = __double2hiint(n[0]);
+  const int differ = (h0 ^ __double2hiint(n[2])) | (h0 ^ __double2hiint(d_1)) | (h0 ^ __double2hiint(d2)) |
+                     (__double2hiint(n[1]) ^ __double2hiint(n[3])) | (__double2hiint(l3) ^ __double2hiint(r3));
+  const double mn = fmin(fmin(fabs(n[0]), fabs(n[2])), fmin(fabs(n[1]), fabs(n[3])));
+  const double md = fmin(fabs(d_1), fabs(d2)), m3 = fmin(fabs(l3), fabs(r3));
+  const bool finite = norm <= 1e280;
+  const bool zero = differ < 0 || fmin(mn, fmin(md, m3)) == 0.0;
+  const bool one = mn >= 12.0002 * norm && md >= 1.00001 * norm && m3 >= 2.00002 * norm;
+  double m = zero ? 0.0 : 1.0;
+  if (__builtin_expect(!(finite && (zero || one)), 0)) m = mono_quotient(yin, n, l3, r3);
+  return m;
 }
 
 // reconstructeno.c:826 c2e_simple_eno(5): ENO5 face value
@@ -254,13 +260,20 @@ __device__ __forceinline__ double eno5(bool right, const double *y) {
 // the stages at one point
 // ---------------------------------------------------------------------------
 // C: y points at the cell, y[-2..2] are read
-template <bool SD>
 __device__ __forceinline__ void stage_c(const double *y, double w[3], double &m0, double &lof0) {
-  double m1;
-  if (cusp(y)) { m0 = 0; m1 = 1; }
-  else { m0 = mono_eno5(y); m1 = m0; }
-  lof0 = weights3<SD>(m0, m1, y, w);
-  if (m0 > 0.0 && m0 < 1.0) {  // reconstructeno.c:702 mono_adjust_unoptimized_weights
+  const double d_1 = y[-1] - y[-2], d0 = y[0] - y[-1], d1 = y[1] - y[0], d2 = y[2] - y[1];
+  const double norm =
+      (fabs(y[-2]) + fabs(y[-1]) + fabs(y[0]) + fabs(y[1]) + fabs(y[2]) + W_SMALL) * SQRT_WENO_EPS;
+  const bool cu = cusp(d_1, d0, d1, d2, norm);
+  m0 = mono_eno5(y, d_1, d2, norm);
+  if (cu) m0 = 0.0;
+  lof0 = cu ? 1.0 : 0.0;
+  if (m0 == 1) {
+    w[0] = w[1] = w[2] = 1.0 / 3;
+    return;
+  }
+  weights3(y, w);
+  if (__builtin_expect(m0 > 0.0 && m0 < 1.0, 0)) {  // reconstructeno.c:702 mono_adjust_unoptimized_weights
     double simpleweight = 1.0 / 3.0;
 #pragma unroll
     for (int c = 0; c < 3; c++) w[c] = (1.0 - m0) * w[c] + m0 * simpleweight;
@@ -269,9 +282,11 @@ __device__ __forceinline__ void stage_c(const double *y, double w[3], double &m0
 
 // D: reconstructeno.c:1962 compute_weights_ratios and the cusp fraction
 __device__ __forceinline__ double stage_d(double w2_s, double w0_sm2, double w0_s, double w2_sp2, double lof0) {
-  double wl = (w2_s + WENO_EPS) / (w0_sm2 + WENO_EPS);
-  double wr = (w0_s + WENO_EPS) / (w2_sp2 + WENO_EPS);
-  double lof = (wmin(wl, wr) - MIN_TR) / (MAX_TR - MIN_TR);
+  double wl = w2_s + WENO_EPS, wr = w0_s + WENO_EPS;
+  div_bounded<1>(&wl, w0_sm2 + WENO_EPS);
+  div_bounded<1>(&wr, w2_sp2 + WENO_EPS);
+  double lof = (wmin(wl, wr) - MIN_TR);
+  lof = div_core(lof, MAX_TR - MIN_TR, rcp_refined(MAX_TR - MIN_TR));
   lof = wmax(0., wmin(lof, 1.0));
   return wmax(lof, lof0);
 }
@@ -283,7 +298,6 @@ __device__ __forceinline__ double dp_jump(double rho, double parm, double par0, 
 }
 
 // E: y points at the cell; lofm/lof0/lofp are the stage-D fractions at s-1, s, s+1
-template <bool SD>
 __device__ __forceinline__ void stage_e(const double *y, double m0, double w0, double w1, double w2, double lofm,
                                         double lof0, double lofp, double dPi, double &outl, double &outr) {
   double shock = wmin((fabs(dPi) - 0.5 * REDUCE_DP) / (0.5 * REDUCE_DP), 1.);
@@ -298,29 +312,25 @@ __device__ __forceinline__ void stage_e(const double *y, double m0, double w0, d
   // compute_optimized_cf_stencil_weights (order 3)
   double wl[3] = {w0 * (1. / 16.), w1 * (5. / 8.), w2 * (5. / 16.)};
   double wr[3] = {w0 * (5. / 16.), w1 * (5. / 8.), w2 * (1. / 16.)};
-  double sl = sum3(wl[0], wl[1], wl[2]), sr = sum3(wr[0], wr[1], wr[2]);
-  div_shared<3, SD>(wl, sl + DBL_MIN);
-  div_shared<3, SD>(wr, sr + DBL_MIN);
-  double l2[2] = {0., 0.}, r2[2] = {0., 0.};
-  bool two = (0.0 < lof);
-  if (two) {
+  div_bounded<3>(wl, sum3(wl[0], wl[1], wl[2]) + DBL_MIN);
+  div_bounded<3>(wr, sum3(wr[0], wr[1], wr[2]) + DBL_MIN);
+  // each side is the blend of the two orders, added to 0. (never -0)
+  if (0.0 < lof) {
+    double l2[2], r2[2];
+    weights2(y, l2, r2);
 #pragma unroll
     for (int c = 0; c < 3; c++) { wl[c] *= (1. - lof); wr[c] *= (1. - lof); }
-    weights2<SD>(m0, y, l2, r2);
     l2[0] *= lof; l2[1] *= lof; r2[0] *= lof; r2[1] *= lof;
+    outl = (0.0 + cvt3(false, wl, y)) + cvt2(false, l2, y);
+    outr = (0.0 + cvt3(true, wr, y)) + cvt2(true, r2, y);
+  } else {
+    outl = 0.0 + cvt3(false, wl, y);
+    outr = 0.0 + cvt3(true, wr, y);
   }
-  double outv[2];
-#pragma unroll
-  for (int side = 0; side < 2; side++) {
-    double prev = 0.0;
-    if (m0 != 0.0) prev = eno5(side == 1, y);
-    double ov = 0.0;
-    ov += cvt3(side == 1, side ? wr : wl, y);
-    if (two) ov += cvt2(side == 1, side ? r2 : l2, y);
-    outv[side] = (1.0 - m0) * ov + m0 * prev;
+  if (__builtin_expect(m0 != 0.0, 0)) {
+    outl = (1.0 - m0) * outl + m0 * eno5(false, y);
+    outr = (1.0 - m0) * outr + m0 * eno5(true, y);
   }
-  outl = outv[0];
-  outr = outv[1];
 }
 
 // ---------------------------------------------------------------------------
@@ -462,7 +472,7 @@ __device__ __forceinline__ void weno_x_body(const double *__restrict__ p, const 
   if (live) {
 #pragma unroll
     for (int a = 0; a < 5; a++) y[a] = yl[s - 2 + a];
-    stage_c<true>(y + 2, w, m0, lof0);
+    stage_c(y + 2, w, m0, lof0);
   }
   // stage D needs the weights of s-2 and s+2 (lanes -2 and +2)
   double w0m2 = __shfl_up(w[0], 2, 64);
@@ -473,7 +483,7 @@ __device__ __forceinline__ void weno_x_body(const double *__restrict__ p, const 
   if (live && lane >= 3 && lane < 3 + XOUT && s >= -1 && s <= n) {
     const double dPi = dpi[zl + s];
     double ol, orr;
-    stage_e<true>(y + 2, m0, w[0], w[1], w[2], lofm, lofd, lofp, dPi, ol, orr);
+    stage_e(y + 2, m0, w[0], w[1], w[2], lofm, lofd, lofp, dPi, ol, orr);
     int64_t z = (int64_t)pl * d.spl + zl + s;
     pleft[z] = ol;
     pright[z] = orr;
@@ -606,7 +616,7 @@ __device__ __forceinline__ void weno_m_body(const double *__restrict__ p, const 
     for (int a = 0; a < 7; a++) yw[a] = yw[a + 1];
     yw[7] = cy;
     double w[3], m0, lof0;
-    stage_c<false>(yw + 5, w, m0, lof0);
+    stage_c(yw + 5, w, m0, lof0);
 #pragma unroll
     for (int a = 0; a < 4; a++) W0[a] = W0[a + 1];
     W0[4] = w[0];
@@ -622,7 +632,7 @@ __device__ __forceinline__ void weno_m_body(const double *__restrict__ p, const 
     LD[2] = stage_d(W2[1], W0[0], W0[2], W2[3], (lofb & 4u) ? 1.0 : 0.0);
     // E(t-3)
     double outl = 0., outr = 0.;
-    if (t - 3 >= e0) stage_e<false>(yw + 2, M0[0], W0[1], W1[0], W2[0], LD[0], LD[1], LD[2], cdp, outl, outr);
+    if (t - 3 >= e0) stage_e(yw + 2, M0[0], W0[1], W1[0], W2[0], LD[0], LD[1], LD[2], cdp, outl, outr);
     const int ts = (t - 3 > e0) ? t - 3 : e0;
     WM_ST(lb, ts) = outl;
     WM_ST(rb, ts) = outr;
