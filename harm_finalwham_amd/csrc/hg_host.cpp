@@ -144,6 +144,7 @@ extern "C" int hg_ctx_destroy(hg_ctx *c) {
   if (c->ly) (void)hipFree(c->ly);
   fixup_free(c);
   diag_free(c);
+  slots_free(c);
   for (hipEvent_t e : c->prof_events) (void)hipEventDestroy(e);
   delete c;
   return 0;
@@ -208,35 +209,6 @@ extern "C" int hg_upload_geometry(hg_ctx *c, const double *gcov, const double *g
     return 1;
   }
   return upload_geometry_tables(c, gcov, gcon, gcovpert, gdet, conn, r_cent);
-}
-
-// AoS host [i][j][k][pl] <-> SoA device [pl][k][j][i]
-int hg::copy_prims(hg_ctx *c, double *dev, const double *host) {
-  const Dims &d = c->d;
-  std::vector<double> t((size_t)d.spl * NPR);
-  for (int ii = 0; ii < d.m1; ii++)
-    for (int jj = 0; jj < d.m2; jj++)
-      for (int kk = 0; kk < d.m3; kk++) {
-        size_t h = (((size_t)ii * d.m2 + jj) * d.m3 + kk) * NPR;
-        size_t g = (size_t)ii + (size_t)jj * d.sj + (size_t)kk * d.sk;
-        for (int pl = 0; pl < NPR; pl++) t[g + pl * d.spl] = host[h + pl];
-      }
-  HIPCHECK(hipMemcpy(dev, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
-  return 0;
-}
-
-int hg::fetch_prims(hg_ctx *c, const double *dev, double *host) {
-  const Dims &d = c->d;
-  std::vector<double> t((size_t)d.spl * NPR);
-  HIPCHECK(hipMemcpy(t.data(), dev, t.size() * sizeof(double), hipMemcpyDeviceToHost));
-  for (int ii = 0; ii < d.m1; ii++)
-    for (int jj = 0; jj < d.m2; jj++)
-      for (int kk = 0; kk < d.m3; kk++) {
-        size_t h = (((size_t)ii * d.m2 + jj) * d.m3 + kk) * NPR;
-        size_t g = (size_t)ii + (size_t)jj * d.sj + (size_t)kk * d.sk;
-        for (int pl = 0; pl < NPR; pl++) host[h + pl] = t[g + pl * d.spl];
-      }
-  return 0;
 }
 
 extern "C" int hg_set_prims(hg_ctx *c, const double *p) {
@@ -527,22 +499,9 @@ extern "C" int hg_fluxcalc(hg_ctx *c, double *F1, double *F2, double *F3, double
   launch_fluxct_fields(c->F[0], c->F[1], c->F[2], c->emf[0], c->emf[1], c->emf[2], d, s);
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipStreamSynchronize(s));
-  std::vector<double> h[3];
-  for (int k = 0; k < 3; k++) {
-    h[k].resize((size_t)d.spl * NPR);
-    HIPCHECK(hipMemcpy(h[k].data(), c->F[k], h[k].size() * sizeof(double), hipMemcpyDeviceToHost));
-  }
   double *outs[3] = {F1, F2, F3};
-  for (int k = 0; k < 3; k++) {
-    if (!outs[k]) continue;
-    for (int ii = 0; ii < d.m1; ii++)
-      for (int jj = 0; jj < d.m2; jj++)
-        for (int kk = 0; kk < d.m3; kk++) {
-          size_t hh = (((size_t)ii * d.m2 + jj) * d.m3 + kk) * NPR;
-          size_t g = (size_t)ii + (size_t)jj * d.sj + (size_t)kk * d.sk;
-          for (int pl = 0; pl < NPR; pl++) outs[k][hh + pl] = h[k][g + pl * d.spl];
-        }
-  }
+  for (int k = 0; k < 3; k++)
+    if (outs[k] && fetch_prims(c, c->F[k], outs[k])) return 1;
   return 0;
 }
 

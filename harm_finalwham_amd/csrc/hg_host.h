@@ -3,11 +3,19 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdarg>
+#include <mutex>
 #include <vector>
 
 #include "harmgpu.h"
 #include "hg_grid.h"
 #include "hg_kernels.h"
+
+// a pinned piece of host memory that states pass through (hg_copy.hip)
+struct HostSlot {
+  void *mem = nullptr;
+  hipEvent_t done = nullptr;
+};
+constexpr int HOST_SLOTS = 8;
 
 struct hg_ctx {
   hg_config cfg;
@@ -72,13 +80,19 @@ struct hg_ctx {
   size_t prof_used = 0;
   std::vector<hipEvent_t> prof_events;
   std::vector<ProfInterval> prof_intervals;
+  // made by the first calls that need them (up to 2 MiB each), freed with the context
+  std::mutex slots_mu;
+  HostSlot slots[HOST_SLOTS];
 };
 
 namespace hg {
 void set_error(const char *fmt, ...);
 int upload_geometry_tables(hg_ctx *c, const double *gcov, const double *gcon, const double *gcovpert,
                            const double *gdet, const double *conn, const double *r_cent);
+// a state between the host layout of hg_set_prims and the device's; both wait
 int copy_prims(hg_ctx *c, double *dev, const double *host);
+int fetch_prims(hg_ctx *c, const double *dev, double *host);
+void slots_free(hg_ctx *c);
 // one step of the context on stream s (kernels only: capturable)
 void enqueue_step(hg_ctx *c, hipStream_t s);
 // the substeps of one step of the context's scheme: their number (at most 4)
@@ -87,7 +101,6 @@ int step_substeps(hg_ctx *c, double *pb[4], double *pf[4], RkStage rk[4]);
 // finite-volume scheme: derive the carried conserved state from p if p was
 // set since (kernels only)
 void ensure_conserved(hg_ctx *c, hipStream_t s);
-int fetch_prims(hg_ctx *c, const double *dev, double *host);
 // returns 1 (with the error set) when the work counter cannot be set up
 // post_fixup buffers (hg_fixup.hip)
 int fixup_alloc(hg_ctx *c);

@@ -240,7 +240,7 @@ class Grid:
         _check(lib().hg_set_prims(self.h, _d(p)))
 
     def get_prims(self):
-        p = np.zeros(self.shape)
+        p = np.empty(self.shape)
         _check(lib().hg_get_prims(self.h, _d(p)))
         return p
 
@@ -251,7 +251,7 @@ class Grid:
         _check(lib().hg_set_conserved(self.h, _d(U)))
 
     def get_conserved(self):
-        U = np.zeros(self.shape)
+        U = np.empty(self.shape)
         _check(lib().hg_get_conserved(self.h, _d(U)))
         return U
 
@@ -319,7 +319,7 @@ class Grid:
         return out
 
     def fluxcalc(self):
-        F = [np.zeros(self.shape) for _ in range(3)]
+        F = [np.empty(self.shape) for _ in range(3)]
         ndt = np.zeros(3)
         _check(lib().hg_fluxcalc(self.h, _d(F[0]), _d(F[1]), _d(F[2]), _d(ndt), None))
         return F, ndt
