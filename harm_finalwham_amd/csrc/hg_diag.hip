@@ -9,9 +9,9 @@
 // step, the RK midpoint state of the final substep) and, for two of its
 // terms, the reference's global p at that point (the state at the start of
 // the step), which the step records when hg_diag_record is on.  The per-zone and per-face terms are formed
-// in parallel with the reference's arithmetic; every sum is then taken by one
-// thread in the reference's loop order, so the sums are bit-identical to the
-// reference's sequential double sums.  The div B normalisation of the
+// in parallel with the reference's arithmetic; every sum has the value of the
+// reference's loop, a sequential double sum in its order (k_dg_sum).  The div B
+// normalisation of the
 // reference is evaluated in x87 extended precision (global.h:505 defines
 // THIRD as a long double); here it is FP64, which leaves a few units in the
 // last place of difference per zone.
@@ -225,63 +225,131 @@ __global__ void __launch_bounds__(256) k_dg_face(const double *__restrict__ p, c
   rec[FREC - 1] = condjet2 ? 1.0 : 0.0;
 }
 
-// pdot alone (diag.c:760-1007 for pl < NPR), one thread per sum, into the
-// record of RK4 substep `stage`
-__global__ void __launch_bounds__(64) k_dg_pdot(DiagView v, int stage) {
-  int t = threadIdx.x;
-  if (t >= 6 * NPR) return;
-  int dir = t / NPR, pl = t % NPR;
-  int n = v.nface[dir];
-  const double *rec = v.face + (int64_t)v.face0[dir] * FREC;
-  double s = 0.0;
-  for (int f = 0; f < n; f++) s += rec[(int64_t)f * FREC + pl];
-  v.stage[stage * 6 * NPR + t] = s;
+// ---------------------------------------------------------------------------
+// sums in loop order
+// ---------------------------------------------------------------------------
+// One lane per sum of a direction's face records: consecutive lanes read
+// consecutive numbers of a record, and 16 records are on their way while the
+// last 16 are added.
+constexpr int FACE_AHEAD = 16;
+template <bool FLAGGED>
+__device__ __forceinline__ double face_sum(const double *__restrict__ rec, int n, int e, bool flagged) {
+  double s = 0.0, x[FACE_AHEAD], fl[FACE_AHEAD];
+  for (int f0 = 0; f0 < n; f0 += FACE_AHEAD) {
+#pragma unroll
+    for (int u = 0; u < FACE_AHEAD; u++) {
+      const int64_t at = (int64_t)(f0 + u < n ? f0 + u : n - 1) * FREC;
+      x[u] = rec[at + e];
+      if (FLAGGED) fl[u] = rec[at + FREC - 1];
+    }
+#pragma unroll
+    for (int u = 0; u < FACE_AHEAD; u++) {
+      const double t = s + x[u];
+      if (f0 + u < n && (!FLAGGED || !flagged || fl[u] != 0.0)) s = t;
+    }
+  }
+  return s;
 }
 
-// every sum by one thread in loop order
-__global__ void __launch_bounds__(1024) k_dg_sum(DiagView v, int64_t nact) {
-  int t = threadIdx.x;
-  if (t < NPR) {
-    const double *a = v.ud + (int64_t)t * nact;
-    double s = 0.0;
-    for (int64_t z = 0; z < nact; z++) s += a[z];
-    v.out[OUT_CONS + t] = s;
-  } else if (t == NPR) {
-    double mx = 0, sum = 0;
-    int64_t imx = 0;
-    for (int64_t z = 0; z < nact; z++) {
-      double dv = v.divb[z];
-      if (dv > mx) {
-        mx = dv;
-        imx = z;
+// pdot alone (diag.c:760-1007 for pl < NPR) into the record of RK4 substep
+// `stage`, one block per direction
+__global__ void __launch_bounds__(64) k_dg_pdot(DiagView v, int stage) {
+  const int dir = blockIdx.x, pl = threadIdx.x;
+  if (pl >= NPR) return;
+  v.stage[stage * 6 * NPR + dir * NPR + pl] =
+      face_sum<false>(v.face + (int64_t)v.face0[dir] * FREC, v.nface[dir], pl, false);
+}
+
+// The sum s = fl(s + x) over n numbers in order.  The chain of additions is
+// the bound, 4.45 ns each; the numbers are brought to it by the other
+// wavefronts of the block, two stretches of LDS in turn, so that it does not
+// wait for memory.  262144 numbers: 1.17 ms, where one thread that loaded and
+// added in turn took 44.  (Adding 64 at a time as integers of the sum's own
+// unit while it stays in one binade and meets no tie gives the same bits and
+// is ten times faster for sums of one sign, but the momenta and fields of a
+// torus cross binades too often: no faster on the whole, not kept.)
+constexpr int SUM_THREADS = 256, CH_N = 3072;
+__device__ double ordered_sum(const double *__restrict__ a, int64_t n) {
+  __shared__ __align__(16) double xs[2][CH_N];
+  const int wave = threadIdx.x >> 6, t = threadIdx.x - 64;
+  constexpr int LOADERS = SUM_THREADS - 64, PER = CH_N / LOADERS;
+  double s = 0.0;
+  for (int64_t base = -CH_N; base < n; base += CH_N) {
+    const int now = (int)((base / CH_N) & 1);
+    if (wave == 0) {
+      if (base >= 0) {
+        const int m = n - base < CH_N ? (int)(n - base) : CH_N;
+        const double2 *p = (const double2 *)xs[now];
+        int k = 0;
+        for (; k + 64 <= m; k += 64, p += 32) {
+          double2 v[32];
+#pragma unroll
+          for (int u = 0; u < 32; u++) v[u] = p[u];
+#pragma unroll
+          for (int u = 0; u < 32; u++) {
+            s += v[u].x;
+            s += v[u].y;
+          }
+        }
+        for (; k < m; k++) s += xs[now][k];
       }
-      sum += dv;
+    } else if (base + CH_N < n) {
+      double x[PER];
+#pragma unroll
+      for (int q = 0; q < PER; q++) {
+        const int64_t z = base + CH_N + q * LOADERS + t;
+        x[q] = z < n ? a[z] : 0.0;
+      }
+#pragma unroll
+      for (int q = 0; q < PER; q++) xs[now ^ 1][q * LOADERS + t] = x[q];
     }
-    v.out[OUT_DIVBMAX] = mx;
-    v.out[OUT_DIVBAVG] = sum / (double)nact;
-    v.out[OUT_DIVBIDX] = (double)imx;
+    __syncthreads();
+  }
+  return s;
+}
+
+// blocks 0..7 the conserved totals, 8 the sum of div B, 9 its first maximum,
+// 10..15 the faces of one direction each (120 sums: pdot, its terms, the jet's)
+constexpr int SUM_BLOCKS = NPR + 2 + 6;
+__global__ void __launch_bounds__(SUM_THREADS) k_dg_sum(DiagView v, int64_t nact) {
+  const int b = blockIdx.x, t = threadIdx.x;
+  if (b <= NPR) {
+    const double s = ordered_sum(b < NPR ? v.ud + (int64_t)b * nact : v.divb, nact);
+    if (t == 0) v.out[b < NPR ? OUT_CONS + b : OUT_DIVBAVG] = b < NPR ? s : s / (double)nact;
+  } else if (b == NPR + 1) {
+    // the first of the largest values above 0 (dump_ener.c:510: dv > max)
+    __shared__ double mx[SUM_THREADS];
+    __shared__ int64_t ix[SUM_THREADS];
+    double m = 0;
+    int64_t im = 0;
+    for (int64_t z = t; z < nact; z += SUM_THREADS) {
+      const double dv = v.divb[z];
+      if (dv > m) {
+        m = dv;
+        im = z;
+      }
+    }
+    mx[t] = m;
+    ix[t] = im;
+    for (int h = SUM_THREADS / 2; h > 0; h >>= 1) {
+      __syncthreads();
+      if (t < h && (mx[t + h] > mx[t] || (mx[t + h] == mx[t] && ix[t + h] < ix[t] && mx[t] > 0.0))) {
+        mx[t] = mx[t + h];
+        ix[t] = ix[t + h];
+      }
+    }
+    if (t == 0) {
+      v.out[OUT_DIVBMAX] = mx[0];
+      v.out[OUT_DIVBIDX] = (double)ix[0];
+    }
   } else {
-    // (dir, kind, fl, pl): kind 0 pdot, 1 terms, 2 jet2 terms
-    int u = t - (NPR + 1);
-    const int per_dir = NPR + 2 * NFLT * NPR;
-    if (u >= 6 * per_dir) return;
-    int dir = u / per_dir, w = u % per_dir;
-    int n = v.nface[dir];
-    const double *rec = v.face + (int64_t)v.face0[dir] * FREC;
-    double s = 0.0;
-    if (w < NPR) {
-      for (int f = 0; f < n; f++) s += rec[(int64_t)f * FREC + w];
-      v.out[OUT_PDOT + dir * NPR + w] = s;
-    } else if (w < NPR + NFLT * NPR) {
-      int e = w - NPR;
-      for (int f = 0; f < n; f++) s += rec[(int64_t)f * FREC + NPR + e];
-      v.out[OUT_TERMS + dir * NFLT * NPR + e] = s;
-    } else {
-      int e = w - NPR - NFLT * NPR;
-      for (int f = 0; f < n; f++)
-        if (rec[(int64_t)f * FREC + FREC - 1] != 0.0) s += rec[(int64_t)f * FREC + NPR + e];
-      v.out[OUT_JET2 + dir * NFLT * NPR + e] = s;
-    }
+    // sum w: pdot 0..7, terms 8..63, the terms again over the jet 64..119
+    const int dir = b - (NPR + 2), w = t;
+    if (w >= NPR + 2 * NFLT * NPR) return;
+    const bool jet = w >= NPR + NFLT * NPR;
+    const double s = face_sum<true>(v.face + (int64_t)v.face0[dir] * FREC, v.nface[dir], jet ? w - NFLT * NPR : w, jet);
+    v.out[w < NPR ? OUT_PDOT + dir * NPR + w
+                  : (jet ? OUT_JET2 + dir * NFLT * NPR + w - NPR - NFLT * NPR : OUT_TERMS + dir * NFLT * NPR + w - NPR)] = s;
   }
 }
 
@@ -348,7 +416,7 @@ void launch_diag_faces(hg_ctx *c, const double *prim, const double *pglob, hipSt
 
 // the pdot of RK4 substep `stage` from the faces just recorded
 void launch_diag_stage(hg_ctx *c, int stage, hipStream_t s) {
-  hipLaunchKernelGGL(k_dg_pdot, dim3(1), dim3(64), 0, s, view(c), stage);
+  hipLaunchKernelGGL(k_dg_pdot, dim3(6), dim3(64), 0, s, view(c), stage);
 }
 
 }  // namespace hg
@@ -386,7 +454,7 @@ extern "C" int hg_diagnostics(hg_ctx *c, double Dt, hg_diag *out, void *stream) 
   // the faces recorded by the last step, else those of the last fluxcalc on p
   if (!(c->dg_record && c->dg_faces_valid))
     launch_diag_faces(c, c->flux_state ? c->flux_state : c->p, c->p, s);
-  hipLaunchKernelGGL(k_dg_sum, dim3(1), dim3(1024), 0, s, v, nact);
+  hipLaunchKernelGGL(k_dg_sum, dim3(SUM_BLOCKS), dim3(SUM_THREADS), 0, s, v, nact);
   double h[OUT_N], hs[4 * 6 * NPR];
   // RK4 with recording: every substep's pdot enters pcum (advance.c:130
   // calls diag_flux with Dt = Cunew[1] dt on each of them)
