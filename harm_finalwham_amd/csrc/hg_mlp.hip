@@ -12,10 +12,12 @@
 //                   the training target log(W_solved / W_guess)
 //   k_mlp_forward   features -> prediction (MFMA; each wavefront keeps the
 //                   network in registers and runs over 16-sample tiles)
-//   k_mlp_backward  forward + backward of a 64-sample chunk on the vector
-//                   units (FP32), per-block weight gradients added to grad[]
-//   k_mlp_adam      Adam update of the FP32 weights
-//   k_mlp_refresh   BF16 copies of the hidden-layer weights
+//   k_mlp_backward  forward + backward of 16-sample tiles on the matrix cores
+//                   (BF16 forward, FP32 gradients), a partial sum of every
+//                   weight's gradient per block
+//   k_mlp_update    the partial sums added up, Adam, the BF16 copies of the
+//                   hidden-layer weights (or the gradient alone)
+//   k_mlp_refresh   the copies alone
 //   k_c2p_learned   the mixed-precision inversion (FP32 Newton, polish,
 //                   double-double primitives) from the learned start where
 //                   the network predicts a large correction and the start's
@@ -107,9 +109,10 @@ __global__ void __launch_bounds__(256) k_mlp_features(int64_t n, double gam, con
 // hidden activations enter layer 2 as BF16 (K = 64).
 // ---------------------------------------------------------------------------
 struct MlpDev {
-  const float *w;       // FP32 parameters (biases, W3, normalisation)
-  const __bf16 *w1b;    // BF16 W1 B-fragments: [nt 4][lane 64][j 8] of the K = 32 layer-1 matrix
-  const __bf16 *w2b;    // BF16 W2 B-fragments: [ks 2][nt 4][lane 64][j 8]
+  float *w;       // FP32 parameters (biases, W3, normalisation)
+  __bf16 *w1b;    // BF16 W1 B-fragments: [nt 4][lane 64][j 8] of the K = 32 layer-1 matrix
+  __bf16 *w2b;    // BF16 W2 B-fragments: [ks 2][nt 4][lane 64][j 8]
+  float *w2q;     // the BF16 W2 in FP32, [64][64]
 };
 
 // the network as one wavefront holds it: the B-fragments of both hidden
@@ -240,154 +243,228 @@ __global__ void __launch_bounds__(64) kg_mlp_forward(const GridView *__restrict_
   mlp_forward_body(n, v.lx, v.ly, m, blockIdx.x - first[g_], first[g_ + 1] - first[g_]);
 }
 
+// BF16 copies of hidden-layer weight e (its value in w1b / w2b at every place
+// of the B-fragments: layer 1 [nt][l][j] = W1x[8 q + j][16 nt + r], lane
+// l = 16 q + r, with W1x the K = 32 matrix whose rows 0..7 and 8..15 are both
+// W1, the input's hi and lo halves, and whose rows 16..31 stay zero; layer 2
+// [ks][nt][l][j] = W2[32 ks + 8 q + j][16 nt + r]) and, for the backward pass,
+// the rounded W2 in FP32
+__device__ __forceinline__ void refresh_bf16(int e, float v, const MlpDev &m) {
+  if (e < OFF_B1) {
+    const int i = e / NH, c = e % NH, nt = c >> 4, r = c & 15;
+    m.w1b[(nt * 64 + r) * 8 + i] = (__bf16)v;
+    m.w1b[(nt * 64 + 16 + r) * 8 + i] = (__bf16)v;
+  } else if (e >= OFF_W2 && e < OFF_B2) {
+    const int k = (e - OFF_W2) / NH, c = (e - OFF_W2) % NH, nt = c >> 4, r = c & 15;
+    const int ks = k >> 5, q = (k >> 3) & 3, j = k & 7;
+    m.w2b[((ks * 4 + nt) * 64 + 16 * q + r) * 8 + j] = (__bf16)v;
+    m.w2q[e - OFF_W2] = (float)(__bf16)v;
+  }
+}
+
 // ---------------------------------------------------------------------------
-// backward pass, 64 samples per block of one wavefront, FP32 on the vector
-// units.  The forward is recomputed from the same BF16-rounded weights and
-// layer inputs the matrix-core forward uses (hi + lo input, BF16 hidden
-// activations; the roundings are treated as the identity when
-// differentiating: the gradient is that of the FP32 master weights).  Activations are staged in LDS (row stride 65 floats, so both
-// per-sample rows and per-unit columns are free of bank conflicts):
-//   A  thread = sample: x, h1, h2, dy
-//   B  thread = unit j: dW3[j], dz2[s][j] in place of h2, db2[j]
-//   C  thread = sample: dz1[s][k] = (W2 dz2)[k] (1 - h1^2)
-//   D  thread = unit k: dW2[k][:], dW1[:][k], db1[k]
-// Each block adds its sums into grad[] once per parameter.
+// backward pass: a block of four wavefronts runs over tiles of 16 samples, and
+// wavefront w has columns 16 w .. 16 w + 15 of every layer.  The forward is the
+// matrix-core one (the roundings to BF16 are treated as the identity when
+// differentiating: the gradient is that of the FP32 master weights); what it
+// differentiates stays FP32, on v_mfma_f32_16x16x4_f32:
+//   dz1 = (dz2 W2^T) (1 - h1^2)   A = dz2, B = W2^T
+//   dW2 = h1^T dz2, dW1 = x^T dz1
+// A C-layout result (sample 4 q + i in lane 16 q + r, register i) is at once a
+// B operand of a product summed over the samples: step i takes sample 4 q + i
+// in slot q, and A is read from LDS in that order.  The gradients stay in
+// accumulators over the block's tiles and go out once per block, to a row of
+// partial sums of its own: sums in a fixed order, no atomics.
+// A minibatch of 2048 is 128 one-tile blocks.  One wavefront per 64 samples on
+// the vector units with an atomic per weight and block took 136 us (32 of them
+// on 1024 SIMDs), Adam and the copies two more launches of 4.7 us; now 7.5 us
+// here and 4 in k_mlp_update, most of both the launch and three or four memory
+// latencies.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ float bfr(float x) { return (float)(__bf16)x; }
 // the value a layer input carries into the matrix cores: hi + lo
 __device__ __forceinline__ float eff(float v) { return (float)bf_hi(v) + (float)bf_lo(v); }
 
-constexpr int LS = NH + 1;  // LDS row stride
+constexpr int BACK_BLOCKS = 256;              // most partial sums
+constexpr int PART = (NTRAIN + 1 + 63) / 64 * 64;  // their stride: the weights, then the loss
 
-__global__ void __launch_bounds__(64) k_mlp_backward(int64_t n, const float *__restrict__ X,
-                                                     const float *__restrict__ Y, const float *__restrict__ w,
-                                                     float inv_n, float loss_scale, float *__restrict__ grad,
-                                                     float *__restrict__ loss) {
-  __shared__ float xs[64][NIN + 1];
-  __shared__ float h1s[64][LS];
-  __shared__ float h2s[64][LS];  // h2, then dz2
-  __shared__ float d1s[64][LS];  // dz1
-  __shared__ float dys[64];
-  const int l = threadIdx.x;
-  const int64_t t = (int64_t)blockIdx.x * 64 + l;
-  const bool live = t < n;
-  // A: forward of sample l
-  {
-    float x[NIN];
+__global__ void __launch_bounds__(256) k_mlp_backward(int64_t n, const float *__restrict__ X,
+                                                      const float *__restrict__ Y, MlpDev m, float inv_n,
+                                                      float loss_scale, float *__restrict__ part) {
+  __shared__ float xs[16][NIN];
+  __shared__ float h1s[16][NH + 4], dz2s[16][NH + 4];
+  __shared__ float ys[4][16];
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6, q = l >> 4, r = l & 15;
+  const int col = 16 * w + r;
+  // thread 8 s + k (of the first 128) has feature k of sample s; a tile's
+  // samples are on their way while the weights, or the tile before, are
+  const int xs_s = threadIdx.x / NIN, xs_k = threadIdx.x % NIN;
+  float nx = 0.f, ny[4] = {0.f, 0.f, 0.f, 0.f};
+  auto fetch = [&](int64_t b) {
+    if (xs_s < 16) nx = b + xs_s < n ? X[(b + xs_s) * NIN + xs_k] : 0.f;
 #pragma unroll
-    for (int i = 0; i < NIN; i++) {
-      x[i] = live ? eff((X[t * NIN + i] - w[OFF_MU + i]) / w[OFF_SD + i]) : 0.f;
-      xs[l][i] = x[i];
-    }
-    for (int j = 0; j < NH; j++) {
-      float s = 0.f;
+    for (int i = 0; i < 4; i++) ny[i] = b + 4 * q + i < n ? Y[b + 4 * q + i] : 0.f;
+  };
+  fetch((int64_t)blockIdx.x * 16);
+  const float mu = m.w[OFF_MU + xs_k], sd = m.w[OFF_SD + xs_k];
+  const bf16x8 w1 = *(const bf16x8 *)(m.w1b + (w * 64 + l) * 8);
+  bf16x8 w2[2];
 #pragma unroll
-      for (int i = 0; i < NIN; i++) s += x[i] * bfr(w[OFF_W1 + i * NH + j]);
-      h1s[l][j] = act(s + w[OFF_B1 + j]);
+  for (int ks = 0; ks < 2; ks++) w2[ks] = *(const bf16x8 *)(m.w2b + ((4 * ks + w) * 64 + l) * 8);
+  float w2t[16];  // W2^T as the B operand of dz2 W2^T: element (4 step + q, col)
+#pragma unroll
+  for (int st = 0; st < 16; st++) w2t[st] = m.w2q[col * NH + 4 * st + q];
+  const float b1 = m.w[OFF_B1 + col], b2 = m.w[OFF_B2 + col], w3 = m.w[OFF_W3 + col], b3 = m.w[OFF_B3];
+  f32x4 gW2[4], gW1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int kt = 0; kt < 4; kt++) gW2[kt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  float gb1 = 0.f, gb2 = 0.f, gw3 = 0.f, gb3 = 0.f, loss = 0.f;
+  for (int64_t base = (int64_t)blockIdx.x * 16; base < n; base += (int64_t)gridDim.x * 16) {
+    if (xs_s < 16) xs[xs_s][xs_k] = base + xs_s < n ? (nx - mu) / sd : 0.f;
+    const float tgt[4] = {ny[0], ny[1], ny[2], ny[3]};
+    fetch(base + (int64_t)gridDim.x * 16);
+    __syncthreads();
+    // forward
+    bf16x8 a;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const float v = (q < 2) ? xs[r][j] : 0.0f;
+      a[j] = (q == 0) ? bf_hi(v) : bf_lo(v);  // q >= 2: bf16(0 - 0) = 0
     }
-    float yp = w[OFF_B3];
-    for (int j = 0; j < NH; j++) {
-      float s = 0.f;
-      for (int k = 0; k < NH; k++) s += bfr(h1s[l][k]) * bfr(w[OFF_W2 + k * NH + j]);
-      float h2 = act(s + w[OFF_B2 + j]);
-      h2s[l][j] = h2;
-      yp += h2 * w[OFF_W3 + j];
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w1, acc, 0, 0, 0);
+    float h1[4], h2[4], dz2[4], dz1[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      h1[i] = act(acc[i] + b1);
+      h1s[4 * q + i][col] = h1[i];
     }
-    float r = live ? yp - Y[t] : 0.f;
-    dys[l] = 2.f * r * inv_n;
-    float lsum = r * r * loss_scale;
-    for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o);
-    if (l == 0) atomicAdd(loss, lsum);
+    __syncthreads();
+    f32x4 acc2 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) {
+      bf16x8 a2;
+#pragma unroll
+      for (int j = 0; j < 8; j++) a2[j] = bf_hi(h1s[r][32 * ks + 8 * q + j]);
+      acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, w2[ks], acc2, 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      h2[i] = act(acc2[i] + b2);
+      float p = h2[i] * w3;
+#pragma unroll
+      for (int off = 8; off >= 1; off >>= 1) p += __shfl_xor(p, off, 64);
+      if (r == 0) ys[w][4 * q + i] = p;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int s = 4 * q + i;
+      const float y = b3 + ((ys[0][s] + ys[1][s]) + (ys[2][s] + ys[3][s]));
+      const float res = base + s < n ? y - tgt[i] : 0.f;
+      const float dy = 2.f * res * inv_n;
+      loss += res * res * loss_scale;
+      gb3 += dy;
+      gw3 += dy * h2[i];
+      dz2[i] = dy * w3 * (1.f - h2[i] * h2[i]);
+      gb2 += dz2[i];
+      dz2s[s][col] = dz2[i];
+    }
+    __syncthreads();
+    // dz1 of columns col
+    f32x4 dh = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int st = 0; st < 16; st++)
+      dh = __builtin_amdgcn_mfma_f32_16x16x4f32(dz2s[r][4 * st + q], w2t[st], dh, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      dz1[i] = dh[i] * (1.f - h1[i] * h1[i]);
+      gb1 += dz1[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const float x = r < NIN ? eff(xs[4 * q + i][r & 7]) : 0.f;
+      gW1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x, dz1[i], gW1, 0, 0, 0);
+#pragma unroll
+      for (int kt = 0; kt < 4; kt++)
+        gW2[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)bf_hi(h1s[4 * q + i][16 * kt + r]), dz2[i], gW2[kt], 0, 0, 0);
+    }
+    __syncthreads();
   }
-  __syncthreads();
-  // B: unit j = l of layer 3 / layer 2 output
-  {
-    const int j = l;
-    const float w3 = w[OFF_W3 + j];
-    float gw3 = 0.f, gb2 = 0.f;
-    for (int s = 0; s < 64; s++) {
-      float h2 = h2s[s][j], dy = dys[s];
-      gw3 += dy * h2;
-      float dz2 = dy * w3 * (1.f - h2 * h2);
-      h2s[s][j] = dz2;
-      gb2 += dz2;
-    }
-    atomicAdd(&grad[OFF_W3 + j], gw3);
-    atomicAdd(&grad[OFF_B2 + j], gb2);
-    if (l == 0) {
-      float gb3 = 0.f;
-      for (int s = 0; s < 64; s++) gb3 += dys[s];
-      atomicAdd(&grad[OFF_B3], gb3);
-    }
+  // out: C layout, row 4 q + i of a 16-row tile, column col
+  float *g = part + (int64_t)blockIdx.x * PART;
+#pragma unroll
+  for (int kt = 0; kt < 4; kt++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) g[OFF_W2 + (16 * kt + 4 * q + i) * NH + col] = gW2[kt][i];
+  if (q < NIN / 4)
+#pragma unroll
+    for (int i = 0; i < 4; i++) g[OFF_W1 + (4 * q + i) * NH + col] = gW1[i];
+#pragma unroll
+  for (int off = 16; off <= 32; off <<= 1) {
+    gb1 += __shfl_xor(gb1, off, 64);
+    gb2 += __shfl_xor(gb2, off, 64);
+    gw3 += __shfl_xor(gw3, off, 64);
+    gb3 += __shfl_xor(gb3, off, 64);
+    loss += __shfl_xor(loss, off, 64);
   }
-  __syncthreads();
-  // C: sample l, back through W2 and the first tanh
-  for (int k = 0; k < NH; k++) {
-    float dh = 0.f;
-    for (int j = 0; j < NH; j++) dh += bfr(w[OFF_W2 + k * NH + j]) * h2s[l][j];
-    float h1 = h1s[l][k];
-    d1s[l][k] = dh * (1.f - h1 * h1);
-  }
-  __syncthreads();
-  // D: unit k = l of the first hidden layer
-  {
-    const int k = l;
-    float g2[NH];
-#pragma unroll
-    for (int j = 0; j < NH; j++) g2[j] = 0.f;
-    float g1[NIN];
-#pragma unroll
-    for (int i = 0; i < NIN; i++) g1[i] = 0.f;
-    float gb1 = 0.f;
-    for (int s = 0; s < 64; s++) {
-      float hk = bfr(h1s[s][k]);
-#pragma unroll
-      for (int j = 0; j < NH; j++) g2[j] += hk * h2s[s][j];
-      float dz1 = d1s[s][k];
-      gb1 += dz1;
-#pragma unroll
-      for (int i = 0; i < NIN; i++) g1[i] += xs[s][i] * dz1;
+  if (q == 0) {
+    g[OFF_B1 + col] = gb1;
+    g[OFF_B2 + col] = gb2;
+    g[OFF_W3 + col] = gw3;
+    if (threadIdx.x == 0) {
+      g[OFF_B3] = gb3;
+      g[NTRAIN] = loss;
     }
-#pragma unroll
-    for (int j = 0; j < NH; j++) atomicAdd(&grad[OFF_W2 + k * NH + j], g2[j]);
-#pragma unroll
-    for (int i = 0; i < NIN; i++) atomicAdd(&grad[OFF_W1 + i * NH + k], g1[i]);
-    atomicAdd(&grad[OFF_B1 + k], gb1);
   }
 }
 
-// BF16 B-fragments of the hidden layers for lane l = 16 q + r, element j:
-// layer 1 [nt][l][j] = W1x[8 q + j][16 nt + r] with W1x the K = 32 matrix
-// whose rows 0..7 and 8..15 are both W1 (the input's hi and lo halves) and
-// rows 16..31 zero; layer 2 [ks][nt][l][j] = W2[32 ks + 8 q + j][16 nt + r]
-__device__ __forceinline__ void refresh_bf16(int e, const float *w, __bf16 *w1b, __bf16 *w2b) {
-  const int j = e & 7, l = (e >> 3) & 63, q = l >> 4, r = l & 15;
-  if (e < 4 * 64 * 8) {
-    const int nt = e >> 9, row = 8 * q + j;
-    w1b[e] = (row < 2 * NIN) ? (__bf16)w[OFF_W1 + (row % NIN) * NH + 16 * nt + r] : (__bf16)0.0f;
+// the nb partial sums of weight e added in a fixed order, eight threads a weight
+// (128 sums are then one round of loads);
+// ADAM: the step and the weight's BF16 copies, else the gradient into grad[].
+// The last number is the loss, added to *loss (first: in its place).
+constexpr int UPDATE_WAYS = 8;
+template <bool ADAM>
+__global__ void __launch_bounds__(64 * UPDATE_WAYS) k_mlp_update(MlpDev m, const float *__restrict__ part, int nb, float lr,
+                                                    float b1t, float b2t, int first, float *__restrict__ m1,
+                                                    float *__restrict__ m2, float *__restrict__ grad,
+                                                    float *__restrict__ loss) {
+  __shared__ float sum[UPDATE_WAYS][64];
+  const int c = threadIdx.x & 63, w = threadIdx.x >> 6, e = blockIdx.x * 64 + c;
+  float s = 0.f;
+  if (e <= NTRAIN) {
+    for (int b = w; b < nb; b += 16 * UPDATE_WAYS) {
+      float v[16];
+#pragma unroll
+      for (int u = 0; u < 16; u++)
+        v[u] = b + u * UPDATE_WAYS < nb ? part[(int64_t)(b + u * UPDATE_WAYS) * PART + e] : 0.f;
+#pragma unroll
+      for (int u = 0; u < 16; u++) s += v[u];
+    }
   }
-  if (e < 8 * 64 * 8) {
-    const int f = e >> 9, ks = f >> 2, nt = f & 3;
-    w2b[e] = (__bf16)w[OFF_W2 + (32 * ks + 8 * q + j) * NH + 16 * nt + r];
-  }
-}
-
-__global__ void k_mlp_adam(float *__restrict__ w, float *__restrict__ g, float *__restrict__ m1,
-                           float *__restrict__ m2, float lr, float b1t, float b2t) {
-  int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < NTRAIN) {
+  sum[w][c] = s;
+  __syncthreads();
+  if (w != 0 || e > NTRAIN) return;
+  float gi = 0.f;
+#pragma unroll
+  for (int u = 0; u < UPDATE_WAYS; u++) gi += sum[u][c];
+  if (e == NTRAIN) {
+    *loss = first ? gi : *loss + gi;
+  } else if (ADAM) {
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    float gi = g[e];
     m1[e] = b1 * m1[e] + (1.f - b1) * gi;
     m2[e] = b2 * m2[e] + (1.f - b2) * gi * gi;
     float mh = m1[e] / (1.f - b1t), vh = m2[e] / (1.f - b2t);
-    w[e] -= lr * mh / (sqrtf(vh) + eps);
-    g[e] = 0.f;
+    const float v = m.w[e] - lr * mh / (sqrtf(vh) + eps);
+    m.w[e] = v;
+    refresh_bf16(e, v, m);
+  } else {
+    grad[e] = gi;
   }
 }
 
-__global__ void k_mlp_refresh(const float *__restrict__ w, __bf16 *__restrict__ w1b, __bf16 *__restrict__ w2b) {
-  refresh_bf16(blockIdx.x * blockDim.x + threadIdx.x, w, w1b, w2b);
+__global__ void k_mlp_refresh(MlpDev m) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < NTRAIN) refresh_bf16(e, m.w[e], m);
 }
 
 // ---------------------------------------------------------------------------
@@ -463,14 +540,24 @@ __global__ void __launch_bounds__(64) k_c2p_learned(int64_t n, double gam, const
 
 }  // namespace
 
+// one allocation holds everything: parameters, gradient, Adam moments, the
+// BF16 copies, the loss, the counts and the partial sums of the backward pass
 struct hg_mlp {
-  float *w = nullptr, *g = nullptr, *m1 = nullptr, *m2 = nullptr, *loss = nullptr;
+  void *mem = nullptr;
+  float *w = nullptr, *g = nullptr, *m1 = nullptr, *m2 = nullptr, *loss = nullptr, *w2q = nullptr, *part = nullptr;
   __bf16 *w1b = nullptr, *w2b = nullptr;
   unsigned long long *counts = nullptr;  // [learned starts, fallbacks]
   int step = 0;
 };
 
-static MlpDev dev_view(const hg_mlp *m) { return MlpDev{m->w, m->w1b, m->w2b}; }
+static MlpDev dev_view(const hg_mlp *m) { return MlpDev{m->w, m->w1b, m->w2b, m->w2q}; }
+
+// blocks of the backward pass: one per 16-sample tile up to BACK_BLOCKS
+static unsigned backward_blocks(int64_t n) {
+  const int64_t tiles = (n + 15) / 16;
+  return (unsigned)(tiles < BACK_BLOCKS ? tiles : BACK_BLOCKS);
+}
+constexpr unsigned UPDATE_BLOCKS = (NTRAIN + 1 + 63) / 64;
 
 // the forward kernel's one-wavefront blocks: one per 16-sample tile up to
 // 8192 (32 per CU), each then loops over its share of the tiles
@@ -490,9 +577,7 @@ static unsigned forward_blocks(int64_t n) {
 
 extern "C" int hg_mlp_destroy(hg_mlp *m) {
   if (!m) return 0;
-  void *b[] = {m->w, m->g, m->m1, m->m2, m->loss, m->w1b, m->w2b, m->counts};
-  for (void *p : b)
-    if (p) (void)hipFree(p);
+  if (m->mem) (void)hipFree(m->mem);
   delete m;
   return 0;
 }
@@ -513,25 +598,38 @@ extern "C" int hg_mlp_create(uint64_t seed, hg_mlp **out) {
   for (int e = 0; e < NH * NH; e++) w[OFF_W2 + e] = (float)(a2 * (2 * uni() - 1));
   for (int e = 0; e < NH; e++) w[OFF_W3 + e] = (float)(a3 * (2 * uni() - 1));
   for (int k = 0; k < NIN; k++) w[OFF_SD + k] = 1.f;
-  hipError_t e = hipMalloc((void **)&m->w, NPARAM * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc((void **)&m->g, NPARAM * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc((void **)&m->m1, NPARAM * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc((void **)&m->m2, NPARAM * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc((void **)&m->loss, sizeof(float));
-  if (e == hipSuccess) e = hipMalloc((void **)&m->w1b, 32 * NH * sizeof(__bf16));
-  if (e == hipSuccess) e = hipMalloc((void **)&m->w2b, NH * NH * sizeof(__bf16));
-  if (e == hipSuccess) e = hipMalloc((void **)&m->counts, 2 * sizeof(unsigned long long));
-  if (e == hipSuccess) e = hipMemcpy(m->w, w.data(), NPARAM * sizeof(float), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemset(m->g, 0, NPARAM * sizeof(float));
-  if (e == hipSuccess) e = hipMemset(m->m1, 0, NPARAM * sizeof(float));
-  if (e == hipSuccess) e = hipMemset(m->m2, 0, NPARAM * sizeof(float));
-  if (e != hipSuccess) {
-    set_error("hg_mlp_create: %s", hipGetErrorString(e));
-    hg_mlp_destroy(m);
-    return 1;
+  // what starts as zero first
+  const size_t np = (NPARAM + 63) / 64 * 64;
+  size_t at = 0;
+  auto take = [&at](size_t bytes) {
+    const size_t here = at;
+    at += (bytes + 255) / 256 * 256;
+    return here;
+  };
+  const size_t o_g = take(np * 4), o_m1 = take(np * 4), o_m2 = take(np * 4), o_w1b = take(32 * NH * sizeof(__bf16)),
+               o_w2b = take(NH * NH * sizeof(__bf16)), o_loss = take(sizeof(float)),
+               o_counts = take(2 * sizeof(unsigned long long)), zeroed = at, o_w = take(np * 4),
+               o_w2q = take(NH * NH * sizeof(float)), o_part = take((size_t)BACK_BLOCKS * PART * sizeof(float));
+  hipError_t e = hipMalloc(&m->mem, at);
+  if (e == hipSuccess) {
+    char *b = (char *)m->mem;
+    m->g = (float *)(b + o_g);
+    m->m1 = (float *)(b + o_m1);
+    m->m2 = (float *)(b + o_m2);
+    m->w1b = (__bf16 *)(b + o_w1b);
+    m->w2b = (__bf16 *)(b + o_w2b);
+    m->loss = (float *)(b + o_loss);
+    m->counts = (unsigned long long *)(b + o_counts);
+    m->w = (float *)(b + o_w);
+    m->w2q = (float *)(b + o_w2q);
+    m->part = (float *)(b + o_part);
+    e = hipMemset(m->mem, 0, zeroed);
   }
-  hipLaunchKernelGGL(k_mlp_refresh, dim3((NH * NH + 255) / 256), dim3(256), 0, 0, m->w, m->w1b, m->w2b);
-  e = hipDeviceSynchronize();
+  if (e == hipSuccess) e = hipMemcpy(m->w, w.data(), NPARAM * sizeof(float), hipMemcpyHostToDevice);
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL(k_mlp_refresh, dim3((NTRAIN + 255) / 256), dim3(256), 0, 0, dev_view(m));
+    e = hipDeviceSynchronize();
+  }
   if (e != hipSuccess) {
     set_error("hg_mlp_create: %s", hipGetErrorString(e));
     hg_mlp_destroy(m);
@@ -554,7 +652,7 @@ extern "C" int hg_mlp_set_params(hg_mlp *m, const float *host) {
   for (int k = 0; k < NIN; k++)
     if (!(host[OFF_SD + k] > 0.f)) { set_error("hg_mlp_set_params: feature scales must be > 0"); return 1; }
   MLPCHECK(hipMemcpy(m->w, host, NPARAM * sizeof(float), hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(k_mlp_refresh, dim3((NH * NH + 255) / 256), dim3(256), 0, 0, m->w, m->w1b, m->w2b);
+  hipLaunchKernelGGL(k_mlp_refresh, dim3((NTRAIN + 255) / 256), dim3(256), 0, 0, dev_view(m));
   MLPCHECK(hipGetLastError());
   MLPCHECK(hipDeviceSynchronize());
   return 0;
@@ -607,15 +705,15 @@ extern "C" int hg_mlp_gradient(hg_mlp *m, int64_t n, const float *X, const float
                                float *loss, void *stream) {
   if (!m || n <= 0 || !X || !Y) { set_error("hg_mlp_gradient: bad arguments"); return 1; }
   hipStream_t s = (hipStream_t)stream;
-  MLPCHECK(hipMemsetAsync(m->g, 0, NPARAM * sizeof(float), s));
-  MLPCHECK(hipMemsetAsync(m->loss, 0, sizeof(float), s));
-  hipLaunchKernelGGL(k_mlp_backward, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, s, n, X, Y, m->w,
-                     (float)(1.0 / (double)n), (float)(1.0 / (double)n), m->g, m->loss);
+  const unsigned nb = backward_blocks(n);
+  hipLaunchKernelGGL(k_mlp_backward, dim3(nb), dim3(256), 0, s, n, X, Y, dev_view(m), (float)(1.0 / (double)n),
+                     (float)(1.0 / (double)n), m->part);
+  hipLaunchKernelGGL(k_mlp_update<false>, dim3(UPDATE_BLOCKS), dim3(64 * UPDATE_WAYS), 0, s, dev_view(m), (const float *)m->part,
+                     (int)nb, 0.f, 0.f, 0.f, 1, m->m1, m->m2, m->g, m->loss);
   MLPCHECK(hipGetLastError());
   MLPCHECK(hipStreamSynchronize(s));
   if (grad_host) MLPCHECK(hipMemcpy(grad_host, m->g, NPARAM * sizeof(float), hipMemcpyDeviceToHost));
   if (loss) MLPCHECK(hipMemcpy(loss, m->loss, sizeof(float), hipMemcpyDeviceToHost));
-  MLPCHECK(hipMemset(m->g, 0, NPARAM * sizeof(float)));
   return 0;
 }
 
@@ -631,17 +729,16 @@ extern "C" int hg_mlp_train(hg_mlp *m, int64_t n, const float *X, const float *Y
   int64_t nb = (n + batch - 1) / batch;
   float last = 0.f;
   for (int ep = 0; ep < epochs; ep++) {
-    MLPCHECK(hipMemsetAsync(m->loss, 0, sizeof(float), s));
     for (int64_t b = 0; b < nb; b++) {
       int64_t off = b * batch, cnt = (off + batch <= n) ? batch : n - off;
-      hipLaunchKernelGGL(k_mlp_backward, dim3((unsigned)((cnt + 63) / 64)), dim3(64), 0, s, cnt,
-                         X + off * NIN, Y + off, m->w, (float)(1.0 / (double)cnt),
-                         (float)(1.0 / (double)cnt / (double)nb), m->g, m->loss);
+      const unsigned blocks = backward_blocks(cnt);
+      hipLaunchKernelGGL(k_mlp_backward, dim3(blocks), dim3(256), 0, s, cnt, X + off * NIN, Y + off, dev_view(m),
+                         (float)(1.0 / (double)cnt), (float)(1.0 / (double)cnt / (double)nb), m->part);
       m->step++;
       float b1t = powf(0.9f, (float)m->step), b2t = powf(0.999f, (float)m->step);
-      hipLaunchKernelGGL(k_mlp_adam, dim3((NTRAIN + 255) / 256), dim3(256), 0, s, m->w, m->g, m->m1, m->m2, lr,
-                         b1t, b2t);
-      hipLaunchKernelGGL(k_mlp_refresh, dim3((NH * NH + 255) / 256), dim3(256), 0, s, m->w, m->w1b, m->w2b);
+      hipLaunchKernelGGL(k_mlp_update<true>, dim3(UPDATE_BLOCKS), dim3(64 * UPDATE_WAYS), 0, s, dev_view(m),
+                         (const float *)m->part, (int)blocks, lr, b1t, b2t, b == 0 ? 1 : 0, m->m1, m->m2, m->g,
+                         m->loss);
     }
     MLPCHECK(hipGetLastError());
     MLPCHECK(hipMemcpyAsync(&last, m->loss, sizeof(float), hipMemcpyDeviceToHost, s));
