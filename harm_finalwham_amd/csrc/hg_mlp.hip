@@ -13,8 +13,8 @@
 //   k_mlp_forward   features -> prediction (MFMA; each wavefront keeps the
 //                   network in registers and runs over 16-sample tiles)
 //   k_mlp_backward  forward + backward of 16-sample tiles on the matrix cores
-//                   (BF16 forward, FP32 gradients), a partial sum of every
-//                   weight's gradient per block
+//                   (FP64, with the BF16 roundings of the inference), a partial
+//                   sum of every weight's gradient per block
 //   k_mlp_update    the partial sums added up, Adam, the BF16 copies of the
 //                   hidden-layer weights (or the gradient alone)
 //   k_mlp_refresh   the copies alone
@@ -28,6 +28,8 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <cstdio>
+#include <cstdlib>
 #include <vector>
 
 #include "harmgpu.h"
@@ -113,6 +115,7 @@ struct MlpDev {
   __bf16 *w1b;    // BF16 W1 B-fragments: [nt 4][lane 64][j 8] of the K = 32 layer-1 matrix
   __bf16 *w2b;    // BF16 W2 B-fragments: [ks 2][nt 4][lane 64][j 8]
   float *w2q;     // the BF16 W2 in FP32, [64][64]
+  float *wlo;     // what the FP32 parameters round off of the trained ones
 };
 
 // the network as one wavefront holds it: the B-fragments of both hidden
@@ -264,35 +267,44 @@ __device__ __forceinline__ void refresh_bf16(int e, float v, const MlpDev &m) {
 
 // ---------------------------------------------------------------------------
 // backward pass: a block of four wavefronts runs over tiles of 16 samples, and
-// wavefront w has columns 16 w .. 16 w + 15 of every layer.  The forward is the
-// matrix-core one (the roundings to BF16 are treated as the identity when
-// differentiating: the gradient is that of the FP32 master weights); what it
-// differentiates stays FP32, on v_mfma_f32_16x16x4_f32:
-//   dz1 = (dz2 W2^T) (1 - h1^2)   A = dz2, B = W2^T
-//   dW2 = h1^T dz2, dW1 = x^T dz1
-// A C-layout result (sample 4 q + i in lane 16 q + r, register i) is at once a
-// B operand of a product summed over the samples: step i takes sample 4 q + i
-// in slot q, and A is read from LDS in that order.  The gradients stay in
-// accumulators over the block's tiles and go out once per block, to a row of
-// partial sums of its own: sums in a fixed order, no atomics.
+// wavefront w has columns 16 w .. 16 w + 15 of every layer.  The forward is
+// recomputed with the BF16-rounded weights and layer inputs of the inference
+// (hi + lo input, BF16 hidden activations; the roundings are treated as the
+// identity when differentiating: the gradient is that of the master weights),
+// and all arithmetic is FP64 on v_mfma_f64_16x16x4_f64:
+//   z2 = h1 W2, dz1 = (dz2 W2^T) (1 - h1^2), dW2 = h1^T dz2, dW1 = x^T dz1
+// A hidden activation or weight then rounds to the BF16 number of the exact
+// computation, where FP32 sums land on the other side now and then and Adam
+// carries that on: two epochs of 128 minibatches end 1.7e-8 from 64-bit
+// training (the parameters' own FP32 rounding), in FP32 4e-4.  It costs 3 us a
+// minibatch of 2048, the block being bound by its launch and a few memory
+// latencies more than by its products.  A C-layout result (sample 4 i + q in lane 16 q + r, register i) is at
+// once a B operand of a product summed over the samples: step i takes sample
+// 4 i + q in slot q, and A is read from LDS in that order.  The gradients stay
+// in accumulators over the block's tiles and go out once per block, to a row
+// of partial sums of its own: sums in a fixed order, no atomics.
 // A minibatch of 2048 is 128 one-tile blocks.  One wavefront per 64 samples on
 // the vector units with an atomic per weight and block took 136 us (32 of them
-// on 1024 SIMDs), Adam and the copies two more launches of 4.7 us; now 7.5 us
-// here and 4 in k_mlp_update, most of both the launch and three or four memory
-// latencies.
+// on 1024 SIMDs), Adam and the copies two more launches of 4.7 us; now 10.8 us
+// here and 4.6 in k_mlp_update.
 // ---------------------------------------------------------------------------
-// the value a layer input carries into the matrix cores: hi + lo
-__device__ __forceinline__ float eff(float v) { return (float)bf_hi(v) + (float)bf_lo(v); }
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-constexpr int BACK_BLOCKS = 256;              // most partial sums
+// the value a layer input carries into the matrix cores: hi + lo
+__device__ __forceinline__ double eff(double v) {
+  const float hi = (float)bf_hi((float)v);
+  return (double)hi + (double)(float)bf_hi((float)(v - (double)hi));
+}
+__device__ __forceinline__ double act64(double x) { return 1.0 - 2.0 / (exp(2.0 * x) + 1.0); }
+
+constexpr int BACK_BLOCKS = 256;                   // most partial sums
 constexpr int PART = (NTRAIN + 1 + 63) / 64 * 64;  // their stride: the weights, then the loss
 
 __global__ void __launch_bounds__(256) k_mlp_backward(int64_t n, const float *__restrict__ X,
-                                                      const float *__restrict__ Y, MlpDev m, float inv_n,
-                                                      float loss_scale, float *__restrict__ part) {
-  __shared__ float xs[16][NIN];
-  __shared__ float h1s[16][NH + 4], dz2s[16][NH + 4];
-  __shared__ float ys[4][16];
+                                                      const float *__restrict__ Y, MlpDev m, double inv_n,
+                                                      double loss_scale, double *__restrict__ part) {
+  __shared__ double xs[16][NIN], dz2s[16][NH + 1], ys[4][16];
+  __shared__ float h1q[16][NH + 4];
   const int l = threadIdx.x & 63, w = threadIdx.x >> 6, q = l >> 4, r = l & 15;
   const int col = 16 * w + r;
   // thread 8 s + k (of the first 128) has feature k of sample s; a tile's
@@ -302,103 +314,94 @@ __global__ void __launch_bounds__(256) k_mlp_backward(int64_t n, const float *__
   auto fetch = [&](int64_t b) {
     if (xs_s < 16) nx = b + xs_s < n ? X[(b + xs_s) * NIN + xs_k] : 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; i++) ny[i] = b + 4 * q + i < n ? Y[b + 4 * q + i] : 0.f;
+    for (int i = 0; i < 4; i++) ny[i] = b + 4 * i + q < n ? Y[b + 4 * i + q] : 0.f;
   };
   fetch((int64_t)blockIdx.x * 16);
-  const float mu = m.w[OFF_MU + xs_k], sd = m.w[OFF_SD + xs_k];
-  const bf16x8 w1 = *(const bf16x8 *)(m.w1b + (w * 64 + l) * 8);
-  bf16x8 w2[2];
+  const double mu = m.w[OFF_MU + xs_k], sd = m.w[OFF_SD + xs_k];
+  const bf16x8 w1 = *(const bf16x8 *)(m.w1b + (w * 64 + r) * 8);  // rows 0..7 of column col
+  float w2[16], w2t[16];  // W2 and W2^T as B operands: elements (4 step + q, col)
 #pragma unroll
-  for (int ks = 0; ks < 2; ks++) w2[ks] = *(const bf16x8 *)(m.w2b + ((4 * ks + w) * 64 + l) * 8);
-  float w2t[16];  // W2^T as the B operand of dz2 W2^T: element (4 step + q, col)
+  for (int st = 0; st < 16; st++) {
+    w2[st] = m.w2q[(4 * st + q) * NH + col];
+    w2t[st] = m.w2q[col * NH + 4 * st + q];
+  }
+  auto par = [&](int e) { return (double)m.w[e] + (double)m.wlo[e]; };
+  const double b1 = par(OFF_B1 + col), b2 = par(OFF_B2 + col), w3 = par(OFF_W3 + col), b3 = par(OFF_B3);
+  f64x4 gW2[4], gW1 = {0., 0., 0., 0.};
 #pragma unroll
-  for (int st = 0; st < 16; st++) w2t[st] = m.w2q[col * NH + 4 * st + q];
-  const float b1 = m.w[OFF_B1 + col], b2 = m.w[OFF_B2 + col], w3 = m.w[OFF_W3 + col], b3 = m.w[OFF_B3];
-  f32x4 gW2[4], gW1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int kt = 0; kt < 4; kt++) gW2[kt] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  float gb1 = 0.f, gb2 = 0.f, gw3 = 0.f, gb3 = 0.f, loss = 0.f;
+  for (int kt = 0; kt < 4; kt++) gW2[kt] = (f64x4){0., 0., 0., 0.};
+  double gb1 = 0., gb2 = 0., gw3 = 0., gb3 = 0., loss = 0.;
   for (int64_t base = (int64_t)blockIdx.x * 16; base < n; base += (int64_t)gridDim.x * 16) {
-    if (xs_s < 16) xs[xs_s][xs_k] = base + xs_s < n ? (nx - mu) / sd : 0.f;
+    if (xs_s < 16) xs[xs_s][xs_k] = base + xs_s < n ? eff(((double)nx - mu) / sd) : 0.;
     const float tgt[4] = {ny[0], ny[1], ny[2], ny[3]};
     fetch(base + (int64_t)gridDim.x * 16);
     __syncthreads();
     // forward
-    bf16x8 a;
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const float v = (q < 2) ? xs[r][j] : 0.0f;
-      a[j] = (q == 0) ? bf_hi(v) : bf_lo(v);  // q >= 2: bf16(0 - 0) = 0
-    }
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w1, acc, 0, 0, 0);
-    float h1[4], h2[4], dz2[4], dz1[4];
+    double h1[4], h2[4], dz2[4], dz1[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      h1[i] = act(acc[i] + b1);
-      h1s[4 * q + i][col] = h1[i];
+      double z = b1;
+#pragma unroll
+      for (int k = 0; k < NIN; k++) z = fma(xs[4 * i + q][k], (double)w1[k], z);
+      h1[i] = act64(z);
+      h1q[4 * i + q][col] = (float)bf_hi((float)h1[i]);
     }
     __syncthreads();
-    f32x4 acc2 = {0.f, 0.f, 0.f, 0.f};
+    f64x4 z2 = {b2, b2, b2, b2};
 #pragma unroll
-    for (int ks = 0; ks < 2; ks++) {
-      bf16x8 a2;
-#pragma unroll
-      for (int j = 0; j < 8; j++) a2[j] = bf_hi(h1s[r][32 * ks + 8 * q + j]);
-      acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, w2[ks], acc2, 0, 0, 0);
-    }
+    for (int st = 0; st < 16; st++)
+      z2 = __builtin_amdgcn_mfma_f64_16x16x4f64((double)h1q[r][4 * st + q], (double)w2[st], z2, 0, 0, 0);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      h2[i] = act(acc2[i] + b2);
-      float p = h2[i] * w3;
+      h2[i] = act64(z2[i]);
+      double p = h2[i] * w3;
 #pragma unroll
       for (int off = 8; off >= 1; off >>= 1) p += __shfl_xor(p, off, 64);
-      if (r == 0) ys[w][4 * q + i] = p;
+      if (r == 0) ys[w][4 * i + q] = p;
     }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const int s = 4 * q + i;
-      const float y = b3 + ((ys[0][s] + ys[1][s]) + (ys[2][s] + ys[3][s]));
-      const float res = base + s < n ? y - tgt[i] : 0.f;
-      const float dy = 2.f * res * inv_n;
+      const int s = 4 * i + q;
+      const double y = b3 + ((ys[0][s] + ys[1][s]) + (ys[2][s] + ys[3][s]));
+      const double res = base + s < n ? y - (double)tgt[i] : 0.;
+      const double dy = 2. * res * inv_n;
       loss += res * res * loss_scale;
       gb3 += dy;
       gw3 += dy * h2[i];
-      dz2[i] = dy * w3 * (1.f - h2[i] * h2[i]);
+      dz2[i] = dy * w3 * (1. - h2[i] * h2[i]);
       gb2 += dz2[i];
       dz2s[s][col] = dz2[i];
     }
     __syncthreads();
     // dz1 of columns col
-    f32x4 dh = {0.f, 0.f, 0.f, 0.f};
+    f64x4 dh = {0., 0., 0., 0.};
 #pragma unroll
     for (int st = 0; st < 16; st++)
-      dh = __builtin_amdgcn_mfma_f32_16x16x4f32(dz2s[r][4 * st + q], w2t[st], dh, 0, 0, 0);
+      dh = __builtin_amdgcn_mfma_f64_16x16x4f64(dz2s[r][4 * st + q], (double)w2t[st], dh, 0, 0, 0);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      dz1[i] = dh[i] * (1.f - h1[i] * h1[i]);
+      dz1[i] = dh[i] * (1. - h1[i] * h1[i]);
       gb1 += dz1[i];
     }
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const float x = r < NIN ? eff(xs[4 * q + i][r & 7]) : 0.f;
-      gW1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x, dz1[i], gW1, 0, 0, 0);
+      const double x = r < NIN ? xs[4 * i + q][r & 7] : 0.;
+      gW1 = __builtin_amdgcn_mfma_f64_16x16x4f64(x, dz1[i], gW1, 0, 0, 0);
 #pragma unroll
       for (int kt = 0; kt < 4; kt++)
-        gW2[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)bf_hi(h1s[4 * q + i][16 * kt + r]), dz2[i], gW2[kt], 0, 0, 0);
+        gW2[kt] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)h1q[4 * i + q][16 * kt + r], dz2[i], gW2[kt], 0, 0, 0);
     }
     __syncthreads();
   }
-  // out: C layout, row 4 q + i of a 16-row tile, column col
-  float *g = part + (int64_t)blockIdx.x * PART;
+  // out: C layout, row 4 i + q of a 16-row tile, column col
+  double *g = part + (int64_t)blockIdx.x * PART;
 #pragma unroll
   for (int kt = 0; kt < 4; kt++)
 #pragma unroll
-    for (int i = 0; i < 4; i++) g[OFF_W2 + (16 * kt + 4 * q + i) * NH + col] = gW2[kt][i];
-  if (q < NIN / 4)
+    for (int i = 0; i < 4; i++) g[OFF_W2 + (16 * kt + 4 * i + q) * NH + col] = gW2[kt][i];
 #pragma unroll
-    for (int i = 0; i < 4; i++) g[OFF_W1 + (4 * q + i) * NH + col] = gW1[i];
+  for (int i = 0; i < NIN / 4; i++) g[OFF_W1 + (4 * i + q) * NH + col] = gW1[i];
 #pragma unroll
   for (int off = 16; off <= 32; off <<= 1) {
     gb1 += __shfl_xor(gb1, off, 64);
@@ -424,19 +427,20 @@ __global__ void __launch_bounds__(256) k_mlp_backward(int64_t n, const float *__
 // The last number is the loss, added to *loss (first: in its place).
 constexpr int UPDATE_WAYS = 8;
 template <bool ADAM>
-__global__ void __launch_bounds__(64 * UPDATE_WAYS) k_mlp_update(MlpDev m, const float *__restrict__ part, int nb, float lr,
-                                                    float b1t, float b2t, int first, float *__restrict__ m1,
-                                                    float *__restrict__ m2, float *__restrict__ grad,
-                                                    float *__restrict__ loss) {
-  __shared__ float sum[UPDATE_WAYS][64];
+__global__ void __launch_bounds__(64 * UPDATE_WAYS) k_mlp_update(MlpDev m, const double *__restrict__ part, int nb,
+                                                                 double lr, double b1t, double b2t, int first,
+                                                                 double *__restrict__ m1, double *__restrict__ m2,
+                                                                 float *__restrict__ grad,
+                                                                 double *__restrict__ loss) {
+  __shared__ double sum[UPDATE_WAYS][64];
   const int c = threadIdx.x & 63, w = threadIdx.x >> 6, e = blockIdx.x * 64 + c;
-  float s = 0.f;
+  double s = 0.;
   if (e <= NTRAIN) {
     for (int b = w; b < nb; b += 16 * UPDATE_WAYS) {
-      float v[16];
+      double v[16];
 #pragma unroll
       for (int u = 0; u < 16; u++)
-        v[u] = b + u * UPDATE_WAYS < nb ? part[(int64_t)(b + u * UPDATE_WAYS) * PART + e] : 0.f;
+        v[u] = b + u * UPDATE_WAYS < nb ? part[(int64_t)(b + u * UPDATE_WAYS) * PART + e] : 0.;
 #pragma unroll
       for (int u = 0; u < 16; u++) s += v[u];
     }
@@ -444,27 +448,33 @@ __global__ void __launch_bounds__(64 * UPDATE_WAYS) k_mlp_update(MlpDev m, const
   sum[w][c] = s;
   __syncthreads();
   if (w != 0 || e > NTRAIN) return;
-  float gi = 0.f;
+  double gs = 0.;
 #pragma unroll
-  for (int u = 0; u < UPDATE_WAYS; u++) gi += sum[u][c];
+  for (int u = 0; u < UPDATE_WAYS; u++) gs += sum[u][c];
   if (e == NTRAIN) {
-    *loss = first ? gi : *loss + gi;
+    *loss = first ? gs : *loss + gs;
   } else if (ADAM) {
-    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    m1[e] = b1 * m1[e] + (1.f - b1) * gi;
-    m2[e] = b2 * m2[e] + (1.f - b2) * gi * gi;
-    float mh = m1[e] / (1.f - b1t), vh = m2[e] / (1.f - b2t);
-    const float v = m.w[e] - lr * mh / (sqrtf(vh) + eps);
+    const double b1 = 0.9, b2 = 0.999, eps = 1e-8;
+    const double mm = b1 * m1[e] + (1. - b1) * gs, vv = b2 * m2[e] + (1. - b2) * gs * gs;
+    m1[e] = mm;
+    m2[e] = vv;
+    // the weight is w + wlo, so that its steps do not round away
+    const double wd = (double)m.w[e] + (double)m.wlo[e] - lr * (mm / (1. - b1t)) / (sqrt(vv / (1. - b2t)) + eps);
+    const float v = (float)wd;
     m.w[e] = v;
+    m.wlo[e] = (float)(wd - (double)v);
     refresh_bf16(e, v, m);
   } else {
-    grad[e] = gi;
+    grad[e] = (float)gs;
   }
 }
 
+// after the parameters were set
 __global__ void k_mlp_refresh(MlpDev m) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < NTRAIN) refresh_bf16(e, m.w[e], m);
+  if (e >= NTRAIN) return;
+  m.wlo[e] = 0.f;
+  refresh_bf16(e, m.w[e], m);
 }
 
 // ---------------------------------------------------------------------------
@@ -544,13 +554,14 @@ __global__ void __launch_bounds__(64) k_c2p_learned(int64_t n, double gam, const
 // BF16 copies, the loss, the counts and the partial sums of the backward pass
 struct hg_mlp {
   void *mem = nullptr;
-  float *w = nullptr, *g = nullptr, *m1 = nullptr, *m2 = nullptr, *loss = nullptr, *w2q = nullptr, *part = nullptr;
+  float *w = nullptr, *g = nullptr, *w2q = nullptr, *wlo = nullptr;
+  double *m1 = nullptr, *m2 = nullptr, *loss = nullptr, *part = nullptr;
   __bf16 *w1b = nullptr, *w2b = nullptr;
   unsigned long long *counts = nullptr;  // [learned starts, fallbacks]
   int step = 0;
 };
 
-static MlpDev dev_view(const hg_mlp *m) { return MlpDev{m->w, m->w1b, m->w2b, m->w2q}; }
+static MlpDev dev_view(const hg_mlp *m) { return MlpDev{m->w, m->w1b, m->w2b, m->w2q, m->wlo}; }
 
 // blocks of the backward pass: one per 16-sample tile up to BACK_BLOCKS
 static unsigned backward_blocks(int64_t n) {
@@ -606,23 +617,24 @@ extern "C" int hg_mlp_create(uint64_t seed, hg_mlp **out) {
     at += (bytes + 255) / 256 * 256;
     return here;
   };
-  const size_t o_g = take(np * 4), o_m1 = take(np * 4), o_m2 = take(np * 4), o_w1b = take(32 * NH * sizeof(__bf16)),
-               o_w2b = take(NH * NH * sizeof(__bf16)), o_loss = take(sizeof(float)),
+  const size_t o_g = take(np * 4), o_m1 = take(np * 8), o_m2 = take(np * 8), o_wlo = take(np * 4), o_w1b = take(32 * NH * sizeof(__bf16)),
+               o_w2b = take(NH * NH * sizeof(__bf16)), o_loss = take(sizeof(double)),
                o_counts = take(2 * sizeof(unsigned long long)), zeroed = at, o_w = take(np * 4),
-               o_w2q = take(NH * NH * sizeof(float)), o_part = take((size_t)BACK_BLOCKS * PART * sizeof(float));
+               o_w2q = take(NH * NH * sizeof(float)), o_part = take((size_t)BACK_BLOCKS * PART * sizeof(double));
   hipError_t e = hipMalloc(&m->mem, at);
   if (e == hipSuccess) {
     char *b = (char *)m->mem;
     m->g = (float *)(b + o_g);
-    m->m1 = (float *)(b + o_m1);
-    m->m2 = (float *)(b + o_m2);
+    m->m1 = (double *)(b + o_m1);
+    m->m2 = (double *)(b + o_m2);
+    m->wlo = (float *)(b + o_wlo);
     m->w1b = (__bf16 *)(b + o_w1b);
     m->w2b = (__bf16 *)(b + o_w2b);
-    m->loss = (float *)(b + o_loss);
+    m->loss = (double *)(b + o_loss);
     m->counts = (unsigned long long *)(b + o_counts);
     m->w = (float *)(b + o_w);
     m->w2q = (float *)(b + o_w2q);
-    m->part = (float *)(b + o_part);
+    m->part = (double *)(b + o_part);
     e = hipMemset(m->mem, 0, zeroed);
   }
   if (e == hipSuccess) e = hipMemcpy(m->w, w.data(), NPARAM * sizeof(float), hipMemcpyHostToDevice);
@@ -706,15 +718,28 @@ extern "C" int hg_mlp_gradient(hg_mlp *m, int64_t n, const float *X, const float
   if (!m || n <= 0 || !X || !Y) { set_error("hg_mlp_gradient: bad arguments"); return 1; }
   hipStream_t s = (hipStream_t)stream;
   const unsigned nb = backward_blocks(n);
-  hipLaunchKernelGGL(k_mlp_backward, dim3(nb), dim3(256), 0, s, n, X, Y, dev_view(m), (float)(1.0 / (double)n),
-                     (float)(1.0 / (double)n), m->part);
-  hipLaunchKernelGGL(k_mlp_update<false>, dim3(UPDATE_BLOCKS), dim3(64 * UPDATE_WAYS), 0, s, dev_view(m), (const float *)m->part,
-                     (int)nb, 0.f, 0.f, 0.f, 1, m->m1, m->m2, m->g, m->loss);
+  hipLaunchKernelGGL(k_mlp_backward, dim3(nb), dim3(256), 0, s, n, X, Y, dev_view(m), 1.0 / (double)n,
+                     1.0 / (double)n, m->part);
+  hipLaunchKernelGGL(k_mlp_update<false>, dim3(UPDATE_BLOCKS), dim3(64 * UPDATE_WAYS), 0, s, dev_view(m), (const double *)m->part,
+                     (int)nb, 0., 0., 0., 1, m->m1, m->m2, m->g, m->loss);
   MLPCHECK(hipGetLastError());
   MLPCHECK(hipStreamSynchronize(s));
   if (grad_host) MLPCHECK(hipMemcpy(grad_host, m->g, NPARAM * sizeof(float), hipMemcpyDeviceToHost));
-  if (loss) MLPCHECK(hipMemcpy(loss, m->loss, sizeof(float), hipMemcpyDeviceToHost));
+  double ls = 0.;
+  if (loss) MLPCHECK(hipMemcpy(&ls, m->loss, sizeof ls, hipMemcpyDeviceToHost));
+  if (loss) *loss = (float)ls;
   return 0;
+}
+
+// the number a caller wrote for a float argument: of the reals that round to
+// it, the one of fewest digits (2e-3f stands for 0.002)
+static double written(float v) {
+  char t[32];
+  for (int digits = 6; digits <= 9; digits++) {
+    snprintf(t, sizeof t, "%.*g", digits, (double)v);
+    if ((float)strtod(t, nullptr) == v) return strtod(t, nullptr);
+  }
+  return v;
 }
 
 // epochs of Adam over the n samples in minibatches of `batch` (in order);
@@ -727,24 +752,25 @@ extern "C" int hg_mlp_train(hg_mlp *m, int64_t n, const float *X, const float *Y
   }
   hipStream_t s = (hipStream_t)stream;
   int64_t nb = (n + batch - 1) / batch;
-  float last = 0.f;
+  const double rate = written(lr);
+  double last = 0.;
   for (int ep = 0; ep < epochs; ep++) {
     for (int64_t b = 0; b < nb; b++) {
       int64_t off = b * batch, cnt = (off + batch <= n) ? batch : n - off;
       const unsigned blocks = backward_blocks(cnt);
       hipLaunchKernelGGL(k_mlp_backward, dim3(blocks), dim3(256), 0, s, cnt, X + off * NIN, Y + off, dev_view(m),
-                         (float)(1.0 / (double)cnt), (float)(1.0 / (double)cnt / (double)nb), m->part);
+                         1.0 / (double)cnt, 1.0 / (double)cnt / (double)nb, m->part);
       m->step++;
-      float b1t = powf(0.9f, (float)m->step), b2t = powf(0.999f, (float)m->step);
+      const double b1t = pow(0.9, (double)m->step), b2t = pow(0.999, (double)m->step);
       hipLaunchKernelGGL(k_mlp_update<true>, dim3(UPDATE_BLOCKS), dim3(64 * UPDATE_WAYS), 0, s, dev_view(m),
-                         (const float *)m->part, (int)blocks, lr, b1t, b2t, b == 0 ? 1 : 0, m->m1, m->m2, m->g,
+                         (const double *)m->part, (int)blocks, rate, b1t, b2t, b == 0 ? 1 : 0, m->m1, m->m2, m->g,
                          m->loss);
     }
     MLPCHECK(hipGetLastError());
-    MLPCHECK(hipMemcpyAsync(&last, m->loss, sizeof(float), hipMemcpyDeviceToHost, s));
+    MLPCHECK(hipMemcpyAsync(&last, m->loss, sizeof last, hipMemcpyDeviceToHost, s));
     MLPCHECK(hipStreamSynchronize(s));
   }
-  if (loss) *loss = last;
+  if (loss) *loss = (float)last;
   return 0;
 }
 
