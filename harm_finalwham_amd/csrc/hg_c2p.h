@@ -23,7 +23,10 @@ constexpr double FAIL_VAL = 1.e30;
 struct C2PInv {
   double Bsq, QdotB, QdotBsq, Qtsq, Qdotn, D, w;
   double Qcon[4], ncon[4], Bcon[4];
-  double Bprim[3];  // alpha * B^i
+  // set by newton_ranges: what the Newton steps need of D, Bsq and w to leave
+  // out the scaling of their divisions
+  bool nice;    // D in [2^-150, 2^150], Bsq zero or in [2^-150, 2^150]
+  double wlim;  // x0 < wlim makes x0 / w <= gsq_big certain
 };
 
 // utoprim_2d_final.c:457 vsq_calc
@@ -33,10 +36,23 @@ __device__ __forceinline__ double vsq_of_W(const C2PInv &c, double W) {
   return ((Wsq * c.Qtsq + c.QdotBsq * (c.Bsq + 2. * W)) / (Wsq * Xsq));
 }
 
+__device__ __forceinline__ void newton_ranges(C2PInv &c) {
+  constexpr double gsq_big = GAMMAFAIL * GAMMAFAIL;
+  c.nice = c.D >= 0x1p-150 && c.D <= 0x1p150 && (c.Bsq == 0. || (c.Bsq >= 0x1p-150 && c.Bsq <= 0x1p150));
+  c.wlim = (c.w >= 0x1p-200 && c.w <= 0x1p200) ? c.w * (gsq_big * (1. - 0x1p-40)) : -1.;
+}
+
+// x0 / w > gsq_big of the reference's loop for x0 >= 0: decided by a product
+// wherever the quotient is further than its rounding from gsq_big
+__device__ __forceinline__ bool w_too_big(const C2PInv &c, double x0) {
+  if (x0 < c.wlim) return false;
+  return x0 / c.w > GAMMAFAIL * GAMMAFAIL;
+}
+
 // One Newton step of utoprim_2d_final.c:1189 func_vsq2 (with the EOS of
 // utoprim_jon_eos.c:107,230,346); returns dx[0..1] and f, df.
-__device__ __forceinline__ void newton_dx(const C2PInv &c, double igr, double W, double vsq,
-                                          double &dx0, double &dx1, double &f, double &df) {
+__device__ __forceinline__ void newton_dx_full(const C2PInv &c, double igr, double W, double vsq,
+                                               double &dx0, double &dx1, double &f, double &df) {
   double Wsq = W * W, D = c.D, Bsq = c.Bsq, QdotBsq = c.QdotBsq;
   double Wp = W - D;
   double gamma = 1.0 / sqrt(1.0 - vsq);
@@ -67,6 +83,78 @@ __device__ __forceinline__ void newton_dx(const C2PInv &c, double igr, double W,
   dx1 = -(-t25 * t11 - 2.0 * t40 * t18) * t21 * t36;
   df = -t11 * t11 - t18 * t18;
   f = -0.5 * df;
+}
+
+// sqrt(x) for x in [2^-60, 2^60]: the steps hipcc lowers it to, without the
+// scaling of tiny arguments and the choice of 0 and infinity around them
+__device__ __forceinline__ double sqrt_core(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  double d = fma(-g, g, x);
+  g = fma(d, h, g);
+  d = fma(-g, g, x);
+  return fma(d, h, g);
+}
+
+// 1 / d for |d| in [2^-300, 2^300] (div_core with a numerator of 1)
+__device__ __forceinline__ double rcp_core(double d) {
+  const double y = rcp_refined(d);
+  return fma(fma(-d, y, 1.0), y, y);
+}
+
+// newton_dx_full bit for bit.  The iteration is a serial chain of seven
+// divisions and a square root, and the instruction count sets its time both
+// where lanes fill the SIMDs and where one wavefront walks the last zones;
+// the scaling around the hardware's division and square root is about a
+// third of it and changes nothing for operands of ordinary size.  The
+// bounds: 1 - vsq in [2^-60, 2^60] and W in [2^-150, 2^150] with D and Bsq as
+// newton_ranges has them keep W^2, Bsq + W, gamma, gamma^2 and 1 + gamma in
+// div_core's ranges; W - D is zero or at least 2^-202; |D vsq| is zero or at
+// least 2^-450.  dPdrho0 = 0 drops out: its products are zeros, added to
+// terms that are not (-0).  A zone outside takes the full step.  2^24 zones
+// in HG_C2P_FP64 take 1.80 ms instead of 2.12 ms.
+__device__ __forceinline__ void newton_dx(const C2PInv &c, double igr, double W, double vsq,
+                                          double &dx0, double &dx1, double &f, double &df) {
+  const double D = c.D, Bsq = c.Bsq, QdotBsq = c.QdotBsq;
+  const double omv = 1.0 - vsq;
+  const double Wsq = W * W;
+  const double Wp = W - D;
+  const double gamma = rcp_core(sqrt_core(omv));
+  const double gammasq = gamma * gamma;
+  const double opg = 1.0 + gamma;
+  const double wmrho0 = div_core(Wp, gammasq, rcp_refined(gammasq)) - div_core(D * vsq, opg, rcp_refined(opg));
+  const double p_tmp = igr * wmrho0;
+  const double dPdW = omv * igr;
+  const double dPdvsq = (D * (gamma * 0.5 - 1.0) - Wp) * igr;
+  const double t2 = -0.5 * Bsq + dPdvsq;
+  const double t3 = Bsq + W;
+  const double t4 = t3 * t3;
+  const double t9 = rcp_core(Wsq);
+  double t11 = c.Qtsq - vsq * t4 + QdotBsq * (Bsq + 2.0 * W) * t9;
+  const double t16 = QdotBsq * t9;
+  double t18 = -c.Qdotn - 0.5 * Bsq * (1.0 + vsq) + 0.5 * t16 - W + p_tmp;
+  const double t21 = rcp_core(t3);
+  const double t23 = rcp_core(W);
+  const double t24 = t16 * t23;
+  const double t25 = -1.0 + dPdW - t24;
+  const double t35 = t25 * t3 + (Bsq - 2.0 * dPdvsq) * (QdotBsq + vsq * Wsq * W) * t9 * t23;
+  const double t36 = rcp_core(t35);
+  const double t40 = (vsq + t24) * t3;
+  double e0 = -(t2 * t11 + t4 * t18) * t21 * t36;
+  double e1 = -(-t25 * t11 - 2.0 * t40 * t18) * t21 * t36;
+  const bool ok = c.nice && omv >= 0x1p-60 && omv <= 0x1p60 && W >= 0x1p-150 && W <= 0x1p150 &&
+                  (vsq == 0. || fabs(vsq) >= 0x1p-300) && fabs(t35) >= 0x1p-300 && fabs(t35) <= 0x1p300;
+  if (ok) {
+    dx0 = e0;
+    dx1 = e1;
+    df = -t11 * t11 - t18 * t18;
+    f = -0.5 * df;
+  } else {
+    newton_dx_full(c, igr, W, vsq, dx0, dx1, f, df);
+  }
 }
 
 // Setup of Utoprim_new_body up to the Newton guess (utoprim_2d_final.c:152-300).
@@ -137,6 +225,7 @@ __device__ __forceinline__ int c2p_setup(const double *U, const GT &G, const dou
     i_increase++;
   }
   c.w = w;
+  newton_ranges(c);
   return 0;
 }
 
@@ -149,9 +238,11 @@ __device__ __forceinline__ int c2p_finish(const C2PInv &c, double W, int retval,
   const double maxnegvsq = (1.0 - 1.0 / (MAXNEGUTSQ + 1.0));
   assign = false;
   if ((retval != 0) || (W == FAIL_VAL)) return retval * 100 + 1;
-  double Wtest = W / c.w;
   assign = true;  // remaining failures return 0 from Utoprim_new_body: guess kept
-  if (Wtest <= 0. || Wtest > gsq_big) { assign = false; return FAIL_CONVW; }
+  if (!(W >= 0x1p-150 && W < c.wlim)) {  // else 0 < W / w <= gsq_big
+    double Wtest = W / c.w;
+    if (Wtest <= 0. || Wtest > gsq_big) { assign = false; return FAIL_CONVW; }
+  }
   double vsq = vsq_of_W(c, W);
   if ((vsq < 0.) && (fabs(vsq) < maxnegvsq)) vsq = 0.0;
   if ((vsq > vsq_big) || (vsq < 0.0)) { assign = false; return FAIL_CONVUTSQ; }
@@ -169,12 +260,32 @@ __device__ __forceinline__ int c2p_finish(const C2PInv &c, double W, int retval,
   }
   prim_out[RHO] = rho0;
   prim_out[UU] = u;
+  double bw[3];
+#pragma unroll
+  for (int i = 0; i < 3; i++) bw[i] = c.QdotB * c.Bcon[i + 1];
+  div_by<3>(bw, W, div_rcp(W));
+  const double gx = gamma / (W + c.Bsq);
 #pragma unroll
   for (int i = 1; i < 4; i++) {
     double Qtcon = c.Qcon[i] + c.ncon[i] * c.Qdotn;
-    prim_out[U1 + i - 1] = gamma / (W + c.Bsq) * (Qtcon + c.QdotB * c.Bcon[i] / W);
+    prim_out[U1 + i - 1] = gx * (Qtcon + bw[i - 1]);
   }
   return flag;
+}
+
+// Utoprimgen's scaling of the evolved conserved variables (utoprimgen.c:23):
+// Ug = U / gdet with the rest mass taken out of the energy, Ut = alpha Ug;
+// returns alpha
+template <class GT>
+__device__ __forceinline__ double c2p_scale(const double *U, const GT &G, double *Ug, double *Ut) {
+#pragma unroll
+  for (int i = 0; i < NPR; i++) Ug[i] = U[i];
+  div_by<NPR>(Ug, G.g, div_rcp(G.g));
+  Ug[UU] -= Ug[RHO];
+  const double alpha = 1.0 / sqrt(-G.gcon[0][0]);
+#pragma unroll
+  for (int i = 0; i < NPR; i++) Ut[i] = alpha * Ug[i];
+  return alpha;
 }
 
 // Full FP64 inversion of one zone (utoprimgen.c:23 with UTOPRIM2DFINAL).
@@ -186,14 +297,9 @@ __device__ __forceinline__ int utoprimgen_fp64_core(const double *U, const GT &G
                                                     int &iters, C2PInv &c, double &x0, double &x1,
                                                     bool &newton) {
   double Ug[NPR], Ut[NPR];
-#pragma unroll
-  for (int i = 0; i < NPR; i++) Ug[i] = U[i] / G.g;
-  Ug[UU] -= Ug[RHO];
+  c2p_scale(U, G, Ug, Ut);
 #pragma unroll
   for (int i = B1; i <= B3; i++) pr[i] = Ug[i];
-  double alpha = 1.0 / sqrt(-G.gcon[0][0]);
-#pragma unroll
-  for (int i = 0; i < NPR; i++) Ut[i] = alpha * Ug[i];
   const double igr = (gam - 1.0) / gam;
   const double gsq_big = GAMMAFAIL * GAMMAFAIL;
   const double vsq_big = (gsq_big - 1.0) / (gsq_big);
@@ -207,9 +313,8 @@ __device__ __forceinline__ int utoprimgen_fp64_core(const double *U, const GT &G
   x0 = fabs(W_last);
   double v0 = vsq_of_W(c, W_last);
   x1 = (v0 > 1.) ? vsq_big : v0;
-  double f = 1., df = 1., errx = 1.;
-  int n_iter = 0;
-  bool keep = true;
+  double f = 1., df = 1.;
+  bool keep = true, far = false;
   while (keep) {
     iters++;
     double dx0, dx1;
@@ -217,16 +322,23 @@ __device__ __forceinline__ int utoprimgen_fp64_core(const double *U, const GT &G
     double xo0 = x0;
     x0 += dx0;
     x1 += dx1;
-    errx = (x0 == 0.) ? fabs(dx0) : fabs(dx0 / x0);
-    x0 = fabs(x0);
-    x0 = (x0 / c.w > gsq_big) ? xo0 : x0;
+    // errx = |dx0 / x0| <= NEWT_TOL by a product, but for quotients within
+    // 2^-40 of the tolerance; errx itself only after the last step allowed
+    const double a0 = fabs(x0), ad = fabs(dx0), lim = NEWT_TOL * a0;
+    bool conv = ad <= lim * (1. - 0x1p-40);
+    far = false;
+    if (!(a0 >= 0x1p-900) || !(conv || ad >= lim * (1. + 0x1p-40)) || iters >= MAX_NEWT_ITER) {
+      const double errx = (x0 == 0.) ? ad : fabs(dx0 / x0);
+      conv = errx <= NEWT_TOL;
+      far = errx > MIN_NEWT_TOL;
+    }
+    x0 = w_too_big(c, a0) ? xo0 : a0;
     x1 = (x1 > 1.) ? vsq_big : x1;
-    if ((fabs(errx) <= NEWT_TOL) || (n_iter >= (MAX_NEWT_ITER - 1))) keep = false;
-    n_iter++;
+    if (conv || (iters >= MAX_NEWT_ITER)) keep = false;
   }
   int retval = 0;
   if (!isfinite(f) || !isfinite(df) || !isfinite(x0) || !isfinite(x1)) retval = 1;
-  else if (fabs(errx) > MIN_NEWT_TOL) retval = 1;
+  else if (far) retval = 1;
   double out[NPR];
   bool assign;
   code = c2p_finish(c, x0, retval, igr, out, assign);
@@ -370,26 +482,29 @@ __device__ __forceinline__ bool newton_f32(const C2PInv &c, double igr, double &
 }
 
 // One Newton step with the residuals t11, t18 of func_vsq2 in double-double
-// and the FP64 Jacobian (newton_dx's terms)
+// and the FP64 Jacobian (newton_dx's terms, reciprocals to an ulp: the
+// Jacobian's rounding moves the step by 1e-15 of itself, the residuals set
+// the root)
 __device__ __forceinline__ void newton_dx_dd(const C2PInv &c, double igr, double W, double vsq, double &dx0,
                                              double &dx1) {
   const double Wsq = W * W, D = c.D, Bsq = c.Bsq, QdotBsq = c.QdotBsq;
-  const double gamma = 1.0 / sqrt(1.0 - vsq);
+  const double gamma = rsqrt_1ulp(1.0 - vsq);
   const double dPdW = (1.0 - vsq) * igr;
   const double dPdvsq = (D * (gamma * 0.5 - 1.0) - (W - D)) * igr;
-  const double t2 = -0.5 * Bsq + dPdvsq, t3 = Bsq + W, t4 = t3 * t3, t9 = 1 / Wsq;
-  const double t16 = QdotBsq * t9, t21 = 1 / t3, t23 = 1 / W, t24 = t16 * t23, t25 = -1.0 + dPdW - t24;
+  const double t2 = -0.5 * Bsq + dPdvsq, t3 = Bsq + W, t4 = t3 * t3, t23 = rcp_1ulp(W), t9 = t23 * t23;
+  const double t16 = QdotBsq * t9, t21 = rcp_1ulp(t3), t24 = t16 * t23, t25 = -1.0 + dPdW - t24;
   const double t35 = t25 * t3 + (Bsq - 2.0 * dPdvsq) * (QdotBsq + vsq * Wsq * W) * t9 * t23;
-  const double t36 = 1 / t35;
+  const double t36 = rcp_1ulp(t35);
   // residuals: t11 = Qtsq - vsq (Bsq + W)^2 + QdotBsq (Bsq + 2 W) / W^2,
   // t18 = -Qdotn - Bsq (1 + vsq) / 2 + QdotBsq / (2 W^2) - W + p(W, vsq)
   const dd Wd = dd_of(W), vd = dd_of(vsq);
   const dd T3 = two_sum(Bsq, W);
-  const dd q = dd_div(dd_of(QdotBsq), two_prod(W, W));
+  const dd q = dd_div_r(dd_of(QdotBsq), two_prod(W, W), t9);
   const dd r11 = dd_add(dd_sub(dd_of(c.Qtsq), dd_mul(vd, dd_mul(T3, T3))), dd_mul(q, two_sum(Bsq, 2.0 * W)));
   const dd omv = two_sum(1.0, -vsq);
-  const dd gd = dd_div(dd_of(1.0), dd_sqrt(omv));
-  const dd wm = dd_sub(dd_mul(two_sum(W, -D), omv), dd_div(two_prod(vsq, D), dd_add(dd_of(1.0), gd)));
+  // D vsq / (1 + gamma) = D vsq s / (1 + s), s = 1 / gamma
+  const dd sd = dd_sqrt(omv);
+  const dd wm = dd_sub(dd_mul(two_sum(W, -D), omv), dd_div(dd_mul(two_prod(vsq, D), sd), dd_add(dd_of(1.0), sd)));
   const dd r18 = dd_add(dd_add(dd_add(dd_of(-c.Qdotn), dd_mul_d(two_sum(1.0, vsq), -0.5 * Bsq)), dd_mul_d(q, 0.5)),
                         dd_add(dd_neg(Wd), dd_mul_d(wm, igr)));
   const double t11 = dd_val(r11), t18 = dd_val(r18);
@@ -411,7 +526,7 @@ __device__ __forceinline__ bool c2p_polish(const C2PInv &c, double igr, double &
     newton_dx(c, igr, x0, x1, dx0, dx1, f, df);
     double xo0 = x0;
     x0 = fabs(x0 + dx0);
-    x0 = (x0 / c.w > gsq_big) ? xo0 : x0;
+    x0 = w_too_big(c, x0) ? xo0 : x0;
     x1 += dx1;
     x1 = (x1 > 1.) ? vsq_big : x1;
     iters++;
@@ -424,7 +539,7 @@ __device__ __forceinline__ bool c2p_polish(const C2PInv &c, double igr, double &
     newton_dx_dd(c, igr, x0, x1, dx0, dx1);
     double xo0 = x0;
     x0 = fabs(x0 + dx0);
-    x0 = (x0 / c.w > gsq_big) ? xo0 : x0;
+    x0 = w_too_big(c, x0) ? xo0 : x0;
     x1 += dx1;
     x1 = (x1 > 1.) ? vsq_big : x1;
     iters++;
@@ -506,6 +621,65 @@ __device__ __forceinline__ int utoprimgen_refined(const double *U, const GT &G, 
     polished = true;
   }
   return code;
+}
+
+// |dW / W| that the rounding of newton_dx's residuals can make at the root:
+// half an ulp of each of their terms through the Jacobian
+__device__ __forceinline__ double newton_noise(const C2PInv &c, double igr, double W, double vsq) {
+  const double D = c.D, Bsq = c.Bsq;
+  const double gamma = rsqrt_1ulp(1.0 - vsq);
+  const double dPdvsq = (D * (gamma * 0.5 - 1.0) - (W - D)) * igr;
+  const double t2 = -0.5 * Bsq + dPdvsq, t3 = Bsq + W, t4 = t3 * t3, t23 = rcp_1ulp(W), t9 = t23 * t23;
+  const double t16 = c.QdotBsq * t9, t24 = t16 * t23, t25 = -1.0 + (1.0 - vsq) * igr - t24;
+  const double t35 = t25 * t3 + (Bsq - 2.0 * dPdvsq) * (c.QdotBsq + vsq * W * W * W) * t9 * t23;
+  const double s11 = fabs(c.Qtsq) + vsq * t4 + t16 * (Bsq + 2.0 * W);
+  const double s18 = fabs(c.Qdotn) + 0.5 * Bsq * (1.0 + vsq) + t16 + W + igr * (W + D);
+  return 0.5 * DBL_EPS * (fabs(t2) * s11 + t4 * s18) * fabs(rcp_1ulp(t3) * rcp_1ulp(t35)) * t23;
+}
+
+constexpr int LISTED_MAX_F64 = 48;       // FP64 steps before the reference's own iteration takes over
+constexpr double LISTED_NOISE = 1e-9;    // largest rounding noise of W the short way accepts
+constexpr double LISTED_MARGIN = 16.0;   // W moved by this many times its noise keeps the code 0
+
+// A zone the FP32 phase or its polish left: utoprimgen_refined's root and
+// primitives without the part of the reference's iteration that walks in the
+// rounding noise of its residual.  Where that noise is above NEWT_TOL
+// (Lorentz factors near 50, magnetisations near 1e3) the reference goes on to
+// 200 steps, 100 us and more for one zone, and the polish then discards where
+// it stopped.  The first steps are the reference's own iterates, to |dW/W| <=
+// 1e-9; from there the polish.  Taken only where every stopping point of the
+// reference inside the noise would give code 0: the FP64 primitives at W and
+// at W moved either way by LISTED_MARGIN times the noise all do.  Every other
+// zone is inverted by utoprimgen_refined from the guess.  The list of 1e6 zones of
+// the benchmark distribution (154, gamma 5/3) takes 42 us instead of 168 us.
+template <class GT>
+__device__ __forceinline__ int utoprimgen_listed(const double *U, const GT &G, double gam, double *pr, int &iters) {
+  C2PInv c;
+  double Ug[NPR], Ut[NPR], W_last;
+  c2p_scale(U, G, Ug, Ut);
+  if (c2p_setup(Ut, G, pr, gam, c, W_last) == 0) {
+    const double igr = (gam - 1.0) / gam;
+    double x0, x1;
+    newton_start(c, W_last, x0, x1);
+    int it = 0;
+    if (c2p_polish(c, igr, x0, x1, LISTED_MAX_F64, it)) {
+      const double noise = newton_noise(c, igr, x0, x1);
+      bool in = noise <= LISTED_NOISE, assign;
+      double out[NPR];
+      for (int k = -1; k <= 1 && in; k++)
+        in = c2p_finish(c, x0 * (1.0 + k * (LISTED_MARGIN * noise)), 0, igr, out, assign) == 0;
+      if (in && c2p_finish_dd(c, x0, igr, out, assign) == 0 && assign) {
+#pragma unroll
+        for (int i = 0; i < B1; i++) pr[i] = out[i];
+#pragma unroll
+        for (int i = B1; i <= B3; i++) pr[i] = Ug[i];
+        iters = it;
+        return 0;
+      }
+    }
+  }
+  bool polished;
+  return utoprimgen_refined(U, G, gam, pr, iters, polished);
 }
 
 }  // namespace hg

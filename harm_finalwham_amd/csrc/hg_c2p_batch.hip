@@ -9,13 +9,17 @@
 //                     (HG_C2P_FP64), or the reference inversion with its root
 //                     converged and the primitives formed in double-double
 //                     (HG_C2P_REFINED)
-//   k_c2p_mixed       persistent work queue: each wavefront takes 4 x 64
-//                     zones at a time from a device counter; per lane the
-//                     FP64 set-up, the FP32 Newton iteration, the polish and
-//                     the double-double primitives; a zone that does not
-//                     converge joins a compacted list instead
-//   k_c2p_listed      persistent over that list: the HG_C2P_REFINED
-//                     inversion from the original guess
+//   k_c2p_mixed       one thread per zone: the FP64 set-up, the FP32 Newton
+//                     iteration, the polish and the FP64 primitives; a zone
+//                     that does not converge joins a compacted list instead.
+//                     The dispatcher hands out the blocks in order, so the
+//                     chip reads the 42 arrays in 42 moving fronts; a work
+//                     queue whose wavefronts each walk their own stretch of
+//                     zones takes 172 us for 1e6 zones, this 96 us, and for
+//                     4096 zones (16 stretches) 35 us against 15 us
+//   k_c2p_listed      persistent over that list, from the original guess: the
+//                     root and primitives of HG_C2P_REFINED, short of the
+//                     reference's walk in rounding noise (utoprimgen_listed)
 //
 // Memory per zone: the inversion reads U (8), the upper triangles of the
 // symmetric gcov and gcon (10 + 10), gdet and the guess's u and u~^i (4),
@@ -164,57 +168,43 @@ __global__ void k_c2p_reset(unsigned long long *ctr) {
   if (threadIdx.x < C2P_NCTR) ctr[threadIdx.x] = 0ull;
 }
 
-constexpr int MIXED_ROUNDS = 4;  // 64-zone rounds per work-queue grab
+constexpr int MIXED_BLOCK = 128;  // 64, 128 and 256 measure alike, and 128 takes a partial last block better
 
-__global__ void __launch_bounds__(256) k_c2p_mixed(int64_t n, double gam, const double *__restrict__ U,
-                                                   const double *__restrict__ gcov,
-                                                   const double *__restrict__ gcon,
-                                                   const double *__restrict__ gdet, double *__restrict__ pr,
-                                                   int *__restrict__ pflag, int *__restrict__ iters,
-                                                   unsigned long long *__restrict__ ctr,
-                                                   uint32_t *__restrict__ list) {
-  const int lane = threadIdx.x & 63;
+__global__ void __launch_bounds__(MIXED_BLOCK) k_c2p_mixed(int64_t n, double gam, const double *__restrict__ U,
+                                                           const double *__restrict__ gcov,
+                                                           const double *__restrict__ gcon,
+                                                           const double *__restrict__ gdet, double *__restrict__ pr,
+                                                           int *__restrict__ pflag, int *__restrict__ iters,
+                                                           unsigned long long *__restrict__ ctr,
+                                                           uint32_t *__restrict__ list) {
+  const int64_t t = blockIdx.x * (int64_t)MIXED_BLOCK + threadIdx.x;
   const double igr = (gam - 1.0) / gam;
-  for (;;) {
-    unsigned long long base = 0;
-    if (lane == 0) base = atomicAdd(&ctr[C2P_WORK], (unsigned long long)(64 * MIXED_ROUNDS));
-    base = __shfl(base, 0, 64);
-    if (base >= (unsigned long long)n) break;
-    for (int r = 0; r < MIXED_ROUNDS; r++) {
-      const int64_t t = (int64_t)base + 64 * r + lane;
-      bool fb = false;
-      if (t < n) {
-        Geom G;
-        double u[NPR], p[NPR], Ug[NPR], Ut[NPR];
-        load_batch_zone(n, t, U, gcov, gcon, gdet, pr, G, u, p);
+  bool fb = false;
+  if (t < n) {
+    Geom G;
+    double u[NPR], p[NPR], Ug[NPR], Ut[NPR];
+    load_batch_zone(n, t, U, gcov, gcon, gdet, pr, G, u, p);
+    c2p_scale(u, G, Ug, Ut);
 #pragma unroll
-        for (int i = 0; i < NPR; i++) Ug[i] = u[i] / G.g;
-        Ug[UU] -= Ug[RHO];
-#pragma unroll
-        for (int i = B1; i <= B3; i++) p[i] = Ug[i];
-        const double alpha = 1.0 / sqrt(-G.gcon[0][0]);
-#pragma unroll
-        for (int i = 0; i < NPR; i++) Ut[i] = alpha * Ug[i];
-        C2PInv c;
-        double W_last;
-        int it = 0, flag = c2p_setup(Ut, G, p, gam, c, W_last);
-        if (flag == 0) {
-          double x0, x1;
-          newton_start(c, W_last, x0, x1);
-          fb = !mixed_zone(c, igr, x0, x1, p, it, flag);
-        }
-        if (!fb) {
-          store_batch_zone(n, t, pr, p, code_assigns(flag));
-          pflag[t] = flag;
-          if (iters) iters[t] = it;
-        }
-      }
-      list_append(fb, t, ctr, list);
+    for (int i = B1; i <= B3; i++) p[i] = Ug[i];
+    C2PInv c;
+    double W_last;
+    int it = 0, flag = c2p_setup(Ut, G, p, gam, c, W_last);
+    if (flag == 0) {
+      double x0, x1;
+      newton_start(c, W_last, x0, x1);
+      fb = !mixed_zone(c, igr, x0, x1, p, it, flag);
+    }
+    if (!fb) {
+      store_batch_zone(n, t, pr, p, code_assigns(flag));
+      pflag[t] = flag;
+      if (iters) iters[t] = it;
     }
   }
+  list_append(fb, t, ctr, list);
 }
 
-// the listed zones: HG_C2P_REFINED from the guess still in pr
+// the listed zones, from the guess still in pr
 __global__ void __launch_bounds__(256) k_c2p_listed(int64_t n, double gam, const double *__restrict__ U,
                                                     const double *__restrict__ gcov,
                                                     const double *__restrict__ gcon,
@@ -235,8 +225,7 @@ __global__ void __launch_bounds__(256) k_c2p_listed(int64_t n, double gam, const
       double u[NPR], p[NPR];
       load_batch_zone(n, t, U, gcov, gcon, gdet, pr, G, u, p);
       int it = 0;
-      bool pol;
-      int flag = utoprimgen_refined(u, G, gam, p, it, pol);
+      int flag = utoprimgen_listed(u, G, gam, p, it);
       store_batch_zone(n, t, pr, p, code_assigns(flag));
       pflag[t] = flag;
       if (iters) iters[t] = it;
@@ -284,12 +273,11 @@ int launch_c2p_batch_mixed(int64_t n, double gam, const double *U, const double 
                            const double *gdet, double *pr, int *pflag, int *iters, void *scratch, hipStream_t s) {
   unsigned long long *ctr = (unsigned long long *)scratch;
   uint32_t *list = (uint32_t *)(ctr + C2P_NCTR);
-  int64_t b1 = 0, b2 = 0;
-  if (persistent_blocks(k_c2p_mixed, (n + 255) / 256, b1)) return 1;
+  int64_t b2 = 0;
   if (persistent_blocks(k_c2p_listed, (n + 255) / 256, b2)) return 1;
   hipLaunchKernelGGL(k_c2p_reset, dim3(1), dim3(64), 0, s, ctr);
-  hipLaunchKernelGGL(k_c2p_mixed, dim3((unsigned)b1), dim3(256), 0, s, n, gam, U, gcov, gcon, gdet, pr, pflag, iters,
-                     ctr, list);
+  hipLaunchKernelGGL(k_c2p_mixed, dim3((unsigned)((n + MIXED_BLOCK - 1) / MIXED_BLOCK)), dim3(MIXED_BLOCK), 0, s, n,
+                     gam, U, gcov, gcon, gdet, pr, pflag, iters, ctr, list);
   hipLaunchKernelGGL(k_c2p_listed, dim3((unsigned)b2), dim3(256), 0, s, n, gam, U, gcov, gcon, gdet, pr, pflag,
                      iters, ctr, (const uint32_t *)list);
   return 0;
@@ -368,7 +356,7 @@ extern "C" int hg_utoprim_batch(int64_t n, double gam, const double *U, const do
     e = hipMallocAsync(&scr, c2p_scratch_bytes(n), s);
     if (e != hipSuccess) { set_error("hg_utoprim_batch: scratch: %s", hipGetErrorString(e)); return 1; }
     int rc = launch_c2p_batch_mixed(n, gam, U, gcov, gcon, gdet, pr, pflag, iters, scr, s);
-    unsigned long long ctr[C2P_NCTR] = {0, 0, 0};
+    unsigned long long ctr[C2P_NCTR] = {0, 0};
     if (!rc) e = hipMemcpyAsync(ctr, scr, sizeof ctr, hipMemcpyDeviceToHost, s);
     hipError_t e2 = hipFreeAsync(scr, s);
     if (e == hipSuccess) e = e2;
@@ -441,7 +429,7 @@ extern "C" int hg_utoprim_batch_noalloc(int64_t n, double gam, const double *U, 
   if (e == hipSuccess) e = hipGetLastError();
   if (e == hipSuccess && cs == hipStreamCaptureStatusNone) {
     if (mode == HG_C2P_MIXED) {
-      unsigned long long ctr[C2P_NCTR] = {0, 0, 0};
+      unsigned long long ctr[C2P_NCTR] = {0, 0};
       void *scr = nullptr;
       if (noalloc_scratch(&scr)) return 1;
       e = hipMemcpyAsync(ctr, scr, sizeof ctr, hipMemcpyDeviceToHost, s);

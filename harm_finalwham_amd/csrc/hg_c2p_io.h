@@ -106,12 +106,7 @@ template <class GT>
 __device__ __forceinline__ int c2p_setup_zone(const double *U, const GT &G, double gam, const double *guess,
                                           C2PInv &c, double &W_last, double &alpha, double *Ug) {
   double Ut[NPR];
-#pragma unroll
-  for (int i = 0; i < NPR; i++) Ug[i] = U[i] / G.g;
-  Ug[UU] -= Ug[RHO];
-  alpha = 1.0 / sqrt(-G.gcon[0][0]);
-#pragma unroll
-  for (int i = 0; i < NPR; i++) Ut[i] = alpha * Ug[i];
+  alpha = c2p_scale(U, G, Ug, Ut);
   return c2p_setup(Ut, G, guess, gam, c, W_last);
 }
 
@@ -142,7 +137,7 @@ __device__ __forceinline__ int learned_start(const C2PInv &c, double igr, double
   }
   if (cand) {
     x0 = fabs(Wm + d0);
-    x0 = (x0 / c.w > gsq_big) ? Wm : x0;
+    x0 = w_too_big(c, x0) ? Wm : x0;
     x1 = xm1 + d1;
     x1 = (x1 > 1.) ? vsq_big : x1;
   } else {

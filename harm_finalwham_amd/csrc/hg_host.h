@@ -120,16 +120,17 @@ unsigned group_blocks_mlp(const GridView &v);
 void launch_group_mlp(const hg_mlp *m, const GridView *views, const unsigned *first, int n, unsigned total,
                       hipStream_t s);
 // batched inversion (hg_c2p_batch.hip).  The mixed path's scratch holds
-// C2P_NCTR counters (work queue, list length, list work queue) and a list of
+// C2P_NCTR counters (list length, list work queue) and a list of
 // n 32-bit zone indices: c2p_scratch_bytes(n) bytes.
-constexpr int C2P_WORK = 0, C2P_LISTLEN = 1, C2P_LISTWORK = 2, C2P_NCTR = 3;
+constexpr int C2P_LISTLEN = 0, C2P_LISTWORK = 1, C2P_NCTR = 2;
 size_t c2p_scratch_bytes(int64_t n);
 int launch_c2p_batch(int64_t n, double gam, const double *U, const double *gcov, const double *gcon,
                      const double *gdet, double *pr, int *pflag, int *iters, bool refined, hipStream_t s);
 int launch_c2p_batch_mixed(int64_t n, double gam, const double *U, const double *gcov, const double *gcon,
                            const double *gdet, double *pr, int *pflag, int *iters, void *scratch, hipStream_t s);
 void launch_c2p_reset(void *scratch, hipStream_t s);
-// the zones a mixed or learned pass listed, inverted by HG_C2P_REFINED
+// the zones a mixed or learned pass listed: the root and primitives of
+// HG_C2P_REFINED
 int launch_c2p_listed(int64_t n, double gam, const double *U, const double *gcov, const double *gcon,
                       const double *gdet, double *pr, int *pflag, int *iters, void *scratch, hipStream_t s);
 void c2p_note_fallbacks(long long nfb);

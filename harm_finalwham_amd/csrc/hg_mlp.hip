@@ -150,12 +150,16 @@ __device__ __forceinline__ float act(float x) {
 }
 __device__ __forceinline__ __bf16 bf_lo(float v) { return (__bf16)(v - (float)(__bf16)v); }
 
-// 16 samples: xin[16][8] (normalised) -> y[16]; h[16][64] float LDS scratch
+// rows of forward16's scratch in LDS: four floats apart in the banks, so the 16
+// lanes of a column block read 16 rows as 16-byte vectors without conflicts
+constexpr int NHS = NH + 4;
+
+// 16 samples: xin[16][8] (normalised) -> y[16]; h[16][NHS] float LDS scratch
 // for the layer-1 activations (the C layout of layer 1 -- sample 4 q + i in
 // lane 16 q + r -- is not the A layout of layer 2, sample r in lane 16 q + r);
 // layer 3 is summed per lane over its columns, then across the 16 lanes of
 // each sample group
-__device__ __forceinline__ void forward16(const MlpRegs &R, const float (*xin)[NIN], float (*h)[NH], float *y) {
+__device__ __forceinline__ void forward16(const MlpRegs &R, const float (*xin)[NIN], float (*h)[NHS], float *y) {
   const int l = threadIdx.x & 63, q = l >> 4, r = l & 15;
   // layer 1
   bf16x8 a;
@@ -210,7 +214,7 @@ __device__ __forceinline__ void forward16(const MlpRegs &R, const float (*xin)[N
 __device__ __forceinline__ void mlp_forward_body(int64_t n, const float *__restrict__ X, float *__restrict__ y,
                                                  const MlpDev &m, unsigned bid, unsigned nblk) {
   __shared__ float xin[16][NIN];
-  __shared__ float h[16][NH];
+  __shared__ __align__(16) float h[16][NHS];
   __shared__ float yo[16];
   const int l = threadIdx.x;
   MlpRegs R;
@@ -496,7 +500,7 @@ __global__ void __launch_bounds__(64) k_c2p_learned(int64_t n, double gam, const
                                                     uint32_t *__restrict__ list,
                                                     unsigned long long *__restrict__ counts) {
   __shared__ float xin[64][NIN];
-  __shared__ float h[16][NH];
+  __shared__ __align__(16) float h[16][NHS];
   __shared__ float yo[64];
   const int l = threadIdx.x;
   const int64_t t = (int64_t)blockIdx.x * 64 + l;
