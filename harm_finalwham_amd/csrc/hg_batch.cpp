@@ -280,16 +280,14 @@ int capture_grouped(hg_graph *g) {
     };
     // one substep of step_ch.c:94-166 on every grid: fluxcalc (directions in
     // turn, every direction's dP/P indicator in one launch), update, the
-    // learned start's features and network, inversion, dt on the final
-    // substep, bound_prim, post_fixup, bound_prim
+    // learned start's features and network, inversion, bound_prim (with dt
+    // on the final substep), post_fixup, bound_prim
     const int order[] = {GK_PREP, GK_DPI, GK_WENO1, GK_FLUX1, GK_WENO2, GK_FLUX2, GK_WENO3, GK_FLUX3,
-                         GK_EMF, g->ucum ? GK_UPDATEU : GK_UPDATE, GK_FEATURES, GK_MLP, GK_INVERT, GK_DT, GK_BOUND1,
-                         GK_BOUND2, GK_BOUND3, GK_FXCHECK, GK_FXRESOLVE, GK_FXAVG, GK_FXAPPLY, GK_BOUND1,
-                         GK_BOUND2, GK_BOUND3};
+                         GK_EMF, g->ucum ? GK_UPDATEU : GK_UPDATE, GK_FEATURES, GK_MLP, GK_INVERT, GK_BOUNDDT, GK_FXCHECK,
+                         GK_FXRESOLVE, GK_FXAVG, GK_FXAPPLY, GK_BOUND};
     for (int step = 0; step < g->nsteps; step++)
       for (int sub = 0; sub < g->ns; sub++)
         for (int k : order) {
-          if (k == GK_DT && sub != g->ns - 1) continue;
           if ((k == GK_FEATURES || k == GK_MLP) && g->mode != 2) continue;
           L(k, sub);
         }

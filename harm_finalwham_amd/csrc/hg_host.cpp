@@ -531,12 +531,13 @@ static void enqueue_substep(hg_ctx *c, double *pi, double *pb, double *pf, const
   launch_invert(c->uf, pb, pf, c->geo, c->floors, rk, finalstep, d, f.gam, f.gammamax, c->counters, c->pflag,
                 c->c2p_mode == HG_C2P_MIXED ? 1 : c->c2p_mode == HG_C2P_LEARNED ? 2 : 0, c->ly, c->fx_count,
                 c->err, c->tune, s);
-  if (finalstep) launch_dt(c->ndt_bits, c->dt, f.defcon, f.safe, s);
   // step_ch.c:127 and :166 call bound_prim twice per substep; the second call
   // is not a repeat of the first: POLEDEATH has zeroed U2 in the rows next to
   // the axis, which the radial inflow check then sees in the corner ghosts
   prof_mark(c, HG_PROF_BOUND, s);
-  launch_bound(pf, c->geo, c->d, f.gammamax, c->err, s);
+  StepDt se{};
+  if (finalstep) se = StepDt{c->ndt_bits, c->dt, f.defcon, f.safe};
+  launch_bound(pf, c->geo, c->d, f.gammamax, c->err, s, se);
   prof_mark(c, HG_PROF_FIXUP, s);
   launch_post_fixup(c, pf, finalstep, s, false);
   prof_mark(c, HG_PROF_BOUND, s);

@@ -18,7 +18,14 @@ struct Tune {
   int concurrent = 1;   // 1: the three directions' fluxes on three streams, 0: one after another
 };
 
-void launch_bound(double *p, const double *geo, const Dims &d, double gammamax, int *err, hipStream_t s);
+// the time step of a final substep, stored by the ghost fill after it
+struct StepDt {
+  const unsigned long long *ndt_bits;
+  double *dt;
+  double defcon, safe;
+};
+void launch_bound(double *p, const double *geo, const Dims &d, double gammamax, int *err, hipStream_t s,
+                  const StepDt &se = StepDt{});
 // point-type reconstruction (lim: HG_LIM_PARA, HG_LIM_MC or another
 // three-point limiter) fused with the flux, over the faces of the standard
 // (fv = false) or the finite-volume scheme's loops
@@ -68,7 +75,6 @@ void launch_invert(const double *ubuf, const double *pb, double *pf, const doubl
 // (8 floats per zone, k_invert's zone order)
 void launch_step_features(const double *ubuf, const double *pb, const double *geo, const Dims &d, double gam,
                           float *X, hipStream_t s);
-void launch_dt(unsigned long long *ndt_bits, double *dtp, double defcon, double safe, hipStream_t s);
 void launch_reset_ndt(unsigned long long *ndt_bits, hipStream_t s);
 
 
@@ -140,7 +146,7 @@ __device__ __forceinline__ int group_of(const unsigned *__restrict__ first, int 
 
 enum GroupClass {
   GK_PREP, GK_DPI, GK_WENO1, GK_WENO2, GK_WENO3, GK_FLUX1, GK_FLUX2, GK_FLUX3, GK_EMF, GK_UPDATE, GK_INVERT,
-  GK_DT, GK_BOUND1, GK_BOUND2, GK_BOUND3, GK_FXCHECK, GK_FXRESOLVE, GK_FXAVG, GK_FXAPPLY, GK_FEATURES, GK_MLP,
+  GK_BOUND, GK_BOUNDDT, GK_FXCHECK, GK_FXRESOLVE, GK_FXAVG, GK_FXAPPLY, GK_FEATURES, GK_MLP,
   GK_UPDATEU,  // the update with ucum (every scheme but the midpoint one)
   GK_NCLASS
 };

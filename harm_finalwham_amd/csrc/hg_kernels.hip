@@ -1,12 +1,12 @@
 // HIP kernels of the per-step GRMHD hot path for gfx950 (FP64 vector ALU).
 //
-//   k_bound_x1/x2/x3   ghost fill (bounds.fishmon.c:29)
+//   k_bound            ghost fill (bounds.fishmon.c:29); on the final substep also
+//                      the time-step update (advance.c:231, step_ch.c:243)
 //   k_flux_mc<dir>     MC reconstruction fused with the Riemann flux (flux.c:469)
 //   k_flux_para<dir>   PARA (para4) reconstruction fused with the Riemann flux
 //   k_flux_lr<dir>     Riemann flux from precomputed interface states (WENO5BND)
 //   k_emf              flux-CT corner EMFs (fluxct.c:10)
 //   k_update           conserved update + source + Noble 2D + fixup1zone (advance.c:58)
-//   k_dt               time-step update (advance.c:231, step_ch.c:243)
 //   k_set_dt           initial time step of the set-up (advance.c:957)
 #include <hip/hip_runtime.h>
 
@@ -98,95 +98,141 @@ __device__ __forceinline__ void block_sum_to(unsigned long long a, unsigned long
 // ---------------------------------------------------------------------------
 // ghost fill, bounds.fishmon.c:29 (EXTRAP 0, POLEDEATH 1, POSDEFMETRIC 0)
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void bound_x1_body(double *__restrict__ p, const double *__restrict__ geo, const Dims &d,
-                                              double gammamax, int *__restrict__ err, unsigned bid) {
-  // threads: ((k * n2 + j) * 2 + side) * nb1 + g: the ghost layers of a row
-  // on consecutive lanes (contiguous in memory, one source zone per side)
-  int64_t t = bid * (int64_t)blockDim.x + threadIdx.x;
-  int64_t total = 2LL * d.nb1 * d.n2 * d.n3;
-  if (t >= total) return;
-  int g = (int)(t % d.nb1);
-  int64_t r = t / d.nb1;
-  int side = (int)(r % 2);
-  r /= 2;
-  int j = (int)(r % d.n2);
-  int k = (int)(r / d.n2);
-  int i = side ? d.n1 + g : -1 - g;
-  int isrc = side ? d.n1 - 1 : 0;
+// One launch fills every ghost zone.  The reference fills along x1, then x2
+// from the rows x1 left, then x3 from both; here each ghost comes from the
+// active zone that order leads back to, by one of three kinds of block:
+//   kind 1  ghosts along x1: 8 lanes per row end carry the x1 rule of its ghost
+//           layers, and write them to the rows and planes that mirror or repeat the row
+//   kind 2  ghosts along x2 of active i: rows, and the planes that repeat them
+//   kind 3  ghosts along x3 of active i and j
+// POLEDEATH clears U2 and B2 of the active row next to the axis after the x1
+// rule has read them.  Inside one launch that order is kept by ownership: the
+// two end zones of such a row are cleared by the lanes of kind 1 that read
+// them, after the read, the others by kind 2.  Every other reader of a
+// cleared component multiplies it by 0 itself, which gives the same bits
+// before and after.  Bound by latency: three launches of 3 to 4 us with 2 us
+// between them on a small grid, one of 4 to 5 us here.
+constexpr int BOUND_LANES = 8;
+HG_HD void bound_blocks(const Dims &d, unsigned nblk[3]) {
+  auto blocks = [](int64_t n) { return (unsigned)((n + 255) / 256); };
+  nblk[0] = d.n1 > 1 ? blocks(2LL * BOUND_LANES * d.n2 * d.n3) : 0u;
+  nblk[1] = d.n2 > 1 ? blocks(2LL * d.nb2 * d.n3 * d.n1) : 0u;
+  nblk[2] = d.n3 > 1 ? blocks(2LL * d.nb3 * d.n2 * d.n1) : 0u;
+}
+
+// pr into zone (i,j) of plane k and of the planes that repeat it
+__device__ __forceinline__ void bound_put(double *__restrict__ p, const Dims &d, int i, int j, int k,
+                                          const double *pr) {
+  const bool up = d.n3 > 1 && k < d.nb3, down = d.n3 > 1 && k >= d.n3 - d.nb3;
+#pragma unroll
+  for (int c = -1; c <= 1; c++) {
+    if ((c < 0 && !down) || (c > 0 && !up)) continue;
+    const int64_t z = d.idx(i, j, k + c * d.n3);
+#pragma unroll
+    for (int pl = 0; pl < NPR; pl++) p[z + pl * d.spl] = pr[pl];
+  }
+}
+
+__device__ __forceinline__ void bound_body(double *p, const double *__restrict__ geo, const Dims &d, double gammamax,
+                                           int *__restrict__ err, unsigned bid) {
+  unsigned nblk[3];
+  bound_blocks(d, nblk);
   double pr[NPR];
-  int64_t src = d.idx(isrc, j, k), dst = d.idx(i, j, k);
+  if (bid < nblk[0]) {
+    const unsigned t = bid * 256u + threadIdx.x;
+    const int g0 = (int)(t % BOUND_LANES);
+    unsigned r = t / BOUND_LANES;
+    const int side = (int)(r & 1u);
+    r >>= 1;
+    const int j = (int)(r % (unsigned)d.n2), k = (int)(r / (unsigned)d.n2);
+    if (k >= d.n3) return;
+    const int isrc = side ? d.n1 - 1 : 0;
+    const int64_t src = d.idx(isrc, j, k);
+    double ps[NPR];
 #pragma unroll
-  for (int pl = 0; pl < NPR; pl++) pr[pl] = p[src + pl * d.spl];
-  Geom G;
-  load_geom(geo, GL_CENT, d.gplane, d.gidx(i, j), G);
-  if (inflow_check_r(pr, G, side ? +1 : -1, gammamax) > 0) atomicOr(err, 1);
-  if (limit_gamma(gammamax, pr, G) > 0) atomicOr(err, 1);
+    for (int pl = 0; pl < NPR; pl++) ps[pl] = p[src + pl * d.spl];
+    const bool pole = d.n2 > 1 && (j == 0 || j == d.n2 - 1);
+    for (int g = g0; g < d.nb1; g += BOUND_LANES) {
+      const int i = side ? d.n1 + g : -1 - g;
 #pragma unroll
-  for (int pl = 0; pl < NPR; pl++) p[dst + pl * d.spl] = pr[pl];
-}
-
-__global__ void k_bound_x1(double *__restrict__ p, const double *__restrict__ geo, Dims d, double gammamax,
-                           int *__restrict__ err) {
-  bound_x1_body(p, geo, d, gammamax, err, blockIdx.x);
-}
-
-__device__ __forceinline__ void bound_x2_body(double *__restrict__ p, const Dims &d, unsigned bid) {
-  // threads: ((slot * n3 + k) * m1 + ii), slot in [0, 2*nb2)
-  int64_t t = bid * (int64_t)blockDim.x + threadIdx.x;
-  int64_t total = 2LL * d.nb2 * d.n3 * d.m1;
-  if (t >= total) return;
-  int ii = t % d.m1;
-  int64_t r = t / d.m1;
-  int k = r % d.n3;
-  int slot = (int)(r / d.n3);
-  int i = ii - d.nb1;
-  int j, jsrc, jact = -1;
-  if (slot < d.nb2) {  // inner: j = -1-slot mirrors row slot
-    j = -1 - slot;
-    jsrc = slot;
-    if (slot == 0) jact = 0;
+      for (int pl = 0; pl < NPR; pl++) pr[pl] = ps[pl];
+      Geom G;
+      load_geom(geo, GL_CENT, d.gplane, d.gidx(i, j), G);
+      if (inflow_check_r(pr, G, side ? +1 : -1, gammamax) > 0) atomicOr(err, 1);
+      if (limit_gamma(gammamax, pr, G) > 0) atomicOr(err, 1);
+      if (pole) {
+        pr[U2] *= 0;
+        pr[B2] *= 0.;
+      }
+      bound_put(p, d, i, j, k, pr);
+      if (d.n2 > 1 && (j < d.nb2 || j >= d.n2 - d.nb2)) {
+        pr[U2] *= 0;
+        pr[B2] *= 0.;
+        if (j < d.nb2) bound_put(p, d, i, -1 - j, k, pr);
+        if (j >= d.n2 - d.nb2) bound_put(p, d, i, 2 * d.n2 - 1 - j, k, pr);
+      }
+    }
+    if (pole && g0 == 0) {
+      p[src + U2 * d.spl] = ps[U2] * 0;
+      p[src + B2 * d.spl] = ps[B2] * 0.;
+    }
+  } else if (bid < nblk[0] + nblk[1]) {
+    const unsigned t = (bid - nblk[0]) * 256u + threadIdx.x;
+    const int i = (int)(t % (unsigned)d.n1);
+    const unsigned r = t / (unsigned)d.n1;
+    const int k = (int)(r % (unsigned)d.n3), slot = (int)(r / (unsigned)d.n3);
+    if (slot >= 2 * d.nb2) return;
+    // inner: j = -1 - slot mirrors row slot; outer: j = n2 + s mirrors n2 - 1 - s
+    const int sl = slot < d.nb2 ? slot : slot - d.nb2;
+    const int j = slot < d.nb2 ? -1 - sl : d.n2 + sl, jsrc = slot < d.nb2 ? sl : d.n2 - 1 - sl;
+    const int64_t src = d.idx(i, jsrc, k);
+#pragma unroll
+    for (int pl = 0; pl < NPR; pl++) pr[pl] = p[src + pl * d.spl];
+    pr[U2] *= 0;
+    pr[B2] *= 0.;
+    bound_put(p, d, i, j, k, pr);
+    if (sl == 0 && !(d.n1 > 1 && (i == 0 || i == d.n1 - 1))) {  // POLEDEATH
+      p[src + U2 * d.spl] = pr[U2];
+      p[src + B2 * d.spl] = pr[B2];
+    }
   } else {
-    int s = slot - d.nb2;  // outer: j = n2+s mirrors row n2-1-s
-    j = d.n2 + s;
-    jsrc = d.n2 - 1 - s;
-    if (s == 0) jact = d.n2 - 1;
-  }
-  int64_t src = d.idx(i, jsrc, k), dst = d.idx(i, j, k);
-  double pr[NPR];
+    const unsigned t = (bid - nblk[0] - nblk[1]) * 256u + threadIdx.x;
+    const int i = (int)(t % (unsigned)d.n1);
+    const unsigned r = t / (unsigned)d.n1;
+    const int j = (int)(r % (unsigned)d.n2), slot = (int)(r / (unsigned)d.n2);
+    if (slot >= 2 * d.nb3) return;
+    const int k = slot < d.nb3 ? -1 - slot : d.n3 + (slot - d.nb3);
+    const int64_t src = d.idx(i, j, slot < d.nb3 ? k + d.n3 : k - d.n3), dst = d.idx(i, j, k);
 #pragma unroll
-  for (int pl = 0; pl < NPR; pl++) pr[pl] = p[src + pl * d.spl];
-  pr[U2] *= 0;
-  pr[B2] *= 0.;
+    for (int pl = 0; pl < NPR; pl++) pr[pl] = p[src + pl * d.spl];
+    if (d.n2 > 1 && (j == 0 || j == d.n2 - 1)) {
+      pr[U2] *= 0;
+      pr[B2] *= 0.;
+    }
 #pragma unroll
-  for (int pl = 0; pl < NPR; pl++) p[dst + pl * d.spl] = pr[pl];
-  if (jact >= 0) {  // POLEDEATH also clears the first active row next to the axis
-    int64_t a = d.idx(i, jact, k);
-    p[a + U2 * d.spl] *= 0;
-    p[a + B2 * d.spl] *= 0.;
+    for (int pl = 0; pl < NPR; pl++) p[dst + pl * d.spl] = pr[pl];
   }
 }
 
-__global__ void k_bound_x2(double *__restrict__ p, Dims d) { bound_x2_body(p, d, blockIdx.x); }
-
-__device__ __forceinline__ void bound_x3_body(double *__restrict__ p, const Dims &d, unsigned bid) {
-  // threads: ((slot * m2 + jj) * m1 + ii), slot in [0, 2*nb3)
-  int64_t t = bid * (int64_t)blockDim.x + threadIdx.x;
-  int64_t total = 2LL * d.nb3 * d.m2 * d.m1;
-  if (t >= total) return;
-  int ii = t % d.m1;
-  int64_t r = t / d.m1;
-  int jj = r % d.m2;
-  int slot = (int)(r / d.m2);
-  int i = ii - d.nb1, j = jj - d.nb2;
-  int k, ksrc;
-  if (slot < d.nb3) { k = -1 - slot; ksrc = d.n3 + k; }
-  else { k = d.n3 + (slot - d.nb3); ksrc = k - d.n3; }
-  int64_t src = d.idx(i, j, ksrc), dst = d.idx(i, j, k);
-#pragma unroll
-  for (int pl = 0; pl < NPR; pl++) p[dst + pl * d.spl] = p[src + pl * d.spl];
+// advance.c:231 ndt = defcon / (1/ndt1 + 1/ndt2 + 1/ndt3); on the final
+// substep step_ch.c:243-247 limits the growth and stores the next dt
+__device__ __forceinline__ void dt_body(const unsigned long long *ndt_bits, double *dtp, double defcon, double safe) {
+  double n1 = __longlong_as_double((long long)ndt_bits[0]);
+  double n2 = __longlong_as_double((long long)ndt_bits[1]);
+  double n3 = __longlong_as_double((long long)ndt_bits[2]);
+  double ndt = defcon * 1. / (1. / n1 + 1. / n2 + 1. / n3);
+  double dt = dtp[0];
+  if (ndt > safe * dt) ndt = safe * dt;
+  dtp[0] = ndt;
 }
 
-__global__ void k_bound_x3(double *__restrict__ p, Dims d) { bound_x3_body(p, d, blockIdx.x); }
+// se: where the final substep's time step goes (the fluxes' ndt and the update
+// that reads dt are done); no address on other substeps
+__global__ void __launch_bounds__(256) k_bound(double *p, const double *__restrict__ geo, Dims d, double gammamax,
+                                               int *__restrict__ err, StepDt se) {
+  if (se.dt && blockIdx.x == 0 && threadIdx.x == 0) dt_body(se.ndt_bits, se.dt, se.defcon, se.safe);
+  bound_body(p, geo, d, gammamax, err, blockIdx.x);
+}
 
 // ---------------------------------------------------------------------------
 // Riemann flux at one face from left/right states, fluxcompute.c:12
@@ -1004,22 +1050,6 @@ __global__ void __launch_bounds__(256) k_invert(const double *__restrict__ ubuf,
                         fx_reset, err, blockIdx.x);
 }
 
-// advance.c:231 ndt = defcon / (1/ndt1 + 1/ndt2 + 1/ndt3); on the final
-// substep step_ch.c:243-247 limits the growth and stores the next dt
-__device__ __forceinline__ void dt_body(unsigned long long *ndt_bits, double *dtp, double defcon, double safe) {
-  double n1 = __longlong_as_double((long long)ndt_bits[0]);
-  double n2 = __longlong_as_double((long long)ndt_bits[1]);
-  double n3 = __longlong_as_double((long long)ndt_bits[2]);
-  double ndt = defcon * 1. / (1. / n1 + 1. / n2 + 1. / n3);
-  double dt = dtp[0];
-  if (ndt > safe * dt) ndt = safe * dt;
-  dtp[0] = ndt;
-}
-
-__global__ void k_dt(unsigned long long *ndt_bits, double *dtp, double defcon, double safe) {
-  dt_body(ndt_bits, dtp, defcon, safe);
-}
-
 // ---------------------------------------------------------------------------
 // grouped launches of the kernels above (GridView, group_of)
 // ---------------------------------------------------------------------------
@@ -1028,22 +1058,14 @@ __global__ void k_dt(unsigned long long *ndt_bits, double *dtp, double defcon, d
   const GridView &v = views[g_];                       \
   const unsigned bid = blockIdx.x - first[g_];
 
-__global__ void __launch_bounds__(128) kg_bound_x1(const GridView *__restrict__ views,
-                                                   const unsigned *__restrict__ first, int n) {
+// first: the bound_prim before post_fixup, which also stores the final
+// substep's time step
+template <bool FIRST>
+__global__ void __launch_bounds__(256) kg_bound(const GridView *__restrict__ views,
+                                                const unsigned *__restrict__ first, int n) {
   HG_GROUP_PRELUDE
-  bound_x1_body(v.pf, v.geo, v.d, v.gammamax, v.err, bid);
-}
-
-__global__ void __launch_bounds__(256) kg_bound_x2(const GridView *__restrict__ views,
-                                                   const unsigned *__restrict__ first, int n) {
-  HG_GROUP_PRELUDE
-  bound_x2_body(v.pf, v.d, bid);
-}
-
-__global__ void __launch_bounds__(256) kg_bound_x3(const GridView *__restrict__ views,
-                                                   const unsigned *__restrict__ first, int n) {
-  HG_GROUP_PRELUDE
-  bound_x3_body(v.pf, v.d, bid);
+  if (FIRST && v.finalstep && bid == 0 && threadIdx.x == 0) dt_body(v.ndt_bits, v.dt, v.defcon, v.safe);
+  bound_body(v.pf, v.geo, v.d, v.gammamax, v.err, bid);
 }
 
 template <int DIR, bool KS>
@@ -1074,12 +1096,6 @@ __global__ void __launch_bounds__(256) kg_invert(const GridView *__restrict__ vi
   HG_GROUP_PRELUDE
   invert_body<false, MODE, KS>(v.uf, v.pb, v.pf, v.geo, v.floors, v.finalstep, v.d, v.gam, v.gammamax, v.counters,
                            v.pflag, nullptr, MODE == INV_LEARNED ? v.ly : nullptr, v.fx.count, v.err, bid);
-}
-
-__global__ void kg_dt(const GridView *__restrict__ views, const unsigned *__restrict__ first, int n) {
-  HG_GROUP_PRELUDE
-  (void)bid;
-  if (threadIdx.x == 0) dt_body(v.ndt_bits, v.dt, v.defcon, v.safe);
 }
 #undef HG_GROUP_PRELUDE
 
@@ -1148,19 +1164,17 @@ static inline unsigned nblocks(int64_t n, int bs) { return (unsigned)((n + bs - 
     else hipLaunchKernelGGL((K<A, B, false>), g, b, 0, s, __VA_ARGS__);              \
   } while (0)
 
-void launch_bound(double *p, const double *geo, const Dims &d, double gammamax, int *err, hipStream_t s) {
-  if (d.n1 > 1) {
-    int64_t n = 2LL * d.nb1 * d.n2 * d.n3;
-    hipLaunchKernelGGL(k_bound_x1, dim3(nblocks(n, 128)), dim3(128), 0, s, p, geo, d, gammamax, err);
-  }
-  if (d.n2 > 1) {
-    int64_t n = 2LL * d.nb2 * d.n3 * d.m1;
-    hipLaunchKernelGGL(k_bound_x2, dim3(nblocks(n, 256)), dim3(256), 0, s, p, d);
-  }
-  if (d.n3 > 1) {
-    int64_t n = 2LL * d.nb3 * d.m2 * d.m1;
-    hipLaunchKernelGGL(k_bound_x3, dim3(nblocks(n, 256)), dim3(256), 0, s, p, d);
-  }
+static unsigned bound_total(const Dims &d) {
+  unsigned nblk[3];
+  bound_blocks(d, nblk);
+  return nblk[0] + nblk[1] + nblk[2];
+}
+
+void launch_bound(double *p, const double *geo, const Dims &d, double gammamax, int *err, hipStream_t s,
+                  const StepDt &se) {
+  // a grid of one zone has no ghosts, but its step has a dt
+  const unsigned nb = bound_total(d);
+  if (nb || se.dt) hipLaunchKernelGGL(k_bound, dim3(nb ? nb : 1), dim3(256), 0, s, p, geo, d, gammamax, err, se);
 }
 
 void launch_flux_point(int dir, int lim, bool fv, const double *p, const double *geo, double *F, const Dims &d,
@@ -1405,10 +1419,6 @@ void launch_step_features(const double *ubuf, const double *pb, const double *ge
   hipLaunchKernelGGL(k_step_features, dim3(nblocks(n, 256)), dim3(256), 0, s, ubuf, pb, geo, d, gam, X);
 }
 
-void launch_dt(unsigned long long *ndt_bits, double *dtp, double defcon, double safe, hipStream_t s) {
-  hipLaunchKernelGGL(k_dt, dim3(1), dim3(1), 0, s, ndt_bits, dtp, defcon, safe);
-}
-
 void launch_reset_ndt(unsigned long long *ndt_bits, hipStream_t s) {
   hipLaunchKernelGGL(k_reset_ndt, dim3(1), dim3(64), 0, s, ndt_bits);
 }
@@ -1420,9 +1430,7 @@ unsigned group_blocks(int k, const GridView &v) {
   const int s1 = d.n1 > 1, s2 = d.n2 > 1, s3 = d.n3 > 1;
   const int64_t act = (int64_t)d.n1 * d.n2 * d.n3;
   switch (k) {
-    case GK_BOUND1: return s1 ? nblocks(2LL * d.nb1 * d.n2 * d.n3, 128) : 0u;
-    case GK_BOUND2: return s2 ? nblocks(2LL * d.nb2 * d.n3 * d.m1, 256) : 0u;
-    case GK_BOUND3: return s3 ? nblocks(2LL * d.nb3 * d.m2 * d.m1, 256) : 0u;
+    case GK_BOUND: case GK_BOUNDDT: return bound_total(d) ? bound_total(d) : 1u;
     case GK_FLUX1: case GK_FLUX2: case GK_FLUX3: {
       const int dir = 1 + k - GK_FLUX1;
       if (!((dir == 1) ? s1 : (dir == 2) ? s2 : s3)) return 0u;
@@ -1431,7 +1439,6 @@ unsigned group_blocks(int k, const GridView &v) {
     }
     case GK_EMF: return nblocks((int64_t)(d.n1 + s1) * (d.n2 + s2) * (d.n3 + s3), 256);
     case GK_UPDATE: case GK_UPDATEU: case GK_INVERT: case GK_FEATURES: return nblocks(act, 256);
-    case GK_DT: return 1u;
     case GK_FXCHECK: case GK_FXRESOLVE: case GK_FXAVG: case GK_FXAPPLY: return group_blocks_fixup(k, v);
     default: return group_blocks_weno(k, v);
   }
@@ -1442,9 +1449,8 @@ void launch_group(int k, const GridView *views, const unsigned *first, int n, un
   if (total == 0) return;
   const dim3 g(total);
   switch (k) {
-    case GK_BOUND1: hipLaunchKernelGGL(kg_bound_x1, g, dim3(128), 0, s, views, first, n); return;
-    case GK_BOUND2: hipLaunchKernelGGL(kg_bound_x2, g, dim3(256), 0, s, views, first, n); return;
-    case GK_BOUND3: hipLaunchKernelGGL(kg_bound_x3, g, dim3(256), 0, s, views, first, n); return;
+    case GK_BOUNDDT: hipLaunchKernelGGL(kg_bound<true>, g, dim3(256), 0, s, views, first, n); return;
+    case GK_BOUND: hipLaunchKernelGGL(kg_bound<false>, g, dim3(256), 0, s, views, first, n); return;
     case GK_FLUX1: HG_LAUNCH_KS(ks, kg_flux_lr, 1, g, dim3(256), views, first, n); return;
     case GK_FLUX2: HG_LAUNCH_KS(ks, kg_flux_lr, 2, g, dim3(256), views, first, n); return;
     case GK_FLUX3: HG_LAUNCH_KS(ks, kg_flux_lr, 3, g, dim3(256), views, first, n); return;
@@ -1457,7 +1463,6 @@ void launch_group(int k, const GridView *views, const unsigned *first, int n, un
       else HG_LAUNCH_KS(ks, kg_invert, INV_FP64, g, dim3(256), views, first, n);
       return;
     case GK_FEATURES: hipLaunchKernelGGL(kg_step_features, g, dim3(256), 0, s, views, first, n); return;
-    case GK_DT: hipLaunchKernelGGL(kg_dt, g, dim3(64), 0, s, views, first, n); return;
     case GK_FXCHECK: case GK_FXRESOLVE: case GK_FXAVG: case GK_FXAPPLY:
       launch_group_fixup(k, views, first, n, total, s);
       return;
