@@ -25,6 +25,7 @@
 //                 read from the primitives as they were before any fix
 //                 (ORDERINDEPENDENT), which no kernel writes until
 //   k_fx_apply    writes the list back.
+// A small grid takes the four steps in one launch (k_fx_all).
 // Flags are int8 in the layout of one primitive; ghost flags are not stored:
 // bound_pflag (boundsint.c:6) for outflow x1, polar x2, periodic x3 is the
 // index map (clamp i, mirror j, wrap k) onto the active zones' inversion codes.
@@ -382,6 +383,52 @@ __global__ void __launch_bounds__(256) k_fx_apply(double *__restrict__ p, Dims d
   fx_apply_body(p, d, b, blockIdx.x, gridDim.x);
 }
 
+// The four kernels as one launch for a grid of at most FX_ONE_ZONES zones: the
+// block that finishes the check last goes on with the lists alone.  On a
+// small grid the lists are short or empty and the launches are all that the
+// four cost: 128^2 zones take 8.5 us and three gaps of 2 to 4 us in four
+// launches, 5.9 us in this one.  The bound keeps the case where every zone is on a
+// list at 128 rounds of one block.  Every block releases what it wrote before
+// it takes its ticket; the last one acquires that before it reads.  The release
+// writes the L2 back, so it is taken once per block (by every wavefront: 8.7 us), and
+// the grouped launch, whose hundreds of blocks share the L2s, keeps the four
+// (41 us in one launch against 29 us).  count[3] is the ticket, zero again when the
+// launch ends.
+constexpr int64_t FX_ONE_ZONES = 32768;
+
+__device__ __forceinline__ bool fx_last_block(unsigned *ticket, unsigned nblk) {
+  __shared__ unsigned mine;
+  __builtin_amdgcn_s_waitcnt(0);  // this wavefront's stores and atomics are in the L2
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __threadfence();  // and written back from it, for the other XCDs
+    mine = atomicAdd(ticket, 1u);
+  }
+  __syncthreads();
+  if (mine != nblk - 1) return false;
+  __threadfence();
+  return true;
+}
+
+__device__ __forceinline__ void fx_all_body(double *p, const double *__restrict__ geo, const Dims &d, const FxBufs &b,
+                                            int finalstep, double gammamax, double gam, double *__restrict__ ucons,
+                                            int *__restrict__ err, unsigned bid, unsigned nblk) {
+  fx_check_body(p, geo, d, b, err, bid);
+  if (!fx_last_block(&b.count[3], nblk)) return;
+  fx_resolve_body(d, b, err);
+  __syncthreads();
+  fx_average_body(p, geo, d, b, finalstep, gammamax, gam, ucons, err, 0, 1);
+  __syncthreads();
+  fx_apply_body(p, d, b, 0, 1);
+  if (threadIdx.x == 0) b.count[3] = 0u;
+}
+
+__global__ void __launch_bounds__(256) k_fx_all(double *p, const double *__restrict__ geo, Dims d, FxBufs b,
+                                                int finalstep, double gammamax, double gam,
+                                                double *__restrict__ ucons, int *__restrict__ err) {
+  fx_all_body(p, geo, d, b, finalstep, gammamax, gam, ucons, err, blockIdx.x, gridDim.x);
+}
+
 // grouped launches (one per class over several grids; the standard scheme,
 // so no carried conserved state)
 #define FX_GROUP_PRELUDE                              \
@@ -444,7 +491,8 @@ int fixup_alloc(hg_ctx *c) {
   get((void **)&c->fx_fix_v, (size_t)act * 5 * sizeof(double));
   get((void **)&c->fx_fix_flag, (size_t)act);
   get((void **)&c->fx_fail_z, (size_t)act * sizeof(int));
-  get((void **)&c->fx_count, 3 * sizeof(unsigned));
+  get((void **)&c->fx_count, 4 * sizeof(unsigned));
+  if (e == hipSuccess) e = hipMemset(c->fx_count, 0, 4 * sizeof(unsigned));
   if (e == hipSuccess) e = hipMemset(c->pflag, 0, (size_t)d.spl);
   if (e != hipSuccess) {
     set_error("hg_ctx_create: %s", hipGetErrorString(e));
@@ -484,6 +532,11 @@ void launch_post_fixup(hg_ctx *c, double *p, int finalstep, hipStream_t s, bool 
   int64_t n = (int64_t)d.n1 * d.n2 * d.n3;
   unsigned nb = (unsigned)((n + 255) / 256);
   if (reset) hipLaunchKernelGGL(k_fx_reset, dim3(1), dim3(64), 0, s, b.count);
+  if (n <= FX_ONE_ZONES) {
+    hipLaunchKernelGGL(k_fx_all, dim3(nb), dim3(256), 0, s, p, c->geo, d, b, finalstep, c->cfg.gammamax, c->cfg.gam,
+                       c->ucons, c->err);
+    return;
+  }
   hipLaunchKernelGGL(k_fx_check, dim3(nb), dim3(256), 0, s, p, c->geo, d, b, c->err);
   hipLaunchKernelGGL(k_fx_resolve, dim3(1), dim3(1024), 0, s, d, b, c->err);
   hipLaunchKernelGGL(k_fx_average, dim3(256), dim3(256), 0, s, p, c->geo, d, b, finalstep, c->cfg.gammamax,

@@ -103,7 +103,7 @@ struct FxBufs {
   double *fix_v;       // their RHO..U3 (5 x cap, structure of arrays)
   int8_t *fix_flag;    // their final flag
   int *fail_z;         // failed inversions that are not candidates
-  unsigned *count;     // [candidates, fixes, failed non-candidates]
+  unsigned *count;     // [candidates, fixes, failed non-candidates, blocks done (k_fx_all)]
   int cap;
 };
 
