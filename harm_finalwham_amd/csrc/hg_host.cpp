@@ -110,6 +110,7 @@ extern "C" int hg_ctx_create(const hg_config *cfg, hg_ctx **out) {
     hipError_t e = hipMalloc((void **)&c->ndt_bits, 3 * sizeof(unsigned long long));
     if (e == hipSuccess) e = hipMalloc((void **)&c->counters, 2 * sizeof(unsigned long long));
     if (e == hipSuccess) e = hipMalloc((void **)&c->err, sizeof(int));
+    if (e == hipSuccess) e = hipHostMalloc((void **)&c->out, sizeof(StepOut), hipHostMallocDefault);
     if (e == hipSuccess) e = hipMemset(c->counters, 0, 2 * sizeof(unsigned long long));
     if (e == hipSuccess) e = hipMemset(c->err, 0, sizeof(int));
     for (int k = 0; k < 2 && e == hipSuccess; k++) {
@@ -135,6 +136,7 @@ extern "C" int hg_ctx_destroy(hg_ctx *c) {
   if (c->ndt_bits) (void)hipFree(c->ndt_bits);
   if (c->counters) (void)hipFree(c->counters);
   if (c->err) (void)hipFree(c->err);
+  if (c->out) (void)hipHostFree(c->out);
   for (int k = 0; k < 2; k++) {
     if (c->xs[k]) (void)hipStreamDestroy(c->xs[k]);
     if (c->ev_join[k]) (void)hipEventDestroy(c->ev_join[k]);
@@ -257,9 +259,7 @@ extern "C" int hg_get_prims(hg_ctx *c, double *p) {
   return fetch_prims(c, c->p, p);
 }
 
-static int check_err(hg_ctx *c) {
-  int e = 0;
-  HIPCHECK(hipMemcpy(&e, c->err, sizeof(int), hipMemcpyDeviceToHost));
+static int report_err(hg_ctx *c, int e) {
   if (e) {
     HIPCHECK(hipMemset(c->err, 0, sizeof(int)));
     set_error("device reported failure mask %d (1: ghost fill, 2: face state, 4: zone update, 8: post_fixup "
@@ -267,6 +267,12 @@ static int check_err(hg_ctx *c) {
     return 1;
   }
   return 0;
+}
+
+static int check_err(hg_ctx *c) {
+  int e = 0;
+  HIPCHECK(hipMemcpy(&e, c->err, sizeof(int), hipMemcpyDeviceToHost));
+  return report_err(c, e);
 }
 
 static int need_geometry(hg_ctx *c, const char *who) {
@@ -435,9 +441,10 @@ static void enqueue_fluxcalc(hg_ctx *c, const double *pb, const Dims &d, bool ca
     prof_mark(c, HG_PROF_PREP, s);
     launch_weno_prep(pb, c->geo, c->aux, d, f.gam, f.doenoflux == HG_ENOFINITEVOLUME, all_dpi, c->ndt_bits, s);
     prof_mark(c, -1, s);
-  } else {
+  } else if (!c->ndt_fresh || captured) {
     launch_reset_ndt(c->ndt_bits, s);
   }
+  c->ndt_fresh = false;
   hipStream_t ds[4] = {nullptr, s, s, s};
   if (conc) {
     (void)hipEventRecord(c->ev_fork, s);
@@ -506,8 +513,9 @@ extern "C" int hg_fluxcalc(hg_ctx *c, double *F1, double *F2, double *F3, double
 }
 
 // one substep of step_ch.c:94-166: advance, bound_prim, post_fixup, bound_prim
+// more: another substep of the same step follows on s
 static void enqueue_substep(hg_ctx *c, double *pi, double *pb, double *pf, const RkStage &rk, int stage,
-                            int finalstep, hipStream_t s) {
+                            int finalstep, bool more, hipStream_t s) {
   const hg_config &f = c->cfg;
   bool captured;
   const Dims d = launch_dims(c, s, captured);
@@ -536,12 +544,17 @@ static void enqueue_substep(hg_ctx *c, double *pi, double *pb, double *pf, const
   // the axis, which the radial inflow check then sees in the corner ghosts
   prof_mark(c, HG_PROF_BOUND, s);
   StepDt se{};
-  if (finalstep) se = StepDt{c->ndt_bits, c->dt, f.defcon, f.safe};
+  if (finalstep) se = StepDt{c->ndt_bits, c->dt, f.defcon, f.safe, nullptr};
   launch_bound(pf, c->geo, c->d, f.gammamax, c->err, s, se);
   prof_mark(c, HG_PROF_FIXUP, s);
   launch_post_fixup(c, pf, finalstep, s, false);
   prof_mark(c, HG_PROF_BOUND, s);
-  launch_bound(pf, c->geo, c->d, f.gammamax, c->err, s);
+  se = StepDt{};
+  if (more && !captured && f.lim != HG_LIM_WENO5BND) {
+    se.reset = c->ndt_bits;
+    c->ndt_fresh = true;
+  }
+  launch_bound(pf, c->geo, c->d, f.gammamax, c->err, s, se);
   prof_mark(c, -1, s);
 }
 
@@ -606,7 +619,7 @@ void hg::enqueue_step(hg_ctx *c, hipStream_t s) {
   double *pb[4], *pf[4];
   RkStage rk[4];
   const int n = step_substeps(c, pb, pf, rk);
-  for (int t = 0; t < n; t++) enqueue_substep(c, c->p, pb[t], pf[t], rk[t], t, t == n - 1, s);
+  for (int t = 0; t < n; t++) enqueue_substep(c, c->p, pb[t], pf[t], rk[t], t, t == n - 1, t < n - 1, s);
 }
 
 extern "C" int hg_set_dt(hg_ctx *c, double dt) {
@@ -658,7 +671,7 @@ extern "C" int hg_advance_substep(hg_ctx *c, int pi, int pb, int pf, const doubl
   const int last = timeorder == numtimeorders - 1;
   if (last) c->unew_in_uf = true;
   RkStage rk{CUf[2], Cunew[0], Cunew[1], Cunew[2], c->ucum, timeorder == 0, last, c->ucons, CUf[0], CUf[1]};
-  enqueue_substep(c, slot[pi], slot[pb], slot[pf], rk, timeorder, last, s);
+  enqueue_substep(c, slot[pi], slot[pb], slot[pf], rk, timeorder, last, false, s);
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipStreamSynchronize(s));
   if (check_err(c)) return 1;
@@ -680,14 +693,20 @@ extern "C" int hg_step(hg_ctx *c, double *dt, int64_t *nfail, int64_t *iters, vo
   // work the caller queued on s (hg_step_async) still reads dt and adds to
   // the counters: let it finish before they are set
   HIPCHECK(hipStreamSynchronize(s));
-  if (hg_set_dt(c, *dt)) return 1;
-  HIPCHECK(hipMemset(c->counters, 0, 2 * sizeof(unsigned long long)));
+  // the state may have been written on the default stream
+  if (s) HIPCHECK(hipStreamSynchronize(nullptr));
+  launch_step_begin(*dt, c->dt, c->ndt_bits, c->counters, s);
+  c->ndt_fresh = true;
   enqueue_step(c, s);
+  launch_step_end(c->dt, c->counters, c->err, c->out, s);
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipStreamSynchronize(s));
-  if (check_err(c)) return 1;
-  if (hg_get_dt(c, dt)) return 1;
-  return hg_get_counters(c, nfail, iters);
+  const StepOut o = *c->out;
+  if (report_err(c, o.err)) return 1;
+  *dt = o.dt;
+  if (nfail) *nfail = (int64_t)o.counters[0];
+  if (iters) *iters = (int64_t)o.counters[1];
+  return 0;
 }
 
 // the final substep's inversions of the last step (advance.c:193-201): the

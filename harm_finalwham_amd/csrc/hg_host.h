@@ -49,6 +49,10 @@ struct hg_ctx {
   double *dt = nullptr;
   unsigned long long *ndt_bits = nullptr, *counters = nullptr;
   int *err = nullptr;
+  hg::StepOut *out = nullptr;  // pinned: what hg_step reads back
+  // ndt_bits hold no direction's limit yet: the next fluxcalc need not reset
+  // them (set by the launch before it on the same stream, never in a capture)
+  bool ndt_fresh = false;
   // post_fixup: inversion codes and checked codes (int8, layout of one
   // primitive), candidate and fix lists (hg_fixup.hip)
   int8_t *pflag = nullptr, *pchk = nullptr;

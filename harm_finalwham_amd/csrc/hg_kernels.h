@@ -19,11 +19,25 @@ struct Tune {
 };
 
 // the time step of a final substep, stored by the ghost fill after it
+// reset: the ndt slots that the next substep's fluxes start from, or none
 struct StepDt {
   const unsigned long long *ndt_bits;
   double *dt;
   double defcon, safe;
+  unsigned long long *reset;
 };
+// hg_step's scalars: dt and cleared counters go in by a kernel's arguments, and
+// the next dt, the counters (cleared again unless a failure is reported) and
+// the failure mask come back through pinned memory.  As copies and a fill
+// these were six calls that each wait for the device, 62 us of a step.
+struct StepOut {
+  double dt;
+  unsigned long long counters[2];
+  int err;
+};
+void launch_step_begin(double dt, double *dtp, unsigned long long *ndt_bits, unsigned long long *counters,
+                       hipStream_t s);
+void launch_step_end(const double *dtp, unsigned long long *counters, const int *err, StepOut *out, hipStream_t s);
 void launch_bound(double *p, const double *geo, const Dims &d, double gammamax, int *err, hipStream_t s,
                   const StepDt &se = StepDt{});
 // point-type reconstruction (lim: HG_LIM_PARA, HG_LIM_MC or another

@@ -226,11 +226,17 @@ __device__ __forceinline__ void dt_body(const unsigned long long *ndt_bits, doub
   dtp[0] = ndt;
 }
 
+__device__ __forceinline__ void reset_ndt_body(unsigned long long *ndt_bits) {
+  if (threadIdx.x < 3) ndt_bits[threadIdx.x] = (unsigned long long)__double_as_longlong(1.e+50);
+}
+
 // se: where the final substep's time step goes (the fluxes' ndt and the update
-// that reads dt are done); no address on other substeps
+// that reads dt are done), or the slots the next substep's fluxes reduce into;
+// no addresses otherwise
 __global__ void __launch_bounds__(256) k_bound(double *p, const double *__restrict__ geo, Dims d, double gammamax,
                                                int *__restrict__ err, StepDt se) {
   if (se.dt && blockIdx.x == 0 && threadIdx.x == 0) dt_body(se.ndt_bits, se.dt, se.defcon, se.safe);
+  if (se.reset && blockIdx.x == 0) reset_ndt_body(se.reset);
   bound_body(p, geo, d, gammamax, err, blockIdx.x);
 }
 
@@ -1099,8 +1105,21 @@ __global__ void __launch_bounds__(256) kg_invert(const GridView *__restrict__ vi
 }
 #undef HG_GROUP_PRELUDE
 
-__global__ void k_reset_ndt(unsigned long long *ndt_bits) {
-  if (threadIdx.x < 3) ndt_bits[threadIdx.x] = (unsigned long long)__double_as_longlong(1.e+50);
+__global__ void k_reset_ndt(unsigned long long *ndt_bits) { reset_ndt_body(ndt_bits); }
+
+__global__ void k_step_begin(double dt, double *dtp, unsigned long long *ndt_bits, unsigned long long *counters) {
+  reset_ndt_body(ndt_bits);
+  if (threadIdx.x < 2) counters[threadIdx.x] = 0ull;
+  if (threadIdx.x == 0) dtp[0] = dt;
+}
+
+__global__ void k_step_end(const double *dtp, unsigned long long *counters, const int *err, StepOut *out) {
+  const int e = *err;
+  out->dt = *dtp;
+  out->counters[0] = counters[0];
+  out->counters[1] = counters[1];
+  out->err = e;
+  if (!e) counters[0] = counters[1] = 0ull;
 }
 
 // ---------------------------------------------------------------------------
@@ -1174,7 +1193,7 @@ void launch_bound(double *p, const double *geo, const Dims &d, double gammamax, 
                   const StepDt &se) {
   // a grid of one zone has no ghosts, but its step has a dt
   const unsigned nb = bound_total(d);
-  if (nb || se.dt) hipLaunchKernelGGL(k_bound, dim3(nb ? nb : 1), dim3(256), 0, s, p, geo, d, gammamax, err, se);
+  if (nb || se.dt || se.reset) hipLaunchKernelGGL(k_bound, dim3(nb ? nb : 1), dim3(256), 0, s, p, geo, d, gammamax, err, se);
 }
 
 void launch_flux_point(int dir, int lim, bool fv, const double *p, const double *geo, double *F, const Dims &d,
@@ -1417,6 +1436,15 @@ void launch_step_features(const double *ubuf, const double *pb, const double *ge
                           float *X, hipStream_t s) {
   int64_t n = (int64_t)d.n1 * d.n2 * d.n3;
   hipLaunchKernelGGL(k_step_features, dim3(nblocks(n, 256)), dim3(256), 0, s, ubuf, pb, geo, d, gam, X);
+}
+
+void launch_step_begin(double dt, double *dtp, unsigned long long *ndt_bits, unsigned long long *counters,
+                       hipStream_t s) {
+  hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(64), 0, s, dt, dtp, ndt_bits, counters);
+}
+
+void launch_step_end(const double *dtp, unsigned long long *counters, const int *err, StepOut *out, hipStream_t s) {
+  hipLaunchKernelGGL(k_step_end, dim3(1), dim3(1), 0, s, dtp, counters, err, out);
 }
 
 void launch_reset_ndt(unsigned long long *ndt_bits, hipStream_t s) {
