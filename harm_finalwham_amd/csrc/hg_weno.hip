@@ -30,6 +30,8 @@
 // All arithmetic is FP64 in the reference's operation order.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include <cfloat>
 
 #include "hg_div.h"
@@ -702,13 +704,22 @@ static void weno_march_shape(int dir, const Dims &d, const Tune &tu, int wide, i
   const int n = (dir == 1) ? d.n1 : (dir == 2) ? d.n2 : d.n3;
   const int64_t lanes = (dir == 1) ? (int64_t)(d.n2 + 2 * s2) * (d.n3 + 2 * s3)
                                    : (int64_t)(d.n1 + 2 * s1) * ((dir == 2) ? d.n3 + 2 * s3 : d.n2 + 2 * s2);
-  // split long lines so that the grid holds enough wavefronts
+  // Split lines so that the launch holds a full device of wavefronts (four per
+  // SIMD, 4096), in segments of at least 4 points: a wavefront walks its
+  // segment point by point after 6 points of run-up, so short of a full device
+  // the time is the segment's length, and beyond it the run-ups'.  Per
+  // step of two substeps, against one segment (two from 96 rows on):
+  // 128^2 430 -> 230 us, 59x19x7 318 -> 260, 64^3 860 -> 725, 128x64x32
+  // 833 -> 711; for 8192 wavefronts 64^3 takes 770 us, with segments of 2
+  // points 48x32x16 292 us instead of 281.
+  nlb = (int)((lanes + 255) / 256);
+  const int64_t fill = 4096 / ((int64_t)nlb * 4 * NPR);
+  const int def = (n + 2 >= 96) ? 2 : 1;
   const int want = (dir == 1) ? tu.weno_xmarch : (dir == 2) ? tu.weno_nseg : tu.weno_nseg3;
-  nseg = want > 0 ? want : ((n + 2 >= 96) ? 2 : 1);
+  nseg = want > 0 ? want : (int)std::max((int64_t)def, std::min(fill, (int64_t)((n + 2) / 4)));
   if (nseg > n + 2) nseg = n + 2;
   seglen = (n + 2 + nseg - 1) / nseg;
   nseg = (n + 2 + seglen - 1) / seglen;  // every segment starts at or before point n
-  nlb = (int)((lanes + 255) / 256);
 }
 
 void launch_weno(int dir, const double *p, double *aux, double *pleft, double *pright, const Dims &d,
