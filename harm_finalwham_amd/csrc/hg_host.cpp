@@ -429,17 +429,22 @@ static void enqueue_fluxcalc(hg_ctx *c, const double *pb, const Dims &d, bool ca
   // caller's: the fork records the context's own events onto its own side
   // streams, which a capture would pull into the graph, and that path is
   // kept out of captures (a graph runs its grids side by side instead).
-  const bool conc = c->tune.concurrent && !c->prof_on && !captured;
+  // A small grid takes its directions' fluxes in one launch instead (flux_dirs),
+  // captured or not.
+  const bool weno = f.lim == HG_LIM_WENO5BND;
+  const bool fv = f.doenoflux == HG_ENOFINITEVOLUME;
+  FluxDirs fd{};
+  const bool dirs = !c->prof_on && flux_dirs(d, fv, f.fluxmethod, c->tune, fd) && (!weno || weno_dirs(c->tune));
+  const bool conc = c->tune.concurrent && !dirs && !c->prof_on && !captured;
   // Run one after another, the three directions' dP/P indicators take one
   // launch with the shared inputs' (fewer launches for the small grids of a
   // graph); a profile keeps them with their directions, as the concurrent
   // step runs them.  The prep kernel also resets the ndt slots.
-  const bool weno = f.lim == HG_LIM_WENO5BND;
   const bool all_dpi = !conc && !c->prof_on;
   if (weno) {
     // the dP/P inputs are shared by the three directions
     prof_mark(c, HG_PROF_PREP, s);
-    launch_weno_prep(pb, c->geo, c->aux, d, f.gam, f.doenoflux == HG_ENOFINITEVOLUME, all_dpi, c->ndt_bits, s);
+    launch_weno_prep(pb, c->geo, c->aux, d, f.gam, fv, all_dpi, c->ndt_bits, s);
     prof_mark(c, -1, s);
   } else if (!c->ndt_fresh || captured) {
     launch_reset_ndt(c->ndt_bits, s);
@@ -455,11 +460,21 @@ static void enqueue_fluxcalc(hg_ctx *c, const double *pb, const Dims &d, bool ca
       }
   }
   double *pls[4] = {nullptr, c->pl, c->pl2, c->pl3}, *prs[4] = {nullptr, c->pr, c->pr2, c->pr3};
+  if (dirs) {
+    for (int k = 0; k < 3; k++) {
+      fd.F[k] = c->F[k];
+      fd.pl[k] = pls[k + 1];
+      fd.pr[k] = prs[k + 1];
+      fd.dx[k] = f.dx[k + 1];
+    }
+    if (weno) launch_weno_dirs(pb, c->aux, fd, d, c->tune, fv, s);
+    launch_flux_dirs(fd, f.lim, fv, pb, c->geo, d, f.gam, f.cour, f.fluxmethod, c->ndt_bits, c->err, s);
+  }
   // concurrent: the side streams' work first; a profile keeps the order 1, 2, 3
   const int order[2][3] = {{1, 2, 3}, {3, 2, 1}};
   for (int o = 0; o < 3; o++) {
     const int dir = order[conc ? 1 : 0][o];
-    if (nn[dir] <= 1) continue;
+    if (dirs || nn[dir] <= 1) continue;
     hipStream_t sd = ds[dir];
     if (f.lim != HG_LIM_WENO5BND) {
       prof_mark(c, HG_PROF_FLUX1 + dir - 1, sd);

@@ -15,7 +15,7 @@ struct Tune {
   int bs_flux = 256, bs_emf = 256, bs_update = 256, bs_invert = 256;
   int weno_xwaves = 4, weno_nseg = 0, weno_nseg3 = 0;  // segments per line along j, along k
   int weno_xmarch = 0;  // along i: 0 = one lane per point (shuffles), n > 0 = marching, n segments
-  int concurrent = 1;   // 1: the three directions' fluxes on three streams, 0: one after another
+  int concurrent = 1;   // 1: the three directions' fluxes side by side, 0: one after another
 };
 
 // the time step of a final substep, stored by the ghost fill after it
@@ -49,6 +49,24 @@ void launch_flux_point(int dir, int lim, bool fv, const double *p, const double 
 // primtoU of every active zone of p into U (same layout)
 void launch_cons_from_prims(const double *p, const double *geo, double *U, const Dims &d, double gam, int *err,
                             hipStream_t s);
+// the fluxes of the active directions in one launch: their arrays, zone sizes
+// and first blocks.  flux_dirs sets the blocks and tells whether the grid takes
+// that launch (small, default launch shapes, LAXF or HLL)
+struct FluxDirs {
+  double *F[3];
+  double *pl[3], *pr[3];  // WENO5BND: the interface states
+  double dx[3];
+  unsigned first[3], nblocks;
+};
+bool flux_dirs(const Dims &d, bool fv, int fluxmethod, const Tune &tu, FluxDirs &f);
+void launch_flux_dirs(const FluxDirs &f, int lim, bool fv, const double *p, const double *geo, const Dims &d,
+                      double gam, double cour, int fluxmethod, unsigned long long *ndt_bits, int *err, hipStream_t s);
+// the reconstruction of the active directions in one launch, after
+// launch_weno_prep formed every direction's indicator (weno_dirs: whether the
+// tuned launch shapes allow it)
+bool weno_dirs(const Tune &tu);
+void launch_weno_dirs(const double *p, const double *aux, const FluxDirs &f, const Dims &d, const Tune &tu, int wide,
+                      hipStream_t s);
 void launch_flux_lr(int dir, const double *pleft, const double *pright, const double *geo, double *F,
                     const Dims &d, double gam, double cour, double dxdir, int fluxmethod,
                     unsigned long long *ndt_bits, int *err, const Tune &tu, bool fv, hipStream_t s);

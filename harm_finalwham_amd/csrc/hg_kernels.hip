@@ -531,8 +531,9 @@ template <int DIR, bool PARA, bool EXT = false, bool KS = false>
 __device__ __forceinline__ void flux_point_body(const double *__restrict__ p, const double *__restrict__ geo,
                                                 double *__restrict__ F, const Dims &d, const FaceRange &fr,
                                                 double gam, double cour, double dxdir, int fluxmethod, int slim,
-                                                unsigned long long *__restrict__ ndt_bits, int *__restrict__ err) {
-  int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+                                                unsigned long long *__restrict__ ndt_bits, int *__restrict__ err,
+                                                unsigned bid) {
+  int64_t t = bid * (int64_t)blockDim.x + threadIdx.x;
   int64_t total = (int64_t)fr.ni * fr.nj * fr.nk;
   double dtij = 1.e+50;
   if (t < total) {
@@ -591,7 +592,7 @@ __global__ void __launch_bounds__(256) k_flux_mc(const double *__restrict__ p, c
                                                  double dxdir, int fluxmethod, int slim,
                                                  unsigned long long *__restrict__ ndt_bits, int *__restrict__ err) {
   FaceRange fr = face_range(d, DIR);
-  flux_point_body<DIR, false, false, KS>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err);
+  flux_point_body<DIR, false, false, KS>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err, blockIdx.x);
 }
 
 template <int DIR, bool KS>
@@ -601,7 +602,7 @@ __global__ void __launch_bounds__(256) k_flux_para(const double *__restrict__ p,
                                                    unsigned long long *__restrict__ ndt_bits,
                                                    int *__restrict__ err) {
   FaceRange fr = face_range(d, DIR);
-  flux_point_body<DIR, true, false, KS>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err);
+  flux_point_body<DIR, true, false, KS>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err, blockIdx.x);
 }
 
 // the finite-volume flux loops (every transverse ghost row)
@@ -612,7 +613,7 @@ __global__ void __launch_bounds__(256) k_flux_pt_fv(const double *__restrict__ p
                                                     unsigned long long *__restrict__ ndt_bits,
                                                     int *__restrict__ err) {
   FaceRange fr = face_range_fv(d, DIR);
-  flux_point_body<DIR, PARA, false, KS>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err);
+  flux_point_body<DIR, PARA, false, KS>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err, blockIdx.x);
 }
 
 // MC or PARA with the FORCE / MUSTA / HLLLAXF1 fluxes
@@ -623,7 +624,7 @@ __global__ void __launch_bounds__(256) k_flux_pt_ext(const double *__restrict__ 
                                                      unsigned long long *__restrict__ ndt_bits,
                                                      int *__restrict__ err) {
   FaceRange fr = fv ? face_range_fv(d, DIR) : face_range(d, DIR);
-  flux_point_body<DIR, PARA, true>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err);
+  flux_point_body<DIR, PARA, true>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err, blockIdx.x);
 }
 
 template <int DIR, bool EXT, bool KS = false>
@@ -700,6 +701,52 @@ __global__ void __launch_bounds__(256) k_flux_lr_ext(const double *__restrict__ 
                                                      int *__restrict__ err) {
   FaceRange fr = fv ? face_range_fv(d, DIR) : face_range(d, DIR);
   flux_lr_body<DIR, true>(pleft, pright, geo, F, d, fr, gam, cour, dxdir, fluxmethod, ndt_bits, err, blockIdx.x);
+}
+
+// The three directions' fluxes of a grid of up to DIRS_BLOCKS blocks in one launch,
+// direction 1's blocks first.  Small grids leave the device idle one direction
+// at a time, and the side streams' fork and join (20 us of a substep) and the
+// extra launches cost more than their work.  A step against the three streams:
+//                   59x19x7   128^2   64^3   128x64x32  128x128x32  256x128x64
+//   WENO5BND (us)   262->182  229->174 731->708 715->689  1209->1210  3852->4059
+//   MC              198->123  168->118 375->347 381->349   595->599   2074->2347
+//   PARA, RK4, FV   459->323  371->265 990->884 998->885  1779->1672  5757->5703
+// 128x64x32 has 3400 (FV: 4600) blocks; on large grids every direction fills the
+// device, and the register count of one kernel for all keeps fewer wavefronts.
+template <bool PARA, bool FV, bool KS>
+__global__ void __launch_bounds__(256) k_flux_pt_dirs(const double *__restrict__ p, const double *__restrict__ geo,
+                                                      FluxDirs f, Dims d, double gam, double cour, int fluxmethod,
+                                                      int slim, unsigned long long *__restrict__ ndt_bits,
+                                                      int *__restrict__ err) {
+  const unsigned b = blockIdx.x;
+  const int dir = b < f.first[1] ? 1 : b < f.first[2] ? 2 : 3;
+  const FaceRange fr = FV ? face_range_fv(d, dir) : face_range(d, dir);
+  if (dir == 1)
+    flux_point_body<1, PARA, false, KS>(p, geo, f.F[0], d, fr, gam, cour, f.dx[0], fluxmethod, slim, ndt_bits, err, b);
+  else if (dir == 2)
+    flux_point_body<2, PARA, false, KS>(p, geo, f.F[1], d, fr, gam, cour, f.dx[1], fluxmethod, slim, ndt_bits + 1,
+                                        err, b - f.first[1]);
+  else
+    flux_point_body<3, PARA, false, KS>(p, geo, f.F[2], d, fr, gam, cour, f.dx[2], fluxmethod, slim, ndt_bits + 2,
+                                        err, b - f.first[2]);
+}
+
+template <bool FV, bool KS>
+__global__ void __launch_bounds__(256) k_flux_lr_dirs(const double *__restrict__ geo, FluxDirs f, Dims d, double gam,
+                                                      double cour, int fluxmethod,
+                                                      unsigned long long *__restrict__ ndt_bits,
+                                                      int *__restrict__ err) {
+  const unsigned b = blockIdx.x;
+  const int dir = b < f.first[1] ? 1 : b < f.first[2] ? 2 : 3;
+  const FaceRange fr = FV ? face_range_fv(d, dir) : face_range(d, dir);
+  if (dir == 1)
+    flux_lr_body<1, false, KS>(f.pl[0], f.pr[0], geo, f.F[0], d, fr, gam, cour, f.dx[0], fluxmethod, ndt_bits, err, b);
+  else if (dir == 2)
+    flux_lr_body<2, false, KS>(f.pl[1], f.pr[1], geo, f.F[1], d, fr, gam, cour, f.dx[1], fluxmethod, ndt_bits + 1,
+                               err, b - f.first[1]);
+  else
+    flux_lr_body<3, false, KS>(f.pl[2], f.pr[2], geo, f.F[2], d, fr, gam, cour, f.dx[2], fluxmethod, ndt_bits + 2,
+                               err, b - f.first[2]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1194,6 +1241,39 @@ void launch_bound(double *p, const double *geo, const Dims &d, double gammamax, 
   // a grid of one zone has no ghosts, but its step has a dt
   const unsigned nb = bound_total(d);
   if (nb || se.dt || se.reset) hipLaunchKernelGGL(k_bound, dim3(nb ? nb : 1), dim3(256), 0, s, p, geo, d, gammamax, err, se);
+}
+
+constexpr unsigned DIRS_BLOCKS = 5000;
+
+bool flux_dirs(const Dims &d, bool fv, int fluxmethod, const Tune &tu, FluxDirs &f) {
+  const int nn[3] = {d.n1, d.n2, d.n3};
+  uint64_t at = 0;
+  for (int k = 0; k < 3; k++) {
+    f.first[k] = (unsigned)at;
+    if (nn[k] > 1) {
+      const FaceRange fr = fv ? face_range_fv(d, k + 1) : face_range(d, k + 1);
+      at += ((uint64_t)fr.ni * fr.nj * fr.nk + 255) / 256;
+    }
+    if (at > DIRS_BLOCKS) return false;
+  }
+  f.nblocks = (unsigned)at;
+  return tu.concurrent && tu.bs_flux == 256 && fluxmethod < 2 && at > 0;
+}
+
+void launch_flux_dirs(const FluxDirs &f, int lim, bool fv, const double *p, const double *geo, const Dims &d,
+                      double gam, double cour, int fluxmethod, unsigned long long *ndt_bits, int *err,
+                      hipStream_t s) {
+  const dim3 g(f.nblocks), b(256);
+  if (lim == HG_LIM_WENO5BND) {
+    if (fv) HG_LAUNCH_KS(d.ks, k_flux_lr_dirs, true, g, b, geo, f, d, gam, cour, fluxmethod, ndt_bits, err);
+    else HG_LAUNCH_KS(d.ks, k_flux_lr_dirs, false, g, b, geo, f, d, gam, cour, fluxmethod, ndt_bits, err);
+  } else if (lim == HG_LIM_PARA) {
+    if (fv) HG_LAUNCH_KS2(d.ks, k_flux_pt_dirs, true, true, g, b, p, geo, f, d, gam, cour, fluxmethod, lim, ndt_bits, err);
+    else HG_LAUNCH_KS2(d.ks, k_flux_pt_dirs, true, false, g, b, p, geo, f, d, gam, cour, fluxmethod, lim, ndt_bits, err);
+  } else {
+    if (fv) HG_LAUNCH_KS2(d.ks, k_flux_pt_dirs, false, true, g, b, p, geo, f, d, gam, cour, fluxmethod, lim, ndt_bits, err);
+    else HG_LAUNCH_KS2(d.ks, k_flux_pt_dirs, false, false, g, b, p, geo, f, d, gam, cour, fluxmethod, lim, ndt_bits, err);
+  }
 }
 
 void launch_flux_point(int dir, int lim, bool fv, const double *p, const double *geo, double *F, const Dims &d,

@@ -759,6 +759,47 @@ void launch_weno(int dir, const double *p, double *aux, double *pleft, double *p
   }
 }
 
+// the three directions of a small grid in one launch (as k_flux_lr_dirs): the
+// long blocks, along j and k, first
+struct WenoDirs {
+  double *pl[3], *pr[3];
+  int nseg[3], seglen[3], nlb[3];
+  unsigned first[3];  // first block along i, j, k (in the order j, k, i)
+};
+
+__global__ void __launch_bounds__(256) k_weno_dirs(const double *__restrict__ p, const double *__restrict__ aux,
+                                                   WenoDirs w, Dims d, int wide) {
+  const unsigned b = blockIdx.x;
+  if (b < w.first[2])
+    weno_m_body<2>(p, aux + 3 * d.spl, w.pl[1], w.pr[1], d, w.nseg[1], w.seglen[1], wide, w.nlb[1], b);
+  else if (b < w.first[0])
+    weno_m_body<3>(p, aux + 4 * d.spl, w.pl[2], w.pr[2], d, w.nseg[2], w.seglen[2], wide, w.nlb[2], b - w.first[2]);
+  else
+    weno_x_body(p, aux + 2 * d.spl, w.pl[0], w.pr[0], d, wide, b - w.first[0]);
+}
+
+bool weno_dirs(const Tune &tu) { return tu.weno_xmarch == 0 && tu.weno_xwaves == 4; }
+
+void launch_weno_dirs(const double *p, const double *aux, const FluxDirs &f, const Dims &d, const Tune &tu, int wide,
+                      hipStream_t s) {
+  const int s2 = d.n2 > 1 ? (wide ? d.nb2 : 1) : 0, s3 = d.n3 > 1 ? (wide ? d.nb3 : 1) : 0;
+  WenoDirs w{};
+  unsigned at = 0;
+  for (int dir = 2; dir <= 3; dir++) {
+    if (((dir == 2) ? d.n2 : d.n3) > 1) {
+      weno_march_shape(dir, d, tu, wide, w.nseg[dir - 1], w.seglen[dir - 1], w.nlb[dir - 1]);
+      at += (unsigned)(((int64_t)w.nlb[dir - 1] * w.nseg[dir - 1] + 7) / 8 * 8 * NPR);
+    }
+    w.first[dir == 2 ? 2 : 0] = at;
+  }
+  if (d.n1 > 1) at += (unsigned)((weno_x_waves(d, s2, s3) + 3) / 4);
+  for (int k = 0; k < 3; k++) {
+    w.pl[k] = f.pl[k];
+    w.pr[k] = f.pr[k];
+  }
+  hipLaunchKernelGGL(k_weno_dirs, dim3(at), dim3(256), 0, s, p, aux, w, d, wide);
+}
+
 void weno_group_shapes(GridView &v, const Tune &tu) {
   v.nseg[1] = v.seglen[1] = v.nlb[1] = 0;
   v.nseg[0] = v.seglen[0] = v.nlb[0] = 0;
