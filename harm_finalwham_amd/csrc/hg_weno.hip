@@ -451,24 +451,34 @@ __host__ __device__ inline int64_t weno_x_waves(const Dims &d, int s2, int s3) {
 __device__ __forceinline__ void weno_x_body(const double *__restrict__ p, const double *__restrict__ dpi,
                                             double *__restrict__ pleft, double *__restrict__ pright, const Dims &d,
                                             int wide, unsigned bid) {
-  const int lane = threadIdx.x & 63;
-  const int64_t wid = (int64_t)bid * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const unsigned lane = threadIdx.x & 63u;
   const int n = d.n1;
   // transverse rows: -1..n, or every ghost row for the finite-volume loops
   const int s2 = d.n2 > 1 ? (wide ? d.nb2 : 1) : 0, s3 = d.n3 > 1 ? (wide ? d.nb3 : 1) : 0;
-  const int c1 = d.n2 + 2 * s2, c2 = d.n3 + 2 * s3;
-  const int lr = n + 8;
-  const int64_t nrows = (int64_t)NPR * c1 * c2;
-  if (wid * XOUT >= nrows * lr) return;  // uniform per wavefront
-  const int64_t v = wid * XOUT + lane;
-  int64_t r = v / lr;
-  const int s = (int)(v - r * lr) - 4;
-  const bool live = r < nrows;
-  if (!live) r = nrows - 1;  // lanes past the last row: in-range indices, no work
-  const int pl = (int)(r % NPR);
-  r /= NPR;
-  const int j = -s2 + (int)(r % c1), k = -s3 + (int)(r / c1);
-  const int64_t zl = d.idx(0, j, k);
+  const unsigned c1 = d.n2 + 2 * s2, c2 = d.n3 + 2 * s3;
+  const unsigned lr = n + 8;
+  // (row, place) of the wavefront's first lane from one uniform division each
+  // (fewer than 8 spl < 2^32 places); the lanes count on from there
+  const unsigned v0 = __builtin_amdgcn_readfirstlane((bid * (blockDim.x >> 6) + (threadIdx.x >> 6)) * XOUT);
+  const unsigned r0 = v0 / lr, q0 = r0 / NPR;
+  if (r0 >= NPR * c1 * c2) return;  // uniform per wavefront
+  unsigned pl = r0 % NPR, k = q0 / c1, j = q0 - k * c1;
+  unsigned place = v0 - r0 * lr + lane;
+  for (unsigned last = v0 - r0 * lr + 63u; last >= lr; last -= lr)
+    if (place >= lr) {
+      place -= lr;
+      if (++pl == NPR) {
+        pl = 0;
+        if (++j == c1) {
+          j = 0;
+          k++;
+        }
+      }
+    }
+  const int s = (int)place - 4;
+  const bool live = k < c2;
+  if (!live) k = c2 - 1;  // lanes past the last row: in-range indices, no work
+  const int64_t zl = d.idx(0, (int)j - s2, (int)k - s3);
   const double *yl = p + (int64_t)pl * d.spl + zl;
   double y[5] = {0., 0., 0., 0., 0.}, w[3] = {1., 1., 1.}, m0 = 0., lof0 = 0.;
   if (live) {
@@ -607,6 +617,10 @@ __device__ __forceinline__ void weno_m_body(const double *__restrict__ p, const 
   double ndp = WM_LDD(db, e0);
   WM_ST(lb, e0) = 0.;
   WM_ST(rb, e0) = 0.;
+#ifndef UN
+#define UN 1
+#endif
+#pragma unroll UN
   for (int t = e0 - 3; t <= tlast; t++) {
     const double cy = ny, cdp = ndp;
     {
