@@ -282,13 +282,15 @@ int capture_grouped(hg_graph *g) {
     // turn, every direction's dP/P indicator in one launch), update, the
     // learned start's features and network, inversion, bound_prim (with dt
     // on the final substep), post_fixup, bound_prim
+    const bool fused = ks && g->mode == 0;  // update_invert_fused
+    const int upd = fused ? (g->ucum ? GK_UPINVU : GK_UPINV) : g->ucum ? GK_UPDATEU : GK_UPDATE;
     const int order[] = {GK_PREP, GK_DPI, GK_WENO1, GK_FLUX1, GK_WENO2, GK_FLUX2, GK_WENO3, GK_FLUX3,
-                         GK_EMF, g->ucum ? GK_UPDATEU : GK_UPDATE, GK_FEATURES, GK_MLP, GK_INVERT, GK_BOUNDDT, GK_FXCHECK,
+                         GK_EMF, upd, GK_FEATURES, GK_MLP, GK_INVERT, GK_BOUNDDT, GK_FXCHECK,
                          GK_FXRESOLVE, GK_FXAVG, GK_FXAPPLY, GK_BOUND};
     for (int step = 0; step < g->nsteps; step++)
       for (int sub = 0; sub < g->ns; sub++)
         for (int k : order) {
-          if ((k == GK_FEATURES || k == GK_MLP) && g->mode != 2) continue;
+          if (((k == GK_FEATURES || k == GK_MLP) && g->mode != 2) || (k == GK_INVERT && fused)) continue;
           L(k, sub);
         }
     HIPTRY(hipGetLastError());

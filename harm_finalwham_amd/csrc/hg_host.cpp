@@ -544,16 +544,22 @@ static void enqueue_substep(hg_ctx *c, double *pi, double *pb, double *pf, const
     c->dg_faces_valid = finalstep != 0;
   }
   prof_mark(c, HG_PROF_UPDATE, s);
-  launch_update(pi, pb, c->uf, c->F[0], c->F[1], c->F[2], c->emf[0], c->emf[1], c->emf[2], c->geo, c->conn, c->dt,
-                rk, d, f.gam, f.dx, c->err, c->tune, s);
-  if (c->c2p_mode == HG_C2P_LEARNED) {
-    // the network's start for every inversion of this substep
-    launch_step_features(c->uf, pb, c->geo, c->d, f.gam, c->lx, s);
-    launch_mlp_forward(c->mlp, (int64_t)c->d.n1 * c->d.n2 * c->d.n3, c->lx, c->ly, s);
+  const int mode = c->c2p_mode == HG_C2P_MIXED ? 1 : c->c2p_mode == HG_C2P_LEARNED ? 2 : 0;
+  if (update_invert_fused(d, mode)) {
+    launch_update_invert(pi, pb, pf, c->uf, c->F[0], c->F[1], c->F[2], c->emf[0], c->emf[1], c->emf[2], c->geo,
+                         c->conn, c->floors, c->dt, rk, finalstep, d, f.gam, f.gammamax, f.dx, c->counters, c->pflag,
+                         c->fx_count, c->err, c->tune, s);
+  } else {
+    launch_update(pi, pb, c->uf, c->F[0], c->F[1], c->F[2], c->emf[0], c->emf[1], c->emf[2], c->geo, c->conn, c->dt,
+                  rk, d, f.gam, f.dx, c->err, c->tune, s);
+    if (mode == 2) {
+      // the network's start for every inversion of this substep
+      launch_step_features(c->uf, pb, c->geo, c->d, f.gam, c->lx, s);
+      launch_mlp_forward(c->mlp, (int64_t)c->d.n1 * c->d.n2 * c->d.n3, c->lx, c->ly, s);
+    }
+    launch_invert(c->uf, pb, pf, c->geo, c->floors, rk, finalstep, d, f.gam, f.gammamax, c->counters, c->pflag, mode,
+                  c->ly, c->fx_count, c->err, c->tune, s);
   }
-  launch_invert(c->uf, pb, pf, c->geo, c->floors, rk, finalstep, d, f.gam, f.gammamax, c->counters, c->pflag,
-                c->c2p_mode == HG_C2P_MIXED ? 1 : c->c2p_mode == HG_C2P_LEARNED ? 2 : 0, c->ly, c->fx_count,
-                c->err, c->tune, s);
   // step_ch.c:127 and :166 call bound_prim twice per substep; the second call
   // is not a repeat of the first: POLEDEATH has zeroed U2 in the rows next to
   // the axis, which the radial inflow check then sees in the corner ghosts

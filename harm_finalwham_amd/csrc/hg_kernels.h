@@ -99,6 +99,15 @@ void launch_update(const double *pi, const double *pb, double *ubuf, const doubl
 // converged root, 2: the same from the learned start (ylearn[zone], the
 // network's log(W / W_guess) in k_invert's zone order); fx_reset (may be
 // null): post_fixup's three list counters, cleared by the kernel
+// update and inversion in one launch: for the Kerr-Schild metric and the FP64
+// inversion (mode 0)
+bool update_invert_fused(const Dims &d, int mode);
+void launch_update_invert(const double *pi, const double *pb, double *pf, double *ubuf, const double *F1,
+                          const double *F2, const double *F3, const double *e1, const double *e2, const double *e3,
+                          const double *geo, const double *conn, const double *floors, const double *dtp,
+                          const RkStage &rk, int finalstep, const Dims &d, double gam, double gammamax,
+                          const double *dx, unsigned long long *counters, int8_t *pflag, unsigned *fx_reset, int *err,
+                          const Tune &tu, hipStream_t s);
 void launch_invert(const double *ubuf, const double *pb, double *pf, const double *geo, const double *floors,
                    const RkStage &rk, int finalstep, const Dims &d, double gam, double gammamax,
                    unsigned long long *counters, int8_t *pflag, int mode, const float *ylearn, unsigned *fx_reset,
@@ -180,6 +189,7 @@ enum GroupClass {
   GK_PREP, GK_DPI, GK_WENO1, GK_WENO2, GK_WENO3, GK_FLUX1, GK_FLUX2, GK_FLUX3, GK_EMF, GK_UPDATE, GK_INVERT,
   GK_BOUND, GK_BOUNDDT, GK_FXCHECK, GK_FXRESOLVE, GK_FXAVG, GK_FXAPPLY, GK_FEATURES, GK_MLP,
   GK_UPDATEU,  // the update with ucum (every scheme but the midpoint one)
+  GK_UPINV, GK_UPINVU,  // update and inversion (update_invert_fused)
   GK_NCLASS
 };
 // blocks of class k on one grid (0: no work there), and one grouped launch of

@@ -815,8 +815,9 @@ __global__ void k_emf(const double *__restrict__ F1, const double *__restrict__ 
 //   k_update: U(pi) + dt * (flux divergence + source) -> Uf
 //   k_invert: Noble 2D inversion of Uf with guess pb, fixup1zone on the
 //             final substep -> pf
-// (one kernel holding both needs more registers than either, and the Uf
-// round trip through HBM costs less than the occupancy it loses)
+// (one kernel holding both for the full metric needs 218 registers against the
+// inversion's 125, and the Uf round trip through HBM costs less than the
+// occupancy it loses; the Kerr-Schild metric's fits 122, k_update_invert)
 // ---------------------------------------------------------------------------
 template <bool UCUM, bool FV, bool KS>
 __device__ __forceinline__ void update_body(const double *__restrict__ pi, const double *__restrict__ pb,
@@ -826,7 +827,8 @@ __device__ __forceinline__ void update_body(const double *__restrict__ pi, const
                                             const double *__restrict__ emf3, const double *__restrict__ geo,
                                             const double *__restrict__ conn, const double *__restrict__ dtp,
                                             const RkStage &rk, const Dims &d, double gam, double idx1, double idx2,
-                                            double idx3, int *__restrict__ err, unsigned bid) {
+                                            double idx3, int *__restrict__ err, unsigned bid, bool store = true,
+                                            double *Ureg = nullptr) {
   int64_t t = bid * (int64_t)blockDim.x + threadIdx.x;
   int64_t total = (int64_t)d.n1 * d.n2 * d.n3;
   if (t < total) {
@@ -959,8 +961,12 @@ __device__ __forceinline__ void update_body(const double *__restrict__ pi, const
       // midpoint scheme: ucum equals Uf on the final substep (Cunew = {0,0,1})
     }
     if (bad) atomicOr(err, 4);
+    if (store)
 #pragma unroll
-    for (int pl = 0; pl < NPR; pl++) ubuf[z + pl * P] = Uf[pl];
+      for (int pl = 0; pl < NPR; pl++) ubuf[z + pl * P] = Uf[pl];
+    if (Ureg)
+#pragma unroll
+      for (int pl = 0; pl < NPR; pl++) Ureg[pl] = Uf[pl];
   }
 }
 
@@ -1023,7 +1029,7 @@ __device__ __forceinline__ void invert_body(const double *__restrict__ ubuf, con
                                             double gam, double gammamax, unsigned long long *__restrict__ counters,
                                             int8_t *__restrict__ pflag, double *__restrict__ ucons,
                                             const float *__restrict__ ylearn, unsigned *__restrict__ fx_reset,
-                                            int *__restrict__ err, unsigned bid) {
+                                            int *__restrict__ err, unsigned bid, const double *Ureg = nullptr) {
   // the post_fixup lists of this substep start empty (launch_post_fixup
   // then skips its own reset)
   if (fx_reset && bid == 0 && threadIdx.x < 3) fx_reset[threadIdx.x] = 0u;
@@ -1042,7 +1048,7 @@ __device__ __forceinline__ void invert_body(const double *__restrict__ ubuf, con
     double Uf[NPR], pr[NPR];
 #pragma unroll
     for (int pl = 0; pl < NPR; pl++) {
-      Uf[pl] = ubuf[z + pl * P];
+      Uf[pl] = Ureg ? Ureg[pl] : ubuf[z + pl * P];
       pr[pl] = pb[z + pl * P];
     }
     bool bad = false;
@@ -1103,6 +1109,31 @@ __global__ void __launch_bounds__(256) k_invert(const double *__restrict__ ubuf,
                         fx_reset, err, blockIdx.x);
 }
 
+// k_update and k_invert of the Kerr-Schild metric in one kernel: Uf stays in
+// registers, stored only where the scheme or hg_dump_inversions reads it, and the
+// guess and metric are read again from the caches.  The phases' live values do
+// not add up (122 VGPRs, four wavefronts per SIMD; 158 where the final substep of
+// the finite-volume scheme corrects its carried state).  A step at 256x128x64
+// takes 3.72 instead of 3.79 ms (WENO5BND), 1.95 instead of 2.07 (MC), 5.62
+// instead of 5.73 (PARA, RK4, finite volume); at 32^2 MC 95 instead of 101 us.
+template <bool UCUM, bool FV, bool FVLAST>
+__global__ void __launch_bounds__(256) k_update_invert(
+    const double *__restrict__ pi, const double *pb, double *pf, double *__restrict__ ubuf,
+    const double *__restrict__ F1, const double *__restrict__ F2, const double *__restrict__ F3,
+    const double *__restrict__ emf1, const double *__restrict__ emf2, const double *__restrict__ emf3,
+    const double *__restrict__ geo, const double *__restrict__ conn, const double *__restrict__ floors,
+    const double *__restrict__ dtp, RkStage rk, Dims d, double gam, double gammamax, double idx1, double idx2,
+    double idx3, int finalstep, unsigned long long *__restrict__ counters, int8_t *__restrict__ pflag,
+    unsigned *__restrict__ fx_reset, int *__restrict__ err) {
+  double U[NPR];
+  update_body<UCUM, FV, true>(pi, pb, ubuf, F1, F2, F3, emf1, emf2, emf3, geo, conn, dtp, rk, d, gam, idx1, idx2, idx3,
+                              err, blockIdx.x, UCUM || finalstep, U);
+  value_barrier(U, NPR);
+  asm volatile("" ::: "memory");
+  invert_body<FVLAST, INV_FP64, true>(ubuf, pb, pf, geo, floors, finalstep, d, gam, gammamax, counters, pflag, rk.ucons,
+                                  nullptr, fx_reset, err, blockIdx.x, U);
+}
+
 // ---------------------------------------------------------------------------
 // grouped launches of the kernels above (GridView, group_of)
 // ---------------------------------------------------------------------------
@@ -1141,6 +1172,20 @@ __global__ void __launch_bounds__(256) kg_update(const GridView *__restrict__ vi
   HG_GROUP_PRELUDE
   update_body<UCUM, false, KS>(v.pi, v.pb, v.uf, v.F[0], v.F[1], v.F[2], v.emf[0], v.emf[1], v.emf[2], v.geo, v.conn,
                             v.dt, v.rk, v.d, v.gam, v.idx[1], v.idx[2], v.idx[3], v.err, bid);
+}
+
+template <bool UCUM>
+__global__ void __launch_bounds__(256) kg_update_invert(const GridView *__restrict__ views,
+                                                        const unsigned *__restrict__ first, int n) {
+  HG_GROUP_PRELUDE
+  double U[NPR];
+  update_body<UCUM, false, true>(v.pi, v.pb, v.uf, v.F[0], v.F[1], v.F[2], v.emf[0], v.emf[1], v.emf[2], v.geo, v.conn,
+                                 v.dt, v.rk, v.d, v.gam, v.idx[1], v.idx[2], v.idx[3], v.err, bid,
+                                 UCUM || v.finalstep, U);
+  value_barrier(U, NPR);
+  asm volatile("" ::: "memory");
+  invert_body<false, INV_FP64, true>(v.uf, v.pb, v.pf, v.geo, v.floors, v.finalstep, v.d, v.gam, v.gammamax, v.counters,
+                                     v.pflag, nullptr, nullptr, v.fx.count, v.err, bid, U);
 }
 
 template <int MODE, bool KS>
@@ -1434,6 +1479,27 @@ void launch_update(const double *pi, const double *pb, double *ubuf, const doubl
                        d, gam, i1, i2, i3, err);
 }
 
+bool update_invert_fused(const Dims &d, int mode) { return d.ks && mode == INV_FP64; }
+
+void launch_update_invert(const double *pi, const double *pb, double *pf, double *ubuf, const double *F1,
+                          const double *F2, const double *F3, const double *e1, const double *e2, const double *e3,
+                          const double *geo, const double *conn, const double *floors, const double *dtp,
+                          const RkStage &rk, int finalstep, const Dims &d, double gam, double gammamax,
+                          const double *dx, unsigned long long *counters, int8_t *pflag, unsigned *fx_reset, int *err,
+                          const Tune &tu, hipStream_t s) {
+  int64_t n = (int64_t)d.n1 * d.n2 * d.n3;
+  dim3 g(nblocks(n, tu.bs_update)), b(tu.bs_update);
+  const double i1 = 1.0 / dx[1], i2 = 1.0 / dx[2], i3 = 1.0 / dx[3];
+#define HG_UI(U, F, L)                                                                                               \
+  hipLaunchKernelGGL((k_update_invert<U, F, L>), g, b, 0, s, pi, pb, pf, ubuf, F1, F2, F3, e1, e2, e3, geo, conn, floors, \
+                     dtp, rk, d, gam, gammamax, i1, i2, i3, finalstep, counters, pflag, fx_reset, err)
+  if (rk.ucons && finalstep) HG_UI(true, true, true);
+  else if (rk.ucons) HG_UI(true, true, false);
+  else if (rk.ucum) HG_UI(true, false, false);
+  else HG_UI(false, false, false);
+#undef HG_UI
+}
+
 template <int MODE>
 static void launch_invert_mode(const double *ubuf, const double *pb, double *pf, const double *geo,
                                const double *floors, const RkStage &rk, int finalstep, const Dims &d, double gam,
@@ -1546,7 +1612,8 @@ unsigned group_blocks(int k, const GridView &v) {
       return nblocks((int64_t)fr.ni * fr.nj * fr.nk, 256);
     }
     case GK_EMF: return nblocks((int64_t)(d.n1 + s1) * (d.n2 + s2) * (d.n3 + s3), 256);
-    case GK_UPDATE: case GK_UPDATEU: case GK_INVERT: case GK_FEATURES: return nblocks(act, 256);
+    case GK_UPDATE: case GK_UPDATEU: case GK_INVERT: case GK_UPINV: case GK_UPINVU: case GK_FEATURES:
+      return nblocks(act, 256);
     case GK_FXCHECK: case GK_FXRESOLVE: case GK_FXAVG: case GK_FXAPPLY: return group_blocks_fixup(k, v);
     default: return group_blocks_weno(k, v);
   }
@@ -1565,6 +1632,8 @@ void launch_group(int k, const GridView *views, const unsigned *first, int n, un
     case GK_EMF: hipLaunchKernelGGL(kg_emf, g, dim3(256), 0, s, views, first, n); return;
     case GK_UPDATE: HG_LAUNCH_KS(ks, kg_update, false, g, dim3(256), views, first, n); return;
     case GK_UPDATEU: HG_LAUNCH_KS(ks, kg_update, true, g, dim3(256), views, first, n); return;
+    case GK_UPINV: hipLaunchKernelGGL(kg_update_invert<false>, g, dim3(256), 0, s, views, first, n); return;
+    case GK_UPINVU: hipLaunchKernelGGL(kg_update_invert<true>, g, dim3(256), 0, s, views, first, n); return;
     case GK_INVERT:
       if (mode == INV_MIXED) HG_LAUNCH_KS(ks, kg_invert, INV_MIXED, g, dim3(256), views, first, n);
       else if (mode == INV_LEARNED) HG_LAUNCH_KS(ks, kg_invert, INV_LEARNED, g, dim3(256), views, first, n);
