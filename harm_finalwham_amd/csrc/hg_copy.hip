@@ -13,9 +13,10 @@
 // spread over them.  A state of up to 2 MiB is one piece, one kernel and one
 // wait.
 //
-// 256x128x64 with 6 ghost layers (182 MB): 4.3 ms in, 5.5 ms out, where one
-// thread transposing on the host around a pageable copy took 71 and 81; 32x32
-// (92 kB) 28 and 25 us against 65 and 66.
+// 256x128x64 with 6 ghost layers (182 MB): 4.2 ms in, 5.5 ms out, where one
+// thread transposing on the host around a pageable copy took 71 and 77; 128^2
+// with 3 (1.1 MB) 55 and 69 us against 135 and 240, 32^2 (92 kB) 20 and 20
+// against 18 and 20.
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -49,27 +50,33 @@ __global__ void __launch_bounds__(256) k_transpose(double *__restrict__ dev, dou
   const int64_t qb = (int64_t)blockIdx.x * TQ;
   const int ib = blockIdx.y * TI;
   const int t = threadIdx.x;
+  // a thread's 8 numbers are all loaded before the first is stored: a state of
+  // one piece waits once for the bus, not 8 times
+  constexpr int NR = TI / 4, NQ = TQ / 8;
+  const int64_t qh = qb + (t & 63);
+  const int ih = t >> 6, id = ib + (t & 31), qd = t >> 5;
+  double v[8] = {0., 0., 0., 0., 0., 0., 0., 0.};
+  static_assert(NR == 8 && NQ == 8, "256 threads");
   if (TO_DEVICE) {
-    for (int i = t >> 6; i < TI; i += 4) {
-      const int64_t q = qb + (t & 63);
-      if (ib + i < ni && q < nq) tile[t & 63][i] = host[(int64_t)(ib + i) * nq + q];
-    }
+#pragma unroll
+    for (int r = 0; r < NR; r++)
+      if (ib + ih + 4 * r < ni && qh < nq) v[r] = host[(int64_t)(ib + ih + 4 * r) * nq + qh];
+#pragma unroll
+    for (int r = 0; r < NR; r++) tile[t & 63][ih + 4 * r] = v[r];
     __syncthreads();
-  }
-  for (int q = t >> 5; q < TQ; q += 8) {
-    const int i = t & 31;
-    if (ib + i < ni && qb + q < nq) {
-      double *a = dev + plane_of(d, q0 + qb + q) + i0 + ib + i;
-      if (TO_DEVICE) *a = tile[q][i];
-      else tile[q][i] = *a;
-    }
-  }
-  if (!TO_DEVICE) {
+#pragma unroll
+    for (int r = 0; r < NQ; r++)
+      if (id < ni && qb + qd + 8 * r < nq) dev[plane_of(d, q0 + qb + qd + 8 * r) + i0 + id] = tile[qd + 8 * r][t & 31];
+  } else {
+#pragma unroll
+    for (int r = 0; r < NQ; r++)
+      if (id < ni && qb + qd + 8 * r < nq) v[r] = dev[plane_of(d, q0 + qb + qd + 8 * r) + i0 + id];
+#pragma unroll
+    for (int r = 0; r < NQ; r++) tile[qd + 8 * r][t & 31] = v[r];
     __syncthreads();
-    for (int i = t >> 6; i < TI; i += 4) {
-      const int64_t q = qb + (t & 63);
-      if (ib + i < ni && q < nq) host[(int64_t)(ib + i) * nq + q] = tile[t & 63][i];
-    }
+#pragma unroll
+    for (int r = 0; r < NR; r++)
+      if (ib + ih + 4 * r < ni && qh < nq) host[(int64_t)(ib + ih + 4 * r) * nq + qh] = tile[t & 63][ih + 4 * r];
   }
 }
 
