@@ -243,7 +243,25 @@ __global__ void __launch_bounds__(256) k_bound(double *p, const double *__restri
 // ---------------------------------------------------------------------------
 // Riemann flux at one face from left/right states, fluxcompute.c:12
 // ---------------------------------------------------------------------------
-template <class GT>
+// One side's results (two sets of fluxes and two speeds), which live through the
+// whole computation of the other: 36 registers, or with PARK a place in LDS (37
+// kB per 256 faces, four blocks to a CU).  With the Kerr-Schild metric that is
+// the step from 164 registers and three wavefronts per SIMD to 128 and four
+// (flux_waves), with the full one from 192 and two to 158 and three.  Worth it
+// where the device is full: 256x128x64 WENO5BND 0.285 -> 0.259 ms per direction
+// and step, the PARA step 5.64 -> 5.32 ms, 128x64x32 WENO5BND 655 -> 634 us, PARA
+// 854 -> 808, MC 327 -> 297 (without the bound; 305 with).  A grid of up to
+// PARK_BLOCKS blocks only pays the round trip (59x19x7 WENO5BND 175.0 -> 176.5
+// us), and so do the large MC kernels, which their stencil loads bound.
+typedef double (*FluxPark)[256];
+__device__ __forceinline__ FluxPark flux_park() {
+  __shared__ double park[2 * NPR + 2][256];
+  return park;
+}
+constexpr unsigned PARK_BLOCKS = 1024;
+constexpr int flux_waves(bool bound, bool ks) { return bound && ks ? 4 : 1; }
+
+template <bool PARK, class GT>
 __device__ __forceinline__ bool face_flux(int dir, GT &G, double *p_l, double *p_r, double gam,
                                           int fluxmethod, double *F, double &ctop) {
   // flux.c:629 BDIRCONT
@@ -265,6 +283,17 @@ __device__ __forceinline__ bool face_flux(int dir, GT &G, double *p_l, double *p
     primtoflux(p_l, ql, M, p1, 0, G, gam, U_l);
     if (vchar(p_l, ql, dir, G, gam, cmax_l, cmin_l)) return true;
   }
+  if constexpr (PARK) {
+    const FluxPark park = flux_park();
+#pragma unroll
+    for (int pl = 0; pl < NPR; pl++) {
+      park[pl][threadIdx.x] = F_l[pl];
+      park[NPR + pl][threadIdx.x] = U_l[pl];
+    }
+    park[2 * NPR][threadIdx.x] = cmax_l;
+    park[2 * NPR + 1][threadIdx.x] = cmin_l;
+    asm volatile("" ::: "memory");
+  }
   geom_barrier(G);
   {
     State qr;
@@ -275,6 +304,17 @@ __device__ __forceinline__ bool face_flux(int dir, GT &G, double *p_l, double *p
     primtoflux(p_r, qr, M, p1, dir, G, gam, F_r);
     primtoflux(p_r, qr, M, p1, 0, G, gam, U_r);
     if (vchar(p_r, qr, dir, G, gam, cmax_r, cmin_r)) return true;
+  }
+  if constexpr (PARK) {
+    const FluxPark park = flux_park();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int pl = 0; pl < NPR; pl++) {
+      F_l[pl] = park[pl][threadIdx.x];
+      U_l[pl] = park[NPR + pl][threadIdx.x];
+    }
+    cmax_l = park[2 * NPR][threadIdx.x];
+    cmin_l = park[2 * NPR + 1][threadIdx.x];
   }
   // wavespeeds.c:325 cminmax_calc
   double lmin = rmin(cmin_l, cmin_r);
@@ -527,7 +567,7 @@ __device__ __forceinline__ void para4(const double y[5], double &lout, double &r
 // point-type reconstruction fused with the Riemann flux (flux.c:469
 // fluxcalc_standard): MC slopes (interppoint.c:387) or PARA interface values
 // (interppoint.c:289), turned into the face states by flux.c:753 getp2interplr
-template <int DIR, bool PARA, bool EXT = false, bool KS = false>
+template <int DIR, bool PARA, bool EXT = false, bool KS = false, bool PARK = false>
 __device__ __forceinline__ void flux_point_body(const double *__restrict__ p, const double *__restrict__ geo,
                                                 double *__restrict__ F, const Dims &d, const FaceRange &fr,
                                                 double gam, double cour, double dxdir, int fluxmethod, int slim,
@@ -574,7 +614,7 @@ __device__ __forceinline__ void flux_point_body(const double *__restrict__ p, co
     double Fz[NPR], ctop;
     bool bad;
     if constexpr (EXT) bad = face_flux_ext(DIR, G, p_l, p_r, gam, fluxmethod, Fz, ctop);
-    else bad = face_flux(DIR, G, p_l, p_r, gam, fluxmethod, Fz, ctop);
+    else bad = face_flux<PARK>(DIR, G, p_l, p_r, gam, fluxmethod, Fz, ctop);
     if (bad) {
       atomicOr(err, 2);
     } else {
@@ -596,24 +636,24 @@ __global__ void __launch_bounds__(256) k_flux_mc(const double *__restrict__ p, c
 }
 
 template <int DIR, bool KS>
-__global__ void __launch_bounds__(256) k_flux_para(const double *__restrict__ p, const double *__restrict__ geo,
+__global__ void __launch_bounds__(256, flux_waves(true, KS)) k_flux_para(const double *__restrict__ p, const double *__restrict__ geo,
                                                    double *__restrict__ F, Dims d, double gam, double cour,
                                                    double dxdir, int fluxmethod, int slim,
                                                    unsigned long long *__restrict__ ndt_bits,
                                                    int *__restrict__ err) {
   FaceRange fr = face_range(d, DIR);
-  flux_point_body<DIR, true, false, KS>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err, blockIdx.x);
+  flux_point_body<DIR, true, false, KS, true>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err, blockIdx.x);
 }
 
 // the finite-volume flux loops (every transverse ghost row)
 template <int DIR, bool PARA, bool KS>
-__global__ void __launch_bounds__(256) k_flux_pt_fv(const double *__restrict__ p, const double *__restrict__ geo,
+__global__ void __launch_bounds__(256, flux_waves(PARA, KS)) k_flux_pt_fv(const double *__restrict__ p, const double *__restrict__ geo,
                                                     double *__restrict__ F, Dims d, double gam, double cour,
                                                     double dxdir, int fluxmethod, int slim,
                                                     unsigned long long *__restrict__ ndt_bits,
                                                     int *__restrict__ err) {
   FaceRange fr = face_range_fv(d, DIR);
-  flux_point_body<DIR, PARA, false, KS>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err, blockIdx.x);
+  flux_point_body<DIR, PARA, false, KS, PARA>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err, blockIdx.x);
 }
 
 // MC or PARA with the FORCE / MUSTA / HLLLAXF1 fluxes
@@ -627,7 +667,7 @@ __global__ void __launch_bounds__(256) k_flux_pt_ext(const double *__restrict__ 
   flux_point_body<DIR, PARA, true>(p, geo, F, d, fr, gam, cour, dxdir, fluxmethod, slim, ndt_bits, err, blockIdx.x);
 }
 
-template <int DIR, bool EXT, bool KS = false>
+template <int DIR, bool EXT, bool KS = false, bool PARK = false>
 __device__ __forceinline__ void flux_lr_body(const double *__restrict__ pleft,
                                                  const double *__restrict__ pright,
                                                  const double *__restrict__ geo, double *__restrict__ F, Dims d,
@@ -657,7 +697,7 @@ __device__ __forceinline__ void flux_lr_body(const double *__restrict__ pleft,
     double Fz[NPR], ctop;
     bool bad;
     if constexpr (EXT) bad = face_flux_ext(DIR, G, p_l, p_r, gam, fluxmethod, Fz, ctop);
-    else bad = face_flux(DIR, G, p_l, p_r, gam, fluxmethod, Fz, ctop);
+    else bad = face_flux<PARK>(DIR, G, p_l, p_r, gam, fluxmethod, Fz, ctop);
     if (bad) {
       atomicOr(err, 2);
     } else {
@@ -670,25 +710,25 @@ __device__ __forceinline__ void flux_lr_body(const double *__restrict__ pleft,
 }
 
 template <int DIR, bool KS>
-__global__ void __launch_bounds__(256) k_flux_lr(const double *__restrict__ pleft,
+__global__ void __launch_bounds__(256, flux_waves(true, KS)) k_flux_lr(const double *__restrict__ pleft,
                                                  const double *__restrict__ pright,
                                                  const double *__restrict__ geo, double *__restrict__ F, Dims d,
                                                  double gam, double cour, double dxdir, int fluxmethod,
                                                  unsigned long long *__restrict__ ndt_bits, int *__restrict__ err) {
   FaceRange fr = face_range(d, DIR);
-  flux_lr_body<DIR, false, KS>(pleft, pright, geo, F, d, fr, gam, cour, dxdir, fluxmethod, ndt_bits, err, blockIdx.x);
+  flux_lr_body<DIR, false, KS, true>(pleft, pright, geo, F, d, fr, gam, cour, dxdir, fluxmethod, ndt_bits, err, blockIdx.x);
 }
 
 // the finite-volume flux loops (every transverse ghost row)
 template <int DIR, bool KS>
-__global__ void __launch_bounds__(256) k_flux_lr_fv(const double *__restrict__ pleft,
+__global__ void __launch_bounds__(256, flux_waves(true, KS)) k_flux_lr_fv(const double *__restrict__ pleft,
                                                     const double *__restrict__ pright,
                                                     const double *__restrict__ geo, double *__restrict__ F, Dims d,
                                                     double gam, double cour, double dxdir, int fluxmethod,
                                                     unsigned long long *__restrict__ ndt_bits,
                                                     int *__restrict__ err) {
   FaceRange fr = face_range_fv(d, DIR);
-  flux_lr_body<DIR, false, KS>(pleft, pright, geo, F, d, fr, gam, cour, dxdir, fluxmethod, ndt_bits, err, blockIdx.x);
+  flux_lr_body<DIR, false, KS, true>(pleft, pright, geo, F, d, fr, gam, cour, dxdir, fluxmethod, ndt_bits, err, blockIdx.x);
 }
 
 // WENO5BND states with the FORCE / MUSTA / HLLLAXF1 fluxes
@@ -713,8 +753,8 @@ __global__ void __launch_bounds__(256) k_flux_lr_ext(const double *__restrict__ 
 //   PARA, RK4, FV   459->323  371->265 990->884 998->885  1779->1672  5757->5703
 // 128x64x32 has 3400 (FV: 4600) blocks; on large grids every direction fills the
 // device, and the register count of one kernel for all keeps fewer wavefronts.
-template <bool PARA, bool FV, bool KS>
-__global__ void __launch_bounds__(256) k_flux_pt_dirs(const double *__restrict__ p, const double *__restrict__ geo,
+template <bool PARA, bool FV, bool PARK, bool KS>
+__global__ void __launch_bounds__(256, flux_waves(PARA && PARK, KS)) k_flux_pt_dirs(const double *__restrict__ p, const double *__restrict__ geo,
                                                       FluxDirs f, Dims d, double gam, double cour, int fluxmethod,
                                                       int slim, unsigned long long *__restrict__ ndt_bits,
                                                       int *__restrict__ err) {
@@ -722,17 +762,17 @@ __global__ void __launch_bounds__(256) k_flux_pt_dirs(const double *__restrict__
   const int dir = b < f.first[1] ? 1 : b < f.first[2] ? 2 : 3;
   const FaceRange fr = FV ? face_range_fv(d, dir) : face_range(d, dir);
   if (dir == 1)
-    flux_point_body<1, PARA, false, KS>(p, geo, f.F[0], d, fr, gam, cour, f.dx[0], fluxmethod, slim, ndt_bits, err, b);
+    flux_point_body<1, PARA, false, KS, PARK>(p, geo, f.F[0], d, fr, gam, cour, f.dx[0], fluxmethod, slim, ndt_bits, err, b);
   else if (dir == 2)
-    flux_point_body<2, PARA, false, KS>(p, geo, f.F[1], d, fr, gam, cour, f.dx[1], fluxmethod, slim, ndt_bits + 1,
+    flux_point_body<2, PARA, false, KS, PARK>(p, geo, f.F[1], d, fr, gam, cour, f.dx[1], fluxmethod, slim, ndt_bits + 1,
                                         err, b - f.first[1]);
   else
-    flux_point_body<3, PARA, false, KS>(p, geo, f.F[2], d, fr, gam, cour, f.dx[2], fluxmethod, slim, ndt_bits + 2,
+    flux_point_body<3, PARA, false, KS, PARK>(p, geo, f.F[2], d, fr, gam, cour, f.dx[2], fluxmethod, slim, ndt_bits + 2,
                                         err, b - f.first[2]);
 }
 
-template <bool FV, bool KS>
-__global__ void __launch_bounds__(256) k_flux_lr_dirs(const double *__restrict__ geo, FluxDirs f, Dims d, double gam,
+template <bool FV, bool PARK, bool KS>
+__global__ void __launch_bounds__(256, flux_waves(PARK, KS)) k_flux_lr_dirs(const double *__restrict__ geo, FluxDirs f, Dims d, double gam,
                                                       double cour, int fluxmethod,
                                                       unsigned long long *__restrict__ ndt_bits,
                                                       int *__restrict__ err) {
@@ -740,12 +780,12 @@ __global__ void __launch_bounds__(256) k_flux_lr_dirs(const double *__restrict__
   const int dir = b < f.first[1] ? 1 : b < f.first[2] ? 2 : 3;
   const FaceRange fr = FV ? face_range_fv(d, dir) : face_range(d, dir);
   if (dir == 1)
-    flux_lr_body<1, false, KS>(f.pl[0], f.pr[0], geo, f.F[0], d, fr, gam, cour, f.dx[0], fluxmethod, ndt_bits, err, b);
+    flux_lr_body<1, false, KS, PARK>(f.pl[0], f.pr[0], geo, f.F[0], d, fr, gam, cour, f.dx[0], fluxmethod, ndt_bits, err, b);
   else if (dir == 2)
-    flux_lr_body<2, false, KS>(f.pl[1], f.pr[1], geo, f.F[1], d, fr, gam, cour, f.dx[1], fluxmethod, ndt_bits + 1,
+    flux_lr_body<2, false, KS, PARK>(f.pl[1], f.pr[1], geo, f.F[1], d, fr, gam, cour, f.dx[1], fluxmethod, ndt_bits + 1,
                                err, b - f.first[1]);
   else
-    flux_lr_body<3, false, KS>(f.pl[2], f.pr[2], geo, f.F[2], d, fr, gam, cour, f.dx[2], fluxmethod, ndt_bits + 2,
+    flux_lr_body<3, false, KS, PARK>(f.pl[2], f.pr[2], geo, f.F[2], d, fr, gam, cour, f.dx[2], fluxmethod, ndt_bits + 2,
                                err, b - f.first[2]);
 }
 
@@ -1153,10 +1193,10 @@ __global__ void __launch_bounds__(256) kg_bound(const GridView *__restrict__ vie
 }
 
 template <int DIR, bool KS>
-__global__ void __launch_bounds__(256) kg_flux_lr(const GridView *__restrict__ views,
+__global__ void __launch_bounds__(256, flux_waves(true, KS)) kg_flux_lr(const GridView *__restrict__ views,
                                                   const unsigned *__restrict__ first, int n) {
   HG_GROUP_PRELUDE
-  flux_lr_body<DIR, false, KS>(v.pl[DIR - 1], v.pr[DIR - 1], v.geo, v.F[DIR - 1], v.d, face_range(v.d, DIR), v.gam,
+  flux_lr_body<DIR, false, KS, true>(v.pl[DIR - 1], v.pr[DIR - 1], v.geo, v.F[DIR - 1], v.d, face_range(v.d, DIR), v.gam,
                            v.cour, v.dx[DIR], v.fluxmethod, v.ndt_bits + DIR - 1, v.err, bid);
 }
 
@@ -1281,6 +1321,12 @@ static unsigned bound_total(const Dims &d) {
   return nblk[0] + nblk[1] + nblk[2];
 }
 
+#define HG_LAUNCH_KS3(ks, K, A, B, C, g, b, ...)                                     \
+  do {                                                                               \
+    if (ks) hipLaunchKernelGGL((K<A, B, C, true>), g, b, 0, s, __VA_ARGS__);         \
+    else hipLaunchKernelGGL((K<A, B, C, false>), g, b, 0, s, __VA_ARGS__);           \
+  } while (0)
+
 void launch_bound(double *p, const double *geo, const Dims &d, double gammamax, int *err, hipStream_t s,
                   const StepDt &se) {
   // a grid of one zone has no ghosts, but its step has a dt
@@ -1309,16 +1355,28 @@ void launch_flux_dirs(const FluxDirs &f, int lim, bool fv, const double *p, cons
                       double gam, double cour, int fluxmethod, unsigned long long *ndt_bits, int *err,
                       hipStream_t s) {
   const dim3 g(f.nblocks), b(256);
+  const bool para = lim == HG_LIM_PARA;
+#define HG_LR(FV, PARK) HG_LAUNCH_KS2(d.ks, k_flux_lr_dirs, FV, PARK, g, b, geo, f, d, gam, cour, fluxmethod, ndt_bits, err)
+#define HG_PT(PARA, FV, PARK)                                                                                        \
+  HG_LAUNCH_KS3(d.ks, k_flux_pt_dirs, PARA, FV, PARK, g, b, p, geo, f, d, gam, cour, fluxmethod, lim, ndt_bits, err)
+#define HG_PARK(L, ...)                       \
+  do {                                        \
+    if (f.nblocks > PARK_BLOCKS) L(__VA_ARGS__, true); \
+    else L(__VA_ARGS__, false);               \
+  } while (0)
   if (lim == HG_LIM_WENO5BND) {
-    if (fv) HG_LAUNCH_KS(d.ks, k_flux_lr_dirs, true, g, b, geo, f, d, gam, cour, fluxmethod, ndt_bits, err);
-    else HG_LAUNCH_KS(d.ks, k_flux_lr_dirs, false, g, b, geo, f, d, gam, cour, fluxmethod, ndt_bits, err);
-  } else if (lim == HG_LIM_PARA) {
-    if (fv) HG_LAUNCH_KS2(d.ks, k_flux_pt_dirs, true, true, g, b, p, geo, f, d, gam, cour, fluxmethod, lim, ndt_bits, err);
-    else HG_LAUNCH_KS2(d.ks, k_flux_pt_dirs, true, false, g, b, p, geo, f, d, gam, cour, fluxmethod, lim, ndt_bits, err);
+    if (fv) HG_PARK(HG_LR, true);
+    else HG_PARK(HG_LR, false);
+  } else if (para) {
+    if (fv) HG_PARK(HG_PT, true, true);
+    else HG_PARK(HG_PT, true, false);
   } else {
-    if (fv) HG_LAUNCH_KS2(d.ks, k_flux_pt_dirs, false, true, g, b, p, geo, f, d, gam, cour, fluxmethod, lim, ndt_bits, err);
-    else HG_LAUNCH_KS2(d.ks, k_flux_pt_dirs, false, false, g, b, p, geo, f, d, gam, cour, fluxmethod, lim, ndt_bits, err);
+    if (fv) HG_PARK(HG_PT, false, true);
+    else HG_PARK(HG_PT, false, false);
   }
+#undef HG_LR
+#undef HG_PT
+#undef HG_PARK
 }
 
 void launch_flux_point(int dir, int lim, bool fv, const double *p, const double *geo, double *F, const Dims &d,
