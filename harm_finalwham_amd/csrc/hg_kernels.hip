@@ -1565,12 +1565,21 @@ static void launch_invert_mode(const double *ubuf, const double *pb, double *pf,
                                unsigned *fx_reset, int *err, const Tune &tu, hipStream_t s) {
   int64_t n = (int64_t)d.n1 * d.n2 * d.n3;
   dim3 gi(nblocks(n, tu.bs_invert)), bi(tu.bs_invert);
-  if (rk.ucons && finalstep)
-    HG_LAUNCH_KS2(d.ks, k_invert, true, MODE, gi, bi, ubuf, pb, pf, geo, floors, finalstep, d, gam, gammamax,
-                       counters, pflag, rk.ucons, ylearn, fx_reset, err);
-  else
-    HG_LAUNCH_KS2(d.ks, k_invert, false, MODE, gi, bi, ubuf, pb, pf, geo, floors, finalstep, d, gam, gammamax,
-                       counters, pflag, nullptr, ylearn, fx_reset, err);
+  const bool fv = rk.ucons && finalstep;
+#define HG_INV(F, KS)                                                                                             \
+  hipLaunchKernelGGL((k_invert<F, MODE, KS>), gi, bi, 0, s, ubuf, pb, pf, geo, floors, finalstep, d, gam, gammamax, \
+                     counters, pflag, F ? rk.ucons : nullptr, ylearn, fx_reset, err)
+  if constexpr (MODE == INV_FP64) {  // with the Kerr-Schild metric: k_update_invert
+    if (fv) HG_INV(true, false);
+    else HG_INV(false, false);
+  } else if (d.ks) {
+    if (fv) HG_INV(true, true);
+    else HG_INV(false, true);
+  } else {
+    if (fv) HG_INV(true, false);
+    else HG_INV(false, false);
+  }
+#undef HG_INV
 }
 
 void launch_invert(const double *ubuf, const double *pb, double *pf, const double *geo, const double *floors,
@@ -1695,7 +1704,7 @@ void launch_group(int k, const GridView *views, const unsigned *first, int n, un
     case GK_INVERT:
       if (mode == INV_MIXED) HG_LAUNCH_KS(ks, kg_invert, INV_MIXED, g, dim3(256), views, first, n);
       else if (mode == INV_LEARNED) HG_LAUNCH_KS(ks, kg_invert, INV_LEARNED, g, dim3(256), views, first, n);
-      else HG_LAUNCH_KS(ks, kg_invert, INV_FP64, g, dim3(256), views, first, n);
+      else hipLaunchKernelGGL((kg_invert<INV_FP64, false>), g, dim3(256), 0, s, views, first, n);
       return;
     case GK_FEATURES: hipLaunchKernelGGL(kg_step_features, g, dim3(256), 0, s, views, first, n); return;
     case GK_FXCHECK: case GK_FXRESOLVE: case GK_FXAVG: case GK_FXAPPLY:
