@@ -59,10 +59,10 @@ def profile_summary(prof, zones):
 
 
 # device kernels of each logical kernel (WENO5BND build)
-DEVICE_KERNELS = {"recon+flux1": ("hg::k_weno_dpi<1>", "hg::k_weno_x", "hg::k_flux_lr<1>"),
-                  "recon+flux2": ("hg::k_weno_dpi<2>", "hg::k_weno_m<2>", "hg::k_flux_lr<2>"),
-                  "recon+flux3": ("hg::k_weno_dpi<3>", "hg::k_weno_m<3>", "hg::k_flux_lr<3>"),
-                  "emf": ("hg::k_emf",), "update": ("hg::k_update<false, false>", "hg::k_invert<false, 0>")}
+DEVICE_KERNELS = {"recon+flux1": ("hg::k_weno_dpi<1>", "hg::k_weno_x", "hg::k_flux_lr<1, true>"),
+                  "recon+flux2": ("hg::k_weno_dpi<2>", "hg::k_weno_m<2>", "hg::k_flux_lr<2, true>"),
+                  "recon+flux3": ("hg::k_weno_dpi<3>", "hg::k_weno_m<3>", "hg::k_flux_lr<3, true>"),
+                  "emf": ("hg::k_emf",), "update": ("hg::k_update_invert<false, false, false>",)}
 TRAFFIC_PROFILE = os.path.join(HERE, "profiles", "hbm_traffic_torus3d_256x128x64_weno_hll.md")
 VALU_PROFILE = os.path.join(HERE, "profiles", "valu_issue_torus3d_256x128x64_weno_hll.md")
 FP64_PEAK_TFLOPS = 78.6
@@ -259,7 +259,7 @@ def c2p_bench(n, reps=3):
     inverted by the plain FP64 kernel (the reference's arithmetic), by the
     converged-root kernel (HG_C2P_REFINED: the reference's codes, root
     converged with double-double residuals) and by the mixed-precision
-    persistent kernel.  Errors are against the converged root."""
+    kernel.  Errors are against the converged root."""
     from harm_finalwham_amd import harmgpu
     import torch
     res = {"n": n, "gam": [], "fp64_ms": [], "refined_ms": [], "mixed_ms": [], "flags_identical": True,

@@ -6,7 +6,10 @@
 //   k_flux_para<dir>   PARA (para4) reconstruction fused with the Riemann flux
 //   k_flux_lr<dir>     Riemann flux from precomputed interface states (WENO5BND)
 //   k_emf              flux-CT corner EMFs (fluxct.c:10)
-//   k_update           conserved update + source + Noble 2D + fixup1zone (advance.c:58)
+//   k_flux_*_dirs      the fluxes of all directions of a small grid
+//   k_update           conserved update + source (advance.c:58)
+//   k_invert           Noble 2D + fixup1zone (advance.c:193)
+//   k_update_invert    both, for the Kerr-Schild metric and the FP64 inversion
 //   k_set_dt           initial time step of the set-up (advance.c:957)
 #include <hip/hip_runtime.h>
 

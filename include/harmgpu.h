@@ -279,11 +279,10 @@ int hg_rdump_write(hg_ctx *ctx, const char *path, const char *header, void *stre
                      iteration in FP32 to |dW/W| <= 2e-6 (or to its rounding
                      floor), then the polish of HG_C2P_REFINED and the
                      primitives from the converged W with the reference's
-                     FP64 formulas (within ~1e-12 of HG_C2P_REFINED's); a
-                     persistent work-queue kernel.  Zones whose FP32 phase or
-                     polish does not converge are inverted by HG_C2P_REFINED
-                     from the guess.
-                     Allocates its scratch (4 n + 24 bytes) stream-ordered on
+                     FP64 formulas (within ~1e-12 of HG_C2P_REFINED's).
+                     Zones whose FP32 phase or polish does not converge get
+                     HG_C2P_REFINED's root and primitives from the guess.
+                     Allocates its scratch (4 n + 16 bytes) stream-ordered on
                      the given stream. */
 #define HG_C2P_FP64 0
 #define HG_C2P_MIXED 1
@@ -296,8 +295,8 @@ int hg_utoprim_batch(int64_t n, double gam, const double *U, const double *gcov,
    for callers that cannot allocate device memory (code under HIP graph
    capture, tight serving loops, harnesses that forbid hipMalloc).  Same
    arguments, kernels and results as hg_utoprim_batch.  HG_C2P_MIXED keeps its
-   work-queue counters and compacted fallback list in a static device array
-   of the library (HG_C2P_NOALLOC_MAX_N zones: 4 * 2^24 + 24 bytes, held on
+   list counters and compacted fallback list in a static device array
+   of the library (HG_C2P_NOALLOC_MAX_N zones: 4 * 2^24 + 16 bytes, held on
    every GPU the library runs on until the process ends); larger n is
    rejected.  Every call on one GPU shares that GPU's array: calls that
    overlap in time on one GPU (other streams, other threads) race and must
