@@ -526,11 +526,12 @@ __device__ __forceinline__ bool c2p_polish(const C2PInv &c, double igr, double &
     newton_dx(c, igr, x0, x1, dx0, dx1, f, df);
     double xo0 = x0;
     x0 = fabs(x0 + dx0);
-    x0 = w_too_big(c, x0) ? xo0 : x0;
+    const bool big = w_too_big(c, x0);  // W stays: not converged, however little it moved
+    x0 = big ? xo0 : x0;
     x1 += dx1;
     x1 = (x1 > 1.) ? vsq_big : x1;
     iters++;
-    ok = fabs(x0 - xo0) <= 1e-9 * x0;
+    ok = !big && fabs(x0 - xo0) <= 1e-9 * x0;
   }
   if (!ok) return false;
   ok = false;
@@ -539,11 +540,12 @@ __device__ __forceinline__ bool c2p_polish(const C2PInv &c, double igr, double &
     newton_dx_dd(c, igr, x0, x1, dx0, dx1);
     double xo0 = x0;
     x0 = fabs(x0 + dx0);
-    x0 = w_too_big(c, x0) ? xo0 : x0;
+    const bool big = w_too_big(c, x0);
+    x0 = big ? xo0 : x0;
     x1 += dx1;
     x1 = (x1 > 1.) ? vsq_big : x1;
     iters++;
-    ok = fabs(x0 - xo0) <= 1e-12 * x0;
+    ok = !big && fabs(x0 - xo0) <= 1e-12 * x0;
   }
   return ok && isfinite(x0) && isfinite(x1);
 }
