@@ -288,6 +288,24 @@ __device__ __forceinline__ double c2p_scale(const double *U, const GT &G, double
   return alpha;
 }
 
+// The reference's stopping test errx = |dx0 / x0| <= NEWT_TOL of the iterate x0
+// that the step dx0 led to: by a product, but for tiny iterates and quotients
+// within 2^-40 of the tolerance.  An infinite step makes both sides infinite and
+// errx a NaN, which is no convergence (the reference puts W back and goes on):
+// the comparison is strict.  far, whether errx is above MIN_NEWT_TOL, is asked
+// of the last step allowed alone.
+__device__ __forceinline__ bool newton_converged(double x0, double dx0, bool last, bool &far) {
+  const double a0 = fabs(x0), ad = fabs(dx0), lim = NEWT_TOL * a0;
+  bool conv = ad < lim * (1. - 0x1p-40);
+  far = false;
+  if (!(a0 >= 0x1p-900) || !(conv || ad >= lim * (1. + 0x1p-40)) || last) {
+    const double errx = (x0 == 0.) ? ad : fabs(dx0 / x0);
+    conv = errx <= NEWT_TOL;
+    far = errx > MIN_NEWT_TOL;
+  }
+  return conv;
+}
+
 // Full FP64 inversion of one zone (utoprimgen.c:23 with UTOPRIM2DFINAL).
 // U: evolved conserved variables (with gdet); pr: guess in, solution out.
 // The core also returns the invariants and the final Newton iterate (x0 = W,
@@ -322,16 +340,8 @@ __device__ __forceinline__ int utoprimgen_fp64_core(const double *U, const GT &G
     double xo0 = x0;
     x0 += dx0;
     x1 += dx1;
-    // errx = |dx0 / x0| <= NEWT_TOL by a product, but for quotients within
-    // 2^-40 of the tolerance; errx itself only after the last step allowed
-    const double a0 = fabs(x0), ad = fabs(dx0), lim = NEWT_TOL * a0;
-    bool conv = ad <= lim * (1. - 0x1p-40);
-    far = false;
-    if (!(a0 >= 0x1p-900) || !(conv || ad >= lim * (1. + 0x1p-40)) || iters >= MAX_NEWT_ITER) {
-      const double errx = (x0 == 0.) ? ad : fabs(dx0 / x0);
-      conv = errx <= NEWT_TOL;
-      far = errx > MIN_NEWT_TOL;
-    }
+    const double a0 = fabs(x0);
+    const bool conv = newton_converged(x0, dx0, iters >= MAX_NEWT_ITER, far);
     x0 = w_too_big(c, a0) ? xo0 : a0;
     x1 = (x1 > 1.) ? vsq_big : x1;
     if (conv || (iters >= MAX_NEWT_ITER)) keep = false;
