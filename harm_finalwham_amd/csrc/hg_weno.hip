@@ -226,8 +226,10 @@ __device__ __forceinline__ double mono_quotient(const double *yin, const double 
 // where every value reaches the cutoff; those two are read off the values
 // before their divisions (norm is cusp's, which is the cutoff but for its
 // order of summing, so that 1.00001 norm is above the cutoff; at least 1e-63,
-// so that no product of the minmods underflows).  Only a point between, or one
-// that is not finite, takes the quotient.
+// so that no product of the minmods underflows).  The smallest minmod is held to
+// W_BIG before it meets the cutoff: lines of 1e63 and more, whose cutoff is not
+// below that, take the quotient, and so does a point between 0 and 1, or one that
+// is not finite.
 __device__ __forceinline__ double mono_eno5(const double *yin, double d_1, double d2, double norm) {
   const double n[4] = {(((-3 * yin[-2] + yin[2]) + (-10 * yin[-1] - 6 * yin[1])) + 18 * yin[0]),
                         (((11 * yin[-2] - yin[2]) + (-20 * yin[-1] + 4 * yin[1])) + 6 * yin[0]),
@@ -240,11 +242,11 @@ __device__ __forceinline__ double mono_eno5(const double *yin, double d_1, doubl
                      (__double2hiint(n[1]) ^ __double2hiint(n[3])) | (__double2hiint(l3) ^ __double2hiint(r3));
   const double mn = fmin(fmin(fabs(n[0]), fabs(n[2])), fmin(fabs(n[1]), fabs(n[3])));
   const double md = fmin(fabs(d_1), fabs(d2)), m3 = fmin(fabs(l3), fabs(r3));
-  const bool finite = norm <= 1e280;
+  const bool below_big = norm <= 0.5 * W_BIG;
   const bool zero = differ < 0 || fmin(mn, fmin(md, m3)) == 0.0;
   const bool one = mn >= 12.0002 * norm && md >= 1.00001 * norm && m3 >= 2.00002 * norm;
   double m = zero ? 0.0 : 1.0;
-  if (__builtin_expect(!(finite && (zero || one)), 0)) m = mono_quotient(yin, n, l3, r3);
+  if (__builtin_expect(!(below_big && (zero || one)), 0)) m = mono_quotient(yin, n, l3, r3);
   return m;
 }
 
