@@ -492,29 +492,26 @@ __device__ __forceinline__ bool newton_f32(const C2PInv &c, double igr, double &
 }
 
 // One Newton step with the residuals t11, t18 of func_vsq2 in double-double
-// and the FP64 Jacobian (newton_dx's terms, reciprocals to an ulp: the
-// Jacobian's rounding moves the step by 1e-15 of itself, the residuals set
-// the root)
+// and the FP64 Jacobian (newton_dx's terms)
 __device__ __forceinline__ void newton_dx_dd(const C2PInv &c, double igr, double W, double vsq, double &dx0,
                                              double &dx1) {
   const double Wsq = W * W, D = c.D, Bsq = c.Bsq, QdotBsq = c.QdotBsq;
-  const double gamma = rsqrt_1ulp(1.0 - vsq);
+  const double gamma = 1.0 / sqrt(1.0 - vsq);
   const double dPdW = (1.0 - vsq) * igr;
   const double dPdvsq = (D * (gamma * 0.5 - 1.0) - (W - D)) * igr;
-  const double t2 = -0.5 * Bsq + dPdvsq, t3 = Bsq + W, t4 = t3 * t3, t23 = rcp_1ulp(W), t9 = t23 * t23;
-  const double t16 = QdotBsq * t9, t21 = rcp_1ulp(t3), t24 = t16 * t23, t25 = -1.0 + dPdW - t24;
+  const double t2 = -0.5 * Bsq + dPdvsq, t3 = Bsq + W, t4 = t3 * t3, t9 = 1 / Wsq;
+  const double t16 = QdotBsq * t9, t21 = 1 / t3, t23 = 1 / W, t24 = t16 * t23, t25 = -1.0 + dPdW - t24;
   const double t35 = t25 * t3 + (Bsq - 2.0 * dPdvsq) * (QdotBsq + vsq * Wsq * W) * t9 * t23;
-  const double t36 = rcp_1ulp(t35);
+  const double t36 = 1 / t35;
   // residuals: t11 = Qtsq - vsq (Bsq + W)^2 + QdotBsq (Bsq + 2 W) / W^2,
   // t18 = -Qdotn - Bsq (1 + vsq) / 2 + QdotBsq / (2 W^2) - W + p(W, vsq)
   const dd Wd = dd_of(W), vd = dd_of(vsq);
   const dd T3 = two_sum(Bsq, W);
-  const dd q = dd_div_r(dd_of(QdotBsq), two_prod(W, W), t9);
+  const dd q = dd_div(dd_of(QdotBsq), two_prod(W, W));
   const dd r11 = dd_add(dd_sub(dd_of(c.Qtsq), dd_mul(vd, dd_mul(T3, T3))), dd_mul(q, two_sum(Bsq, 2.0 * W)));
   const dd omv = two_sum(1.0, -vsq);
-  // D vsq / (1 + gamma) = D vsq s / (1 + s), s = 1 / gamma
-  const dd sd = dd_sqrt(omv);
-  const dd wm = dd_sub(dd_mul(two_sum(W, -D), omv), dd_div(dd_mul(two_prod(vsq, D), sd), dd_add(dd_of(1.0), sd)));
+  const dd gd = dd_div(dd_of(1.0), dd_sqrt(omv));
+  const dd wm = dd_sub(dd_mul(two_sum(W, -D), omv), dd_div(two_prod(vsq, D), dd_add(dd_of(1.0), gd)));
   const dd r18 = dd_add(dd_add(dd_add(dd_of(-c.Qdotn), dd_mul_d(two_sum(1.0, vsq), -0.5 * Bsq)), dd_mul_d(q, 0.5)),
                         dd_add(dd_neg(Wd), dd_mul_d(wm, igr)));
   const double t11 = dd_val(r11), t18 = dd_val(r18);
