@@ -659,14 +659,17 @@ constexpr double LISTED_MARGIN = 16.0;   // W moved by this many times its noise
 // 1e-9; from there the polish.  Taken only where every stopping point of the
 // reference inside the noise would give code 0: the FP64 primitives at W and
 // at W moved either way by LISTED_MARGIN times the noise all do.  Every other
-// zone is inverted by utoprimgen_refined from the guess.  The list of 1e6 zones of
-// the benchmark distribution (154, gamma 5/3) takes 42 us instead of 168 us.
-template <class GT>
+// zone is inverted by utoprimgen_refined from the guess, and so is every zone of a
+// caller that asks for the counts: they are the reference's, walk included.  The
+// list of 1e6 zones of the benchmark distribution (154, gamma 5/3) takes 42 us
+// instead of 168 us without them; 1.5e6 listed zones gave the same bits and codes
+// either way.
+template <bool COUNTED, class GT>
 __device__ __forceinline__ int utoprimgen_listed(const double *U, const GT &G, double gam, double *pr, int &iters) {
   C2PInv c;
   double Ug[NPR], Ut[NPR], W_last;
   c2p_scale(U, G, Ug, Ut);
-  if (c2p_setup(Ut, G, pr, gam, c, W_last) == 0) {
+  if (!COUNTED && c2p_setup(Ut, G, pr, gam, c, W_last) == 0) {
     const double igr = (gam - 1.0) / gam;
     double x0, x1;
     newton_start(c, W_last, x0, x1);
@@ -682,7 +685,6 @@ __device__ __forceinline__ int utoprimgen_listed(const double *U, const GT &G, d
         for (int i = 0; i < B1; i++) pr[i] = out[i];
 #pragma unroll
         for (int i = B1; i <= B3; i++) pr[i] = Ug[i];
-        iters = it;
         return 0;
       }
     }

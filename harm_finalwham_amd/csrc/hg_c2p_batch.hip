@@ -19,7 +19,8 @@
 //                     4096 zones (16 stretches) 35 us against 15 us
 //   k_c2p_listed      persistent over that list, from the original guess: the
 //                     root and primitives of HG_C2P_REFINED, short of the
-//                     reference's walk in rounding noise (utoprimgen_listed)
+//                     reference's walk in rounding noise unless the counts are
+//                     asked for (utoprimgen_listed)
 //
 // Memory per zone: the inversion reads U (8), the upper triangles of the
 // symmetric gcov and gcon (10 + 10), gdet and the guess's u and u~^i (4),
@@ -213,7 +214,8 @@ __global__ void __launch_bounds__(MIXED_BLOCK) k_c2p_mixed(int64_t n, double gam
   list_append(fb, t, ctr, list);
 }
 
-// the listed zones, from the guess still in pr
+// the listed zones, from the guess still in pr; COUNTED: iters is given
+template <bool COUNTED>
 __global__ void __launch_bounds__(256) k_c2p_listed(int64_t n, double gam, const double *__restrict__ U,
                                                     const double *__restrict__ gcov,
                                                     const double *__restrict__ gcon,
@@ -234,10 +236,10 @@ __global__ void __launch_bounds__(256) k_c2p_listed(int64_t n, double gam, const
       double u[NPR], p[NPR];
       load_batch_zone(n, t, U, gcov, gcon, gdet, pr, G, u, p);
       int it = 0;
-      int flag = utoprimgen_listed(u, G, gam, p, it);
+      int flag = utoprimgen_listed<COUNTED>(u, G, gam, p, it);
       store_batch_zone(n, t, pr, p, code_assigns(flag));
       pflag[t] = flag;
-      if (iters) iters[t] = it;
+      if (COUNTED) iters[t] = it;
     }
   }
 }
@@ -282,28 +284,31 @@ int launch_c2p_batch_mixed(int64_t n, double gam, const double *U, const double 
                            const double *gdet, double *pr, int *pflag, int *iters, void *scratch, hipStream_t s) {
   unsigned long long *ctr = (unsigned long long *)scratch;
   uint32_t *list = (uint32_t *)(ctr + C2P_NCTR);
-  int64_t b2 = 0;
-  if (persistent_blocks(k_c2p_listed, (n + 255) / 256, b2)) return 1;
   hipLaunchKernelGGL(k_c2p_reset, dim3(1), dim3(64), 0, s, ctr);
   hipLaunchKernelGGL(k_c2p_mixed, dim3((unsigned)((n + MIXED_BLOCK - 1) / MIXED_BLOCK)), dim3(MIXED_BLOCK), 0, s, n,
                      gam, U, gcov, gcon, gdet, pr, pflag, iters, ctr, list);
-  hipLaunchKernelGGL(k_c2p_listed, dim3((unsigned)b2), dim3(256), 0, s, n, gam, U, gcov, gcon, gdet, pr, pflag,
-                     iters, ctr, (const uint32_t *)list);
-  return 0;
+  return launch_c2p_listed(n, gam, U, gcov, gcon, gdet, pr, pflag, iters, scratch, s);
 }
 
 void launch_c2p_reset(void *scratch, hipStream_t s) {
   hipLaunchKernelGGL(k_c2p_reset, dim3(1), dim3(64), 0, s, (unsigned long long *)scratch);
 }
 
-int launch_c2p_listed(int64_t n, double gam, const double *U, const double *gcov, const double *gcon,
-                      const double *gdet, double *pr, int *pflag, int *iters, void *scratch, hipStream_t s) {
+template <bool COUNTED>
+static int launch_listed(int64_t n, double gam, const double *U, const double *gcov, const double *gcon,
+                         const double *gdet, double *pr, int *pflag, int *iters, void *scratch, hipStream_t s) {
   unsigned long long *ctr = (unsigned long long *)scratch;
   int64_t b = 0;
-  if (persistent_blocks(k_c2p_listed, (n + 255) / 256, b)) return 1;
-  hipLaunchKernelGGL(k_c2p_listed, dim3((unsigned)b), dim3(256), 0, s, n, gam, U, gcov, gcon, gdet, pr, pflag, iters,
-                     ctr, (const uint32_t *)(ctr + C2P_NCTR));
+  if (persistent_blocks(k_c2p_listed<COUNTED>, (n + 255) / 256, b)) return 1;
+  hipLaunchKernelGGL(k_c2p_listed<COUNTED>, dim3((unsigned)b), dim3(256), 0, s, n, gam, U, gcov, gcon, gdet, pr, pflag,
+                     iters, ctr, (const uint32_t *)(ctr + C2P_NCTR));
   return 0;
+}
+
+int launch_c2p_listed(int64_t n, double gam, const double *U, const double *gcov, const double *gcon,
+                      const double *gdet, double *pr, int *pflag, int *iters, void *scratch, hipStream_t s) {
+  return iters ? launch_listed<true>(n, gam, U, gcov, gcon, gdet, pr, pflag, iters, scratch, s)
+               : launch_listed<false>(n, gam, U, gcov, gcon, gdet, pr, pflag, iters, scratch, s);
 }
 
 void c2p_note_fallbacks(long long nfb) {

@@ -281,7 +281,9 @@ int hg_rdump_write(hg_ctx *ctx, const char *path, const char *header, void *stre
                      primitives from the converged W with the reference's
                      FP64 formulas (within ~1e-12 of HG_C2P_REFINED's).
                      Zones whose FP32 phase or polish does not converge get
-                     HG_C2P_REFINED's root and primitives from the guess.
+                     HG_C2P_REFINED's root and primitives from the guess, and
+                     its count: without iters the library need not walk the
+                     reference's last steps for them.
                      Allocates its scratch (4 n + 16 bytes) stream-ordered on
                      the given stream. */
 #define HG_C2P_FP64 0
@@ -373,8 +375,8 @@ int hg_mlp_train(hg_mlp *m, int64_t n, const float *X, const float *Y, int epoch
    FP32 iteration continues from there, else the FP32 iteration starts from
    the plain start (the reference's, from the guess).  The polish and
    double-double primitives of HG_C2P_REFINED follow.  A zone whose FP32
-   phase or polish does not converge is inverted by HG_C2P_REFINED from its
-   plain guess.  The values therefore agree with HG_C2P_REFINED to ~1e-12
+   phase or polish does not converge gets HG_C2P_REFINED's root, primitives and
+   count from its plain guess, as in HG_C2P_MIXED.  The values therefore agree with HG_C2P_REFINED to ~1e-12
    (the same converged root), not bit for bit.  iters counts Newton steps and
    the learned start's evaluation.  counts (may be NULL) receives [zones solved from the learned
    start, zones inverted by the fallback].  Allocates its scratch (4 n + 24
