@@ -17,7 +17,7 @@
 //                   sum of every weight's gradient per block
 //   k_mlp_update    the partial sums added up, Adam, the BF16 copies of the
 //                   hidden-layer weights (or the gradient alone)
-//   k_mlp_refresh   the copies alone
+//   k_mlp_set       the parameters a caller sets, and the copies
 //   k_c2p_learned   the mixed-precision inversion (FP32 Newton, polish,
 //                   double-double primitives) from the learned start where
 //                   the network predicts a large correction and the start's
@@ -475,12 +475,18 @@ __global__ void __launch_bounds__(64 * UPDATE_WAYS) k_mlp_update(MlpDev m, const
   }
 }
 
-// after the parameters were set
-__global__ void k_mlp_refresh(MlpDev m) {
+// the parameters a caller sets.  One that has the value it had keeps what its
+// FP32 number rounds off, so that setting the parameters just read leaves a
+// training as it is.
+__global__ void k_mlp_set(MlpDev m, const float *__restrict__ src) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= NTRAIN) return;
-  m.wlo[e] = 0.f;
-  refresh_bf16(e, m.w[e], m);
+  if (e >= NPARAM) return;
+  const float v = src[e];
+  if (e < NTRAIN) {
+    if (__float_as_int(v) != __float_as_int(m.w[e])) m.wlo[e] = 0.f;
+    refresh_bf16(e, v, m);
+  }
+  m.w[e] = v;
 }
 
 constexpr int COUNT_SLOTS = 64, COUNT_STRIDE = 8;
@@ -561,11 +567,13 @@ __global__ void __launch_bounds__(64) k_c2p_learned(int64_t n, double gam, const
 
 }  // namespace
 
-// one allocation holds everything: parameters, gradient, Adam moments, the
-// BF16 copies, the loss, the counts and the partial sums of the backward pass
+// one allocation holds everything: parameters, gradient, Adam moments, what the
+// parameters round off and as many zeros (which stand for it in a gradient at
+// the parameters themselves: a branch in the kernel costs a minibatch 1.2 us),
+// the BF16 copies, the loss, the counts and the partial sums of the backward pass
 struct hg_mlp {
   void *mem = nullptr;
-  float *w = nullptr, *g = nullptr, *w2q = nullptr, *wlo = nullptr;
+  float *w = nullptr, *g = nullptr, *w2q = nullptr, *wlo = nullptr, *zero = nullptr;
   double *m1 = nullptr, *m2 = nullptr, *loss = nullptr, *part = nullptr;
   __bf16 *w1b = nullptr, *w2b = nullptr;
   unsigned long long *counts = nullptr;  // learned starts, in COUNT_SLOTS parts
@@ -573,6 +581,15 @@ struct hg_mlp {
 };
 
 static MlpDev dev_view(const hg_mlp *m) { return MlpDev{m->w, m->w1b, m->w2b, m->w2q, m->wlo}; }
+
+// parameters from the host, through the room of the partial sums
+static hipError_t upload_params(hg_mlp *m, const float *host) {
+  hipError_t e = hipMemcpy(m->part, host, NPARAM * sizeof(float), hipMemcpyHostToDevice);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_mlp_set, dim3((NPARAM + 255) / 256), dim3(256), 0, 0, dev_view(m), (const float *)m->part);
+  e = hipGetLastError();
+  return e == hipSuccess ? hipDeviceSynchronize() : e;
+}
 
 // blocks of the backward pass: one per 16-sample tile up to BACK_BLOCKS
 static unsigned backward_blocks(int64_t n) {
@@ -628,10 +645,12 @@ extern "C" int hg_mlp_create(uint64_t seed, hg_mlp **out) {
     at += (bytes + 255) / 256 * 256;
     return here;
   };
-  const size_t o_g = take(np * 4), o_m1 = take(np * 8), o_m2 = take(np * 8), o_wlo = take(np * 4), o_w1b = take(32 * NH * sizeof(__bf16)),
+  const size_t o_g = take(np * 4), o_m1 = take(np * 8), o_m2 = take(np * 8), o_wlo = take(np * 4),
+               o_w1b = take(32 * NH * sizeof(__bf16)),
                o_w2b = take(NH * NH * sizeof(__bf16)), o_loss = take(sizeof(double)),
                o_counts = take(COUNT_SLOTS * COUNT_STRIDE * sizeof(unsigned long long)), zeroed = at, o_w = take(np * 4),
-               o_w2q = take(NH * NH * sizeof(float)), o_part = take((size_t)BACK_BLOCKS * PART * sizeof(double));
+               o_w2q = take(NH * NH * sizeof(float)), o_part = take((size_t)BACK_BLOCKS * PART * sizeof(double)),
+               o_zero = take(np * 4);
   hipError_t e = hipMalloc(&m->mem, at);
   if (e == hipSuccess) {
     char *b = (char *)m->mem;
@@ -639,6 +658,7 @@ extern "C" int hg_mlp_create(uint64_t seed, hg_mlp **out) {
     m->m1 = (double *)(b + o_m1);
     m->m2 = (double *)(b + o_m2);
     m->wlo = (float *)(b + o_wlo);
+    m->zero = (float *)(b + o_zero);
     m->w1b = (__bf16 *)(b + o_w1b);
     m->w2b = (__bf16 *)(b + o_w2b);
     m->loss = (double *)(b + o_loss);
@@ -647,12 +667,9 @@ extern "C" int hg_mlp_create(uint64_t seed, hg_mlp **out) {
     m->w2q = (float *)(b + o_w2q);
     m->part = (double *)(b + o_part);
     e = hipMemset(m->mem, 0, zeroed);
+    if (e == hipSuccess) e = hipMemset(m->zero, 0, np * 4);
   }
-  if (e == hipSuccess) e = hipMemcpy(m->w, w.data(), NPARAM * sizeof(float), hipMemcpyHostToDevice);
-  if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_mlp_refresh, dim3((NTRAIN + 255) / 256), dim3(256), 0, 0, dev_view(m));
-    e = hipDeviceSynchronize();
-  }
+  if (e == hipSuccess) e = upload_params(m, w.data());
   if (e != hipSuccess) {
     set_error("hg_mlp_create: %s", hipGetErrorString(e));
     hg_mlp_destroy(m);
@@ -674,10 +691,7 @@ extern "C" int hg_mlp_set_params(hg_mlp *m, const float *host) {
   if (!m || !host) { set_error("hg_mlp_set_params: null argument"); return 1; }
   for (int k = 0; k < NIN; k++)
     if (!(host[OFF_SD + k] > 0.f)) { set_error("hg_mlp_set_params: feature scales must be > 0"); return 1; }
-  MLPCHECK(hipMemcpy(m->w, host, NPARAM * sizeof(float), hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(k_mlp_refresh, dim3((NTRAIN + 255) / 256), dim3(256), 0, 0, dev_view(m));
-  MLPCHECK(hipGetLastError());
-  MLPCHECK(hipDeviceSynchronize());
+  MLPCHECK(upload_params(m, host));
   return 0;
 }
 
@@ -729,9 +743,11 @@ extern "C" int hg_mlp_gradient(hg_mlp *m, int64_t n, const float *X, const float
   if (!m || n <= 0 || !X || !Y) { set_error("hg_mlp_gradient: bad arguments"); return 1; }
   hipStream_t s = (hipStream_t)stream;
   const unsigned nb = backward_blocks(n);
-  hipLaunchKernelGGL(k_mlp_backward, dim3(nb), dim3(256), 0, s, n, X, Y, dev_view(m), 1.0 / (double)n,
+  MlpDev at = dev_view(m);
+  at.wlo = m->zero;  // at the parameters that hg_mlp_get_params returns
+  hipLaunchKernelGGL(k_mlp_backward, dim3(nb), dim3(256), 0, s, n, X, Y, at, 1.0 / (double)n,
                      1.0 / (double)n, m->part);
-  hipLaunchKernelGGL(k_mlp_update<false>, dim3(UPDATE_BLOCKS), dim3(64 * UPDATE_WAYS), 0, s, dev_view(m), (const double *)m->part,
+  hipLaunchKernelGGL(k_mlp_update<false>, dim3(UPDATE_BLOCKS), dim3(64 * UPDATE_WAYS), 0, s, at, (const double *)m->part,
                      (int)nb, 0., 0., 0., 1, m->m1, m->m2, m->g, m->loss);
   MLPCHECK(hipGetLastError());
   MLPCHECK(hipStreamSynchronize(s));

@@ -336,8 +336,9 @@ int hg_c2p_fallbacks(int64_t *nfallback);
    Utoprim_new_body).  A perceptron 8 -> 64 -> 64 -> 1 (tanh) maps invariants
    of the conserved state and the plain guess to y = log(W / W_guess); the
    hidden layers run on the matrix cores with BF16 weights (each input as a
-   hi + lo BF16 pair) and FP32 accumulation, the FP32 master weights are
-   trained on the GPU (Adam) from inversions this library solved.
+   hi + lo BF16 pair) and FP32 accumulation.  The weights are trained on the
+   GPU (Adam, in FP64) from inversions this library solved: a trained weight
+   carries what its FP32 number rounds off, which no other call sees.
    Parameter block (FP32, hg_mlp_nparams() = 4817 entries):
      W1[8][64] b1[64] W2[64][64] b2[64] W3[64] b3 mu[8] sd[8]
    where the network sees (x - mu) / sd.  Features x per zone:
@@ -351,6 +352,9 @@ int hg_mlp_create(uint64_t seed, hg_mlp **out);
 int hg_mlp_destroy(hg_mlp *m);
 int hg_mlp_nparams(void);
 int hg_mlp_get_params(const hg_mlp *m, float *host);
+/* sets the parameters; Adam's moments and step count stay, and a weight set to
+   the value it has keeps what that rounds off: setting what hg_mlp_get_params
+   returned changes nothing */
 int hg_mlp_set_params(hg_mlp *m, const float *host);
 /* features X[n][8] of n inversions from their plain guess p_guess[8][n];
    with solved primitives p_solved[8][n] (may be NULL) also the training
@@ -360,9 +364,9 @@ int hg_mlp_features(int64_t n, double gam, const double *U, const double *gcov, 
                     const double *gdet, const double *p_guess, const double *p_solved, float *X, float *y,
                     int32_t *ok, void *stream);
 int hg_mlp_forward(const hg_mlp *m, int64_t n, const float *X, float *y, void *stream);
-/* gradient of mean((y - Y)^2) with respect to the parameter block (host
-   copy in grad_host, may be NULL; normalisation entries are 0), the loss in
-   *loss; the weights are not changed */
+/* gradient of mean((y - Y)^2) with respect to the parameter block, at the
+   parameters hg_mlp_get_params returns (host copy in grad_host, may be NULL;
+   normalisation entries are 0), the loss in *loss; the weights are not changed */
 int hg_mlp_gradient(hg_mlp *m, int64_t n, const float *X, const float *Y, float *grad_host, float *loss,
                     void *stream);
 /* `epochs` passes of Adam over minibatches of `batch` (>= 64) samples in order */
