@@ -28,8 +28,6 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
-#include <cstdio>
-#include <cstdlib>
 #include <vector>
 
 #include "harmgpu.h"
@@ -758,28 +756,16 @@ extern "C" int hg_mlp_gradient(hg_mlp *m, int64_t n, const float *X, const float
   return 0;
 }
 
-// the number a caller wrote for a float argument: of the reals that round to
-// it, the one of fewest digits (2e-3f stands for 0.002)
-static double written(float v) {
-  char t[32];
-  for (int digits = 6; digits <= 9; digits++) {
-    snprintf(t, sizeof t, "%.*g", digits, (double)v);
-    if ((float)strtod(t, nullptr) == v) return strtod(t, nullptr);
-  }
-  return v;
-}
-
 // epochs of Adam over the n samples in minibatches of `batch` (in order);
 // *loss receives the mean minibatch loss of the last epoch
-extern "C" int hg_mlp_train(hg_mlp *m, int64_t n, const float *X, const float *Y, int epochs, int batch,
-                            float lr, float *loss, void *stream) {
+extern "C" int hg_mlp_train_rate(hg_mlp *m, int64_t n, const float *X, const float *Y, int epochs, int batch,
+                                 double rate, float *loss, void *stream) {
   if (!m || n <= 0 || !X || !Y || epochs < 0 || batch < 64) {
     set_error("hg_mlp_train: bad arguments (batch >= 64)");
     return 1;
   }
   hipStream_t s = (hipStream_t)stream;
   int64_t nb = (n + batch - 1) / batch;
-  const double rate = written(lr);
   double last = 0.;
   for (int ep = 0; ep < epochs; ep++) {
     for (int64_t b = 0; b < nb; b++) {
@@ -799,6 +785,11 @@ extern "C" int hg_mlp_train(hg_mlp *m, int64_t n, const float *X, const float *Y
   }
   if (loss) *loss = (float)last;
   return 0;
+}
+
+extern "C" int hg_mlp_train(hg_mlp *m, int64_t n, const float *X, const float *Y, int epochs, int batch, float lr,
+                            float *loss, void *stream) {
+  return hg_mlp_train_rate(m, n, X, Y, epochs, batch, (double)lr, loss, stream);
 }
 
 extern "C" int hg_utoprim_batch_learned(const hg_mlp *m, int64_t n, double gam, const double *U,

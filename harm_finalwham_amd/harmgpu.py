@@ -25,7 +25,7 @@ EXPORTS = ["hg_ctx_create", "hg_ctx_destroy", "hg_upload_geometry", "hg_mks_geom
            "hg_profile", "hg_profile_read", "hg_profile_class_name", "hg_c2p_fallbacks",
            "hg_graph_create", "hg_graph_create_grouped", "hg_graph_launch", "hg_graph_destroy", "hg_get_tune", "hg_set_tune", "hg_autotune",
            "hg_mlp_create", "hg_mlp_destroy", "hg_mlp_nparams", "hg_mlp_get_params", "hg_mlp_set_params",
-           "hg_mlp_features", "hg_mlp_forward", "hg_mlp_gradient", "hg_mlp_train",
+           "hg_mlp_features", "hg_mlp_forward", "hg_mlp_gradient", "hg_mlp_train", "hg_mlp_train_rate",
            "hg_utoprim_batch_learned", "hg_post_fixup", "hg_get_pflag", "hg_diagnostics", "hg_diag_record", "hg_rdump_parse",
            "hg_rdump_read", "hg_set_conserved", "hg_get_conserved", "hg_rdump_write", "hg_advance_substep",
            "hg_dump_inversions", "hg_utoprim_batch_noalloc", "hg_set_inversion", "hg_check_division"]
@@ -166,6 +166,7 @@ def lib():
     L.hg_mlp_forward.argtypes = [vp, C.c_int64, vp, vp, vp]
     L.hg_mlp_gradient.argtypes = [vp, C.c_int64, vp, vp, fp, fp, vp]
     L.hg_mlp_train.argtypes = [vp, C.c_int64, vp, vp, C.c_int, C.c_int, C.c_float, fp, vp]
+    L.hg_mlp_train_rate.argtypes = [vp, C.c_int64, vp, vp, C.c_int, C.c_int, C.c_double, fp, vp]
     L.hg_utoprim_batch_learned.argtypes = [vp, C.c_int64, C.c_double, vp, vp, vp, vp, vp, vp, vp, vp, i64p, vp]
     L.hg_profile_read.argtypes = [vp, d, i64p]
     L.hg_profile_class_name.argtypes = [C.c_int]
@@ -521,8 +522,8 @@ class Mlp:
         """Adam over the samples in order, minibatches of `batch`; returns the
         mean loss of the last epoch."""
         loss = C.c_float()
-        _check(lib().hg_mlp_train(self.h, X.shape[0], C.c_void_p(X.data_ptr()), C.c_void_p(Y.data_ptr()),
-                                  epochs, batch, lr, C.byref(loss), stream))
+        _check(lib().hg_mlp_train_rate(self.h, X.shape[0], C.c_void_p(X.data_ptr()), C.c_void_p(Y.data_ptr()),
+                                       epochs, batch, lr, C.byref(loss), stream))
         return loss.value
 
     def close(self):

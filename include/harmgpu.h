@@ -372,6 +372,11 @@ int hg_mlp_gradient(hg_mlp *m, int64_t n, const float *X, const float *Y, float 
 /* `epochs` passes of Adam over minibatches of `batch` (>= 64) samples in order */
 int hg_mlp_train(hg_mlp *m, int64_t n, const float *X, const float *Y, int epochs, int batch, float lr,
                  float *loss, void *stream);
+/* the same at a rate in double precision, which is that of the updates: 2e-3f
+   is 5e-8 away from 0.002, and a training in which a weight's BF16 copy then
+   rounds the other way ends elsewhere */
+int hg_mlp_train_rate(hg_mlp *m, int64_t n, const float *X, const float *Y, int epochs, int batch, double rate,
+                      float *loss, void *stream);
 /* hg_utoprim_batch's HG_C2P_MIXED inversion with a learned start.  Where
    the network predicts |y| > 0.25 (the plain guess off by more than ~28% in
    W), the Newton step of the FP64 system is evaluated at W_guess exp(y); when
