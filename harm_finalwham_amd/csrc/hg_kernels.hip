@@ -247,19 +247,22 @@ __global__ void __launch_bounds__(256) k_bound(double *p, const double *__restri
 // Riemann flux at one face from left/right states, fluxcompute.c:12
 // ---------------------------------------------------------------------------
 // One side's results (two sets of fluxes and two speeds), which live through the
-// whole computation of the other: 36 registers, or with PARK a place in LDS (37
-// kB per 256 faces, four blocks to a CU).  With the Kerr-Schild metric that is
-// the step from 164 registers and three wavefronts per SIMD to 128 and four
-// (flux_waves), with the full one from 192 and two to 158 and three.  Worth it
-// where the device is full: 256x128x64 WENO5BND 0.285 -> 0.259 ms per direction
-// and step, the PARA step 5.64 -> 5.32 ms, 128x64x32 WENO5BND 655 -> 634 us, PARA
-// 854 -> 808, MC 327 -> 297 (without the bound; 305 with).  A grid of up to
-// PARK_BLOCKS blocks only pays the round trip (59x19x7 WENO5BND 175.0 -> 176.5
-// us), and so do the large MC kernels, which their stencil loads bound.
-typedef double (*FluxPark)[256];
-__device__ __forceinline__ FluxPark flux_park() {
-  __shared__ double park[2 * NPR + 2][256];
-  return park;
+// whole computation of the other: 36 registers, or with PARK a place in LDS (9.2
+// kB per wavefront, the launch's dynamic size: 16 wavefronts to a CU whatever the
+// block).  With the Kerr-Schild metric that is the step from 164 registers and
+// three wavefronts per SIMD to 128 and four (flux_waves), with the full one from
+// 192 and two to 158 and three.  Worth it where the device is full: 256x128x64
+// WENO5BND 0.285 -> 0.259 ms per direction and step, the PARA step 5.64 -> 5.32
+// ms, 128x64x32 WENO5BND 655 -> 634 us, PARA 854 -> 808, MC 327 -> 297 (without
+// the bound; 305 with).  A grid of up to PARK_BLOCKS blocks only pays the round
+// trip (59x19x7 WENO5BND 175.0 -> 176.5 us), and so do the large MC kernels,
+// which their stencil loads bound.
+constexpr int PARK_N = 2 * NPR + 2;
+constexpr size_t park_bytes(bool park, unsigned threads) { return park ? threads * PARK_N * sizeof(double) : 0; }
+// number pl of a lane's place is 64 doubles from number pl - 1
+__device__ __forceinline__ double *flux_park() {
+  extern __shared__ double park[];
+  return park + (threadIdx.x >> 6) * (PARK_N * 64) + (threadIdx.x & 63);
 }
 constexpr unsigned PARK_BLOCKS = 1024;
 constexpr int flux_waves(bool bound, bool ks) { return bound && ks ? 4 : 1; }
@@ -287,14 +290,14 @@ __device__ __forceinline__ bool face_flux(int dir, GT &G, double *p_l, double *p
     if (vchar(p_l, ql, dir, G, gam, cmax_l, cmin_l)) return true;
   }
   if constexpr (PARK) {
-    const FluxPark park = flux_park();
+    double *park = flux_park();
 #pragma unroll
     for (int pl = 0; pl < NPR; pl++) {
-      park[pl][threadIdx.x] = F_l[pl];
-      park[NPR + pl][threadIdx.x] = U_l[pl];
+      park[pl * 64] = F_l[pl];
+      park[(NPR + pl) * 64] = U_l[pl];
     }
-    park[2 * NPR][threadIdx.x] = cmax_l;
-    park[2 * NPR + 1][threadIdx.x] = cmin_l;
+    park[2 * NPR * 64] = cmax_l;
+    park[(2 * NPR + 1) * 64] = cmin_l;
     asm volatile("" ::: "memory");
   }
   geom_barrier(G);
@@ -309,15 +312,15 @@ __device__ __forceinline__ bool face_flux(int dir, GT &G, double *p_l, double *p
     if (vchar(p_r, qr, dir, G, gam, cmax_r, cmin_r)) return true;
   }
   if constexpr (PARK) {
-    const FluxPark park = flux_park();
+    const double *park = flux_park();
     asm volatile("" ::: "memory");
 #pragma unroll
     for (int pl = 0; pl < NPR; pl++) {
-      F_l[pl] = park[pl][threadIdx.x];
-      U_l[pl] = park[NPR + pl][threadIdx.x];
+      F_l[pl] = park[pl * 64];
+      U_l[pl] = park[(NPR + pl) * 64];
     }
-    cmax_l = park[2 * NPR][threadIdx.x];
-    cmin_l = park[2 * NPR + 1][threadIdx.x];
+    cmax_l = park[2 * NPR * 64];
+    cmin_l = park[(2 * NPR + 1) * 64];
   }
   // wavespeeds.c:325 cminmax_calc
   double lmin = rmin(cmin_l, cmin_r);
@@ -1306,16 +1309,16 @@ void launch_gather_inversions(const double *ubuf, const double *pb, const double
 static inline unsigned nblocks(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
 // the instance of a kernel template for the grid's metric (Dims::ks, GeomT):
-// its last template argument
-#define HG_LAUNCH_KS(ks, K, A, g, b, ...)                                            \
+// its last template argument; lds: dynamic LDS (park_bytes of a parking kernel)
+#define HG_LAUNCH_KS(ks, K, A, g, b, lds, ...)                                       \
   do {                                                                               \
-    if (ks) hipLaunchKernelGGL((K<A, true>), g, b, 0, s, __VA_ARGS__);               \
-    else hipLaunchKernelGGL((K<A, false>), g, b, 0, s, __VA_ARGS__);                 \
+    if (ks) hipLaunchKernelGGL((K<A, true>), g, b, lds, s, __VA_ARGS__);             \
+    else hipLaunchKernelGGL((K<A, false>), g, b, lds, s, __VA_ARGS__);               \
   } while (0)
-#define HG_LAUNCH_KS2(ks, K, A, B, g, b, ...)                                        \
+#define HG_LAUNCH_KS2(ks, K, A, B, g, b, lds, ...)                                   \
   do {                                                                               \
-    if (ks) hipLaunchKernelGGL((K<A, B, true>), g, b, 0, s, __VA_ARGS__);            \
-    else hipLaunchKernelGGL((K<A, B, false>), g, b, 0, s, __VA_ARGS__);              \
+    if (ks) hipLaunchKernelGGL((K<A, B, true>), g, b, lds, s, __VA_ARGS__);          \
+    else hipLaunchKernelGGL((K<A, B, false>), g, b, lds, s, __VA_ARGS__);            \
   } while (0)
 
 static unsigned bound_total(const Dims &d) {
@@ -1324,10 +1327,10 @@ static unsigned bound_total(const Dims &d) {
   return nblk[0] + nblk[1] + nblk[2];
 }
 
-#define HG_LAUNCH_KS3(ks, K, A, B, C, g, b, ...)                                     \
+#define HG_LAUNCH_KS3(ks, K, A, B, C, g, b, lds, ...)                                \
   do {                                                                               \
-    if (ks) hipLaunchKernelGGL((K<A, B, C, true>), g, b, 0, s, __VA_ARGS__);         \
-    else hipLaunchKernelGGL((K<A, B, C, false>), g, b, 0, s, __VA_ARGS__);           \
+    if (ks) hipLaunchKernelGGL((K<A, B, C, true>), g, b, lds, s, __VA_ARGS__);       \
+    else hipLaunchKernelGGL((K<A, B, C, false>), g, b, lds, s, __VA_ARGS__);         \
   } while (0)
 
 void launch_bound(double *p, const double *geo, const Dims &d, double gammamax, int *err, hipStream_t s,
@@ -1359,9 +1362,9 @@ void launch_flux_dirs(const FluxDirs &f, int lim, bool fv, const double *p, cons
                       hipStream_t s) {
   const dim3 g(f.nblocks), b(256);
   const bool para = lim == HG_LIM_PARA;
-#define HG_LR(FV, PARK) HG_LAUNCH_KS2(d.ks, k_flux_lr_dirs, FV, PARK, g, b, geo, f, d, gam, cour, fluxmethod, ndt_bits, err)
+#define HG_LR(FV, PARK) HG_LAUNCH_KS2(d.ks, k_flux_lr_dirs, FV, PARK, g, b, park_bytes(PARK, 256), geo, f, d, gam, cour, fluxmethod, ndt_bits, err)
 #define HG_PT(PARA, FV, PARK)                                                                                        \
-  HG_LAUNCH_KS3(d.ks, k_flux_pt_dirs, PARA, FV, PARK, g, b, p, geo, f, d, gam, cour, fluxmethod, lim, ndt_bits, err)
+  HG_LAUNCH_KS3(d.ks, k_flux_pt_dirs, PARA, FV, PARK, g, b, park_bytes(PARK, 256), p, geo, f, d, gam, cour, fluxmethod, lim, ndt_bits, err)
 #define HG_PARK(L, ...)                       \
   do {                                        \
     if (f.nblocks > PARK_BLOCKS) L(__VA_ARGS__, true); \
@@ -1389,6 +1392,7 @@ void launch_flux_point(int dir, int lim, bool fv, const double *p, const double 
   int64_t n = (int64_t)fr.ni * fr.nj * fr.nk;
   dim3 g(nblocks(n, tu.bs_flux)), b(tu.bs_flux);
   const bool para = lim == HG_LIM_PARA;
+  const size_t lds = park_bytes(true, b.x);
   if (fluxmethod >= 2) {
     if (para) {
       if (dir == 1) hipLaunchKernelGGL((k_flux_pt_ext<1, true>), g, b, 0, s, p, geo, F, d, (int)fv, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
@@ -1403,25 +1407,25 @@ void launch_flux_point(int dir, int lim, bool fv, const double *p, const double 
   }
   if (fv) {
     if (para) {
-      if (dir == 1) HG_LAUNCH_KS2(d.ks, k_flux_pt_fv, 1, true, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
-      if (dir == 2) HG_LAUNCH_KS2(d.ks, k_flux_pt_fv, 2, true, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
-      if (dir == 3) HG_LAUNCH_KS2(d.ks, k_flux_pt_fv, 3, true, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+      if (dir == 1) HG_LAUNCH_KS2(d.ks, k_flux_pt_fv, 1, true, g, b, lds, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+      if (dir == 2) HG_LAUNCH_KS2(d.ks, k_flux_pt_fv, 2, true, g, b, lds, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+      if (dir == 3) HG_LAUNCH_KS2(d.ks, k_flux_pt_fv, 3, true, g, b, lds, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
     } else {
-      if (dir == 1) HG_LAUNCH_KS2(d.ks, k_flux_pt_fv, 1, false, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
-      if (dir == 2) HG_LAUNCH_KS2(d.ks, k_flux_pt_fv, 2, false, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
-      if (dir == 3) HG_LAUNCH_KS2(d.ks, k_flux_pt_fv, 3, false, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+      if (dir == 1) HG_LAUNCH_KS2(d.ks, k_flux_pt_fv, 1, false, g, b, 0, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+      if (dir == 2) HG_LAUNCH_KS2(d.ks, k_flux_pt_fv, 2, false, g, b, 0, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+      if (dir == 3) HG_LAUNCH_KS2(d.ks, k_flux_pt_fv, 3, false, g, b, 0, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
     }
     return;
   }
   if (para) {
-    if (dir == 1) HG_LAUNCH_KS(d.ks, k_flux_para, 1, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
-    if (dir == 2) HG_LAUNCH_KS(d.ks, k_flux_para, 2, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
-    if (dir == 3) HG_LAUNCH_KS(d.ks, k_flux_para, 3, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+    if (dir == 1) HG_LAUNCH_KS(d.ks, k_flux_para, 1, g, b, lds, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+    if (dir == 2) HG_LAUNCH_KS(d.ks, k_flux_para, 2, g, b, lds, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+    if (dir == 3) HG_LAUNCH_KS(d.ks, k_flux_para, 3, g, b, lds, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
     return;
   }
-  if (dir == 1) HG_LAUNCH_KS(d.ks, k_flux_mc, 1, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
-  if (dir == 2) HG_LAUNCH_KS(d.ks, k_flux_mc, 2, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
-  if (dir == 3) HG_LAUNCH_KS(d.ks, k_flux_mc, 3, g, b, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+  if (dir == 1) HG_LAUNCH_KS(d.ks, k_flux_mc, 1, g, b, 0, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+  if (dir == 2) HG_LAUNCH_KS(d.ks, k_flux_mc, 2, g, b, 0, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
+  if (dir == 3) HG_LAUNCH_KS(d.ks, k_flux_mc, 3, g, b, 0, p, geo, F, d, gam, cour, dxdir, fluxmethod, lim, ndt_bits, err);
 }
 
 // initbase.c:18 init_conservatives (primtoU of every active zone) into the
@@ -1459,6 +1463,7 @@ void launch_flux_lr(int dir, const double *pleft, const double *pright, const do
   FaceRange fr = fv ? face_range_fv(d, dir) : face_range(d, dir);
   int64_t n = (int64_t)fr.ni * fr.nj * fr.nk;
   dim3 g(nblocks(n, tu.bs_flux)), b(tu.bs_flux);
+  const size_t lds = park_bytes(true, b.x);
   if (fluxmethod >= 2) {
     if (dir == 1) hipLaunchKernelGGL(k_flux_lr_ext<1>, g, b, 0, s, pleft, pright, geo, F, d, (int)fv, gam, cour, dxdir, fluxmethod, ndt_bits, err);
     if (dir == 2) hipLaunchKernelGGL(k_flux_lr_ext<2>, g, b, 0, s, pleft, pright, geo, F, d, (int)fv, gam, cour, dxdir, fluxmethod, ndt_bits, err);
@@ -1466,14 +1471,14 @@ void launch_flux_lr(int dir, const double *pleft, const double *pright, const do
     return;
   }
   if (fv) {
-    if (dir == 1) HG_LAUNCH_KS(d.ks, k_flux_lr_fv, 1, g, b, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
-    if (dir == 2) HG_LAUNCH_KS(d.ks, k_flux_lr_fv, 2, g, b, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
-    if (dir == 3) HG_LAUNCH_KS(d.ks, k_flux_lr_fv, 3, g, b, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
+    if (dir == 1) HG_LAUNCH_KS(d.ks, k_flux_lr_fv, 1, g, b, lds, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
+    if (dir == 2) HG_LAUNCH_KS(d.ks, k_flux_lr_fv, 2, g, b, lds, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
+    if (dir == 3) HG_LAUNCH_KS(d.ks, k_flux_lr_fv, 3, g, b, lds, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
     return;
   }
-  if (dir == 1) HG_LAUNCH_KS(d.ks, k_flux_lr, 1, g, b, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
-  if (dir == 2) HG_LAUNCH_KS(d.ks, k_flux_lr, 2, g, b, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
-  if (dir == 3) HG_LAUNCH_KS(d.ks, k_flux_lr, 3, g, b, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
+  if (dir == 1) HG_LAUNCH_KS(d.ks, k_flux_lr, 1, g, b, lds, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
+  if (dir == 2) HG_LAUNCH_KS(d.ks, k_flux_lr, 2, g, b, lds, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
+  if (dir == 3) HG_LAUNCH_KS(d.ks, k_flux_lr, 3, g, b, lds, pleft, pright, geo, F, d, gam, cour, dxdir, fluxmethod, ndt_bits, err);
 }
 
 void launch_emf(const double *F1, const double *F2, const double *F3, const double *geo, const double *corn,
@@ -1530,13 +1535,13 @@ void launch_update(const double *pi, const double *pb, double *ubuf, const doubl
   dim3 g(nblocks(n, tu.bs_update)), b(tu.bs_update);
   const double i1 = 1.0 / dx[1], i2 = 1.0 / dx[2], i3 = 1.0 / dx[3];
   if (rk.ucons)
-    HG_LAUNCH_KS2(d.ks, k_update, true, true, g, b, pi, pb, ubuf, F1, F2, F3, e1, e2, e3, geo, conn, dtp, rk, d,
+    HG_LAUNCH_KS2(d.ks, k_update, true, true, g, b, 0, pi, pb, ubuf, F1, F2, F3, e1, e2, e3, geo, conn, dtp, rk, d,
                        gam, i1, i2, i3, err);
   else if (rk.ucum)
-    HG_LAUNCH_KS2(d.ks, k_update, true, false, g, b, pi, pb, ubuf, F1, F2, F3, e1, e2, e3, geo, conn, dtp, rk,
+    HG_LAUNCH_KS2(d.ks, k_update, true, false, g, b, 0, pi, pb, ubuf, F1, F2, F3, e1, e2, e3, geo, conn, dtp, rk,
                        d, gam, i1, i2, i3, err);
   else
-    HG_LAUNCH_KS2(d.ks, k_update, false, false, g, b, pi, pb, ubuf, F1, F2, F3, e1, e2, e3, geo, conn, dtp, rk,
+    HG_LAUNCH_KS2(d.ks, k_update, false, false, g, b, 0, pi, pb, ubuf, F1, F2, F3, e1, e2, e3, geo, conn, dtp, rk,
                        d, gam, i1, i2, i3, err);
 }
 
@@ -1696,17 +1701,17 @@ void launch_group(int k, const GridView *views, const unsigned *first, int n, un
   switch (k) {
     case GK_BOUNDDT: hipLaunchKernelGGL(kg_bound<true>, g, dim3(256), 0, s, views, first, n); return;
     case GK_BOUND: hipLaunchKernelGGL(kg_bound<false>, g, dim3(256), 0, s, views, first, n); return;
-    case GK_FLUX1: HG_LAUNCH_KS(ks, kg_flux_lr, 1, g, dim3(256), views, first, n); return;
-    case GK_FLUX2: HG_LAUNCH_KS(ks, kg_flux_lr, 2, g, dim3(256), views, first, n); return;
-    case GK_FLUX3: HG_LAUNCH_KS(ks, kg_flux_lr, 3, g, dim3(256), views, first, n); return;
+    case GK_FLUX1: HG_LAUNCH_KS(ks, kg_flux_lr, 1, g, dim3(256), park_bytes(true, 256), views, first, n); return;
+    case GK_FLUX2: HG_LAUNCH_KS(ks, kg_flux_lr, 2, g, dim3(256), park_bytes(true, 256), views, first, n); return;
+    case GK_FLUX3: HG_LAUNCH_KS(ks, kg_flux_lr, 3, g, dim3(256), park_bytes(true, 256), views, first, n); return;
     case GK_EMF: hipLaunchKernelGGL(kg_emf, g, dim3(256), 0, s, views, first, n); return;
-    case GK_UPDATE: HG_LAUNCH_KS(ks, kg_update, false, g, dim3(256), views, first, n); return;
-    case GK_UPDATEU: HG_LAUNCH_KS(ks, kg_update, true, g, dim3(256), views, first, n); return;
+    case GK_UPDATE: HG_LAUNCH_KS(ks, kg_update, false, g, dim3(256), 0, views, first, n); return;
+    case GK_UPDATEU: HG_LAUNCH_KS(ks, kg_update, true, g, dim3(256), 0, views, first, n); return;
     case GK_UPINV: hipLaunchKernelGGL(kg_update_invert<false>, g, dim3(256), 0, s, views, first, n); return;
     case GK_UPINVU: hipLaunchKernelGGL(kg_update_invert<true>, g, dim3(256), 0, s, views, first, n); return;
     case GK_INVERT:
-      if (mode == INV_MIXED) HG_LAUNCH_KS(ks, kg_invert, INV_MIXED, g, dim3(256), views, first, n);
-      else if (mode == INV_LEARNED) HG_LAUNCH_KS(ks, kg_invert, INV_LEARNED, g, dim3(256), views, first, n);
+      if (mode == INV_MIXED) HG_LAUNCH_KS(ks, kg_invert, INV_MIXED, g, dim3(256), 0, views, first, n);
+      else if (mode == INV_LEARNED) HG_LAUNCH_KS(ks, kg_invert, INV_LEARNED, g, dim3(256), 0, views, first, n);
       else hipLaunchKernelGGL((kg_invert<INV_FP64, false>), g, dim3(256), 0, s, views, first, n);
       return;
     case GK_FEATURES: hipLaunchKernelGGL(kg_step_features, g, dim3(256), 0, s, views, first, n); return;
