@@ -606,8 +606,11 @@ extern "C" int hg_autotune(hg_ctx *c, int nsteps, hg_tune *best, void *stream) {
                               {&Tune::weno_xmarch, {0, 2, 4}}, {&Tune::weno_nseg3, {1, 2, 3, 4}}};
     if (c->cfg.lim == HG_LIM_MC) axes.resize(4);
     else if (c->d.n3 == 1) axes.pop_back();  // no reconstruction along k
+    // one kernel updates and inverts: bs_invert is not read, only noise would pick it
+    const bool fused = update_invert_fused(c->d, c->c2p_mode == HG_C2P_FP64 ? 0 : 1);
     for (const Axis &ax : axes) {
       if (rc) break;
+      if (fused && ax.field == &Tune::bs_invert) continue;
       for (int v : ax.values) {
         if (cur.*(ax.field) == v) continue;
         Tune trial = cur;

@@ -439,21 +439,27 @@ int hg_graph_launch(hg_graph *g, void *stream);
 int hg_graph_destroy(hg_graph *g);
 
 /* Launch shapes of the step (no effect on results): block sizes of the flux,
-   EMF, update and inversion kernels (64, 128 or 256), wavefronts per block of
-   the i-direction reconstruction (1, 2 or 4), segments per line of the j
-   and of the k reconstruction (0 = by line length), and the scheme along i
-   (weno_xmarch 0: one lane per point with wavefront shuffles; n > 0: lanes
-   across j and k marching along i in n segments).  hg_autotune times nsteps steps per
-   candidate (coordinate descent) from the current state, restores the state
-   (primitives, intermediate states, the finite-volume scheme's carried
-   conserved state, unew, failure codes), dt and counters, keeps the fastest
-   shapes and returns them in *best (may be NULL).  Diagnostics recording is
-   paused during the trials.  No counterpart in the reference. */
+   EMF, update and inversion kernels (64, 128 or 256; with the Kerr-Schild
+   metric's zeros and HG_C2P_FP64 one kernel updates and inverts, in blocks of
+   bs_update, and bs_invert is read by captured steps alone), wavefronts per
+   block of the i-direction reconstruction (1, 2 or 4), segments per line of the
+   j and of the k reconstruction (0 = by line length and grid), and the scheme
+   along i (weno_xmarch 0: one lane per point with wavefront shuffles; n > 0:
+   lanes across j and k marching along i in n segments).  hg_autotune times
+   nsteps steps per candidate (coordinate descent) of each shape the step reads,
+   from the current state, restores the state (primitives, intermediate states,
+   the finite-volume scheme's carried conserved state, unew, failure codes), dt
+   and counters, keeps the fastest shapes and returns them in *best (may be
+   NULL).  Diagnostics recording is paused during the trials.  No counterpart in
+   the reference. */
 typedef struct {
   int bs_flux, bs_emf, bs_update, bs_invert;
   int weno_xwaves, weno_nseg, weno_nseg3;
   int weno_xmarch;
-  int concurrent; /* 1: the three directions' fluxes on three streams, 0: in turn */
+  /* 1: the directions' fluxes side by side: in one launch on small grids (up to
+     5000 blocks, LAXF or HLL, bs_flux 256, for WENO5BND weno_xwaves 4 and
+     weno_xmarch 0), else on three streams; 0: one direction after another */
+  int concurrent;
 } hg_tune;
 int hg_get_tune(const hg_ctx *ctx, hg_tune *t);
 int hg_set_tune(hg_ctx *ctx, const hg_tune *t);
