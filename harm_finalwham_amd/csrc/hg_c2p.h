@@ -85,26 +85,6 @@ __device__ __forceinline__ void newton_dx_full(const C2PInv &c, double igr, doub
   f = -0.5 * df;
 }
 
-// sqrt(x) for x in [2^-60, 2^60]: the steps hipcc lowers it to, without the
-// scaling of tiny arguments and the choice of 0 and infinity around them
-__device__ __forceinline__ double sqrt_core(double x) {
-  const double y = __builtin_amdgcn_rsq(x);
-  double g = x * y, h = 0.5 * y;
-  const double r = fma(-h, g, 0.5);
-  g = fma(g, r, g);
-  h = fma(h, r, h);
-  double d = fma(-g, g, x);
-  g = fma(d, h, g);
-  d = fma(-g, g, x);
-  return fma(d, h, g);
-}
-
-// 1 / d for |d| in [2^-300, 2^300] (div_core with a numerator of 1)
-__device__ __forceinline__ double rcp_core(double d) {
-  const double y = rcp_refined(d);
-  return fma(fma(-d, y, 1.0), y, y);
-}
-
 // newton_dx_full bit for bit.  The iteration is a serial chain of seven
 // divisions and a square root, and the instruction count sets its time both
 // where lanes fill the SIMDs and where one wavefront walks the last zones;

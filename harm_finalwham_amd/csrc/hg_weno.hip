@@ -63,7 +63,7 @@ __device__ __forceinline__ double sum5(const double *a) { return ((a[0] + a[4]) 
 // The quotients of the weights.  Every numerator and divisor of these
 // functions but the smoothness indicators' is bounded by the step that formed
 // it, so the hardware division's scaling and fix-up steps have nothing to do
-// and are left out (div_core, hg_div.h):
+// and are left out (div_bounded and div_weights, hg_div.h):
 //   indicators over their sum   si in [0, ss]; div_weights looks at the range
 //   1 / t^2, t = si + 1e-26     si is such a quotient, in [0, 1]
 //   w / sum of w                w = 1 / t^2 in [0.99, 1e52]
@@ -73,34 +73,6 @@ __device__ __forceinline__ double sum5(const double *a) { return ((a[0] + a[4]) 
 // (cusp, mono_eno5) the reconstruction at 256x128x64 went from 0.428 / 0.514 /
 // 0.538 to 0.310 / 0.355 / 0.355 ms along i / j / k: FP64 issue bounds it, and
 // about 33 full divisions a point were half of that.
-template <int K>
-__device__ __forceinline__ void div_bounded(double *x, double d) {
-  const double y = rcp_refined(d);
-#pragma unroll
-  for (int k = 0; k < K; k++) x[k] = div_core(x[k], d, y);
-}
-__device__ __forceinline__ double rcp_bounded(double d) {
-  const double y = rcp_refined(d);
-  return fma(fma(-d, y, 1.0), y, y);
-}
-// indicators si >= e >= 0 over d = their sum ss + DBL_MIN: in the steps' range
-// when e >= 2^-600 and d <= 2^600, or when ss = 0 (a line of zeros: every
-// quotient is +0); full divisions otherwise
-template <int K>
-__device__ __forceinline__ void div_weights(double *si, double ss, double e) {
-  const double d = ss + DBL_MIN;
-  double q[K];
-#pragma unroll
-  for (int k = 0; k < K; k++) q[k] = si[k];
-  div_bounded<K>(q, d);
-  if (__builtin_expect((e >= 0x1p-600 && d <= 0x1p600) || ss == 0.0, 1)) {
-#pragma unroll
-    for (int k = 0; k < K; k++) si[k] = q[k];
-  } else {
-#pragma unroll
-    for (int k = 0; k < K; k++) si[k] /= d;
-  }
-}
 // indicators normalised by their sum -> weights normalised by theirs
 template <int K>
 __device__ __forceinline__ void norm_weights(const double *si, double *w) {
@@ -108,7 +80,7 @@ __device__ __forceinline__ void norm_weights(const double *si, double *w) {
   for (int s = 0; s < K; s++) {
     double t = si[s] + WENO_EPS / 1.;
     t *= t;
-    w[s] = rcp_bounded(t);
+    w[s] = rcp_core(t);
   }
   div_bounded<K>(w, K == 3 ? sum3(w[0], w[1], w[K - 1]) : w[0] + w[1]);
 }

@@ -450,9 +450,9 @@ def make_c2p_batch(n, gam=4.0 / 3.0, a=0.9375, seed=1, device="cuda"):
 
 
 def check_division(n, seed=1):
-    """hg_check_division: mismatches of the shared-reciprocal division
-    against the hardware's x / d over n generated operand sets ([shared
-    divisor, reciprocal, divisor 12, sets on the shortcut])."""
+    """hg_check_division: mismatches of the arithmetic without scaling steps
+    against the hardware's own over n generated operand sets ([quotients,
+    reciprocals and roots, divisor 12 and decisions, sets on the shortcut])."""
     r = np.zeros(4, dtype=np.int64)
     _check(lib().hg_check_division(int(n), int(seed), r.ctypes.data_as(C.POINTER(C.c_int64))))
     return [int(v) for v in r]

@@ -467,13 +467,16 @@ int hg_autotune(hg_ctx *ctx, int nsteps, hg_tune *best, void *stream);
 
 const char *hg_last_error(void);
 
-/* Device self-check of the shared-reciprocal FP64 division the WENO5BND
-   kernels use (a test hook, no counterpart in the reference): n generated
-   operand sets from seed; result[0], [1], [2] count the mismatches against
-   the hardware's own x / d of three numerators sharing one divisor, of 1 / d,
-   and of four signed numerators of the divisor 12 (a zero quotient compared
-   without its sign); result[3] counts the sets inside the shortcut's
-   ranges.  n at most 2^32. */
+/* Device self-check of the FP64 arithmetic that leaves out the scaling steps of
+   the hardware's division and square root (a test hook, no counterpart in the
+   reference): n generated operand sets from seed; result[0], [1], [2] count the
+   mismatches, bit for bit, against the full operations: [0] of quotients (three
+   numerators of one divisor anywhere; the quotients of the WENO5BND weights and
+   of the Newton steps over their ranges), [1] of reciprocals and square roots,
+   [2] of four signed numerators of the divisor 12, and of the Newton loop's
+   decisions taken by a product (its stopping test and its cap on W, infinities
+   and NaN included); result[3] counts the sets inside the shortcut's ranges.
+   n at most 2^32. */
 int hg_check_division(int64_t n, uint64_t seed, int64_t result[4]);
 
 /* Kernel-class timing, no counterpart in the reference (its timing is the
