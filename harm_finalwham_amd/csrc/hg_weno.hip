@@ -591,10 +591,7 @@ __device__ __forceinline__ void weno_m_body(const double *__restrict__ p, const 
   double ndp = WM_LDD(db, e0);
   WM_ST(lb, e0) = 0.;
   WM_ST(rb, e0) = 0.;
-#ifndef UN
-#define UN 1
-#endif
-#pragma unroll UN
+#pragma unroll 1
   for (int t = e0 - 3; t <= tlast; t++) {
     const double cy = ny, cdp = ndp;
     {
