@@ -118,10 +118,13 @@ int move_state(hg_ctx *c, double *dev, double *host) {
   }
   // two calls on one context share its slots
   std::lock_guard<std::mutex> lk(c->slots_mu);
+  // the kernels run where the state is, whichever device the caller has set
+  int caller = c->device;
+  (void)hipGetDevice(&caller);
+  hipError_t e = caller == c->device ? hipSuccess : hipSetDevice(c->device);
   const size_t bytes = pieces.size() == 1 ? (size_t)d.m1 * Q * sizeof(double) : SLOT;
   size_t want = pieces.size() < (size_t)HOST_SLOTS ? pieces.size() : (size_t)HOST_SLOTS;
-  hipError_t e = hipSuccess;
-  for (size_t k = 0; k < want; k++) {
+  for (size_t k = 0; k < want && e == hipSuccess; k++) {
     HostSlot &s = c->slots[k];
     if (!s.mem) {
       if (!s.done) e = hipEventCreateWithFlags(&s.done, hipEventDisableTiming);
@@ -135,13 +138,11 @@ int move_state(hg_ctx *c, double *dev, double *host) {
       }
     }
   }
-  int dev_id = 0;
-  if (e == hipSuccess) e = hipGetDevice(&dev_id);
   if (e == hipSuccess) {
     std::atomic<size_t> next{0};
     std::vector<hipError_t> err(want, hipSuccess);
     auto work = [&](size_t k) {
-      if (k) err[k] = hipSetDevice(dev_id);  // a new thread starts on device 0
+      if (k) err[k] = hipSetDevice(c->device);  // a new thread starts on device 0
       for (size_t n; err[k] == hipSuccess && (n = next.fetch_add(1)) < pieces.size();)
         err[k] = move_piece<TO_DEVICE>(d, dev, host, pieces[n], c->slots[k]);
     };
@@ -157,6 +158,7 @@ int move_state(hg_ctx *c, double *dev, double *host) {
     for (hipError_t k : err)
       if (e == hipSuccess) e = k;
   }
+  if (caller != c->device) (void)hipSetDevice(caller);
   if (e != hipSuccess) {
     set_error("copying a state: %s", hipGetErrorString(e));
     return 1;

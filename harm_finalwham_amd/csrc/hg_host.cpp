@@ -82,6 +82,7 @@ extern "C" int hg_ctx_create(const hg_config *cfg, hg_ctx **out) {
   c->cfg = *cfg;
   c->d = make_dims(cfg->n1, cfg->n2, cfg->n3, cfg->nb);
   const Dims &d = c->d;
+  (void)hipGetDevice(&c->device);
   size_t ns = (size_t)d.spl * NPR, nz = (size_t)d.spl;
   int rc = 0;
   rc |= dalloc(&c->p, ns);

@@ -20,6 +20,7 @@ constexpr int HOST_SLOTS = 8;
 struct hg_ctx {
   hg_config cfg;
   hg::Dims d;
+  int device = 0;  // the one its memory is on
   double *p = nullptr, *pk = nullptr;        // primitives and the first intermediate state
   double *pk2 = nullptr, *ucum = nullptr;    // RK4 only: second intermediate state, ucum
   // finite-volume scheme: carried conserved state; stale until derived from
