@@ -511,28 +511,30 @@ __device__ __forceinline__ bool c2p_polish(const C2PInv &c, double igr, double &
   for (int k = 0; k < n64 && !ok; k++) {
     double dx0, dx1, f, df;
     newton_dx(c, igr, x0, x1, dx0, dx1, f, df);
-    double xo0 = x0;
-    x0 = fabs(x0 + dx0);
-    const bool big = w_too_big(c, x0);  // W stays: not converged, however little it moved
+    const double xo0 = x0, xn = x0 + dx0;
+    x0 = fabs(xn);
+    // W put back, or turned round from below zero: not converged, however little
+    // it moved (a step of -2 W does not move it)
+    const bool big = w_too_big(c, x0), held = big || xn < 0.;
     x0 = big ? xo0 : x0;
     x1 += dx1;
     x1 = (x1 > 1.) ? vsq_big : x1;
     iters++;
-    ok = !big && fabs(x0 - xo0) <= 1e-9 * x0;
+    ok = !held && fabs(x0 - xo0) <= 1e-9 * x0;
   }
   if (!ok) return false;
   ok = false;
   for (int k = 0; k < POLISH_MAX_DD && !ok; k++) {
     double dx0, dx1;
     newton_dx_dd(c, igr, x0, x1, dx0, dx1);
-    double xo0 = x0;
-    x0 = fabs(x0 + dx0);
-    const bool big = w_too_big(c, x0);
+    const double xo0 = x0, xn = x0 + dx0;
+    x0 = fabs(xn);
+    const bool big = w_too_big(c, x0), held = big || xn < 0.;
     x0 = big ? xo0 : x0;
     x1 += dx1;
     x1 = (x1 > 1.) ? vsq_big : x1;
     iters++;
-    ok = !big && fabs(x0 - xo0) <= 1e-12 * x0;
+    ok = !held && fabs(x0 - xo0) <= 1e-12 * x0;
   }
   return ok && isfinite(x0) && isfinite(x1);
 }
