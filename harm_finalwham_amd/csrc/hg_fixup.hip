@@ -379,16 +379,31 @@ __device__ __forceinline__ void fx_apply_body(double *__restrict__ p, const Dims
   }
 }
 
+// whether the lists were too long for one block, told to the host when it changes
+constexpr unsigned FX_LONG_FIXES = 256, FX_LONG_CANDIDATES = 2048;
+__device__ __forceinline__ void fx_note(const FxBufs &b) {
+  const unsigned lng = b.count[1] > FX_LONG_FIXES || b.count[0] > FX_LONG_CANDIDATES;
+  if (lng != b.count[4]) {
+    b.count[4] = lng;
+    *b.lists_long = (int)lng;
+  }
+}
+
 __global__ void __launch_bounds__(256) k_fx_apply(double *__restrict__ p, Dims d, FxBufs b) {
   fx_apply_body(p, d, b, blockIdx.x, gridDim.x);
+  if (blockIdx.x == 0 && threadIdx.x == 0) fx_note(b);
 }
 
 // The four kernels as one launch for a grid of at most FX_ONE_ZONES zones: the
 // block that finishes the check last goes on with the lists alone.  On a
 // small grid the lists are short or empty and the launches are all that the
 // four cost: 128^2 zones take 8.5 us and three gaps of 2 to 4 us in four
-// launches, 5.9 us in this one.  The bound keeps the case where every zone is on a
-// list at 128 rounds of one block.  Every block releases what it wrote before
+// launches, 5.9 us in this one.  One block is slow with long lists: hg_post_fixup
+// of 32^3 zones takes 93 us with none failed and 132 in four launches, 171 and
+// 173 with 1 % failed, 450 and 163 with 10 %; 128^2 fast zones, all candidates,
+// take 237 and 158.  So the host takes the four while the last lists it heard of
+// were long (fx_note); that is late by the launches queued since, and a captured
+// launch stays what it was, with the same results.  Every block releases what it wrote before
 // it takes its ticket; the last one acquires that before it reads.  The release
 // writes the L2 back, so it is taken once per block (by every wavefront: 8.7 us), and
 // the grouped launch, whose hundreds of blocks share the L2s, keeps the four
@@ -420,7 +435,10 @@ __device__ __forceinline__ void fx_all_body(double *p, const double *__restrict_
   fx_average_body(p, geo, d, b, finalstep, gammamax, gam, ucons, err, 0, 1);
   __syncthreads();
   fx_apply_body(p, d, b, 0, 1);
-  if (threadIdx.x == 0) b.count[3] = 0u;
+  if (threadIdx.x == 0) {
+    b.count[3] = 0u;
+    fx_note(b);
+  }
 }
 
 __global__ void __launch_bounds__(256) k_fx_all(double *p, const double *__restrict__ geo, Dims d, FxBufs b,
@@ -491,8 +509,8 @@ int fixup_alloc(hg_ctx *c) {
   get((void **)&c->fx_fix_v, (size_t)act * 5 * sizeof(double));
   get((void **)&c->fx_fix_flag, (size_t)act);
   get((void **)&c->fx_fail_z, (size_t)act * sizeof(int));
-  get((void **)&c->fx_count, 4 * sizeof(unsigned));
-  if (e == hipSuccess) e = hipMemset(c->fx_count, 0, 4 * sizeof(unsigned));
+  get((void **)&c->fx_count, 5 * sizeof(unsigned));
+  if (e == hipSuccess) e = hipMemset(c->fx_count, 0, 5 * sizeof(unsigned));
   if (e == hipSuccess) e = hipMemset(c->pflag, 0, (size_t)d.spl);
   if (e != hipSuccess) {
     set_error("hg_ctx_create: %s", hipGetErrorString(e));
@@ -520,6 +538,7 @@ FxBufs fixup_bufs(hg_ctx *c) {
   b.fix_flag = c->fx_fix_flag;
   b.fail_z = c->fx_fail_z;
   b.count = c->fx_count;
+  b.lists_long = &c->out->fx_long;
   b.cap = (int)((int64_t)c->d.n1 * c->d.n2 * c->d.n3);
   return b;
 }
@@ -532,7 +551,7 @@ void launch_post_fixup(hg_ctx *c, double *p, int finalstep, hipStream_t s, bool 
   int64_t n = (int64_t)d.n1 * d.n2 * d.n3;
   unsigned nb = (unsigned)((n + 255) / 256);
   if (reset) hipLaunchKernelGGL(k_fx_reset, dim3(1), dim3(64), 0, s, b.count);
-  if (n <= FX_ONE_ZONES) {
+  if (n <= FX_ONE_ZONES && !*(volatile const int *)&c->out->fx_long) {
     hipLaunchKernelGGL(k_fx_all, dim3(nb), dim3(256), 0, s, p, c->geo, d, b, finalstep, c->cfg.gammamax, c->cfg.gam,
                        c->ucons, c->err);
     return;

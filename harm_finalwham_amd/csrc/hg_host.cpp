@@ -112,6 +112,7 @@ extern "C" int hg_ctx_create(const hg_config *cfg, hg_ctx **out) {
     if (e == hipSuccess) e = hipMalloc((void **)&c->counters, 2 * sizeof(unsigned long long));
     if (e == hipSuccess) e = hipMalloc((void **)&c->err, sizeof(int));
     if (e == hipSuccess) e = hipHostMalloc((void **)&c->out, sizeof(StepOut), hipHostMallocDefault);
+    if (e == hipSuccess) *c->out = StepOut{};
     if (e == hipSuccess) e = hipMemset(c->counters, 0, 2 * sizeof(unsigned long long));
     if (e == hipSuccess) e = hipMemset(c->err, 0, sizeof(int));
     for (int k = 0; k < 2 && e == hipSuccess; k++) {

@@ -34,6 +34,7 @@ struct StepOut {
   double dt;
   unsigned long long counters[2];
   int err;
+  int fx_long;  // post_fixup: FxBufs::lists_long
 };
 void launch_step_begin(double dt, double *dtp, unsigned long long *ndt_bits, unsigned long long *counters,
                        hipStream_t s);
@@ -144,7 +145,8 @@ struct FxBufs {
   double *fix_v;       // their RHO..U3 (5 x cap, structure of arrays)
   int8_t *fix_flag;    // their final flag
   int *fail_z;         // failed inversions that are not candidates
-  unsigned *count;     // [candidates, fixes, failed non-candidates, blocks done (k_fx_all)]
+  unsigned *count;     // [candidates, fixes, failed non-candidates, blocks done (k_fx_all), lists long]
+  int *lists_long;     // the last of these for the host (pinned), written when it changes
   int cap;
 };
 
