@@ -17,7 +17,7 @@
 //                   sum of every weight's gradient per block
 //   k_mlp_update    the partial sums added up, Adam, the BF16 copies of the
 //                   hidden-layer weights (or the gradient alone)
-//   k_mlp_set       the parameters a caller sets, and the copies
+//   k_mlp_set       the parameters a caller sets, the copies, the zeros of a gradient
 //   k_c2p_learned   the mixed-precision inversion (FP32 Newton, polish,
 //                   double-double primitives) from the learned start where
 //                   the network predicts a large correction and the start's
@@ -476,13 +476,14 @@ __global__ void __launch_bounds__(64 * UPDATE_WAYS) k_mlp_update(MlpDev m, const
 // the parameters a caller sets.  One that has the value it had keeps what its
 // FP32 number rounds off, so that setting the parameters just read leaves a
 // training as it is.
-__global__ void k_mlp_set(MlpDev m, const float *__restrict__ src) {
+__global__ void k_mlp_set(MlpDev m, const float *__restrict__ src, float *__restrict__ zero) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= NPARAM) return;
   const float v = src[e];
   if (e < NTRAIN) {
     if (__float_as_int(v) != __float_as_int(m.w[e])) m.wlo[e] = 0.f;
     refresh_bf16(e, v, m);
+    zero[e] = 0.f;
   }
   m.w[e] = v;
 }
@@ -584,7 +585,8 @@ static MlpDev dev_view(const hg_mlp *m) { return MlpDev{m->w, m->w1b, m->w2b, m-
 static hipError_t upload_params(hg_mlp *m, const float *host) {
   hipError_t e = hipMemcpy(m->part, host, NPARAM * sizeof(float), hipMemcpyHostToDevice);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_mlp_set, dim3((NPARAM + 255) / 256), dim3(256), 0, 0, dev_view(m), (const float *)m->part);
+  hipLaunchKernelGGL(k_mlp_set, dim3((NPARAM + 255) / 256), dim3(256), 0, 0, dev_view(m), (const float *)m->part,
+                     m->zero);
   e = hipGetLastError();
   return e == hipSuccess ? hipDeviceSynchronize() : e;
 }
@@ -665,7 +667,6 @@ extern "C" int hg_mlp_create(uint64_t seed, hg_mlp **out) {
     m->w2q = (float *)(b + o_w2q);
     m->part = (double *)(b + o_part);
     e = hipMemset(m->mem, 0, zeroed);
-    if (e == hipSuccess) e = hipMemset(m->zero, 0, np * 4);
   }
   if (e == hipSuccess) e = upload_params(m, w.data());
   if (e != hipSuccess) {
