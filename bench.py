@@ -209,9 +209,11 @@ def torus_scheme_cpu_baseline():
     return reference_timing(3, "PARA + HLL + RK4 finite volume")
 
 
-def _c2p_solve(b, gam, mode, reps, mlp=None):
+def _c2p_solve(b, gam, mode, reps, mlp=None, counted=True):
     """Best-of-reps kernel time (HIP events on the launch stream) of one
-    batched inversion; returns (pr, pflag, iters, ms, counts)."""
+    batched inversion; returns (pr, pflag, iters, ms, counts).  counted: with
+    the step counts, for which the mixed modes take the reference's whole walk
+    in the zones of their list."""
     import torch
     from harm_finalwham_amd import harmgpu
     best, cnt = None, None
@@ -225,8 +227,8 @@ def _c2p_solve(b, gam, mode, reps, mlp=None):
         torch.cuda.synchronize()
         e0.record()
         if mlp is None:
-            harmgpu.utoprim_batch(b["U"], b["gcov"], b["gcon"], b["gdet"], b["gcovpert"], pr, pflag, iters, gam=gam,
-                                  mode=mode)
+            harmgpu.utoprim_batch(b["U"], b["gcov"], b["gcon"], b["gdet"], b["gcovpert"], pr, pflag,
+                                  iters if counted else None, gam=gam, mode=mode)
         else:
             cnt = harmgpu.utoprim_batch_learned(mlp, b["U"], b["gcov"], b["gcon"], b["gdet"], b["gcovpert"], pr,
                                                 pflag, iters, gam=gam)
@@ -262,7 +264,8 @@ def c2p_bench(n, reps=3):
     kernel.  Errors are against the converged root."""
     from harm_finalwham_amd import harmgpu
     import torch
-    res = {"n": n, "gam": [], "fp64_ms": [], "refined_ms": [], "mixed_ms": [], "flags_identical": True,
+    res = {"n": n, "gam": [], "fp64_ms": [], "refined_ms": [], "mixed_ms": [],
+           "mixed_ms_without_counts": [], "flags_identical": True,
            "fallbacks": 0, "max_err_vs_converged": {"fp64": [0.0, 0.0, 0.0], "mixed": [0.0, 0.0, 0.0]},
            "fp64_iters_per_zone": [], "mixed_iters_per_zone": [], "mixed_wavefront_max_iters": []}
     for gam in (4.0 / 3.0, 5.0 / 3.0):
@@ -271,6 +274,7 @@ def c2p_bench(n, reps=3):
         pre, fre, _, tre, _ = _c2p_solve(b, gam, harmgpu.HG_C2P_REFINED, reps)
         pmx, fmx, imx, tmx, _ = _c2p_solve(b, gam, harmgpu.HG_C2P_MIXED, reps)
         res["fallbacks"] += harmgpu.c2p_fallbacks()
+        res["mixed_ms_without_counts"].append(_c2p_solve(b, gam, harmgpu.HG_C2P_MIXED, reps, counted=False)[3])
         res["gam"].append(gam)
         res["fp64_ms"].append(t64)
         res["refined_ms"].append(tre)
