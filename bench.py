@@ -249,10 +249,10 @@ def c2p_errors(p, pref, fref, gam):
             float((d[2:5].amax(dim=0) / ref[2:5].amax(dim=0).clamp(min=1.0)).max())]
 
 
-# algorithmic bytes per inversion: U 8, the upper triangles of gcov and gcon
-# 10 + 10, gdet, the guess's u and u~^i 4 doubles in; the solution 8 doubles,
+# algorithmic bytes per inversion: U 8, the upper triangles of the spatial gcov
+# and of gcon 6 + 10, gdet, the guess's u and u~^i 4 doubles in; the solution 8 doubles,
 # the code and the step count out
-C2P_BYTES = (8 + 10 + 10 + 1 + 4 + 8) * 8 + 4 + 4
+C2P_BYTES = (8 + 6 + 10 + 1 + 4 + 8) * 8 + 4 + 4
 
 
 def c2p_bench(n, reps=3):

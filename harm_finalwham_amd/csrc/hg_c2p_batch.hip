@@ -23,11 +23,11 @@
 //                     asked for (utoprimgen_listed)
 //
 // Memory per zone: the inversion reads U (8), the upper triangles of the
-// symmetric gcov and gcon (10 + 10), gdet and the guess's u and u~^i (4),
+// spatial gcov and of gcon (6 + 10), gdet and the guess's u and u~^i (4),
 // and writes the field (3), the solved rho, u, u~^i (5, only where the
 // reference assigns them), the failure code and the iteration count:
-// 336 bytes.  gcovpert and the guess's rho and field are not read (the
-// inversion does not use them).
+// 304 bytes.  g_{t mu}, gcovpert and the guess's rho and field are not read:
+// g_{t mu} would only meet B^t = 0, the others the inversion does not use.
 #include <hip/hip_runtime.h>
 
 #include <atomic>

@@ -289,8 +289,8 @@ __device__ __forceinline__ void refresh_bf16(int e, float v, const MlpDev &m) {
 // of partial sums of its own: sums in a fixed order, no atomics.
 // A minibatch of 2048 is 128 one-tile blocks.  One wavefront per 64 samples on
 // the vector units with an atomic per weight and block took 136 us (32 of them
-// on 1024 SIMDs), Adam and the copies two more launches of 4.7 us; now 10.8 us
-// here and 4.6 in k_mlp_update.
+// on 1024 SIMDs), Adam and the copies two more launches of 4.7 us; now 11.6 us
+// here and 3.9 in k_mlp_update.
 // ---------------------------------------------------------------------------
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 

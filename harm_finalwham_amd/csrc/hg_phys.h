@@ -29,7 +29,8 @@ constexpr int FAIL_CONVW = 2, FAIL_CONVUTSQ = 3, FAIL_CONVGUESSUTSQ = 4, FAIL_RH
 // them +0 at every point (upload_geometry_tables looks).  The sums below then
 // leave those terms out: a term with such a factor is a zero, adding a zero
 // changes nothing but the sign of a zero sum, and the sums that start from 0.
-// never hold -0, so every value that is not itself a zero keeps its bits.  Of
+// never hold -0, so every value that is not itself a zero keeps its bits (of
+// finite states: an infinity times a left-out zero would be a NaN).  Of
 // 96 products in the Maxwell tensor 27 are left, of 34 numbers per place 18
 // are read, and the flux kernels take 164 VGPRs instead of 192 (three waves a
 // SIMD instead of two).  With the quotients below sharing their divisors'

@@ -259,7 +259,8 @@ int hg_rdump_write(hg_ctx *ctx, const char *path, const char *header, void *stre
 /* Batched Noble-2D inversion on device memory (utoprimgen.c:23 for each of
    n independent zones).  All arrays are structure-of-arrays over n zones:
      U[8][n] evolved conserved variables (with gdet), gcov[16][n], gcon[16][n]
-     (symmetric: only the upper triangles, rows 4a+b with a <= b, are read),
+     (symmetric: only the upper triangles, rows 4a+b with a <= b, are read, of
+     gcov those with a > 0),
      gdet[n], gcovpert[n] (the tt component; not read), pr[8][n] guess in /
      solution out (the inversion reads the guess's u and u~^i; it writes the
      field, and rho, u, u~^i where the reference assigns them: codes 0, 9, 10,
@@ -388,7 +389,7 @@ int hg_mlp_train_rate(hg_mlp *m, int64_t n, const float *X, const float *Y, int 
    count from its plain guess, as in HG_C2P_MIXED.  The values therefore agree with HG_C2P_REFINED to ~1e-12
    (the same converged root), not bit for bit.  iters counts Newton steps and
    the learned start's evaluation.  counts (may be NULL) receives [zones solved from the learned
-   start, zones inverted by the fallback].  Allocates its scratch (4 n + 24
+   start, zones inverted by the fallback].  Allocates its scratch (4 n + 16
    bytes) stream-ordered on the given stream. */
 int hg_utoprim_batch_learned(const hg_mlp *m, int64_t n, double gam, const double *U, const double *gcov,
                              const double *gcon, const double *gdet, const double *gcovpert, double *pr,
